@@ -23,12 +23,35 @@ static __constant__ double c_shape[27] = {0.6494, 0.7957, 0.6494, 0.7957, 1.0000
 
 /* the 26 attempts by rank = call order of SCORE_Kernel.cpp:4611-4638:
  * offsets, infector code and overshoot class (1 face 0.0682, 2 edge 0.0542, 3 corner 0.0484) */
-static __constant__ int8_t c_dx[26] = {-1, 0, 1, -1, 1, -1, 0, 1, -1, 0, 1, -1, 0, 1, -1, 0, 1, -1, 0, 1, -1, 0, 1, -1, 0, 1};
-static __constant__ int8_t c_dy[26] = {-1, -1, -1, 0, 0, 1, 1, 1, 1, 1, 1, -1, -1, -1, 0, 0, 0, -1, -1, -1, 0, 0, 0, 1, 1, 1};
-static __constant__ int8_t c_dz[26] = {0, 0, 0, 0, 0, 0, 0, 0, -1, -1, -1, -1, -1, -1, -1, -1, -1, 1, 1, 1, 1, 1, 1, 1, 1, 1};
-static __constant__ uint8_t c_code[26] = {16, 15, 14, 13, 12, 11, 10, 9, 19, 18, 17, 25, 24, 23, 22, 21, 20,
-                                   8, 7, 6, 5, 4, 3, 2, 1, 0};
-static __constant__ uint8_t c_cls[26] = {2, 1, 2, 1, 1, 2, 1, 2, 3, 2, 3, 3, 2, 3, 2, 1, 2, 3, 2, 3, 2, 1, 2, 3, 2, 3};
+
+/* The same tables packed into literals, two bits per rank: a per-lane index into
+ * a constant array is a memory load, a shift of a literal is not. */
+static constexpr int8_t k_dx[26] = {-1, 0, 1, -1, 1, -1, 0, 1, -1, 0, 1, -1, 0, 1, -1, 0, 1, -1, 0, 1, -1, 0, 1, -1, 0, 1};
+static constexpr int8_t k_dy[26] = {-1, -1, -1, 0, 0, 1, 1, 1, 1, 1, 1, -1, -1, -1, 0, 0, 0, -1, -1, -1, 0, 0, 0, 1, 1, 1};
+static constexpr int8_t k_dz[26] = {0, 0, 0, 0, 0, 0, 0, 0, -1, -1, -1, -1, -1, -1, -1, -1, -1, 1, 1, 1, 1, 1, 1, 1, 1, 1};
+static constexpr unsigned long long pack_dir(const int8_t *v, int n) {
+    return n == 0 ? 0ull : pack_dir(v, n - 1) | (unsigned long long)(v[n - 1] + 1) << (2 * (n - 1));
+}
+static __device__ __forceinline__ int dir_dx(uint32_t r) {
+    constexpr unsigned long long t = pack_dir(k_dx, 26);
+    return (int)((uint32_t)(t >> (2u * r)) & 3u) - 1;
+}
+static __device__ __forceinline__ int dir_dy(uint32_t r) {
+    constexpr unsigned long long t = pack_dir(k_dy, 26);
+    return (int)((uint32_t)(t >> (2u * r)) & 3u) - 1;
+}
+static __device__ __forceinline__ int dir_dz(uint32_t r) {
+    constexpr unsigned long long t = pack_dir(k_dz, 26);
+    return (int)((uint32_t)(t >> (2u * r)) & 3u) - 1;
+}
+/* number of nonzero offsets: 1 face, 2 edge, 3 corner */
+static __device__ __forceinline__ int dir_class(uint32_t r) {
+    return (dir_dx(r) & 1) + (dir_dy(r) & 1) + (dir_dz(r) & 1);
+}
+/* the infector code of the attempt */
+static __device__ __forceinline__ uint32_t dir_code(uint32_t r) {
+    return (r < 8u ? 16u : r < 11u ? 27u : r < 17u ? 36u : 25u) - r;
+}
 
 static __device__ __forceinline__ uint32_t lanemask_lt_count(uint64_t m) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -229,14 +252,18 @@ static __device__ __forceinline__ uint32_t predict_values(const GmDev &d, const 
     return cs;
 }
 
+/* f after n >= 1 additions of inc */
+static __device__ __forceinline__ double advanced(double f, double inc, uint32_t n) {
+    return n == 1u ? f + inc : gm_radd_n(f, inc, n);
+}
+
 /* rxFrac of a parent after its completing addition in step k: n = k - s0 + 1
  * additions of its increment to the value it was anchored with before step s0 */
 static __device__ __forceinline__ double parent_fin(const GmDev &d, uint32_t slot, uint32_t k) {
     const GmRec *r = d.rec + slot;
     const RecA a = rec_a(r);
     const double inc = r->inc;
-    const uint32_t n = k - a.s0 + 1u;
-    return n == 1u ? a.frac0 + inc : gm_radd_n(a.frac0, inc, n);
+    return advanced(a.frac0, inc, k - a.s0 + 1u);
 }
 
 /* the stored code of completion step cs predicted at step kp */
@@ -271,7 +298,7 @@ static __device__ __forceinline__ void predict_slot(const GmDev &d, const GmSwee
     d.cstep[s] = cs_code(d, cs, A.k);
 }
 
-/* the arguments of the step the device is at */
+/* with several regions: the arguments of the step the device is at */
 static __device__ __forceinline__ GmSweepArgs step_args(const GmDev &d, const GmSweepArgs &A) {
     GmSweepArgs B = A;
     B.k = d.st->kcur;
@@ -410,14 +437,19 @@ static __device__ __forceinline__ void infect_one(const GmDev &d, const GmPParam
                                                   uint32_t t, uint32_t g, uint32_t tx, uint32_t ty, uint32_t tz,
                                                   uint32_t gslot, bool fresh_weight = false) {
     const double overshoot = pfin - 1.0;
-    const int cls = c_cls[r];
+    const int cls = dir_class(r);
     const double carry = cls == 1 ? overshoot * 0.0682 : (cls == 2 ? overshoot * 0.0542 : overshoot * 0.0484);
     double Pn = pP;
     if (fresh_weight || pq0.z != g) Pn = pair_weight(d, pp, pq0.w, g);
-    const uint32_t inf = c_code[r];
+    const uint32_t inf = dir_code(r);
     double inc = 0.0;
     gm_cs_t cs = (gm_cs_t)GM_CS_DEFERRED;
-    if (!is_pending(Pn)) cs = cs_code(d, predict_values(d, A, k + 1u, carry, Pn, g, inf, inc), k + 1u);
+    if (!is_pending(Pn)) {
+        const uint32_t step = predict_values(d, A, k + 1u, carry, Pn, g, inf, inc);
+        /* the window's lists of completed cells were made at its start */
+        if (step < A.wend) atomicOr(&d.st->err, GM_ERRF_MISSED);
+        cs = cs_code(d, step, k + 1u);
+    }
     GmRec *rec = d.rec + gslot;
     rec_set_a(rec, carry, k + 1u, inf);
     rec_set_b(rec, inc);
@@ -450,41 +482,53 @@ static __device__ __forceinline__ void infect_one(const GmDev &d, const GmPParam
  * last cell is reported so the host can update rhomax (update_myrhomax,
  * SCORE_RecoveryModels.cpp:146-165).  Consecutive parents often share their
  * nucleus and deformed grain (siblings), so each run of equal ids among
- * neighbouring lanes makes one atomic.  Every lane of the wave takes part. */
-static __device__ __forceinline__ void retire_batch(const GmDev &d, const uint4 &q0, bool valid) {
-    GmStats *st = d.st;
+ * neighbouring lanes makes one atomic.  Every lane of the wave takes part in
+ * retire_begin, which issues the atomics; retire_end looks at what they returned,
+ * so that other work can lie between.  top_hit, if given, is set when top_grain loses its last cell. */
+struct Retired {
+    uint32_t n, old;            /* cells this lane took from its deformed grain's count (0: none), the count before */
+};
+static __device__ __forceinline__ Retired retire_begin(const GmDev &d, const uint4 &q0, bool valid) {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t g = q0.z, r = q0.w;
     const uint32_t gprev = __shfl_up(g, 1, 64), rprev = __shfl_up(r, 1, 64);
     const uint64_t gstart = __ballot(valid && (lane == 0 || g != gprev));
     const uint64_t rstart = __ballot(valid && (lane == 0 || r != rprev));
     const uint64_t vmask = __ballot(valid);
-    if (!valid) return;
+    Retired ret = {0u, 0u};
+    if (!valid) return ret;
     const uint64_t above = lane == 63 ? 0ull : (~0ull << (lane + 1)); /* lanes after this one */
     if ((gstart >> lane) & 1ull) {
         /* run length: up to the next run start or the last valid lane */
         const uint64_t nxt = (gstart | ~vmask) & above;
         const uint32_t end = nxt ? (uint32_t)__ffsll((long long)nxt) - 1u : 64u;
-        const uint32_t n = end - lane;
-        const uint32_t old = atomicSub(&d.defcnt[g], n);
-        if (old == n) {
-            const uint32_t i = atomicAdd(&st->nzeroed, 1u);
-            if (i < GM_ZEROED_INLINE) st->zeroed_ids[i] = g;
-            if (i < d.ndefg) d.zlist[i] = g;
-        } else if (old < n) {
-            /* only a cell held by two records retires twice; the count wraps
-             * as SCORE's uint32 does and the host re-reads them all */
-            st->cwrap = 1u;
-        }
+        ret.n = end - lane;
+        ret.old = atomicSub(&d.defcnt[g], ret.n);
     }
     if ((rstart >> lane) & 1ull) {
         const uint64_t nxt = (rstart | ~vmask) & above;
         const uint32_t end = nxt ? (uint32_t)__ffsll((long long)nxt) - 1u : 64u;
         atomicAdd(&d.rxcnt[r], end - lane);
     }
+    return ret;
+}
+static __device__ __forceinline__ void retire_end(const GmDev &d, uint32_t g, const Retired &ret,
+                                                  uint32_t top_grain = 0xFFFFFFFFu, uint32_t *top_hit = nullptr) {
+    GmStats *st = d.st;
+    if (!ret.n) return;
+    if (ret.old == ret.n) {
+        const uint32_t i = atomicAdd(&st->nzeroed, 1u);
+        if (i < GM_ZEROED_INLINE) st->zeroed_ids[i] = g;
+        if (i < d.ndefg) d.zlist[i] = g;
+        if (top_hit && g == top_grain) *top_hit = 1u;
+    } else if (ret.old < ret.n) {
+        /* only a cell held by two records retires twice; the count wraps
+         * as SCORE's uint32 does and the host re-reads them all */
+        st->cwrap = 1u;
+    }
 }
 
-/* The row of the step just done, and whether the next one may run without the
+/* With several regions: the row of the step just done, and whether the next one may run without the
  * host: not after an error, a count that wrapped, the exhaustion of the grain
  * that sets rhomax (any_top), Xcells reaching a threshold the host acts on, a
  * weight the window cannot wait for, or lists outgrowing their allocations.
@@ -500,14 +544,9 @@ static __device__ void step_finish(const GmDev &d, const GmWindow &w, const GmSt
     st->npend0 = npend;
     const double xc = st->xcells + (double)(r.nfullI + r.nfullB);
     st->xcells = xc;
-    /* the next step's arrivals may go to either list */
-    const uint32_t kn = st->kcur;
-    const uint64_t narr = (kn >= 1u && kn <= d.arr_last) ? (uint64_t)d.arr_off[kn + 1u] - d.arr_off[kn] : 0ull;
-    const uint64_t slots = (uint64_t)r.nI + r.nB + narr;
-    const uint64_t nIn = (uint64_t)r.nI + narr < 0xFFFFFFC0ull ? (uint64_t)r.nI + narr : 0xFFFFFFC0ull;
-    /* with several regions each list is swept in whole 8-tile chunks */
-    const uint64_t tiles = d.nreg > 1u ? slots / 64u + (uint64_t)GM_SW_TPC * (d.nlists + 1u)
-                                       : (uint64_t)gm_tiles_inside((uint32_t)nIn) + ((uint64_t)r.nB + narr + 63) / 64 + GM_SW_TPC;
+    const uint64_t slots = (uint64_t)r.nI + r.nB;
+    /* each list is swept in whole 8-tile chunks */
+    const uint64_t tiles = slots / 64u + (uint64_t)GM_SW_TPC * (d.nlists + 1u);
     bool halt = r.err != 0u || __hip_atomic_load(&st->cwrap, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u ||
                 any_top || xc >= w.xstop;
     halt = halt || (npend != 0u && !w.defer) || npend > w.pend_limit;

@@ -208,6 +208,7 @@ struct score_gm_handle {
      * capacities (2T lists, region r's Inside list 2r and Border list 2r+1) */
     std::vector<GmRegion> reg;
     std::vector<uint32_t> lbase, lcap, lrcap, lrbase;
+    uint32_t last_full = 0xFFFFFFFFu; /* most cells completed in one step of the last window */
 };
 
 namespace {
@@ -319,6 +320,7 @@ void free_device(score_gm_handle *h) {
                     d.par, d.recI, d.recB, d.mF, d.mR, d.pmI, d.pmB, d.bcnt, d.rho, d.defq,
                     d.rxq, d.defcnt, d.rxcnt, d.zlist, d.hkeys, d.hvals, d.pend_slot, d.pend_key, d.nflag, d.nI_, d.nB_,
                     d.scan_bsum, d.st, d.arr_ids, d.arr_off, d.nsite, d.nucP,
+                    d.win, d.wcnt, d.wpre, d.wwave, d.rcnt, d.rpre, d.rgone, d.rmrg, d.acnt, d.btot, d.ccnt,
                     d.reg, d.pmH, d.L.base, d.L.cap, d.L.rcap, d.L.rbase, d.L.n, d.L.nold, d.L.rlen,
                     d.L.win, d.L.occ, d.L.tile, d.L.tile_s, d.L.par, d.L.rst, d.L.rbuf, d.L.rs, d.L.bstart, d.L.breg,
                     d.L.hoff, d.plist};
@@ -817,19 +819,21 @@ int ensure_step_capacity(score_gm_handle *h) {
         dfree(h, d.mF); dfree(h, d.mR);
         d.mF = d.mR = nullptr;
         int rc;
-        if ((rc = dalloc(h, &d.mF, nc)) || (rc = dalloc(h, &d.mR, nc))) return rc;
+        if ((d.nreg > 1 && (rc = dalloc(h, &d.mF, nc))) || (rc = dalloc(h, &d.mR, nc))) return rc;
         d.tileCap = nc;
     }
     const uint32_t parents = h->nI + h->nB + na;
     if (parents > d.parentCap) {
         uint32_t nc = std::max<uint32_t>(parents, d.parentCap + d.parentCap / 2);
         dfree(h, d.pmI); dfree(h, d.pmB); dfree(h, d.pslot); dfree(h, d.par); dfree(h, d.pmH); dfree(h, d.plist);
-        d.pmI = d.pmB = d.pslot = d.pmH = d.plist = nullptr;
+        dfree(h, d.ccnt);
+        d.pmI = d.pmB = d.pslot = d.pmH = d.plist = d.ccnt = nullptr;
         d.par = nullptr;
         d.parentCap = 0;
         int rc;
         if ((rc = dalloc(h, &d.pmI, nc)) || (rc = dalloc(h, &d.pmB, nc)) || (rc = dalloc(h, &d.pslot, nc)) ||
-            (rc = dalloc(h, &d.par, (size_t)GM_PAR_PLANES * nc)) || (d.nreg > 1 && ((rc = dalloc(h, &d.pmH, nc)) || (rc = dalloc(h, &d.plist, nc)))))
+            (rc = dalloc(h, &d.par, (size_t)(d.nreg > 1 ? GM_PAR_PLANES : GM_PAR1_PLANES) * nc)) || (d.nreg > 1 && ((rc = dalloc(h, &d.pmH, nc)) || (rc = dalloc(h, &d.plist, nc)))) ||
+            (d.nreg <= 1 && (rc = dalloc(h, &d.ccnt, (size_t)nc / 64 + 1))))
             return rc;
         d.parentCap = nc;
     }
@@ -1037,8 +1041,9 @@ void advance_scalars(score_gm_handle *h) {
 /* Steps that may follow the current one in a launch window: the termination
  * tests on t and the step count must not fire and the scalars must stay
  * bit-identical, found by running the scalar updates ahead on a copy; and a
- * cell infected in the window must not be able to complete before its
- * deferred prediction at the window's end.  Only the Rollett-Holm model
+ * cell infected in the window must not be able to complete before the window's
+ * end, since its lists of completed cells are made at its start (with several
+ * regions: before its deferred prediction).  Only the Rollett-Holm model
  * qualifies: its time step does not depend on the weights of new pairs. */
 uint32_t window_length(score_gm_handle *h, uint32_t wmax, const GmSweepParams &sp) {
     if (h->prof || wmax <= 1 || h->p.mobility_model != SCORE_GM_MOB_ROLLETTHOLM) return 1;
@@ -1061,6 +1066,8 @@ uint32_t window_length(score_gm_handle *h, uint32_t wmax, const GmSweepParams &s
         h->step++;
         /* a step at a multiple of the horizon re-anchors, so it starts a window */
         if (done(h) || !same_scalars(sweep_params(h), sp) || h->step % h->d.horizon == 0) break;
+        /* nuclei that arrive complete in their first step, so that step starts a window */
+        if (arrivals_at(h, h->step)) break;
         n++;
     }
     h->t = t0; h->T = T0; h->G = G0; h->b = b0; h->Gbhalfsq = gb0; h->dt = dt0; h->pzmin = pz0; h->fr = fr0;
@@ -1148,6 +1155,36 @@ bool wait_steps(score_gm_handle *h, uint32_t need) {
     }
 }
 
+/* Cuts the window's passes into blocks for lists of at most nI and nB slots: one
+ * 512-slot chunk per wave of a sweep block while GM_SW_BLOCKS blocks (8 on every
+ * CU) cover the lists, then more chunks per wave, and beyond GM_SW_MAXCPW (the
+ * masks a wave of the recycling pass keeps in LDS) more blocks.  The infection
+ * passes take 64 parents per block and stride over more; they get twice the
+ * blocks the last window's largest step filled. */
+GmPart window_part(const score_gm_handle *h, uint32_t nI, uint32_t nB, uint32_t W) {
+    GmPart P;
+    P.chI = (uint32_t)(((uint64_t)nI + GM_SW_CHUNK - 1) / GM_SW_CHUNK);
+    P.chB = (uint32_t)(((uint64_t)nB + GM_SW_CHUNK - 1) / GM_SW_CHUNK);
+    const uint64_t ch = (uint64_t)P.chI + P.chB, per = GM_SW_WAVES * (uint64_t)(GM_SW_BLOCKS - 1);
+    P.cpw = (uint32_t)std::min<uint64_t>(GM_SW_MAXCPW, std::max<uint64_t>(1, (ch + per - 1) / per));
+    const uint32_t cpb = GM_SW_WAVES * P.cpw;
+    P.nbI = (P.chI + cpb - 1) / cpb;
+    P.nb = P.nbI + (P.chB + cpb - 1) / cpb;
+    if (P.nb == 0) P.nbI = P.nb = 1;
+    P.W = W;
+    const uint64_t slots = (uint64_t)nI + nB, est = std::min<uint64_t>(slots, 2ull * h->last_full + 1024u);
+    P.nbp = (uint32_t)std::min<uint64_t>(GM_PB, est / 64 + 1);
+    P.nbd = std::min<uint32_t>(GM_DB, P.nbp);
+    return P;
+}
+
+/* entries of a row of sweep-block tables: enough for window_part of full lists */
+uint32_t sweep_block_rows(const GmDev &d) {
+    const uint64_t ch = ((uint64_t)d.capI + GM_SW_CHUNK - 1) / GM_SW_CHUNK + ((uint64_t)d.capB + GM_SW_CHUNK - 1) / GM_SW_CHUNK;
+    const uint64_t nb = ch / (GM_SW_WAVES * GM_SW_MAXCPW) + 2;
+    return (uint32_t)((std::max<uint64_t>(nb, GM_SW_BLOCKS) + 63) / 64 * 64);
+}
+
 int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
     *nsteps = 0;
     if (h->err) return h->err;
@@ -1202,6 +1239,10 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
     const uint32_t nBe = W == 1 ? h->nB : (uint32_t)std::min<uint64_t>(capBe, h->nB + h->nB / 2 + 4096u);
     a.nI = nIe;
     a.nB = nBe;
+    a.wend = d.nreg > 1 ? 0u : h->step + W;
+    const uint32_t na = arrivals_at(h, h->step);
+    const GmPart P = window_part(h, (uint32_t)std::min<uint64_t>(d.capI, (uint64_t)h->nI + na),
+                                 (uint32_t)std::min<uint64_t>(d.capB, (uint64_t)h->nB + na), W);
     GmWindow w;
     memset(&w, 0, sizeof(w));
     w.xstop = window_xstop(h);
@@ -1218,26 +1259,30 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
      * nothing, whatever the host sees in time. */
     const bool paced = !prof && W > GM_LEAD + 1;
     if (paced) __atomic_store_n(h->hprog, 0u, __ATOMIC_RELAXED);
-    if ((e = gm_launch_window_begin(d, h->step, h->Xcells, h->stream)) != hipSuccess)
-        return h->err = hip_fail(e, "growth step");
+    if (d.nreg > 1)
+        e = gm_launch_window_begin(d, h->step, h->Xcells, h->stream);
+    else
+        e = gm_launch_window(d, P, a, na != 0, h->Xcells, h->stream, ev);
+    if (e != hipSuccess) return h->err = hip_fail(e, "growth step");
+    uint32_t launched = 0;
     for (uint32_t j = 0; j < W; j++) {
         if (paced && j > GM_LEAD && !wait_steps(h, j - GM_LEAD)) break;
-        GmSweepArgs aj = a;
-        if (j) aj.reanchor = 0;
+        launched = j + 1;
         if (d.nreg > 1) {
+            GmSweepArgs aj = a;
+            if (j) aj.reanchor = 0;
             if ((e = gm_launch_rg_sweep(d, aj, std::max(slots0, nIe + nBe), h->stream, ev)) != hipSuccess ||
                 (e = gm_launch_rg_infect(d, h->pp, aj, std::max(slots0, nIe + nBe), h->stream, ev)) != hipSuccess ||
                 (e = gm_launch_step_tail(d, w, h->stream)) != hipSuccess)
                 return h->err = hip_fail(e, "growth step");
             continue;
         }
-        if ((e = gm_launch_sweep(d, aj, h->stream, ev)) != hipSuccess ||
-            (e = gm_launch_infect(d, h->pp, aj, std::max(slots0, nIe + nBe), h->stream, ev)) != hipSuccess ||
-            (e = gm_launch_step_tail(d, w, h->stream)) != hipSuccess)
+        if ((e = gm_launch_infect(d, h->pp, a, P, w, j, h->stream, ev)) != hipSuccess)
             return h->err = hip_fail(e, "growth step");
     }
-    if ((e = gm_launch_stats_out(d, h->hst_dev, h->stream)) != hipSuccess ||
-        (e = hipStreamSynchronize(h->stream)) != hipSuccess)
+    e = d.nreg > 1 ? gm_launch_stats_out(d, h->hst_dev, h->stream)
+                   : gm_launch_window_end(d, P, launched, h->hst_dev, h->stream);
+    if (e != hipSuccess || (e = hipStreamSynchronize(h->stream)) != hipSuccess)
         return h->err = hip_fail(e, "growth step");
     h->last_sp = sp;
     h->have_last_sp = true;
@@ -1284,6 +1329,8 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
         const GmStepRow &last = st.rows[nexec - 1];
         h->nI = last.nI;
         h->nB = last.nB;
+        h->last_full = 0;
+        for (uint32_t j = 0; j < nexec; j++) h->last_full = std::max(h->last_full, st.rows[j].nfullI + st.rows[j].nfullB);
     }
     if ((rc = grow_pcache(h))) return h->err = rc;
     if (st.novf) {
@@ -1610,8 +1657,8 @@ int score_gm_create(const score_gm_domain *dom, const score_gm_params *prm, int 
         (rc = dalloc(h, &d.rec, capTot)) ||
         (rc = dalloc(h, &d.dlist, d.dlistCap)) ||
         (rc = dalloc(h, &d.dmap, (size_t)d.dnbx * d.dnby * d.dnbz * 32)) || (rc = dalloc(h, &d.pslot, d.parentCap)) ||
-        (rc = dalloc(h, &d.par, (size_t)GM_PAR_PLANES * d.parentCap)) || (rc = dalloc(h, &d.recI, d.recCapI)) || (rc = dalloc(h, &d.recB, d.recCapB)) ||
-        (rc = dalloc(h, &d.mF, d.tileCap)) || (rc = dalloc(h, &d.mR, d.tileCap)) || (rc = dalloc(h, &d.pmI, d.parentCap)) ||
+        (rc = dalloc(h, &d.par, (size_t)(multi ? GM_PAR_PLANES : GM_PAR1_PLANES) * d.parentCap)) || (rc = dalloc(h, &d.recI, d.recCapI)) || (rc = dalloc(h, &d.recB, d.recCapB)) ||
+        (multi && (rc = dalloc(h, &d.mF, d.tileCap))) || (rc = dalloc(h, &d.mR, d.tileCap)) || (rc = dalloc(h, &d.pmI, d.parentCap)) ||
         (rc = dalloc(h, &d.pmB, d.parentCap)) || (rc = dalloc(h, &d.bcnt, GM_BCNT_ROWS * GM_MAX_BLOCKS)) ||
         (rc = dalloc(h, &d.rho, d.ndefg)) || (rc = dalloc(h, &d.defq, 4 * (size_t)d.ndefg)) ||
         (rc = dalloc(h, &d.rxq, 4 * (size_t)d.nrxg + 4)) || (rc = dalloc(h, &d.defcnt, d.ndefg)) ||
@@ -1624,6 +1671,19 @@ int score_gm_create(const score_gm_domain *dom, const score_gm_params *prm, int 
         free_device(h);
         delete h;
         return rc;
+    }
+    if (!multi) {
+        d.swb = sweep_block_rows(d);
+        if ((rc = dalloc(h, &d.win, 1)) || (rc = dalloc(h, &d.wcnt, (size_t)(GM_WMAX + 1) * d.swb)) ||
+            (rc = dalloc(h, &d.wpre, (size_t)(GM_WMAX + 1) * d.swb)) ||
+            (rc = dalloc(h, &d.wwave, (size_t)GM_SW_WAVES * GM_WMAX * d.swb)) ||
+            (rc = dalloc(h, &d.rcnt, 2 * (size_t)d.swb)) || (rc = dalloc(h, &d.rpre, 2 * (size_t)d.swb)) ||
+            (rc = dalloc(h, &d.rgone, d.swb)) || (rc = dalloc(h, &d.rmrg, d.swb)) || (rc = dalloc(h, &d.acnt, 2 * GM_PB)) ||
+            (rc = dalloc(h, &d.btot, GM_DB)) || (rc = dalloc(h, &d.ccnt, (size_t)d.parentCap / 64 + 1))) {
+            free_device(h);
+            delete h;
+            return rc;
+        }
     }
     if (multi) {
         const uint32_t L = d.nlists;
@@ -2035,6 +2095,11 @@ int score_gm_footprint(const score_gm_domain *dom, const score_gm_params *prm, u
     const uint64_t hcap = pow2_at_least(std::max<uint64_t>(65536, 4ull * dom->n_rxg));
     const uint64_t front = std::max<uint64_t>(65536, N / 4);
     uint64_t b = 0;
+    if (prm->n_regions <= 1) {
+        /* the window sweep's tables */
+        const uint64_t rows = std::max<uint64_t>(capTot / (GM_SW_CHUNK * GM_SW_WAVES * GM_SW_MAXCPW) + 67, GM_SW_BLOCKS);
+        b += sizeof(GmWin) + 4 * rows * (2 * (GM_WMAX + 1) + GM_SW_WAVES * GM_WMAX + 6) + 16 * GM_PB + front / 16 + 4;
+    }
     if (prm->n_regions > 1) {
         /* the lists of every region (build_regions), halo masks and tables */
         const uint32_t T = (uint32_t)prm->n_regions, npy = smallest_y_factor(T), npz = T / npy;
@@ -2051,6 +2116,7 @@ int score_gm_footprint(const score_gm_domain *dom, const score_gm_params *prm, u
                 rbuf += (uint64_t)(prm->rel_cell_caching * (double)vol * prm->maxfill * kFullRecyclingAtt) +
                         (uint64_t)((double)cb * prm->maxfill * kFullRecyclingAtt);
             }
+        b += 8 * (capTot / 64 + GM_SW_TPC); /* completed masks */
         b += 4 * front + (sizeof(GmRegion) + 4ull * (GM_RROWS + GM_NHALO + 26)) * (T + 1) + 16ull * GM_SW_TPC * 2 * T;
     }
     b += 8 * N;                                   /* grid, claim */
@@ -2059,7 +2125,7 @@ int score_gm_footprint(const score_gm_domain *dom, const score_gm_params *prm, u
     b += (sizeof(gm_cs_t) + sizeof(GmRec)) * capTot; /* completion steps, records */
     b += (4 + 16 * GM_PAR_PLANES + 8) * front;    /* parents: slots, data, winner masks */
     b += 4 * std::min<uint64_t>(N, 1u << 20);     /* deferred-cell list */
-    b += 16 * (capTot / 64 + GM_SW_TPC);          /* tile masks */
+    b += 8 * (capTot / 64 + GM_SW_TPC);           /* tile masks */
     b += 4 * rbuf;                                /* recycled slots */
     b += 4 * GM_BCNT_ROWS * GM_MAX_BLOCKS;
     b += 52ull * dom->n_defg + 52ull * (dom->n_rxg + 1);

@@ -110,6 +110,16 @@ static inline __host__ __device__ uint32_t gm_tiles_inside(uint32_t nI) {
 #define GM_PEND_INLINE 2048       /* new P-cache keys returned with the per-step stats */
 #define GM_NK 9                   /* kernels per step (SCORE_GM_K_* order) */
 #define GM_WMAX 16                /* steps per launch window at most (also below imin - 1) */
+/* the window sweep of one-region handles (gm_kernels.hip) */
+#define GM_SW_WAVES (GM_BLOCK / 64)
+#define GM_SW_CHUNK (64u * GM_SW_TPC) /* slots a wave takes at a time */
+#define GM_SW_BLOCKS 2048u        /* sweep blocks up to GM_SW_MAXCPW chunks per wave */
+#define GM_SW_MAXCPW 32u
+#define GM_SW_PACK 31u            /* chunks whose per-lane counts fit a byte */
+#define GM_SW_FOLD 256u           /* sweep blocks up to which no scan pass runs between counting and compaction */
+#define GM_PB 2048u               /* blocks of the propose pass at most */
+#define GM_DB 1024u               /* blocks of the decide and commit passes at most */
+#define GM_RECYCLE_BLOCKS 2048u   /* blocks of the decide launch that write recycled slots */
 
 /* One front record: SCORE's `cell` (SCORE_Kernel.h:124-137) with rxFrac held as
  * anchor + increment.  The first 32-byte sector holds
@@ -141,6 +151,12 @@ static_assert(__builtin_offsetof(GmRec, inc) == 16 && __builtin_offsetof(GmRec, 
  *               (written by the decide pass for parents that won a target) and
  *               the mobility weight
  *   GM_PAR_XYZ  (x, y, z, Border flag or list) */
+/* with one region two planes:
+ *   GM_PAR1_CELL (x | y << 16, z | Border flag << 16, defg, rxg)
+ *   GM_PAR1_FP   (fin, P), fin for the parents that found a deformed neighbour */
+#define GM_PAR1_CELL 0u
+#define GM_PAR1_FP 1u
+#define GM_PAR1_PLANES 2u
 #define GM_PAR_IDS 0u
 #define GM_PAR_FP 1u
 #define GM_PAR_XYZ 2u
@@ -204,6 +220,32 @@ struct GmWindow {
     uint32_t pend_limit;      /* new P-cache entries that keep the cache at most half full */
     uint32_t defer;           /* pending weights may wait for the end of the window */
     uint32_t pad;
+};
+
+/* How a window's passes are cut up, fixed over the window: sweep blocks of
+ * GM_SW_WAVES waves with cpw chunks each, nbI of them over the Inside list's chI
+ * chunks, the rest over the Border list's chB; W steps; blocks of the propose and
+ * decide passes. */
+struct GmPart {
+    uint32_t nbI, nb, cpw, chI, chB, W, nbp, nbd;
+};
+
+/* the front lists as a step of the window finds them */
+struct GmWinStep {
+    uint32_t nI, nB;            /* list lengths */
+    uint32_t totRecI, totRecB;  /* INACTIVE slots */
+    uint32_t recLenI, recLenB;  /* of which may be handed out */
+};
+
+/* what the passes of a window share, all on the device */
+struct GmWin {
+    uint32_t full[GM_WMAX], fullI[GM_WMAX]; /* cells completing in each step, in all and of the Inside list */
+    uint32_t off[GM_WMAX + 1];  /* completed cells before each step: its list starts at pslot[off[i]] */
+    uint32_t npend0;            /* new weight-cache entries before the current step */
+    uint32_t top_hit;           /* the grain that sets rhomax lost its last cell */
+    GmWinStep step[GM_WMAX + 1];
+    unsigned long long nret0;   /* retirements before the window */
+    double xcells0;             /* Xcells before the window */
 };
 
 /* Several memory regions (SCORE with OMP_NUM_THREADS = T > 1, ompshar_ca2regions,
@@ -274,16 +316,28 @@ struct GmDev {
     uint32_t horizon;           /* steps, in [16, GM_CS_HORIZON_MAX] */
     GmRec *rec;
     /* per-step lists */
-    uint32_t *pslot;            /* completed cells (global slots), Inside then Border, ascending each */
+    uint32_t *pslot;            /* completed cells (global slots), Inside then Border, ascending each; with one
+                                 * region those of all steps of the window, step after step */
     uint4 *par;                 /* the same cells' parent data: GM_PAR_PLANES planes */
     uint32_t *recI, *recB;      /* recycled slots (list-relative), ascending, capped */
-    uint64_t *mF, *mR;          /* per 64-slot tile: completed / INACTIVE masks */
+    uint64_t *mF, *mR;          /* per 64-slot tile: completed (several regions only) / INACTIVE masks */
     uint32_t *pmI, *pmB;        /* per parent: winning ranks into Inside / Border */
     /* pslot, par, pmI and pmB hold parentCap entries */
     uint32_t *bcnt;             /* per-block counts and offsets, 8 x GM_MAX_BLOCKS */
     uint32_t *dlist;            /* slots of the cells left DEFERRED in a window (dlistCap entries) */
     uint32_t dlistCap;
     uint32_t tileCap, parentCap;
+    /* window sweep (one region): rows of swb entries, one per sweep block */
+    uint32_t swb;
+    GmWin *win;
+    uint32_t *wcnt, *wpre;      /* GM_WMAX+1 rows: cells completing in step i (row GM_WMAX: INACTIVE slots), and the
+                                 * exclusive prefixes over the blocks */
+    uint32_t *wwave;            /* GM_WMAX counts per wave of each block */
+    uint32_t *rcnt, *rpre;      /* INACTIVE slots of each block and before it in its list; two rows, by the step's parity */
+    uint32_t *rgone, *rmrg;     /* slots the step before handed out; steps whose completed cells are in the block's masks */
+    uint32_t *acnt;             /* attempts per propose block, two rows by the step's parity */
+    uint2 *btot;                /* winners into Inside, Border per decide block */
+    uint32_t *ccnt;             /* the same per 64 parents, Inside << 16 | Border */
     /* grains */
     double *rho, *defq, *rxq;
     uint32_t *defcnt, *rxcnt;
@@ -339,12 +393,15 @@ struct GmSweepArgs {
     uint32_t stepcap;           /* last step a completion can fall in */
     uint32_t next_only;         /* every following step re-anchors: predict only whether a cell
                                  * completes in the step it is predicted for (else FAR) */
-    uint32_t pad;
+    uint32_t wend;              /* the step after the window (one region): no cell infected in it completes before */
 };
 
 /* launchers (gm_kernels.hip); all asynchronous on `s`.  With `ev` non-null,
  * ev[i] is recorded before kernel i of the step and ev[GM_NK] after the last. */
-hipError_t gm_launch_sweep(const GmDev &d, const GmSweepArgs &a, hipStream_t s, hipEvent_t *ev);
+/* the start of a one-region window: re-anchoring (a.reanchor), the arrivals of
+ * step a.k, and the window sweep */
+hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &a, bool arrivals, double xcells,
+                            hipStream_t s, hipEvent_t *ev);
 /* every active cell advanced to step a.k with its old increment and predicted again */
 hipError_t gm_launch_reanchor(const GmDev &d, const GmSweepArgs &a, hipStream_t s);
 /* the same two halves of a step with several regions (gm_regions.hip) */
@@ -356,20 +413,20 @@ hipError_t gm_launch_rg_infect(const GmDev &d, const GmPParams &pp, const GmSwee
 hipError_t gm_launch_rg_prefix(const GmDev &d, hipStream_t s);
 /* with several regions: nuclei the host placed, records scattered to their slots */
 hipError_t gm_launch_rg_place(const GmDev &d, const uint32_t *slots, const GmRec *recs, uint32_t n, hipStream_t s);
-hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, uint32_t parents_upper,
-                            hipStream_t s, hipEvent_t *ev);
-/* start of a window: step index and Xcells; clears the window's accumulators */
+/* step j of a one-region window: infections and retirements */
+hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P,
+                            const GmWindow &w, uint32_t j, hipStream_t s, hipEvent_t *ev);
+/* its end after `launched` steps: the last step's row, the stats into the host's mirror */
+hipError_t gm_launch_window_end(const GmDev &d, const GmPart &P, uint32_t launched, GmStats *out, hipStream_t s);
+/* start of a window with several regions: step index and Xcells; clears the window's accumulators */
 hipError_t gm_launch_window_begin(const GmDev &d, uint32_t k, double xcells, hipStream_t s);
-/* end of every step of a window: records the step's row, advances the step
+/* end of every step of a window with several regions: records the step's row, advances the step
  * index, and sets halt when the host must act before the next step */
 hipError_t gm_launch_step_tail(const GmDev &d, const GmWindow &w, hipStream_t s);
 /* cells left DEFERRED in a window, with their weights now resolved: replayed to
  * step a.k under the window's scalars and predicted */
 hipError_t gm_launch_predict_deferred(const GmDev &d, const GmSweepArgs &a, uint32_t ndeferred, hipStream_t s);
 hipError_t gm_launch_nucleate(const GmDev &d, const uint32_t *site, const double *nucP, uint32_t nrxg, hipStream_t s);
-/* one block per step, between the re-anchoring and the sweep: the nuclei arriving
- * at the step the device is at, placed in pool order and predicted under a's scalars */
-hipError_t gm_launch_arrivals(const GmDev &d, const GmSweepArgs &a, hipStream_t s);
 hipError_t gm_launch_resolve_pending(const GmDev &d, const double *vals, uint32_t npend, hipStream_t s);
 hipError_t gm_launch_stats_out(const GmDev &d, GmStats *out, hipStream_t s);
 /* SCORE's view of slots [base, base+n) before step k, unpacked into per-field arrays */

@@ -5,36 +5,44 @@
  * is, in serial order: sweep the Inside list, sweep the Border list, let every
  * completed Inside cell infect its 26 neighbours in list order, then every
  * completed Border cell.  A target is won by the first attempt in that order
- * that finds it deformed.  The same outcome is computed by nine kernels:
+ * that finds it deformed.  Steps run in launch windows of up to GM_WMAX; the same
+ * outcome is computed by
  *
- *   k_reanchor     only in steps whose scalars changed: every active cell is
- *                  advanced to the step with its old increment and predicted
- *                  again with the new one, one thread per slot.
- *   k_sweep        pass over the occupied slots of both lists, statically
- *                  partitioned over the grid.  A slot costs one 4-byte read (its
- *                  predicted completion step).  Completed and INACTIVE slots are
- *                  balloted into per-tile masks and counted per block.
- *   k_sweep_scan   one block scans the per-block counts into offsets.
- *   k_compact      one wave per sweep block writes the completed slots in FullRX
- *                  order (Inside list, then Border) at those offsets.
- *   k_propose      copies what the infection needs of each completed cell (ids,
- *                  rxFrac, P, coordinates) into a dense parent array; then every
- *                  (parent p, direction rank r) attempt on a deformed cell
- *                  (one bit of a brick-blocked bitmap) does
- *                  atomicMin(claim[target], p*32 + r): the key orders attempts
- *                  exactly as the serial loop issues them.
+ * per window
+ *   k_reanchor     only where the scalars changed: every active cell is advanced to
+ *                  the step with its old increment and predicted again with the new
+ *                  one, one thread per slot.
+ *   k_arrivals     only where nuclei arrive at the window's first step.
+ *   k_sweep        pass over the completion codes of the occupied slots: per block,
+ *                  the cells that complete in each step of the window and the
+ *                  INACTIVE slots.
+ *   k_sweep_scan   one block scans the per-block counts into offsets (short fronts:
+ *                  each block of the next pass adds up what it needs).
+ *   k_compact      the completed slots of every step in FullRX order (Inside list,
+ *                  then Border), and the INACTIVE slots as masks.
+ *   k_window_end   closes the last step and hands the stats to the host.
+ * per step
+ *   k_propose      block 0 closes the step before (its row, list lengths, recycling
+ *                  tables).  The others copy what the infection needs of each
+ *                  completed cell (ids, rxFrac after the completing addition, P,
+ *                  coordinates) into dense parent planes; every (parent p, direction
+ *                  rank r) attempt on a deformed cell (one bit of a brick-blocked
+ *                  bitmap) does atomicMin(claim[target], p*32 + r): the key orders
+ *                  attempts exactly as the serial loop issues them.
  *   k_decide       an attempt wins iff its key is the minimum; winners per parent
- *                  and destination list as bit masks, counted per block; a
- *                  parent that won gets its rxFrac after the completing
- *                  addition, replayed from its anchor.
- *   k_decide_scan  one block scans those counts: rank k into a list takes the
- *                  k-th recycled slot, else appends.
- *   k_recycle      writes the recycled slots that will be handed out: the first
- *                  min(winners, cap) INACTIVE slots of each list, ascending.
- *   k_commit       one thread per winner writes the new record with its
- *                  increment and completion step (certified from the real
- *                  sums, gm_radd_count_to_one), and clears the cell's bitmap
- *                  bit; then the parents retire.
+ *                  and destination list as bit masks, counted per 64 parents and per
+ *                  block.  Further blocks write the recycled slots that may be handed
+ *                  out, ascending.
+ *   k_commit       the winners before a block rank its own: rank k into a list takes
+ *                  the k-th recycled slot, else appends.  One thread per winner writes
+ *                  the new record with its increment and completion step (certified
+ *                  from the real sums, gm_radd_count_to_one), and clears the cell's
+ *                  bitmap bit; the parents retire.
+ *
+ * Three passes a step, where sweep, scan, compaction, ranking scan, recycling and
+ * the step's row were seven more launches: on the 24x20x18 domain of ten nuclei a
+ * step went from 48 to 24 us, at 100^3 from 62 to 33, at 320^3 from 90 to 62, at
+ * 512^3 from 165 to 135.
  *
  * No kernel waits on another block: every cross-block dependency is a kernel
  * boundary, so the passes use only relaxed device atomics.  FP64 throughout,
@@ -67,9 +75,7 @@ hipError_t gm_launch_fill_u64(unsigned long long *p, unsigned long long v, size_
  * step k with its old increment (its anchor moves to k) and predicted again
  * with the new one.  One thread per occupied slot.  Codes of cells that
  * completed before step k are turned into INACTIVE. */
-__global__ void __launch_bounds__(GM_BLOCK) k_reanchor(GmDev d, GmSweepArgs A0) {
-    if (d.st->halt) return;
-    const GmSweepArgs A = step_args(d, A0);
+__global__ void __launch_bounds__(GM_BLOCK) k_reanchor(GmDev d, GmSweepArgs A) {
     const uint32_t nI = d.st->nI, n = nI + d.st->nB;
     const uint32_t kc = A.k & (GM_CS_MOD - 1u);
     for (uint32_t i = blockIdx.x * GM_BLOCK + threadIdx.x; i < n; i += gridDim.x * GM_BLOCK) {
@@ -95,217 +101,340 @@ __global__ void __launch_bounds__(GM_BLOCK) k_reanchor(GmDev d, GmSweepArgs A0) 
     }
 }
 
-/* list lengths of the current step as tiles: the Inside list rounded up to
- * whole sweep chunks (tI), then the Border list (T in all) */
-static __device__ __forceinline__ void step_tiles(uint32_t nI, uint32_t nB, uint32_t &tI, uint32_t &T) {
-    tI = gm_tiles_inside(nI);
-    T = tI + (nB + 63) / 64;
+/* ------------------------------------------------------------ window sweep
+ * A cell infected inside a launch window cannot complete before the window ends
+ * (window_length, gm_host.cpp), so one pass over the completion codes at the
+ * window's start finds the completed cells of all its steps: SCORE's sweep
+ * (calcGrowthStepInside / Border, SCORE_Kernel.cpp:4046-4249) with its FullRX
+ * lists, W steps at a time.  The 2-byte codes are read twice per window instead
+ * of once per step.
+ *
+ * Blocks of GM_BLOCK threads own consecutive 512-slot chunks of one list, P.cpw
+ * per wave: blocks [0, P.nbI) the Inside list, [P.nbI, P.nb) the Border list, so
+ * block order is FullRX order.  A lane takes eight slots with one 16-byte load. */
+
+/* chunks [c0, c1) of wave w of block b, within its list; chunk c of the Border
+ * list is chunk P.chI + c in tile numbering */
+struct WaveChunks {
+    uint32_t c0, c1, slot0, n, tile0;
+};
+static __device__ __forceinline__ WaveChunks wave_chunks(const GmDev &d, const GmPart &P, uint32_t b, uint32_t w) {
+    const bool inB = b >= P.nbI;
+    const uint32_t first = ((inB ? b - P.nbI : b) * GM_SW_WAVES + w) * P.cpw, nch = inB ? P.chB : P.chI;
+    WaveChunks r;
+    r.c0 = first < nch ? first : nch;
+    r.c1 = first + P.cpw < nch ? first + P.cpw : nch;
+    r.slot0 = inB ? d.capI : 0u;
+    r.n = inB ? d.st->nB : d.st->nI;
+    r.tile0 = (inB ? P.chI : 0u) * GM_SW_TPC;
+    return r;
 }
 
-/* per-block list counts: [0] full Inside, [1] recycled Inside, [2] full Border,
- * [3] recycled Border, [4] cells without a valid prediction; each GM_MAX_BLOCKS long */
-#define BC_FI 0
-#define BC_RI 1
-#define BC_FB 2
-#define BC_RB 3
-#define BC_UN 4
-/* rows of the infection pass: winners into Inside / Border, attempts */
-#define BC_WI 5
-#define BC_WB 6
-#define BC_WA 7
-
-static __device__ __forceinline__ uint32_t tile_slot0(const GmDev &d, uint32_t tile, uint32_t tI) {
-    return tile < tI ? tile * 64u : d.capI + (tile - tI) * 64u;
+/* the eight codes of a lane in chunk c, INACTIVE... (0xFFFF) beyond the list's
+ * length, and how many of them are occupied */
+static __device__ __forceinline__ uint4 chunk_codes(const GmDev &d, const WaveChunks &r, uint32_t c, uint32_t lane,
+                                                    uint32_t &nocc) {
+    const uint32_t i = c * GM_SW_CHUNK + 8u * lane;
+    nocc = r.n > i ? (r.n - i < 8u ? r.n - i : 8u) : 0u;
+    return nocc ? *reinterpret_cast<const uint4 *>(d.cstep + r.slot0 + i)
+                : make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu);
 }
 
-/* pass 1: every occupied slot, eight per lane with one 16-byte load of 2-byte
- * codes: a wave reads a 512-slot chunk of GM_SW_TPC = 8 tiles per load, and
- * GM_SW_UNROLL chunks at once.  Each lane classifies its eight slots without
- * branches (completed bits 0-7, INACTIVE bits 8-15); tile t's masks are balloted
- * from lanes 8t..8t+7, lane t keeps them and one store writes the chunk's.  The
- * Inside list spans tI tiles (whole chunks), the Border list follows from tile tI. */
-#ifndef GM_SW_UNROLL
-#define GM_SW_UNROLL 2
-#endif
-static_assert(GM_SW_TPC == 8, "a 16-byte load of 2-byte codes covers 8 slots per lane");
-__global__ void __launch_bounds__(GM_BLOCK) k_sweep(GmDev d, GmSweepArgs A0) {
-    __shared__ uint32_t red[GM_BLOCK / 64][5];
-    __shared__ uint64_t sF[GM_BLOCK / 64][8], sR[GM_BLOCK / 64][8];
-    if (d.st->halt) return;
-    const GmSweepArgs A = step_args(d, A0);
-    const uint32_t nI = d.st->nI, nB = d.st->nB;
-    uint32_t tI, T;
-    step_tiles(nI, nB, tI, T);
-    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint32_t lo, hi;
-    part_of(T, GM_SW_TPC, lo, hi); /* whole chunks, except an end at T */
-    /* chunks [c_lo, c_hi); a block left empty (lo == hi == T) has none */
-    const uint32_t c_lo = lo / GM_SW_TPC, c_hi = lo < hi ? (hi + GM_SW_TPC - 1u) / GM_SW_TPC : c_lo;
-    const uint32_t kc = A.k & (GM_CS_MOD - 1u), horizon = d.horizon;
-    uint32_t cFI = 0, cRI = 0, cFB = 0, cRB = 0, unknown = 0;
-    for (uint32_t c0 = c_lo + w; c0 < c_hi; c0 += (GM_BLOCK / 64) * GM_SW_UNROLL) {
-        uint4 cs[GM_SW_UNROLL];
-        uint32_t nocc[GM_SW_UNROLL];
+static __device__ __forceinline__ uint32_t code_at(const uint4 &cs, int q) {
+    const uint32_t wd = q < 2 ? cs.x : q < 4 ? cs.y : q < 6 ? cs.z : cs.w;
+    return (wd >> (16 * (q & 1))) & 0xFFFFu;
+}
+
+/* pass 1: per block, the cells that complete in each step of the window and the
+ * INACTIVE slots (row GM_WMAX); per wave, the completing cells of each step.
+ * Block 0 also clears the window's accumulators.  A slot without a prediction
+ * (UNKNOWN) raises GM_ERRF_MISSED. */
+__global__ void __launch_bounds__(GM_BLOCK) k_sweep(GmDev d, GmPart P, uint32_t k0, double xcells) {
+    __shared__ uint32_t red[GM_SW_WAVES][GM_WMAX + 1];
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6, b = blockIdx.x;
+    if (b == 0 && threadIdx.x == 0) {
+        GmStats *st = d.st;
+        st->halt = 0;
+        st->nexec = 0;
+        st->ndeferred = 0;
+        st->npend = 0;
+        st->pone = 0;
+        st->nzeroed = 0;
+        st->cwrap = 0;
+        st->novf = 0;
+        d.win->nret0 = st->nret;
+        d.win->xcells0 = xcells;
+        d.win->npend0 = 0;
+        d.win->top_hit = 0;
+    }
+    const WaveChunks r = wave_chunks(d, P, b, w);
+    const uint32_t kc = k0 & (GM_CS_MOD - 1u), horizon = d.horizon;
+    uint32_t mine = 0, nrec = 0; /* lane i: step i's cells in the wave */
+    bool unknown = false;
+    for (uint32_t cb = r.c0; cb < r.c1; cb += GM_SW_PACK) {
+        const uint32_t ce = cb + GM_SW_PACK < r.c1 ? cb + GM_SW_PACK : r.c1;
+        /* counts of the lane's slots by step, a byte each (at most 8 per chunk) */
+        unsigned long long a0 = 0ull, a1 = 0ull;
+        for (uint32_t c = cb; c < ce; c++) {
+            uint32_t nocc;
+            const uint4 cs = chunk_codes(d, r, c, lane, nocc);
 #pragma unroll
-        for (int u = 0; u < GM_SW_UNROLL; u++) {
-            const uint32_t c = c0 + u * (GM_BLOCK / 64);
-            const uint32_t tile0 = c * GM_SW_TPC;
-            const uint32_t base = tile_slot0(d, tile0, tI) + 8u * lane;
-            /* slots below lim are occupied and inside this block's tiles */
-            const uint32_t lend = tile0 < tI ? nI : d.capI + nB;
-            const uint32_t tend = tile_slot0(d, tile0, tI) + 64u * (hi - tile0 < GM_SW_TPC ? hi - tile0 : GM_SW_TPC);
-            const uint32_t lim = c < c_hi ? (lend < tend ? lend : tend) : 0u;
-            nocc[u] = lim > base ? (lim - base < 8u ? lim - base : 8u) : 0u; /* occupied slots of this lane */
-            cs[u] = nocc[u] ? *reinterpret_cast<const uint4 *>(d.cstep + base)
-                            : make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu);
-        }
-#pragma unroll
-        for (int u = 0; u < GM_SW_UNROLL; u++) {
-            const uint32_t c = c0 + u * (GM_BLOCK / 64);
-            if (c >= c_hi) break;
-            const uint32_t pack = sweep_classify(cs[u], nocc[u], kc, horizon, unknown);
-            const uint32_t tile0 = c * GM_SW_TPC;
-            /* per-lane counts, summed over the wave once at the end */
-            const uint32_t nf = (uint32_t)__popc(pack & 0xFFu), nr = (uint32_t)__popc(pack >> 8);
-            if (tile0 >= tI) {
-                cFB += nf;
-                cRB += nr;
-            } else {
-                cFI += nf;
-                cRI += nr;
-            }
-            uint64_t myF, myR;
-            sweep_masks(pack, sF[w], sR[w], myF, myR);
-            if (lane < GM_SW_TPC && tile0 + lane < hi) {
-                d.mF[tile0 + lane] = myF;
-                d.mR[tile0 + lane] = myR;
+            for (int q = 0; q < 8; q++) {
+                const uint32_t x = code_at(cs, q);
+                const bool in = (uint32_t)q < nocc;
+                const uint32_t di = (x - kc) & (GM_CS_MOD - 1u);
+                const unsigned long long one = in && x < GM_CS_MOD && di < P.W ? 1ull << (8u * (di & 7u)) : 0ull;
+                if (di < 8u) a0 += one;
+                else a1 += one;
+                nrec += in && cs_inactive(x, kc, horizon) ? 1u : 0u;
+                unknown |= in && x == GM_CS_UNKNOWN;
             }
         }
+        /* wave sums: two 16-bit fields per register (at most 64 * 8 * GM_SW_PACK) */
+        uint32_t s[GM_WMAX / 2];
+#pragma unroll
+        for (int i = 0; i < GM_WMAX / 2; i++) {
+            const unsigned long long a = i < 4 ? a0 : a1;
+            const uint32_t f = (uint32_t)(a >> (16 * (i & 3))) & 0xFFFFu;
+            s[i] = (f & 0xFFu) | (f & 0xFF00u) << 8;
+        }
+#pragma unroll
+        for (int i = 0; i < GM_WMAX / 2; i++) {
+            if (2u * i >= P.W) break;
+            for (int o = 32; o > 0; o >>= 1) s[i] += (uint32_t)__shfl_xor((int)s[i], o, 64);
+            if ((lane >> 1) == (uint32_t)i) mine += (lane & 1u) ? s[i] >> 16 : s[i] & 0xFFFFu;
+        }
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        unknown += __shfl_down(unknown, o, 64);
-        cFI += __shfl_down(cFI, o, 64);
-        cRI += __shfl_down(cRI, o, 64);
-        cFB += __shfl_down(cFB, o, 64);
-        cRB += __shfl_down(cRB, o, 64);
+    for (int o = 32; o > 0; o >>= 1) nrec += __shfl_xor(nrec, o, 64);
+    if (__any(unknown) && lane == 0) atomicOr(&d.st->err, GM_ERRF_MISSED);
+    if (lane < P.W) {
+        red[w][lane] = mine;
+        d.wwave[((size_t)b * GM_SW_WAVES + w) * GM_WMAX + lane] = mine;
     }
-    if (lane == 0) {
-        red[w][0] = cFI; red[w][1] = cRI; red[w][2] = cFB; red[w][3] = cRB; red[w][4] = unknown;
+    if (lane == 0) red[w][GM_WMAX] = nrec;
+    __syncthreads();
+    const uint32_t t = threadIdx.x;
+    if (t < P.W || t == GM_WMAX) {
+        uint32_t v = 0;
+        for (uint32_t q = 0; q < GM_SW_WAVES; q++) v += red[q][t];
+        d.wcnt[(size_t)t * d.swb + b] = v;
+    }
+}
+
+/* What the window's steps need of the counts' totals: cells completing in step
+ * i, where its list starts, the lists' lengths and recyclable slots before step
+ * 0.  One thread. */
+static __device__ void window_totals(const GmDev &d, const GmPart &P, const uint32_t *tot, uint32_t recI, uint32_t recB,
+                                     const uint32_t *totI) {
+    GmWin *win = d.win;
+    uint32_t off = 0, err = 0;
+    for (uint32_t i = 0; i < P.W; i++) {
+        win->full[i] = tot[i];
+        win->fullI[i] = totI[i];
+        win->off[i] = off;
+        off += tot[i];
+        /* infection keys are p*32 + rank in 32 bits, p < full */
+        if (tot[i] > (1u << 27)) err = GM_ERRF_KEYS;
+    }
+    win->off[P.W] = off;
+    if (err) atomicOr(&d.st->err, err);
+    GmWinStep &s = win->step[0];
+    s.nI = d.st->nI;
+    s.nB = d.st->nB;
+    s.totRecI = recI;
+    s.totRecB = recB;
+    s.recLenI = recI < d.recCapI ? recI : d.recCapI;
+    s.recLenB = recB < d.recCapB ? recB : d.recCapB;
+}
+
+/* pass 2, where the window has more than GM_SW_FOLD blocks: one block, a wave
+ * per row of counts, 32 consecutive entries per lane; exclusive prefixes over
+ * the blocks.  The INACTIVE counts and their prefixes within each list go to the
+ * recycling tables of step 0.  (With fewer blocks each block of pass 3 adds up
+ * what it needs, which saves this launch: 6 us a step before.) */
+__global__ void __launch_bounds__(1024) k_sweep_scan(GmDev d, GmPart P) {
+    __shared__ uint32_t stot[GM_WMAX + 1], stotI[GM_WMAX + 1];
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    for (uint32_t row = w; row <= P.W; row += 16u) {
+        const bool rec = row == P.W;
+        const uint32_t rr = rec ? (uint32_t)GM_WMAX : row;
+        const uint32_t *cnt = d.wcnt + (size_t)rr * d.swb;
+        uint32_t carry = 0, atI = 0;
+        for (uint32_t b0 = 0; b0 < P.nb; b0 += 2048u) {
+            const uint32_t i0 = b0 + lane * 32u;
+            uint32_t v[32], sum = 0;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                uint4 q = make_uint4(0u, 0u, 0u, 0u);
+                if (i0 + 4u * i < P.nb) q = *reinterpret_cast<const uint4 *>(cnt + i0 + 4u * i);
+                v[4 * i] = q.x; v[4 * i + 1] = q.y; v[4 * i + 2] = q.z; v[4 * i + 3] = q.w;
+            }
+#pragma unroll
+            for (int i = 0; i < 32; i++) {
+                if (i0 + i >= P.nb) v[i] = 0;
+                sum += v[i];
+            }
+            const uint32_t incl = wave_incl_scan(sum);
+            uint32_t run = carry + incl - sum;
+            /* the prefix at the first Border block */
+            const uint32_t atLane = (P.nbI - b0) / 32u;
+            uint32_t here = 0;
+#pragma unroll
+            for (int i = 0; i < 32; i++) {
+                const uint32_t x = v[i];
+                v[i] = run;
+                if (i0 + i == P.nbI) here = run;
+                run += x;
+            }
+            if (P.nbI >= b0 && P.nbI < b0 + 2048u) atI = __shfl(here, (int)atLane, 64);
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const uint32_t b = i0 + 4u * i;
+                if (b >= P.nb) continue;
+                uint4 q = make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+                if (rec) { /* within the list; the counts themselves are step 0's */
+                    *reinterpret_cast<uint4 *>(d.rcnt + b) = *reinterpret_cast<const uint4 *>(cnt + b);
+                    *reinterpret_cast<uint4 *>(d.rgone + b) = make_uint4(0u, 0u, 0u, 0u);
+                    *reinterpret_cast<uint4 *>(d.rmrg + b) = make_uint4(0u, 0u, 0u, 0u);
+                    q.x -= b >= P.nbI ? atI : 0u;
+                    q.y -= b + 1u >= P.nbI ? atI : 0u;
+                    q.z -= b + 2u >= P.nbI ? atI : 0u;
+                    q.w -= b + 3u >= P.nbI ? atI : 0u;
+                }
+                *reinterpret_cast<uint4 *>((rec ? d.rpre : d.wpre + (size_t)rr * d.swb) + b) = q;
+            }
+            carry += __shfl(incl, 63, 64);
+        }
+        if (P.nbI >= P.nb) atI = carry;
+        if (lane == 0) {
+            stot[row] = carry;
+            stotI[row] = atI;
+        }
     }
     __syncthreads();
-    if (threadIdx.x < 5) {
-        uint32_t t = 0;
-        for (int i = 0; i < GM_BLOCK / 64; i++) t += red[i][threadIdx.x];
-        d.bcnt[threadIdx.x * GM_MAX_BLOCKS + blockIdx.x] = t;
-    }
+    if (threadIdx.x == 0) window_totals(d, P, stot, stotI[P.W], stot[P.W] - stotI[P.W], stotI);
 }
 
-/* pass 2: per-block offsets and the list lengths.  Cells the sweep met without
- * a prediction (UNKNOWN) raise GM_ERRF_MISSED. */
-__global__ void __launch_bounds__(1024) k_sweep_scan(GmDev d, uint32_t nb) {
-    if (d.st->halt) return;
-    uint32_t tot[5];
-    scan_block_counts<5>(d.bcnt, nb, tot);
-    if (threadIdx.x == 0) {
-        GmStats *st = d.st;
-        if (tot[BC_UN]) st->err |= GM_ERRF_MISSED;
-        /* infection keys are p*32 + rank in 32 bits, p < nfull */
-        if ((uint64_t)tot[BC_FI] + tot[BC_FB] > (1ull << 27)) st->err |= GM_ERRF_KEYS;
-        st->nfullI = tot[BC_FI];
-        st->totRecI = tot[BC_RI];
-        st->nfullB = tot[BC_FB];
-        st->totRecB = tot[BC_RB];
-        st->recLenI = tot[BC_RI] < d.recCapI ? tot[BC_RI] : d.recCapI;
-        st->recLenB = tot[BC_RB] < d.recCapB ? tot[BC_RB] : d.recCapB;
-    }
-}
-
-/* Running offsets of the tiles [batch, batch+64) of a sweep block: lane t
- * holds tile batch+t and gets, per list count c (BC_FI..BC_RB), the offset of
- * its tile's first entry; run[] advances past the batch. */
-static __device__ __forceinline__ void tile_offsets(const GmDev &d, uint32_t tI, uint32_t t, bool valid, uint64_t &bf,
-                                                    uint64_t &br, uint32_t *run, uint32_t *off) {
-    bf = valid ? d.mF[t] : 0ull;
-    br = valid ? d.mR[t] : 0ull;
-    const bool isB = t >= tI;
-    const uint32_t cf = (uint32_t)__popcll(bf), cr = (uint32_t)__popcll(br);
-    const uint32_t v[4] = {isB ? 0u : cf, isB ? 0u : cr, isB ? cf : 0u, isB ? cr : 0u};
+/* pass 3: append_to_fullrx_*_list (SCORE_Kernel.cpp:3994-4042, :4133-4180) of
+ * every step as ordered compaction: step i's completed slots ascending, Inside
+ * then Border, at pslot[win->off[i]...]; and the INACTIVE mask of every 64-slot
+ * tile, from which the steps hand out recycled slots.  FOLD: the block adds up
+ * the counts of at most GM_SW_FOLD blocks itself. */
+template <bool FOLD>
+__global__ void __launch_bounds__(GM_BLOCK) k_compact(GmDev d, GmPart P, uint32_t k0) {
+    __shared__ uint32_t stot[GM_WMAX + 1], spre[GM_WMAX + 1], stotI[GM_WMAX + 1], base[GM_WMAX];
+    __shared__ uint32_t run[GM_SW_WAVES][GM_WMAX];
+    __shared__ uint64_t sR[GM_SW_WAVES][8];
+    /* per lane 16 counters of 16 bits, rows of 40 bytes against bank conflicts */
+    __shared__ __align__(8) uint32_t sl[GM_SW_WAVES][64][10];
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6, b = blockIdx.x, t = threadIdx.x;
+    if (FOLD) {
+        for (uint32_t row = w; row <= P.W; row += GM_SW_WAVES) {
+            const bool rec = row == P.W;
+            const uint32_t *cnt = d.wcnt + (size_t)(rec ? (uint32_t)GM_WMAX : row) * d.swb;
+            const uint32_t i0 = 4u * lane;
+            uint4 q = make_uint4(0u, 0u, 0u, 0u);
+            if (i0 < P.nb) q = *reinterpret_cast<const uint4 *>(cnt + i0);
+            const uint32_t v[4] = {q.x, q.y, q.z, q.w};
+            uint32_t a = 0, p = 0, pI = 0;
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-        const uint32_t incl = wave_incl_scan(v[c]);
-        off[c] = run[c] + incl - v[c];
-        run[c] += __shfl(incl, 63, 64);
-    }
-}
-
-/* pass 3: append_to_fullrx_*_list (SCORE_Kernel.cpp:3994-4042, :4133-4180) as
- * ordered compaction: the completed slots in ascending order, Inside then
- * Border, in one array.  One wave per sweep block, one lane per tile: the lane
- * writes its tile's completed slots at its offset. */
-__global__ void __launch_bounds__(64) k_compact(GmDev d) {
-    if (d.st->halt) return;
-    const uint32_t lane = threadIdx.x;
-    uint32_t tI, T;
-    step_tiles(d.st->nI, d.st->nB, tI, T);
-    uint32_t lo, hi;
-    part_of(T, GM_SW_TPC, lo, hi);
-    uint32_t run[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) run[c] = d.bcnt[c * GM_MAX_BLOCKS + blockIdx.x];
-    run[BC_FB] += d.st->nfullI; /* Border parents follow the Inside ones */
-    for (uint32_t batch = lo; batch < hi; batch += 64) {
-        const uint32_t t = batch + lane;
-        uint64_t bf, br;
-        uint32_t off[4];
-        tile_offsets(d, tI, t, t < hi, bf, br, run, off);
-        const uint32_t s0 = tile_slot0(d, t, tI);
-        uint32_t o = off[t >= tI ? BC_FB : BC_FI];
-        for (uint64_t m = bf; m; m &= m - 1ull) d.pslot[o++] = s0 + (uint32_t)__ffsll((long long)m) - 1u;
-    }
-}
-
-/* append_to_recycling_*_list (SCORE_Kernel.cpp:4037-4041, :4175-4179): the
- * recycled slots in ascending order, of which only the first min(winners, cap)
- * are ever handed out; written after the winners are counted, so each sweep
- * block writes only the part of its INACTIVE slots that falls below that. */
-__global__ void __launch_bounds__(64) k_recycle(GmDev d) {
-    const GmStats *st = d.st;
-    if (st->halt) return;
-    const uint32_t lane = threadIdx.x;
-    /* the sweep's tiles and partition: the lengths before this step's appends */
-    uint32_t tI, T;
-    step_tiles(st->nIold, st->nBold, tI, T);
-    const uint32_t limI = st->winI < st->recLenI ? st->winI : st->recLenI;
-    const uint32_t limB = st->winB < st->recLenB ? st->winB : st->recLenB;
-    uint32_t run[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) run[c] = d.bcnt[c * GM_MAX_BLOCKS + blockIdx.x];
-    uint32_t lo, hi;
-    part_of(T, GM_SW_TPC, lo, hi);
-    for (uint32_t batch = lo; batch < hi; batch += 64) {
-        if (run[BC_RI] >= limI && run[BC_RB] >= limB) return; /* nothing further is handed out */
-        const uint32_t t = batch + lane;
-        uint64_t bf, br;
-        uint32_t off[4];
-        tile_offsets(d, tI, t, t < hi, bf, br, run, off);
-        const uint32_t s0 = tile_slot0(d, t, tI);
-        if (t >= tI) {
-            uint32_t o = off[BC_RB];
-            for (uint64_t m = br; m && o < limB; m &= m - 1ull) d.recB[o++] = s0 - d.capI + (uint32_t)__ffsll((long long)m) - 1u;
-        } else {
-            uint32_t o = off[BC_RI];
-            for (uint64_t m = br; m && o < limI; m &= m - 1ull) d.recI[o++] = s0 + (uint32_t)__ffsll((long long)m) - 1u;
+            for (uint32_t i = 0; i < 4; i++) {
+                const uint32_t x = i0 + i < P.nb ? v[i] : 0u;
+                a += x;
+                p += i0 + i < b ? x : 0u;
+                pI += i0 + i < P.nbI ? x : 0u;
+            }
+            for (int o = 32; o > 0; o >>= 1) {
+                a += __shfl_xor(a, o, 64);
+                p += __shfl_xor(p, o, 64);
+                pI += __shfl_xor(pI, o, 64);
+            }
+            if (lane == 0) {
+                stot[row] = a;
+                spre[row] = p;
+                stotI[row] = pI;
+            }
         }
+        __syncthreads();
+        if (t < P.W) {
+            uint32_t o = spre[t];
+            d.wpre[(size_t)t * d.swb + b] = o;
+            for (uint32_t i = 0; i < t; i++) o += stot[i];
+            base[t] = o;
+        }
+        if (t == GM_WMAX) {
+            d.rcnt[b] = d.wcnt[(size_t)GM_WMAX * d.swb + b];
+            d.rpre[b] = spre[P.W] - (b >= P.nbI ? stotI[P.W] : 0u);
+            d.rgone[b] = 0;
+            d.rmrg[b] = 0;
+        }
+        if (b == 0 && t == 64u) window_totals(d, P, stot, stotI[P.W], stot[P.W] - stotI[P.W], stotI);
+    } else if (t < P.W) {
+        base[t] = d.win->off[t] + d.wpre[(size_t)t * d.swb + b];
     }
-}
-
-/* grid of the sweep, compaction and recycling passes for lists of about nI, nB */
-#ifndef GM_SW_CHUNKS
-#define GM_SW_CHUNKS 2 /* 512-slot chunks per sweep wave */
-#endif
-static uint32_t sweep_blocks(uint32_t nI, uint32_t nB) {
-    const uint32_t T = gm_tiles_inside(nI) + (nB + 63) / 64;
-    return grid_for(T, GM_SW_TPC * (GM_BLOCK / 64) * GM_SW_CHUNKS);
+    __syncthreads();
+    if (lane < P.W) {
+        uint32_t o = base[lane];
+        const uint32_t *ww = d.wwave + (size_t)b * GM_SW_WAVES * GM_WMAX + lane;
+        for (uint32_t q = 0; q < w; q++) o += ww[q * GM_WMAX];
+        run[w][lane] = o;
+    }
+    wave_sync();
+    const WaveChunks r = wave_chunks(d, P, b, w);
+    const uint32_t kc = k0 & (GM_CS_MOD - 1u), horizon = d.horizon;
+    for (uint32_t c = r.c0; c < r.c1; c++) {
+        uint32_t nocc;
+        const uint4 cs = chunk_codes(d, r, c, lane, nocc);
+        unsigned long long cnt = 0ull; /* 16 counters of 4 bits (at most 8 each) */
+        uint32_t full = 0, rec = 0;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const uint32_t x = code_at(cs, q);
+            const bool in = (uint32_t)q < nocc;
+            const uint32_t di = (x - kc) & (GM_CS_MOD - 1u);
+            const bool f = in && x < GM_CS_MOD && di < P.W;
+            cnt += f ? 1ull << (4u * (di & 15u)) : 0ull;
+            full |= f ? 1u << q : 0u;
+            rec |= in && cs_inactive(x, kc, horizon) ? 1u << q : 0u;
+        }
+        reinterpret_cast<uint8_t *>(sR[w])[lane] = (uint8_t)rec;
+        wave_sync();
+        if (lane < GM_SW_TPC) d.mR[r.tile0 + c * GM_SW_TPC + lane] = sR[w][lane];
+        if (!__any(full != 0u)) {
+            wave_sync();
+            continue;
+        }
+        uint32_t incl[GM_WMAX / 2];
+#pragma unroll
+        for (int i = 0; i < GM_WMAX / 2; i++) {
+            if (2u * i >= P.W) break;
+            const uint32_t f = (uint32_t)(cnt >> (8 * i));
+            const uint32_t v = (f & 0xFu) | (f & 0xF0u) << 12;
+            incl[i] = wave_incl_scan(v);
+            sl[w][lane][i] = incl[i] - v;
+        }
+        wave_sync();
+        uint16_t *mineRow = reinterpret_cast<uint16_t *>(sl[w][lane]);
+        const uint32_t slot = r.slot0 + c * GM_SW_CHUNK + 8u * lane;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            if (!((full >> q) & 1u)) continue;
+            const uint32_t di = (code_at(cs, q) - kc) & (GM_CS_MOD - 1u);
+            const uint32_t o = mineRow[di];
+            mineRow[di] = (uint16_t)(o + 1u);
+            d.pslot[run[w][di] + o] = slot + (uint32_t)q;
+        }
+        wave_sync();
+        if (lane == 63u) {
+#pragma unroll
+            for (int i = 0; i < GM_WMAX / 2; i++) {
+                if (2u * i >= P.W) break;
+                run[w][2 * i] += incl[i] & 0xFFFFu;
+                run[w][2 * i + 1] += incl[i] >> 16;
+            }
+        }
+        wave_sync();
+    }
 }
 
 hipError_t gm_launch_reanchor(const GmDev &d, const GmSweepArgs &a, hipStream_t s) {
@@ -313,20 +442,25 @@ hipError_t gm_launch_reanchor(const GmDev &d, const GmSweepArgs &a, hipStream_t 
     return hipGetLastError();
 }
 
-hipError_t gm_launch_sweep(const GmDev &d, const GmSweepArgs &a, hipStream_t s, hipEvent_t *ev) {
+__global__ void k_arrivals(GmDev d, GmSweepArgs A);
+
+hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &a, bool arrivals, double xcells,
+                            hipStream_t s, hipEvent_t *ev) {
     hipError_t e;
-    GmSweepArgs A = a;
-    A.reanchor = 0;
     if ((e = mark(ev, 0, s)) != hipSuccess) return e;
-    if (a.reanchor) k_reanchor<<<grid_for(a.nI + a.nB, GM_BLOCK), GM_BLOCK, 0, s>>>(d, a);
-    if ((e = gm_launch_arrivals(d, A, s)) != hipSuccess) return e;
-    const uint32_t nb = sweep_blocks(a.nI, a.nB);
+    if (a.reanchor && (e = gm_launch_reanchor(d, a, s)) != hipSuccess) return e;
+    if (arrivals) {
+        k_arrivals<<<1, 1024, 0, s>>>(d, a);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
     if ((e = mark(ev, 1, s)) != hipSuccess) return e;
-    k_sweep<<<nb, GM_BLOCK, 0, s>>>(d, A);
+    k_sweep<<<P.nb, GM_BLOCK, 0, s>>>(d, P, a.k, xcells);
     if ((e = mark(ev, 2, s)) != hipSuccess) return e;
-    k_sweep_scan<<<1, 1024, 0, s>>>(d, nb);
+    const bool fold = P.nb <= GM_SW_FOLD;
+    if (!fold) k_sweep_scan<<<1, 1024, 0, s>>>(d, P);
     if ((e = mark(ev, 3, s)) != hipSuccess) return e;
-    k_compact<<<nb, 64, 0, s>>>(d);
+    if (fold) k_compact<true><<<P.nb, GM_BLOCK, 0, s>>>(d, P, a.k);
+    else k_compact<false><<<P.nb, GM_BLOCK, 0, s>>>(d, P, a.k);
     return hipGetLastError();
 }
 
@@ -360,7 +494,7 @@ hipError_t gm_launch_dmap_init(const GmDev &d, hipStream_t s) {
  * targets outside z, and send strictly interior targets to the Inside list. */
 static __device__ __forceinline__ bool attempt_target(const GmDev &d, bool fromB, uint32_t x, uint32_t y, uint32_t z,
                                                       int r, uint32_t &tx_, uint32_t &ty_, uint32_t &tz_, bool &toB) {
-    int tx = (int)x + c_dx[r], ty = (int)y + c_dy[r], tz = (int)z + c_dz[r];
+    int tx = (int)x + dir_dx(r), ty = (int)y + dir_dy(r), tz = (int)z + dir_dz(r);
     const int nx = (int)d.nx, ny = (int)d.ny, nz = (int)d.nz;
     if (fromB) {
         if (tx < 0) tx += nx;
@@ -382,228 +516,633 @@ static __device__ __forceinline__ bool attempt_target(const GmDev &d, bool fromB
 }
 
 
-/* GM_PG lanes per parent: lane 0 copies what the infection needs of the
- * completed cell from its record into the dense parent array (FullRX order);
- * lane l makes the attempts of rank l, l+GM_PG, ... (< 26), so the bitmap reads
- * of a lane are independent and a wave keeps 64/GM_PG parents in flight.  Every
- * attempt on a deformed cell claims its target (the smallest key p*32+r is the
- * serial winner); their mask over the ranks is kept in pmI for the decide pass. */
-__global__ void __launch_bounds__(GM_BLOCK) k_propose(GmDev d) {
-    if (d.st->halt) return;
-    const uint32_t nfull = d.st->nfullI + d.st->nfullB;
-    /* the step's parents retire into the log at [nret, nret + nfull) */
-    const unsigned long long nret = d.st->nret;
-    const bool logged = nret + nfull <= d.rlogCap;
-    if (!logged && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&d.st->err, GM_ERRF_RLOG_FULL);
-    const uint32_t lg = threadIdx.x & (GM_PG - 1);
-    const uint32_t ngroups = gridDim.x * (GM_BLOCK / GM_PG);
-    for (uint32_t p = blockIdx.x * (GM_BLOCK / GM_PG) + threadIdx.x / GM_PG; p < nfull; p += ngroups) {
-        uint4 q2 = make_uint4(0u, 0u, 0u, 0u);
-        if (lg == 0) {
-            const uint32_t s = d.pslot[p];
-            const GmRec *r = d.rec + s;
-            const RecC c = rec_c(r);
-            const uint32_t rxg = r->rxg;
-            const uint32_t cell = c.cell;
-            const uint32_t z = cell / d.nxy, rem = cell - z * d.nxy, y = rem / d.nx, x = rem - y * d.nx;
-            q2 = make_uint4(x, y, z, s >= d.capI ? 1u : 0u);
-            par_plane(d, GM_PAR_IDS)[p] = make_uint4(s, cell, c.defg, rxg);
-            /* the value after the completing addition follows in k_decide */
-            reinterpret_cast<double2 *>(par_plane(d, GM_PAR_FP))[p] = make_double2(0.0, c.P);
-            par_plane(d, GM_PAR_XYZ)[p] = q2;
-            if (logged) d.rlog[nret + p] = make_uint2(cell, d.ndefg + rxg);
-        }
-        q2.x = (uint32_t)__shfl((int)q2.x, 0, GM_PG);
-        q2.y = (uint32_t)__shfl((int)q2.y, 0, GM_PG);
-        q2.z = (uint32_t)__shfl((int)q2.z, 0, GM_PG);
-        q2.w = (uint32_t)__shfl((int)q2.w, 0, GM_PG);
-        const bool fromB = q2.w != 0u;
-        const uint32_t gsh = (threadIdx.x & 63) & ~(GM_PG - 1); /* first lane of the group in the wave */
-        uint32_t am = 0;
+/* sum over the block (GM_BLOCK threads) of three values; every thread gets them */
+static __device__ __forceinline__ void block_sum3(uint32_t &a, uint32_t &b, uint32_t &c, uint32_t (*sh)[3]) {
+    for (int o = 32; o > 0; o >>= 1) {
+        a += __shfl_xor(a, o, 64);
+        b += __shfl_xor(b, o, 64);
+        c += __shfl_xor(c, o, 64);
+    }
+    const uint32_t w = threadIdx.x >> 6;
+    __syncthreads();
+    if ((threadIdx.x & 63u) == 0) {
+        sh[w][0] = a;
+        sh[w][1] = b;
+        sh[w][2] = c;
+    }
+    __syncthreads();
+    a = b = c = 0;
 #pragma unroll
-        for (uint32_t i = 0; i < GM_PG_ITERS; i++) {
-            const uint32_t rk = lg + GM_PG * i;
-            bool att = false;
-            if (rk < 26) {
-                uint32_t tx, ty, tz;
-                bool toB;
-                if (attempt_target(d, fromB, q2.x, q2.y, q2.z, (int)rk, tx, ty, tz, toB) && is_deformed(d, tx, ty, tz)) {
-                    att = true;
-                    atomicMin(&d.claim[cell_of(d, tx, ty, tz)], p * 32u + rk);
-                }
-            }
-            am |= (uint32_t)((__ballot(att) >> gsh) & ((1ull << GM_PG) - 1u)) << (GM_PG * i);
-        }
-        if (lg == 0) d.pmI[p] = am;
+    for (int i = 0; i < GM_BLOCK / 64; i++) {
+        a += sh[i][0];
+        b += sh[i][1];
+        c += sh[i][2];
     }
 }
 
-/* One lane per parent: which of its attempts won, as 26-bit masks per
- * destination list; per-block totals for the ranking scan and the attempts.
- * A parent that won a target gets its value after the completing addition, the
- * carry's source, in the parent array.  The partition into blocks is the commit
- * pass's. */
-__global__ void __launch_bounds__(64) k_decide(GmDev d) {
-    if (d.st->halt) return;
-    const uint32_t nfull = d.st->nfullI + d.st->nfullB;
-    const uint32_t k = d.st->kcur;
-    uint32_t lo, hi;
-    part_of(nfull, GM_PCHUNK, lo, hi);
-    uint32_t cI = 0, cB = 0, cA = 0;
-    for (uint32_t p = lo + threadIdx.x; p < hi; p += 64) {
-        const uint4 q2 = par_plane(d, GM_PAR_XYZ)[p];
-        const uint32_t am = d.pmI[p];
-        const uint32_t ps = d.pslot[p]; /* loaded with the rest, used if the parent wins */
-        uint32_t mI = 0, mB = 0;
+/* Closes step js of the window, by one block after the step's commit pass: its
+ * row for the host's master section, the lists' lengths and, with `next`, the
+ * recycling tables of step js+1: per sweep block, how many of its INACTIVE slots
+ * step js handed out (the first min(winners, cap) of each list, ascending), how
+ * many it has now that step js's completed cells are INACTIVE, and their prefix
+ * within the list. */
+static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, bool next) {
+    __shared__ uint32_t sh[GM_BLOCK / 64][3];
+    __shared__ unsigned long long ws[GM_BLOCK / 64];
+    GmStats *st = d.st;
+    GmWin *win = d.win;
+    const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    uint32_t wI = 0, wB = 0, na = 0;
+    for (uint32_t i = t; i < P.nbd; i += GM_BLOCK) {
+        const uint2 v = d.btot[i];
+        wI += v.x;
+        wB += v.y;
+    }
+    for (uint32_t i = t; i < P.nbp; i += GM_BLOCK) na += d.acnt[(js & 1u) * GM_PB + i];
+    block_sum3(wI, wB, na, sh);
+    const GmWinStep o = win->step[js];
+    const uint32_t limI = wI < o.recLenI ? wI : o.recLenI, limB = wB < o.recLenB ? wB : o.recLenB;
+    const uint32_t rp = (js & 1u) * d.swb, rn = ((js + 1u) & 1u) * d.swb;
+    unsigned long long carry = 0ull; /* Inside | Border totals */
+    if (next) {
+        for (uint32_t b0 = 0; b0 < P.nb; b0 += 8u * GM_BLOCK) {
+            const uint32_t i0 = b0 + 8u * t;
+            uint32_t R[8], pre[8], full[8];
+            if (i0 < P.nb) {
+                const uint4 *q = reinterpret_cast<const uint4 *>(d.rcnt + rp + i0);
+                const uint4 *u = reinterpret_cast<const uint4 *>(d.rpre + rp + i0);
+                const uint4 *f = reinterpret_cast<const uint4 *>(d.wcnt + (size_t)js * d.swb + i0);
+                const uint4 q0 = q[0], q1 = q[1], u0 = u[0], u1 = u[1], f0 = f[0], f1 = f[1];
+                R[0] = q0.x; R[1] = q0.y; R[2] = q0.z; R[3] = q0.w; R[4] = q1.x; R[5] = q1.y; R[6] = q1.z; R[7] = q1.w;
+                pre[0] = u0.x; pre[1] = u0.y; pre[2] = u0.z; pre[3] = u0.w;
+                pre[4] = u1.x; pre[5] = u1.y; pre[6] = u1.z; pre[7] = u1.w;
+                full[0] = f0.x; full[1] = f0.y; full[2] = f0.z; full[3] = f0.w;
+                full[4] = f1.x; full[5] = f1.y; full[6] = f1.z; full[7] = f1.w;
+            }
+            unsigned long long sum = 0ull;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const uint32_t b = i0 + i;
+                if (b >= P.nb) {
+                    R[i] = pre[i] = 0;
+                    continue;
+                }
+                const uint32_t lim = b < P.nbI ? limI : limB;
+                const uint32_t left = pre[i] < lim ? lim - pre[i] : 0u;
+                pre[i] = left < R[i] ? left : R[i]; /* handed out */
+                R[i] = R[i] - pre[i] + full[i];
+                sum += b < P.nbI ? (unsigned long long)R[i] << 32 : (unsigned long long)R[i];
+            }
+            unsigned long long incl = sum;
+            for (int s = 1; s < 64; s <<= 1) {
+                const unsigned long long v = (unsigned long long)__shfl_up((long long)incl, s, 64);
+                if (lane >= (uint32_t)s) incl += v;
+            }
+            __syncthreads();
+            if (lane == 63u) ws[w] = incl;
+            __syncthreads();
+            unsigned long long before = carry + incl - sum;
+            for (uint32_t i = 0; i < GM_BLOCK / 64; i++) {
+                if (i < w) before += ws[i];
+                carry += ws[i];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const uint32_t b = i0 + i;
+                if (b >= P.nb) break;
+                d.rgone[b] = pre[i];
+                d.rcnt[rn + b] = R[i];
+                d.rpre[rn + b] = b < P.nbI ? (uint32_t)(before >> 32) : (uint32_t)before;
+                before += b < P.nbI ? (unsigned long long)R[i] << 32 : (unsigned long long)R[i];
+            }
+        }
+    }
+    if (t != 0) return;
+    GmStepRow r;
+    r.nI = o.nI + (wI - limI);
+    r.nB = o.nB + (wB - limB);
+    r.nfullI = win->fullI[js];
+    r.nfullB = win->full[js] - win->fullI[js];
+    r.totRecI = o.totRecI;
+    r.totRecB = o.totRecB;
+    r.recLenI = o.recLenI;
+    r.recLenB = o.recLenB;
+    r.winI = wI;
+    r.winB = wB;
+    r.npend = st->npend - win->npend0;
+    r.nattempt = na;
+    r.nzeroed = st->nzeroed < d.ndefg ? st->nzeroed : d.ndefg;
+    r.err = st->err;
+    r.nplaced = st->nplaced;
+    r.pone = st->pone;
+    r.pkey = st->arr_pkey;
+    st->rows[js] = r;
+    st->nplaced = 0;
+    st->pone = 0;
+    st->arr_pkey = 0ull;
+    win->npend0 = st->npend;
+    st->nI = r.nI;
+    st->nB = r.nB;
+    st->nret += (unsigned long long)win->full[js];
+    st->nexec = js + 1u;
+    if (next) {
+        GmWinStep &s = win->step[js + 1u];
+        s.nI = r.nI;
+        s.nB = r.nB;
+        s.totRecI = (uint32_t)(carry >> 32);
+        s.totRecB = (uint32_t)carry;
+        s.recLenI = s.totRecI < d.recCapI ? s.totRecI : d.recCapI;
+        s.recLenB = s.totRecB < d.recCapB ? s.totRecB : d.recCapB;
+    }
+}
+
+/* Whether step j of the window must not run: the host has to act on what step
+ * j-1 left (an error, a count that wrapped, the exhaustion of the grain that
+ * sets rhomax, Xcells at a threshold, weights the window cannot wait for).  Every
+ * input was written by an earlier kernel, so all blocks of the propose pass find
+ * the same; it records the answer in st->halt for the step's other passes. */
+static __device__ __forceinline__ bool must_halt(const GmDev &d, const GmWindow &w, uint32_t j) {
+    const GmStats *st = d.st;
+    const GmWin *win = d.win;
+    /* every word loaded before the first test */
+    const uint32_t flags = st->err | st->cwrap | st->novf | win->top_hit, npend = st->npend;
+    const double xc = win->xcells0 + (double)win->off[j];
+    return (flags != 0u) | ((npend != 0u) & !w.defer) | (npend > w.pend_limit) | ((j != 0u) & (xc >= w.xstop));
+}
+
+/* The deformed bits around a cell: nine per plane, bit (dy+1)*3 + dx+1, for the
+ * cell's own plane, the one below and the one above, in the order of the attempts'
+ * ranks (SCORE_Kernel.cpp:4611-4638: the own plane without the cell itself, the
+ * lower plane with its row y+1 first, the upper plane). */
+static __device__ __forceinline__ uint32_t rank_mask(uint32_t m, uint32_t dn, uint32_t up) {
+    const uint32_t lower = (dn >> 6 & 7u) | (dn & 7u) << 3 | (dn >> 3 & 7u) << 6;
+    return (m & 0xFu) | (m >> 1 & 0xF0u) | lower << 8 | up << 17;
+}
+
+/* A strictly interior cell's neighbourhood in the bitmap.  A brick holds 16 x 8
+ * cells of a plane in 16 bytes, a row of 16 cells in 16 bits, so one 16-byte load
+ * a plane usually covers the nine cells; a cell at a brick's edge also loads from
+ * the bricks beside it.  The loads of all planes are issued together (load), so
+ * that the caller can work until it needs them (mask). */
+struct Neighbourhood {
+    uint4 c[3], cx[3];          /* planes z, z-1, z+1: the cell's brick, the one beside it along x */
+    uint32_t ry[3], rxy[3];     /* the word with the adjacent row of the bricks beside along y */
+    uint32_t xi, yi;
+    __device__ __forceinline__ void load(const GmDev &d, uint32_t x, uint32_t y, uint32_t z) {
+        const uint4 *D = reinterpret_cast<const uint4 *>(d.dmap);
+        xi = x & 15u;
+        yi = y & 7u;
+        const uint32_t row = (x >> 4) + d.dnbx * (y >> 3), layer = d.dnbx * d.dnby;
+        uint32_t at[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const uint32_t zi = i == 0 ? z : i == 1 ? z - 1u : z + 1u;
+            at[i] = (row + layer * (zi >> 3)) * 8u + (zi & 7u);
+            c[i] = D[at[i]];
+            cx[i] = make_uint4(0u, 0u, 0u, 0u);
+            ry[i] = rxy[i] = 0;
+        }
+        const bool ex = xi == 0u || xi == 15u, ey = yi == 0u || yi == 7u;
+        const uint32_t sx = xi ? 8u : 0u - 8u, sy = (yi ? 8u : 0u - 8u) * d.dnbx, yw = yi ? 0u : 3u;
+        if (ex) {
+#pragma unroll
+            for (int i = 0; i < 3; i++) cx[i] = D[at[i] + sx];
+        }
+        if (ey) {
+#pragma unroll
+            for (int i = 0; i < 3; i++) ry[i] = d.dmap[(at[i] + sy) * 4u + yw];
+        }
+        if (ex && ey) {
+#pragma unroll
+            for (int i = 0; i < 3; i++) rxy[i] = d.dmap[(at[i] + sx + sy) * 4u + yw];
+        }
+    }
+    /* three rows of 16 bits, y-1 first */
+    __device__ __forceinline__ unsigned long long rows(const uint4 &q, uint32_t r) const {
+        const unsigned long long lo = (unsigned long long)q.y << 32 | q.x, hi = (unsigned long long)q.w << 32 | q.z;
+        const uint32_t s = 16u * (yi - 1u);
+        unsigned long long v = s < 64u ? lo >> (s & 63u) : hi >> (s & 63u);
+        if (s != 0u && s < 64u) v |= hi << (64u - s);
+        if (yi == 0u) v = lo << 16 | r >> 16;
+        if (yi == 7u) v = hi >> 32 | (unsigned long long)(r & 0xFFFFu) << 32;
+        return v;
+    }
+    __device__ __forceinline__ uint32_t plane(int i) const {
+        const unsigned long long one = 0x0000000100010001ull;
+        const unsigned long long T = rows(c[i], ry[i]), TX = rows(cx[i], rxy[i]);
+        unsigned long long U = T >> ((xi - 1u) & 63u);
+        if (xi == 0u) U = (T & 3u * one) << 1 | (TX >> 15 & one);
+        if (xi == 15u) U = (T >> 14 & 3u * one) | (TX & one) << 2;
+        return (uint32_t)(U & 7u) | (uint32_t)(U >> 13 & 0x38u) | (uint32_t)(U >> 26 & 0x1C0u);
+    }
+    __device__ __forceinline__ uint32_t mask() const { return rank_mask(plane(0), plane(1), plane(2)); }
+};
+
+/* The attempts of a Border cell on a face of the domain: x and y wrap, planes
+ * outside z have none.  27 single words, all loaded together. */
+static __device__ __forceinline__ uint32_t face_attempts(const GmDev &d, uint32_t x, uint32_t y, uint32_t z) {
+    const uint32_t xs[3] = {x ? x - 1u : d.nx - 1u, x, x + 1u < d.nx ? x + 1u : 0u};
+    const uint32_t ys[3] = {y ? y - 1u : d.ny - 1u, y, y + 1u < d.ny ? y + 1u : 0u};
+    uint32_t wd[27];
+#pragma unroll
+    for (int i = 0; i < 27; i++) {
+        const uint32_t zz = i < 9 ? z : i < 18 ? (z ? z - 1u : z) : (z + 1u < d.nz ? z + 1u : z);
+        const uint32_t yy = ys[i / 3 % 3], xx = xs[i % 3];
+        wd[i] = d.dmap[((xx >> 4) + d.dnbx * ((yy >> 3) + d.dnby * (zz >> 3))) * 32u + (zz & 7u) * 4u + ((yy & 7u) >> 1)];
+    }
+    uint32_t m[3] = {0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 27; i++)
+        m[i / 9] |= (wd[i] >> ((xs[i % 3] & 15u) + 16u * (ys[i / 3 % 3] & 1u)) & 1u) << (i % 9);
+    return rank_mask(m[0], z ? m[1] : 0u, z + 1u < d.nz ? m[2] : 0u);
+}
+
+/* Step j's attempts, one lane per parent.  What the infection needs of the parent
+ * goes to the dense parent planes (FullRX order), with its rxFrac after the
+ * completing addition, replayed from the anchor.  Every attempt on a deformed cell
+ * claims its target (the smallest key p*32+r is the serial winner); their mask
+ * over the ranks is kept in pmI for the decide pass.  Few of the 26 neighbours are
+ * still deformed (1.04 per parent on the 512^3 workload), so the cost is finding
+ * them: a strictly interior parent reads its 3x3x3 bits with three 16-byte loads
+ * (26 single tests before).  Wave w
+ * of a block takes chunks of 64 parents w*nbp apart, so that a short list spreads
+ * over the CUs.  Block 0 closes the step before. */
+__global__ void __launch_bounds__(GM_BLOCK) k_propose(GmDev d, GmPart P, GmWindow wd, uint32_t j, uint32_t k) {
+    __shared__ uint32_t satt[GM_BLOCK / 64];
+    GmStats *st = d.st;
+    const GmWin *win = d.win;
+    const uint32_t nfull = win->full[j], off = win->off[j];
+    const bool halt = must_halt(d, wd, j);
+    if (blockIdx.x == 0) {
+        if (j) close_step(d, P, j - 1u, !halt);
+        if (threadIdx.x == 0) {
+            st->halt = halt ? 1u : 0u;
+            if (d.prog)
+                __hip_atomic_store(d.prog, (j << 1) | (halt ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        return;
+    }
+    if (halt) return;
+    /* the step's parents retire into the log at [nret, nret + nfull) */
+    const unsigned long long nret = win->nret0 + off;
+    const bool logged = nret + nfull <= d.rlogCap;
+    const uint32_t blk = blockIdx.x - 1u, lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    if (!logged && blk == 0 && threadIdx.x == 0) atomicOr(&st->err, GM_ERRF_RLOG_FULL);
+    uint32_t natt = 0;
+    for (uint32_t c = w * P.nbp + blk; c * 64u < nfull; c += P.nbp * (GM_BLOCK / 64u)) {
+        const uint32_t p = c * 64u + lane;
+        if (p >= nfull) break;
+        const uint32_t s = d.pslot[off + p];
+        const GmRec *r = d.rec + s;
+        const RecC rc = rec_c(r);
+        const RecA ra = rec_a(r);
+        const double inc = r->inc;
+        const uint32_t rxg = r->rxg, cell = rc.cell;
+        const uint32_t z = cell / d.nxy, rem = cell - z * d.nxy, y = rem / d.nx, x = rem - y * d.nx;
+        const bool fromB = s >= d.capI;
+        const bool interior = (x - 1u < d.nx - 2u) & (y - 1u < d.ny - 2u) & (z - 1u < d.nz - 2u);
+        Neighbourhood nb;
+        if (interior) nb.load(d, x, y, z);
+        /* rxFrac after the completing addition, while the bits are on their way */
+        const double fin = advanced(ra.frac0, inc, k - ra.s0 + 1u);
+        const uint32_t am = interior ? nb.mask() : face_attempts(d, x, y, z);
         for (uint32_t m = am; m; m &= m - 1u) {
             const uint32_t rk = (uint32_t)__ffs(m) - 1u;
-            uint32_t tx, ty, tz;
-            bool toB;
-            attempt_target(d, q2.w != 0u, q2.x, q2.y, q2.z, (int)rk, tx, ty, tz, toB);
-            if (d.claim[cell_of(d, tx, ty, tz)] == p * 32u + rk) {
-                if (toB) mB |= 1u << rk;
-                else mI |= 1u << rk;
+            uint32_t t = cell + (uint32_t)(dir_dx(rk) + dir_dy(rk) * (int)d.nx + dir_dz(rk) * (int)d.nxy);
+            if (!interior) {
+                uint32_t tx, ty, tz;
+                bool toB;
+                attempt_target(d, true, x, y, z, (int)rk, tx, ty, tz, toB);
+                t = cell_of(d, tx, ty, tz);
+            }
+            atomicMin(&d.claim[t], p * 32u + rk);
+        }
+        natt += (uint32_t)__popc(am);
+        d.pmI[p] = am;
+        par_plane(d, GM_PAR1_CELL)[p] = make_uint4(x | y << 16, z | (fromB ? 1u << 16 : 0u), rc.defg, rxg);
+        reinterpret_cast<double2 *>(par_plane(d, GM_PAR1_FP))[p] = make_double2(fin, rc.P);
+        if (logged) d.rlog[nret + p] = make_uint2(cell, d.ndefg + rxg);
+    }
+    for (int o = 32; o > 0; o >>= 1) natt += __shfl_xor(natt, o, 64);
+    if (lane == 0) satt[w] = natt;
+    __syncthreads();
+    if (threadIdx.x == 0) d.acnt[(j & 1u) * GM_PB + blk] = satt[0] + satt[1] + satt[2] + satt[3];
+}
+
+/* exclusive prefix of v over the block (GM_BLOCK threads) and the total */
+static __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t *sh, uint32_t &tot) {
+    const uint32_t incl = wave_incl_scan(v), w = threadIdx.x >> 6;
+    __syncthreads();
+    if ((threadIdx.x & 63u) == 63u) sh[w] = incl;
+    __syncthreads();
+    uint32_t pre = 0;
+    tot = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < GM_BLOCK / 64; i++) {
+        if (i < w) pre += sh[i];
+        tot += sh[i];
+    }
+    return pre + incl - v;
+}
+
+/* append_to_recycling_*_list (SCORE_Kernel.cpp:4037-4041, :4175-4179): the
+ * recycled slots in ascending order, of which only the first min(winners, cap)
+ * are ever handed out.  Runs beside the decide pass, so the winners are not
+ * counted yet: their upper bound is the step's attempts (1.03 per winner).  A
+ * block takes sweep blocks r, r + nrec, ... and keeps their INACTIVE masks up to
+ * date within the window: the slots the step before handed out leave (the first
+ * rgone of them), the cells completed since the masks were last brought up to date
+ * join, and the part of the slots that lies below the bound is written.  Sweep
+ * blocks beyond it are left alone and catch up when they are reached. */
+static __device__ void recycle_blocks(const GmDev &d, const GmPart &P, uint32_t j, uint32_t r, uint32_t nrec,
+                                      unsigned long long *sm) {
+    __shared__ uint32_t sh[GM_BLOCK / 64], sn[GM_BLOCK / 64][3];
+    const GmWin *win = d.win;
+    const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    const uint32_t rp = (j & 1u) * d.swb, nt = GM_SW_WAVES * P.cpw * GM_SW_TPC;
+    uint32_t *so = reinterpret_cast<uint32_t *>(sm + nt);
+    const uint32_t recI = win->step[j].recLenI, recB = win->step[j].recLenB;
+    uint32_t na = 0, z0 = 0, z1 = 0;
+    for (uint32_t i = 4u * t; i < P.nbp; i += 4u * GM_BLOCK) {
+        const uint4 q = *reinterpret_cast<const uint4 *>(d.acnt + (j & 1u) * GM_PB + i);
+        na += q.x + (i + 1u < P.nbp ? q.y : 0u) + (i + 2u < P.nbp ? q.z : 0u) + (i + 3u < P.nbp ? q.w : 0u);
+    }
+    block_sum3(na, z0, z1, sn);
+    for (uint32_t b = r; b < P.nb; b += nrec) {
+        const bool inB = b >= P.nbI;
+        const uint32_t pre = d.rpre[rp + b], gone = j ? d.rgone[b] : 0u, rec = inB ? recB : recI;
+        const uint32_t bound = na < rec ? na : rec;
+        if (gone == 0u && pre >= bound) continue;
+        const uint32_t nch = inB ? P.chB : P.chI, ch0 = (inB ? b - P.nbI : b) * GM_SW_WAVES * P.cpw;
+        const uint32_t n = (ch0 + GM_SW_WAVES * P.cpw < nch ? GM_SW_WAVES * P.cpw : nch - ch0) * GM_SW_TPC;
+        const uint32_t t0 = ((inB ? P.chI : 0u) + ch0) * GM_SW_TPC, merged = d.rmrg[b];
+        const uint32_t rel0 = ch0 * GM_SW_CHUNK, slot0 = (inB ? d.capI : 0u) + rel0;
+        uint32_t run = 0;
+        __syncthreads();
+        for (uint32_t i0 = 0; i0 < n; i0 += GM_BLOCK) {
+            const uint32_t i = i0 + t;
+            unsigned long long m = i < n ? d.mR[t0 + i] : 0ull;
+            if (run < gone) {
+                const uint32_t c = (uint32_t)__popcll(m);
+                uint32_t tot;
+                const uint32_t before = run + block_excl_scan(c, sh, tot);
+                if (before + c <= gone) m = 0ull;
+                else
+                    for (uint32_t q = before < gone ? gone - before : 0u; q; q--) m &= m - 1ull;
+                run += tot;
+            }
+            if (i < n) sm[i] = m;
+        }
+        __syncthreads();
+        for (uint32_t i = merged; i < j; i++) {
+            const uint32_t nf = d.wcnt[(size_t)i * d.swb + b];
+            const uint32_t *list = d.pslot + win->off[i] + d.wpre[(size_t)i * d.swb + b];
+            for (uint32_t q = t; q < nf; q += GM_BLOCK) {
+                const uint32_t s = list[q] - slot0;
+                atomicOr(&sm[s >> 6], 1ull << (s & 63u));
             }
         }
-        d.pmI[p] = mI;
-        d.pmB[p] = mB;
-        if (mI | mB) reinterpret_cast<double *>(par_plane(d, GM_PAR_FP))[2 * (size_t)p] = parent_fin(d, ps, k);
-        cI += (uint32_t)__popc(mI);
-        cB += (uint32_t)__popc(mB);
-        cA += (uint32_t)__popc(am);
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        cI += __shfl_down(cI, o, 64);
-        cB += __shfl_down(cB, o, 64);
-        cA += __shfl_down(cA, o, 64);
-    }
-    if (threadIdx.x == 0) {
-        d.bcnt[BC_WI * GM_MAX_BLOCKS + blockIdx.x] = cI;
-        d.bcnt[BC_WB * GM_MAX_BLOCKS + blockIdx.x] = cB;
-        d.bcnt[BC_WA * GM_MAX_BLOCKS + blockIdx.x] = cA;
+        __syncthreads();
+        run = pre;
+        for (uint32_t i0 = 0; i0 < n; i0 += GM_BLOCK) {
+            const uint32_t i = i0 + t;
+            const unsigned long long m = i < n ? sm[i] : 0ull;
+            if (i < n) d.mR[t0 + i] = m;
+            uint32_t tot;
+            const uint32_t o = run + block_excl_scan((uint32_t)__popcll(m), sh, tot);
+            if (i < n) so[i] = o;
+            run += tot;
+        }
+        if (t == 0) d.rmrg[b] = j;
+        __syncthreads();
+        /* tile by tile, a lane per slot */
+        uint32_t *out = inB ? d.recB : d.recI;
+        for (uint32_t i = w; i < n; i += GM_SW_WAVES) {
+            const unsigned long long m = sm[i];
+            const uint32_t o = so[i];
+            if (o >= bound) break;
+            const uint32_t q = o + lanemask_lt_count(m);
+            if ((m >> lane & 1ull) && q < bound) out[q] = rel0 + 64u * i + lane;
+        }
     }
 }
 
-/* one block: offsets of every block's winners in each list, the new list lengths
- * (recycled slots first, then appended) */
-__global__ void __launch_bounds__(1024) k_decide_scan(GmDev d, uint32_t nb) {
-    if (d.st->halt) return;
-    uint32_t tot[3];
-    scan_block_counts<3>(d.bcnt + BC_WI * GM_MAX_BLOCKS, nb, tot);
-    if (threadIdx.x == 0) {
-        GmStats *st = d.st;
-        st->winI = tot[0];
-        st->winB = tot[1];
-        st->nattempt = tot[2];
-        /* the commit pass reads the lengths before this step's appends */
-        st->nIold = st->nI;
-        st->nBold = st->nB;
-        if (tot[0] > st->recLenI) st->nI += tot[0] - st->recLenI;
-        if (tot[1] > st->recLenB) st->nB += tot[1] - st->recLenB;
+/* chunks of 64 parents that a block of the decide and commit passes takes */
+static __device__ __forceinline__ uint32_t chunks_per_block(uint32_t nfull, uint32_t nbd) {
+    return ((nfull + 63u) / 64u + nbd - 1u) / nbd;
+}
+
+/* The first nrec blocks write the recycled slots; the rest find which attempts
+ * won.  A wave takes 64 parents at a time and flattens their attempts into a list,
+ * a lane per attempt, so that all claims are loaded together (a loop over each
+ * parent's attempts waits once per attempt of its busiest parent).  Winners as
+ * 26-bit masks per destination list, their counts per 64 parents (Inside << 16 |
+ * Border) and per block, from which the commit pass ranks them. */
+__global__ void __launch_bounds__(GM_BLOCK) k_decide(GmDev d, GmPart P, uint32_t j, uint32_t nrec) {
+    extern __shared__ unsigned long long smask[];
+    struct Wave {
+        uint2 xyz[64];
+        uint32_t mI[64], mB[64];
+        uint16_t wl[26 * 64];
+    };
+    __shared__ Wave sw[GM_BLOCK / 64];
+    __shared__ uint32_t sh[GM_BLOCK / 64][3];
+    const uint32_t halt = d.st->halt, nfull = d.win->full[j];
+    if (halt) return;
+    if (blockIdx.x < nrec) {
+        recycle_blocks(d, P, j, blockIdx.x, nrec, smask);
+        return;
     }
+    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u, blk = blockIdx.x - nrec;
+    const uint32_t nch = (nfull + 63u) / 64u;
+    const uint32_t cpd = chunks_per_block(nfull, P.nbd);
+    const uint32_t c0 = blk * cpd, c1 = c0 + cpd < nch ? c0 + cpd : nch;
+    Wave &W = sw[w];
+    uint32_t tI = 0, tB = 0, dummy = 0;
+    for (uint32_t c = c0 + w; c < c1; c += GM_BLOCK / 64u) {
+        const uint32_t p = c * 64u + lane;
+        const bool valid = p < nfull;
+        const uint32_t am = valid ? d.pmI[p] : 0u;
+        W.xyz[lane] = valid ? *reinterpret_cast<const uint2 *>(par_plane(d, GM_PAR1_CELL) + p) : make_uint2(0u, 0u);
+        W.mI[lane] = 0;
+        W.mB[lane] = 0;
+        const uint32_t na = (uint32_t)__popc(am), incl = wave_incl_scan(na);
+        const uint32_t n = __shfl(incl, 63, 64);
+        uint32_t pos = incl - na;
+        for (uint32_t m = am; m; m &= m - 1u) W.wl[pos++] = (uint16_t)(lane | ((uint32_t)__ffs(m) - 1u) << 8);
+        wave_sync();
+        for (uint32_t i = lane; i < n; i += 64u) {
+            const uint32_t e = W.wl[i], q = e & 0xFFu, rk = e >> 8;
+            const uint2 v = W.xyz[q];
+            uint32_t tx, ty, tz;
+            bool toB;
+            attempt_target(d, (v.y >> 16) != 0u, v.x & 0xFFFFu, v.x >> 16, v.y & 0xFFFFu, (int)rk, tx, ty, tz, toB);
+            if (d.claim[cell_of(d, tx, ty, tz)] == (c * 64u + q) * 32u + rk)
+                atomicOr(toB ? &W.mB[q] : &W.mI[q], 1u << rk);
+        }
+        wave_sync();
+        const uint32_t mI = W.mI[lane], mB = W.mB[lane];
+        if (valid) {
+            d.pmI[p] = mI;
+            d.pmB[p] = mB;
+        }
+        uint32_t cnt = (uint32_t)__popc(mI) << 16 | (uint32_t)__popc(mB);
+        for (int o = 32; o > 0; o >>= 1) cnt += (uint32_t)__shfl_xor((int)cnt, o, 64);
+        if (lane == 0) {
+            d.ccnt[c] = cnt;
+            tI += cnt >> 16;
+            tB += cnt & 0xFFFFu;
+        }
+        wave_sync();
+    }
+    block_sum3(tI, tB, dummy, sh);
+    if (threadIdx.x == 0) d.btot[blk] = make_uint2(tI, tB);
 }
 
 /* New records as omp_infect_OutOfRXFront* write them (SCORE_Kernel.cpp:4281-4310,
  * :4402-4426), slots as omp_getNextFreeSlotIn* hand them out (:3757-3874); then
- * the parents retire as updateFullRX* does it (:4640-4653).  One wave per block
- * takes the block's parents (the partition of k_decide) 64 at a time; their
- * winners are flattened into a list so that every lane commits one infection.
- * Each lane loads its own parent's data with its winner masks and shares it
- * through LDS, and a winner issues its target's grid load and its slot lookup
- * together, so a wave waits on few dependent memory round trips. */
-__global__ void __launch_bounds__(64) k_commit(GmDev d, GmPParams pp, GmSweepArgs A) {
-    __shared__ uint32_t sI[64], sB[64], oI[64], oB[64];
-    __shared__ uint4 sq0[64], sq2[64];
-    __shared__ double sfin[64], sP[64];
-    __shared__ uint16_t wl[26 * 64];
+ * the parents retire as updateFullRX* does it (:4640-4653).  A wave takes 64
+ * parents at a time; their winners are flattened into a list so that every lane
+ * commits one infection.  Each lane loads its own parent's data with its winner
+ * masks and shares it through LDS, and a winner issues its target's grid load and
+ * its slot lookup together, so a wave waits on few dependent memory round trips.
+ * A winner's rank in its list is the winners before it: the blocks of the decide
+ * pass before its own (added up by the block), the chunks before its own in that
+ * block, the parents before its own in the chunk. */
+__global__ void __launch_bounds__(GM_BLOCK) k_commit(GmDev d, GmPParams pp, GmSweepArgs A, GmPart P, uint32_t j,
+                                                     uint32_t top_grain) {
+    struct Wave {
+        uint32_t sI[64], sB[64], oI[64], oB[64];
+        uint4 sq0[64];
+        double sfin[64], sP[64];
+        uint16_t wl[26 * 64];
+    };
+    __shared__ Wave sw[GM_BLOCK / 64];
+    __shared__ uint32_t sh[GM_BLOCK / 64][3];
     GmStats *st = d.st;
-    if (st->halt) return;
-    const uint32_t k = st->kcur;
-    const uint32_t nfull = st->nfullI + st->nfullB;
-    const uint32_t recLenI = st->recLenI, recLenB = st->recLenB;
-    const uint32_t nI = st->nIold, nB = st->nBold;
-    const uint32_t lane = threadIdx.x;
-    uint32_t lo, hi;
-    part_of(nfull, GM_PCHUNK, lo, hi);
-    uint32_t runI = d.bcnt[BC_WI * GM_MAX_BLOCKS + blockIdx.x], runB = d.bcnt[BC_WB * GM_MAX_BLOCKS + blockIdx.x];
-    for (uint32_t batch = lo; batch < hi; batch += 64) {
-        const uint32_t pt = batch + lane;
-        const bool valid = pt < hi;
-        const uint32_t mI = valid ? d.pmI[pt] : 0u, mB = valid ? d.pmB[pt] : 0u;
-        /* this lane's parent: slot, cell, defg, rxg | fin, P | x, y, z, fromB */
-        uint4 q0 = make_uint4(0u, 0u, 0xFFFFFFFFu, 0xFFFFFFFFu), q2 = make_uint4(0u, 0u, 0u, 0u);
-        double2 fp = make_double2(0.0, 0.0);
-        if (valid) {
-            q0 = par_plane(d, GM_PAR_IDS)[pt];
-            fp = reinterpret_cast<const double2 *>(par_plane(d, GM_PAR_FP))[pt];
-            q2 = par_plane(d, GM_PAR_XYZ)[pt];
+    const uint32_t halt = st->halt, nfull = d.win->full[j], nch = (nfull + 63u) / 64u;
+    const GmWinStep ws = d.win->step[j];
+    if (halt) return;
+    const uint32_t k = A.k;
+    const uint32_t cpd = chunks_per_block(nfull, P.nbd), db = blockIdx.x;
+    const uint32_t c0 = db * cpd, c1 = c0 + cpd < nch ? c0 + cpd : nch;
+    if (c0 >= nch) return;
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    /* a lane's parent: winner masks | x | y, z | fromB, defg, rxg | fin, P; the
+     * wave's first chunk is loaded before the winners of earlier blocks are added up */
+    uint32_t mI, mB;
+    uint4 q0;
+    double2 fp;
+    auto load = [&](uint32_t c) {
+        const uint32_t pt = c * 64u + lane;
+        mI = mB = 0;
+        q0 = make_uint4(0u, 0u, 0xFFFFFFFFu, 0xFFFFFFFFu);
+        fp = make_double2(0.0, 0.0);
+        if (c < c1 && pt < nfull) {
+            mI = d.pmI[pt];
+            mB = d.pmB[pt];
+            q0 = par_plane(d, GM_PAR1_CELL)[pt];
+            fp = reinterpret_cast<const double2 *>(par_plane(d, GM_PAR1_FP))[pt];
         }
+    };
+    load(c0 + wv);
+    uint32_t runI = 0, runB = 0, dummy = 0;
+    for (uint32_t i0 = threadIdx.x; i0 < db; i0 += 4u * GM_BLOCK) {
+        uint2 v[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; i++) {
+            v[i] = make_uint2(0u, 0u);
+            if (i0 + i * GM_BLOCK < db) v[i] = d.btot[i0 + i * GM_BLOCK];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; i++) {
+            runI += v[i].x;
+            runB += v[i].y;
+        }
+    }
+    block_sum3(runI, runB, dummy, sh);
+    uint32_t cdone = c0; /* chunks of this block counted in runI, runB */
+    Wave &W = sw[wv];
+    for (uint32_t c = c0 + wv; c < c1; c += GM_BLOCK / 64u) {
+        if (c != c0 + wv) load(c);
+        const bool valid = c * 64u + lane < nfull;
+        uint32_t bI = 0, bB = 0;
+        for (uint32_t i = cdone + lane; i < c; i += 64u) {
+            const uint32_t v = d.ccnt[i];
+            bI += v >> 16;
+            bB += v & 0xFFFFu;
+        }
+        cdone = c;
+        /* the parents' counts: issued here, looked at after the new records */
+        const Retired gone = retire_begin(d, q0, valid);
+        for (int o = 32; o > 0; o >>= 1) {
+            bI += __shfl_xor(bI, o, 64);
+            bB += __shfl_xor(bB, o, 64);
+        }
+        runI += bI;
+        runB += bB;
         const uint32_t cI = (uint32_t)__popc(mI), cB = (uint32_t)__popc(mB);
         /* one scan of both counts (each batch total < 2^16) */
         const uint32_t packed = (cI << 16) | cB;
         const uint32_t incl = wave_incl_scan(packed);
         const uint32_t ex = incl - packed, tot = __shfl(incl, 63, 64);
         const uint32_t totI = tot >> 16, totB = tot & 0xFFFFu;
-        oI[lane] = runI + (ex >> 16);
-        oB[lane] = runB + (ex & 0xFFFFu);
-        sI[lane] = mI;
-        sB[lane] = mB;
-        sq0[lane] = q0;
-        sq2[lane] = q2;
-        sfin[lane] = fp.x;
-        sP[lane] = fp.y;
+        W.oI[lane] = runI + (ex >> 16);
+        W.oB[lane] = runB + (ex & 0xFFFFu);
+        W.sI[lane] = mI;
+        W.sB[lane] = mB;
+        W.sq0[lane] = q0;
+        W.sfin[lane] = fp.x;
+        W.sP[lane] = fp.y;
         /* winners of this parent at [exI + exB, ...) in the flat list, by rank */
         uint32_t pos = (ex >> 16) + (ex & 0xFFFFu);
-        for (uint32_t m = mI | mB; m; m &= m - 1u) wl[pos++] = (uint16_t)(lane | ((uint32_t)__ffs(m) - 1u) << 8);
-        __syncthreads();
+        for (uint32_t m = mI | mB; m; m &= m - 1u) W.wl[pos++] = (uint16_t)(lane | ((uint32_t)__ffs(m) - 1u) << 8);
+        wave_sync();
         const uint32_t nw = totI + totB;
-        for (uint32_t w = lane; w < nw; w += 64) {
-            const uint32_t e = wl[w], j = e & 0xFFu, r = e >> 8, bit = 1u << r;
-            const uint4 pq0 = sq0[j], pq2 = sq2[j];
+        for (uint32_t w = lane; w < nw; w += 64u) {
+            const uint32_t e = W.wl[w], q = e & 0xFFu, r = e >> 8, bit = 1u << r;
+            const uint4 pq0 = W.sq0[q];
             uint32_t tx, ty, tz;
             bool toB;
-            attempt_target(d, pq2.w != 0u, pq2.x, pq2.y, pq2.z, (int)r, tx, ty, tz, toB);
+            attempt_target(d, (pq0.y >> 16) != 0u, pq0.x & 0xFFFFu, pq0.x >> 16, pq0.y & 0xFFFFu, (int)r, tx, ty, tz,
+                           toB);
             const uint32_t t = cell_of(d, tx, ty, tz);
             const uint32_t g = d.grid[t];
             /* rank k into a list takes its k-th recycled slot, else appends */
-            const uint32_t wI = sI[j];
+            const uint32_t wI = W.sI[q];
             const bool intoI = (wI & bit) != 0u;
-            const uint32_t wm = intoI ? wI : sB[j];
-            const uint32_t rank = (intoI ? oI[j] : oB[j]) + (uint32_t)__popc(wm & (bit - 1u));
-            const uint32_t recLen = intoI ? recLenI : recLenB;
+            const uint32_t wm = intoI ? wI : W.sB[q];
+            const uint32_t rank = (intoI ? W.oI[q] : W.oB[q]) + (uint32_t)__popc(wm & (bit - 1u));
+            const uint32_t recLen = intoI ? ws.recLenI : ws.recLenB;
             const uint32_t *recl = intoI ? d.recI : d.recB;
-            const uint32_t rel = rank < recLen ? recl[rank] : (intoI ? nI : nB) + (rank - recLen);
+            const uint32_t rel = rank < recLen ? recl[rank] : (intoI ? ws.nI : ws.nB) + (rank - recLen);
             if (rel >= (intoI ? d.capI : d.capB)) {
                 atomicOr(&st->err, intoI ? GM_ERRF_INSIDE_FULL : GM_ERRF_BORDER_FULL);
                 continue;
             }
             const uint32_t gslot = intoI ? rel : d.capI + rel;
-            infect_one(d, pp, A, k, sfin[j], sP[j], pq0, r, t, g, tx, ty, tz, gslot);
+            infect_one(d, pp, A, k, W.sfin[q], W.sP[q], pq0, r, t, g, tx, ty, tz, gslot);
         }
-        retire_batch(d, q0, valid);
-        runI += totI;
-        runB += totB;
-        __syncthreads();
+        retire_end(d, q0.z, gone, top_grain, &d.win->top_hit);
+        wave_sync();
     }
 }
 
-hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, uint32_t parents_upper,
-                            hipStream_t s, hipEvent_t *ev) {
+hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P,
+                            const GmWindow &w, uint32_t j, hipStream_t s, hipEvent_t *ev) {
     hipError_t e;
-    if ((e = mark(ev, 4, s)) != hipSuccess) return e;
-    k_propose<<<grid_for(parents_upper, GM_BLOCK / GM_PG), GM_BLOCK, 0, s>>>(d);
-    const uint32_t nb = grid_for(parents_upper, GM_PCHUNK);
-    if ((e = mark(ev, 5, s)) != hipSuccess) return e;
-    k_decide<<<nb, 64, 0, s>>>(d);
-    if ((e = mark(ev, 6, s)) != hipSuccess) return e;
-    k_decide_scan<<<1, 1024, 0, s>>>(d, nb);
-    /* the sweep's grid, for the recycling lists */
-    if ((e = mark(ev, 7, s)) != hipSuccess) return e;
-    k_recycle<<<sweep_blocks(a.nI, a.nB), 64, 0, s>>>(d);
-    if ((e = mark(ev, 8, s)) != hipSuccess) return e;
     GmSweepArgs A = a;
-    A.reanchor = 0;
-    k_commit<<<nb, 64, 0, s>>>(d, pp, A);
+    A.k = a.k + j;
+    if ((e = mark(ev, 4, s)) != hipSuccess) return e;
+    k_propose<<<P.nbp + 1u, GM_BLOCK, 0, s>>>(d, P, w, j, A.k);
+    if ((e = mark(ev, 5, s)) != hipSuccess) return e;
+    const uint32_t nrec = P.nb < GM_RECYCLE_BLOCKS ? P.nb : GM_RECYCLE_BLOCKS;
+    /* a sweep block's INACTIVE masks and the offsets of its tiles */
+    const size_t lds = (size_t)GM_SW_WAVES * P.cpw * GM_SW_TPC * (sizeof(unsigned long long) + sizeof(uint32_t));
+    k_decide<<<nrec + P.nbd, GM_BLOCK, lds, s>>>(d, P, j, nrec);
+    for (int i = 6; i <= 8; i++)
+        if ((e = mark(ev, i, s)) != hipSuccess) return e;
+    k_commit<<<P.nbd, GM_BLOCK, 0, s>>>(d, pp, A, P, j, w.top_grain);
     if ((e = mark(ev, 9, s)) != hipSuccess) return e;
     return hipGetLastError();
 }
@@ -831,7 +1370,7 @@ hipError_t gm_launch_resolve_pending(const GmDev &d, const double *vals, uint32_
 /* the stats into the host's pinned mirror (mapped, coherent), word by word:
  * cheaper than a copy command at the end of every window.  Only the filled part
  * of the inline id and key arrays crosses the bus; the host reads no more. */
-__global__ void __launch_bounds__(GM_BLOCK) k_stats_out(GmDev d, uint32_t *out) {
+static __device__ __forceinline__ void copy_stats(const GmDev &d, uint32_t *out) {
     const uint32_t *in = reinterpret_cast<const uint32_t *>(d.st);
     const GmStats *st = d.st;
     const uint32_t nz = st->nzeroed < GM_ZEROED_INLINE ? st->nzeroed : GM_ZEROED_INLINE;
@@ -844,8 +1383,24 @@ __global__ void __launch_bounds__(GM_BLOCK) k_stats_out(GmDev d, uint32_t *out) 
     }
 }
 
+__global__ void __launch_bounds__(GM_BLOCK) k_stats_out(GmDev d, uint32_t *out) { copy_stats(d, out); }
+
 hipError_t gm_launch_stats_out(const GmDev &d, GmStats *out, hipStream_t s) {
     k_stats_out<<<1, GM_BLOCK, 0, s>>>(d, reinterpret_cast<uint32_t *>(out));
+    return hipGetLastError();
+}
+
+/* The end of a window of `launched` steps: its last step is closed, unless the
+ * window halted (the propose pass that halted it closed the step before), and
+ * the stats go to the host's mirror. */
+__global__ void __launch_bounds__(GM_BLOCK) k_window_end(GmDev d, GmPart P, uint32_t launched, uint32_t *out) {
+    if (!d.st->halt && d.st->nexec + 1u == launched) close_step(d, P, launched - 1u, false);
+    __syncthreads();
+    copy_stats(d, out);
+}
+
+hipError_t gm_launch_window_end(const GmDev &d, const GmPart &P, uint32_t launched, GmStats *out, hipStream_t s) {
+    k_window_end<<<1, GM_BLOCK, 0, s>>>(d, P, launched, reinterpret_cast<uint32_t *>(out));
     return hipGetLastError();
 }
 
@@ -1110,13 +1665,11 @@ hipError_t gm_launch_status(const GmDev &d, uint32_t nI, uint32_t nB, uint32_t k
  * (SCORE_Kernel.cpp:6632).  One block: every nucleus of the step claims its
  * cell (the lowest pool id wins), then the winners are ranked in pool order,
  * 1024 at a time, and each record is predicted under the step's scalars. */
-__global__ void __launch_bounds__(1024) k_arrivals(GmDev d, GmSweepArgs A0) {
+__global__ void __launch_bounds__(1024) k_arrivals(GmDev d, GmSweepArgs A) {
     __shared__ uint32_t ws[16][2];
     GmStats *st = d.st;
-    if (st->halt) return;
-    const uint32_t k = st->kcur;
+    const uint32_t k = A.k; /* the first step of a window */
     if (k == 0u || k > d.arr_last) return;
-    const GmSweepArgs A = step_args(d, A0);
     const uint32_t lo = d.arr_off[k], hi = d.arr_off[k + 1u];
     if (lo == hi) return;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
@@ -1191,12 +1744,6 @@ __global__ void __launch_bounds__(1024) k_arrivals(GmDev d, GmSweepArgs A0) {
         st->nB = runB < d.capB ? runB : d.capB;
         st->nplaced = placed;
     }
-}
-
-hipError_t gm_launch_arrivals(const GmDev &d, const GmSweepArgs &a, hipStream_t s) {
-    if (d.arr_last == 0u) return hipSuccess;
-    k_arrivals<<<1, 1024, 0, s>>>(d, a);
-    return hipGetLastError();
 }
 
 /* ----------------------------------------------------------- launch windows

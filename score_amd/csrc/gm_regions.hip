@@ -180,7 +180,7 @@ static __device__ __forceinline__ RgBox rg_box(const GmDev &d, uint32_t r) {
 static __device__ __forceinline__ bool rg_target(const GmDev &d, const RgBox &B, uint32_t l, uint32_t x, uint32_t y,
                                                   uint32_t z, int rk, RgTarget &o) {
     const uint32_t r = l >> 1;
-    int tx = (int)x + c_dx[rk], ty = (int)y + c_dy[rk], tz = (int)z + c_dz[rk];
+    int tx = (int)x + dir_dx(rk), ty = (int)y + dir_dy(rk), tz = (int)z + dir_dz(rk);
     const int nx = (int)d.nx, ny = (int)d.ny, nz = (int)d.nz;
     const int lo0 = B.lo0, lo1 = B.lo1, lo2 = B.lo2, hi0 = B.hi0, hi1 = B.hi1, hi2 = B.hi2;
     o.khi = 0u;
@@ -204,7 +204,7 @@ static __device__ __forceinline__ bool rg_target(const GmDev &d, const RgBox &B,
             /* the target lies in the region or next to it: the neighbour in the
              * direction it left along y (none with one slab along y, whose
              * region spans every y) and z */
-            const int uy = (int)y + c_dy[rk], uz = (int)z + c_dz[rk];
+            const int uy = (int)y + dir_dy(rk), uz = (int)z + dir_dz(rk);
             const int sy = d.npy == 1u ? 0 : (uy < lo1 ? -1 : (uy > hi1 ? 1 : 0));
             const int sz = uz < lo2 ? -1 : (uz > hi2 ? 1 : 0);
             const GmRegion &R = d.reg[r];
@@ -843,7 +843,7 @@ __global__ void __launch_bounds__(64) k_rg_commit(GmDev d, GmPParams pp, GmSweep
             }
             infect_one(d, pp, A, k, sfin[j], sP[j], pq0, r, t, g, o.x, o.y, o.z, bs + rel, o.khi != 0u);
         }
-        retire_batch(d, q0, valid);
+        retire_end(d, q0.z, retire_begin(d, q0, valid));
 #pragma unroll
         for (int c = 0; c < GM_RROWS; c++) run[c] += bt[c];
         __syncthreads();
