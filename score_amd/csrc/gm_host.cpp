@@ -417,8 +417,16 @@ int validate(const score_gm_domain *dom, const score_gm_params *prm) {
     for (uint32_t i = 0; i < dom->n_rxg; i++)
         if (dom->rxg_ori[i] >= dom->n_ori || dom->rxg_site[i] >= N)
             return fail(SCORE_GM_ERR_ARG, "nucleus orientation or site out of range");
+    return 0;
+}
+
+const char *const kBadGrid = "cellgrid holds a non-deformed id";
+
+/* the cell grid's ids, where no device pass checks them (k_grid_init) */
+int validate_grid(const score_gm_domain *dom) {
+    const uint64_t N = (uint64_t)dom->nx * dom->ny * dom->nz;
     for (uint64_t i = 0; i < N; i++)
-        if (dom->cellgrid[i] >= dom->n_defg) return fail(SCORE_GM_ERR_ARG, "cellgrid holds a non-deformed id");
+        if (dom->cellgrid[i] >= dom->n_defg) return fail(SCORE_GM_ERR_ARG, kBadGrid);
     return 0;
 }
 
@@ -1498,11 +1506,8 @@ int score_gm_device_count(void) {
     return usable;
 }
 
-int score_gm_create(const score_gm_domain *dom, const score_gm_params *prm, int device, score_gm_handle **out) {
-    if (!out) return fail(SCORE_GM_ERR_ARG, "null output handle");
-    *out = nullptr;
-    int rc = validate(dom, prm);
-    if (rc) return rc;
+static int create_handle(const score_gm_domain *dom, const score_gm_params *prm, int device, score_gm_handle **out) {
+    int rc;
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || device < 0 || device >= ndev) {
         (void)hipGetLastError();
@@ -1566,9 +1571,9 @@ int score_gm_create(const score_gm_domain *dom, const score_gm_params *prm, int 
     for (uint32_t i = 0; i < d.nrxg; i++)
         memcpy(&h->rxq[4 * (size_t)i], &dom->ori_quat[4 * (size_t)dom->rxg_ori[i]], 4 * sizeof(double));
 
-    /* initial grain counts after solve_REPLACE_CA_STRUCTURE (SCORE_Kernel.cpp:6390-6420) */
+    /* initial grain counts after solve_REPLACE_CA_STRUCTURE (SCORE_Kernel.cpp:6390-6420),
+     * counted on the device */
     std::vector<uint32_t> defcnt(d.ndefg, 0u);
-    for (uint64_t i = 0; i < d.N; i++) defcnt[dom->cellgrid[i]]++;
 
     /* nucleus weights with glibc (calc_mobilityweight, SCORE_GrowthMachine.cpp:152); a
      * nucleus keeps the deformed grain of its site until it arrives, since a cell
@@ -1584,6 +1589,10 @@ int score_gm_create(const score_gm_domain *dom, const score_gm_params *prm, int 
         for (uint32_t k = 0; k < d.nrxg; k++) {
             const uint32_t w = dom->rxg_site[k];
             const uint32_t g = dom->cellgrid[w];
+            if (g >= d.ndefg) {
+                delete h;
+                return fail(SCORE_GM_ERR_ARG, kBadGrid);
+            }
             nucP[k] = mobility_weight(h->p, &h->rxq[4 * (size_t)k], &h->defq[4 * (size_t)g]);
             const uint32_t ks = dom->rxg_step ? dom->rxg_step[k] : 0u;
             if (ks > last) last = ks;
@@ -1722,18 +1731,18 @@ int score_gm_create(const score_gm_domain *dom, const score_gm_params *prm, int 
         hipStream_t s = h->stream;
         HIPCHK(hipMemcpyAsync(d.grid, dom->cellgrid, sizeof(uint32_t) * d.N, hipMemcpyHostToDevice, s));
         HIPCHK(gm_launch_fill_u32(d.claim, GM_FREE_CLAIM, d.N, s));
-        HIPCHK(gm_launch_dmap_init(d, s));
+        HIPCHK(gm_launch_fill_u32(d.defcnt, 0u, d.ndefg, s));
+        HIPCHK(gm_launch_fill_u32((uint32_t *)d.st, 0u, sizeof(GmStats) / 4, s));
+        HIPCHK(gm_launch_grid_init(d, s));
+        HIPCHK(hipMemcpyAsync(defcnt.data(), d.defcnt, sizeof(uint32_t) * d.ndefg, hipMemcpyDeviceToHost, s));
         /* two INACTIVE codes per word (capTot is a multiple of 64) */
         HIPCHK(gm_launch_fill_u32((uint32_t *)d.cstep, 0xFFFFFFFFu, capTot / 2, s));
-        HIPCHK(gm_launch_fill_u64((unsigned long long *)d.rec, 0ull, capTot * (sizeof(GmRec) / 8), s));
         HIPCHK(hipMemcpyAsync(d.rho, dom->defg_rho, sizeof(double) * d.ndefg, hipMemcpyHostToDevice, s));
         HIPCHK(hipMemcpyAsync(d.defq, h->defq.data(), sizeof(double) * 4 * d.ndefg, hipMemcpyHostToDevice, s));
         HIPCHK(hipMemcpyAsync(d.rxq, h->rxq.data(), sizeof(double) * h->rxq.size(), hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemcpyAsync(d.defcnt, defcnt.data(), sizeof(uint32_t) * d.ndefg, hipMemcpyHostToDevice, s));
         HIPCHK(gm_launch_fill_u32(d.rxcnt, 0u, (size_t)d.nrxg + 1, s));
         HIPCHK(gm_launch_fill_u64(d.hkeys, 0ull, d.hcap, s));
         HIPCHK(gm_launch_fill_u64((unsigned long long *)d.hvals, GM_PENDING_TAG, d.hcap, s));
-        HIPCHK(gm_launch_fill_u32((uint32_t *)d.st, 0u, sizeof(GmStats) / 4, s));
         int r2;
         if ((r2 = dalloc(h, &d_site, (size_t)d.nrxg + 1)) || (r2 = dalloc(h, &d_nucP, (size_t)d.nrxg + 1))) return r2;
         if (d.nrxg) {
@@ -1761,6 +1770,7 @@ int score_gm_create(const score_gm_domain *dom, const score_gm_params *prm, int 
     dfree(h, d_nucP);
     dfree(h, d.nflag); dfree(h, d.nI_); dfree(h, d.nB_);
     d.nflag = d.nI_ = d.nB_ = nullptr;
+    if (rc == 0 && (h->hst->err & GM_ERRF_GRID)) rc = fail(SCORE_GM_ERR_ARG, kBadGrid);
     if (rc == 0 && h->hst->err) rc = fail(SCORE_GM_ERR_CAPACITY, "Border front list full while placing nuclei");
     if (rc) {
         free_device(h);
@@ -1793,6 +1803,22 @@ int score_gm_create(const score_gm_domain *dom, const score_gm_params *prm, int 
     if (h->regPmax >= h->Pmax) h->Pmax = h->regPmax;
     *out = h;
     return SCORE_GM_OK;
+}
+
+int score_gm_create(const score_gm_domain *dom, const score_gm_params *prm, int device, score_gm_handle **out) {
+    if (!out) return fail(SCORE_GM_ERR_ARG, "null output handle");
+    *out = nullptr;
+    int rc = validate(dom, prm);
+    if (rc) return rc;
+    rc = create_handle(dom, prm, device, out);
+    /* a domain that could not be set up is refused for its cell grid first, which
+     * the device checks only once the handle's memory is there */
+    if (rc && rc != SCORE_GM_ERR_ARG) {
+        const std::string why = g_last_error;
+        if (validate_grid(dom)) return SCORE_GM_ERR_ARG;
+        g_last_error = why;
+    }
+    return rc;
 }
 
 int score_gm_step(score_gm_handle *h, uint32_t max_steps, int32_t *completed) {
@@ -2085,7 +2111,7 @@ int score_gm_batch_run(score_gm_batch_item *items, uint32_t n, int32_t device, u
 int score_gm_footprint(const score_gm_domain *dom, const score_gm_params *prm, uint64_t *bytes) {
     if (!bytes) return fail(SCORE_GM_ERR_ARG, "null argument");
     int rc = validate(dom, prm);
-    if (rc) return rc;
+    if (rc || (rc = validate_grid(dom))) return rc;
     const uint64_t N = (uint64_t)dom->nx * dom->ny * dom->nz;
     uint64_t capB = 2ull * ((uint64_t)dom->nx * dom->ny + (uint64_t)dom->nx * dom->nz + (uint64_t)dom->ny * dom->nz);
     uint64_t capTot = (N + 63) / 64 * 64 + (capB + 63) / 64 * 64 + 512;

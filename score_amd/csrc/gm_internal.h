@@ -74,6 +74,7 @@ static_assert(GM_CS_HORIZON_MAX <= GM_CS_MOD / 2, "a past code must not wrap int
 #define GM_ERRF_MISSED 0x8u       /* a prediction lies in the past: internal error */
 #define GM_ERRF_KEYS 0x10u        /* more completed cells in one step than infection keys hold (2^27; 2^23 with regions) */
 #define GM_ERRF_RLOG_FULL 0x20u   /* more retirements than the log holds (only cells retired twice can do it) */
+#define GM_ERRF_GRID 0x80u        /* the cell grid holds an id that is no deformed grain's */
 #define GM_ERRF_HALO 0x40u        /* an infection into another region found no halo to park in: internal error */
 
 /* the mobility-weight cache probes at most this many slots from a key's home;
@@ -119,6 +120,7 @@ static inline __host__ __device__ uint32_t gm_tiles_inside(uint32_t nI) {
 #define GM_SW_FOLD 256u           /* sweep blocks up to which no scan pass runs between counting and compaction */
 #define GM_PB 2048u               /* blocks of the propose pass at most */
 #define GM_DB 1024u               /* blocks of the decide and commit passes at most */
+#define GM_GRID_BLOCKS 2048u      /* blocks of the pass over the cell grid at most */
 #define GM_RECYCLE_BLOCKS 2048u   /* blocks of the decide launch that write recycled slots */
 
 /* One front record: SCORE's `cell` (SCORE_Kernel.h:124-137) with rxFrac held as
@@ -437,7 +439,9 @@ struct GmFrontOut {
 };
 hipError_t gm_launch_materialize(const GmDev &d, uint32_t k, uint32_t base, uint32_t n, const GmFrontOut &o,
                                  hipStream_t s);
-hipError_t gm_launch_dmap_init(const GmDev &d, hipStream_t s);
+/* the deformed-cell bitmap, the grains' cell counts (d.defcnt, zeroed before) and
+ * the check of the cell grid; raises GM_ERRF_GRID (d.st, zeroed before) */
+hipError_t gm_launch_grid_init(const GmDev &d, hipStream_t s);
 /* ompshar_defragmentation on the list whose slot 0 is global slot `base`:
  * first_inactive leaves in st->dfirst the first INACTIVE slot in [lo, hi), or hi;
  * move compacts the ACTIVE slots of (first, nnever) to [first, first+count) through
