@@ -85,24 +85,25 @@ static __device__ __forceinline__ uint32_t hash_slot(unsigned long long k, uint3
 
 /* largest |component| over the six Grimmer candidates of q_def^-1 * q_rx
  * (SCORE_Math.cpp:230-239, :558-608); only + - * fabs and compares, so the
- * value is bit-identical to the host's. */
-static __device__ double grimmer_omega(const double *p, const double *q, double fac) {
+ * value is bit-identical to the host's.  The 24 candidates are the sums and
+ * differences of two components times 1/sqrt(2), of all four (left to right) times
+ * 1/2, and the components.  Rounding is monotone and symmetric, so no sign pattern
+ * exceeds the one that adds the magnitudes, and among the pairs the two largest
+ * magnitudes win: three candidates remain (24 kept 48 registers alive, which held
+ * the commit pass at 12 waves a CU). */
+static __device__ __forceinline__ double grimmer_omega(const double *p, const double *q, double fac) {
     double m0 = q[0], m1 = -1.0 * q[1], m2 = -1.0 * q[2], m3 = -1.0 * q[3];
-    double a = m0 * p[0] - m1 * p[1] - m2 * p[2] - m3 * p[3];
-    double b = p[0] * m1 + m0 * p[1] + (m2 * p[3] - m3 * p[2]);
-    double c = p[0] * m2 + m0 * p[2] + (-(m1 * p[3]) + m3 * p[1]);
-    double d = p[0] * m3 + m0 * p[3] + (m1 * p[2] - m2 * p[1]);
-    double v[24];
-    v[0] = (a + b) * fac; v[1] = (a - b) * fac; v[2] = (c + d) * fac; v[3] = (c - d) * fac;
-    v[4] = (a + c) * fac; v[5] = (a - c) * fac; v[6] = (b + d) * fac; v[7] = (b - d) * fac;
-    v[8] = (a + d) * fac; v[9] = (a - d) * fac; v[10] = (b + c) * fac; v[11] = (b - c) * fac;
-    v[12] = (a + b + c + d) * 0.5; v[13] = (a + b - c - d) * 0.5; v[14] = (a - b + c - d) * 0.5; v[15] = (a - b - c + d) * 0.5;
-    v[16] = (a + b + c - d) * 0.5; v[17] = (a + b - c + d) * 0.5; v[18] = (a - b + c + d) * 0.5; v[19] = (a - b - c - d) * 0.5;
-    v[20] = a; v[21] = b; v[22] = c; v[23] = d;
-    double omega = 0.0;
-#pragma unroll
-    for (int i = 0; i < 24; i++)
-        if (fabs(v[i]) > omega) omega = fabs(v[i]);
+    const double a = fabs(m0 * p[0] - m1 * p[1] - m2 * p[2] - m3 * p[3]);
+    const double b = fabs(p[0] * m1 + m0 * p[1] + (m2 * p[3] - m3 * p[2]));
+    const double c = fabs(p[0] * m2 + m0 * p[2] + (-(m1 * p[3]) + m3 * p[1]));
+    const double d = fabs(p[0] * m3 + m0 * p[3] + (m1 * p[2] - m2 * p[1]));
+    const double ab = a > b ? a : b, ba = a > b ? b : a, cd = c > d ? c : d, dc = c > d ? d : c;
+    const double l1 = ab > cd ? ab : cd;
+    const double lo = ab > cd ? cd : ab, in = ab > cd ? ba : dc;
+    const double l2 = lo > in ? lo : in;
+    const double two = (l1 + l2) * fac, four = (((a + b) + c) + d) * 0.5;
+    double omega = l1 > two ? l1 : two;
+    if (four > omega) omega = four;
     return omega;
 }
 
@@ -432,34 +433,43 @@ static_assert(GM_PG == 4 || GM_PG == 8 || GM_PG == 16, "lanes per parent");
  * complete before the window ends, and is predicted then.  fresh_weight: the
  * weight is looked up whatever the deformed grain, as the halo synchronisation
  * does (SCORE_Kernel.cpp:4853). */
-static __device__ __forceinline__ void infect_one(const GmDev &d, const GmPParams &pp, const GmSweepArgs &A,
-                                                  uint32_t k, double pfin, double pP, const uint4 &pq0, uint32_t r,
-                                                  uint32_t t, uint32_t g, uint32_t tx, uint32_t ty, uint32_t tz,
-                                                  uint32_t gslot, bool fresh_weight = false) {
+struct NewCell {
+    double carry, P, inc;
+    uint32_t inf;
+    gm_cs_t cs;
+};
+static __device__ __forceinline__ NewCell new_cell(const GmDev &d, const GmPParams &pp, const GmSweepArgs &A, uint32_t k,
+                                                   double pfin, double pP, const uint4 &pq0, uint32_t r, uint32_t g,
+                                                   bool fresh_weight = false) {
     const double overshoot = pfin - 1.0;
     const int cls = dir_class(r);
-    const double carry = cls == 1 ? overshoot * 0.0682 : (cls == 2 ? overshoot * 0.0542 : overshoot * 0.0484);
-    double Pn = pP;
-    if (fresh_weight || pq0.z != g) Pn = pair_weight(d, pp, pq0.w, g);
-    const uint32_t inf = dir_code(r);
-    double inc = 0.0;
-    gm_cs_t cs = (gm_cs_t)GM_CS_DEFERRED;
-    if (!is_pending(Pn)) {
-        const uint32_t step = predict_values(d, A, k + 1u, carry, Pn, g, inf, inc);
+    NewCell n;
+    n.carry = cls == 1 ? overshoot * 0.0682 : (cls == 2 ? overshoot * 0.0542 : overshoot * 0.0484);
+    n.P = pP;
+    if (fresh_weight || pq0.z != g) n.P = pair_weight(d, pp, pq0.w, g);
+    n.inf = dir_code(r);
+    n.inc = 0.0;
+    n.cs = (gm_cs_t)GM_CS_DEFERRED;
+    if (!is_pending(n.P)) {
+        const uint32_t step = predict_values(d, A, k + 1u, n.carry, n.P, g, n.inf, n.inc);
         /* the window's lists of completed cells were made at its start */
         if (step < A.wend) atomicOr(&d.st->err, GM_ERRF_MISSED);
-        cs = cs_code(d, step, k + 1u);
+        n.cs = cs_code(d, step, k + 1u);
     }
+    return n;
+}
+static __device__ __forceinline__ void put_cell(const GmDev &d, uint32_t k, const NewCell &n, const uint4 &pq0, uint32_t t,
+                                                uint32_t g, uint32_t tx, uint32_t ty, uint32_t tz, uint32_t gslot) {
     GmRec *rec = d.rec + gslot;
-    rec_set_a(rec, carry, k + 1u, inf);
-    rec_set_b(rec, inc);
-    rec_set_c(rec, Pn, t, g);
+    rec_set_a(rec, n.carry, k + 1u, n.inf);
+    rec_set_b(rec, n.inc);
+    rec_set_c(rec, n.P, t, g);
     *reinterpret_cast<uint4 *>(&rec->rxg) = make_uint4(pq0.w, 0u, 0u, 0u);
-    d.cstep[gslot] = cs;
+    d.cstep[gslot] = n.cs;
     /* DEFERRED cells go to the deferred list with one atomic per wave: the
      * list's counter is a single address, and atomics on one address are
      * served one after another */
-    const bool deferred = cs == GM_CS_DEFERRED;
+    const bool deferred = n.cs == GM_CS_DEFERRED;
     const uint64_t dm = __ballot(deferred);
     if (dm) {
         const uint32_t lead = (uint32_t)__ffsll((long long)dm) - 1u;
@@ -476,52 +486,55 @@ static __device__ __forceinline__ void infect_one(const GmDev &d, const GmPParam
 
 
 /* Retires a batch of parents (updateFullRX*, SCORE_Kernel.cpp:4640-4653): each
- * lane's parent, q0 = (slot, cell, defg, rxg), moves a cell from its deformed
- * grain's count to its nucleus' (its slot reads as INACTIVE from the next step
- * on by its completion code, cs_inactive).  A deformed grain losing its
- * last cell is reported so the host can update rhomax (update_myrhomax,
- * SCORE_RecoveryModels.cpp:146-165).  Consecutive parents often share their
- * nucleus and deformed grain (siblings), so each run of equal ids among
- * neighbouring lanes makes one atomic.  Every lane of the wave takes part in
- * retire_begin, which issues the atomics; retire_end looks at what they returned,
- * so that other work can lie between.  top_hit, if given, is set when top_grain loses its last cell. */
-struct Retired {
-    uint32_t n, old;            /* cells this lane took from its deformed grain's count (0: none), the count before */
-};
-static __device__ __forceinline__ Retired retire_begin(const GmDev &d, const uint4 &q0, bool valid) {
+ * lane's parent moves a cell from its deformed grain g's count to its nucleus r's
+ * (its slot reads as INACTIVE from the next step on by its completion code,
+ * cs_inactive).  Consecutive parents often share their nucleus and deformed grain
+ * (siblings), so each run of equal ids among neighbouring lanes makes one atomic.
+ * runs: this lane's run length of g (0: the lane starts none), and the nucleus'
+ * count is done.  Every lane of the wave takes part. */
+static __device__ __forceinline__ uint32_t retire_runs(const GmDev &d, uint32_t g, uint32_t r, bool valid) {
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t g = q0.z, r = q0.w;
     const uint32_t gprev = __shfl_up(g, 1, 64), rprev = __shfl_up(r, 1, 64);
     const uint64_t gstart = __ballot(valid && (lane == 0 || g != gprev));
     const uint64_t rstart = __ballot(valid && (lane == 0 || r != rprev));
     const uint64_t vmask = __ballot(valid);
-    Retired ret = {0u, 0u};
-    if (!valid) return ret;
+    if (!valid) return 0u;
     const uint64_t above = lane == 63 ? 0ull : (~0ull << (lane + 1)); /* lanes after this one */
-    if ((gstart >> lane) & 1ull) {
-        /* run length: up to the next run start or the last valid lane */
-        const uint64_t nxt = (gstart | ~vmask) & above;
-        const uint32_t end = nxt ? (uint32_t)__ffsll((long long)nxt) - 1u : 64u;
-        ret.n = end - lane;
-        ret.old = atomicSub(&d.defcnt[g], ret.n);
-    }
     if ((rstart >> lane) & 1ull) {
+        /* run length: up to the next run start or the last valid lane */
         const uint64_t nxt = (rstart | ~vmask) & above;
         const uint32_t end = nxt ? (uint32_t)__ffsll((long long)nxt) - 1u : 64u;
         atomicAdd(&d.rxcnt[r], end - lane);
     }
-    return ret;
+    if (!((gstart >> lane) & 1ull)) return 0u;
+    const uint64_t nxt = (gstart | ~vmask) & above;
+    return (nxt ? (uint32_t)__ffsll((long long)nxt) - 1u : 64u) - lane;
 }
-static __device__ __forceinline__ void retire_end(const GmDev &d, uint32_t g, const Retired &ret,
-                                                  uint32_t top_grain = 0xFFFFFFFFu, uint32_t *top_hit = nullptr) {
+
+/* One region: the deformed grains' counts are taken down in GM_SUBS parts each,
+ * part `sub` by this block.  Atomics on one address are served one after another,
+ * and a step takes some 30 to 50 cells from every grain: with one counter a grain,
+ * whose old value told when the grain was exhausted, the commit pass took 21.6 us
+ * at 320^3 and 11.8 at 100^3, without it 13.5 and 8.8.  Which grains are exhausted
+ * is only asked of the one that sets rhomax: it is counted per step
+ * (k_decide, k_commit), and its successor found when it is gone (k_window_end). */
+static __device__ __forceinline__ void retire(const GmDev &d, uint32_t g, uint32_t r, bool valid, uint32_t sub) {
+    const uint32_t n = retire_runs(d, g, r, valid);
+    if (n) atomicAdd(&d.defsub[(size_t)sub * d.ndefg + g], n);
+}
+
+/* Several regions: a deformed grain losing its last cell is reported so the host
+ * can update rhomax (update_myrhomax, SCORE_RecoveryModels.cpp:146-165). */
+static __device__ __forceinline__ void retire_batch(const GmDev &d, const uint4 &q0, bool valid) {
     GmStats *st = d.st;
-    if (!ret.n) return;
-    if (ret.old == ret.n) {
+    const uint32_t g = q0.z, n = retire_runs(d, g, q0.w, valid);
+    if (!n) return;
+    const uint32_t old = atomicSub(&d.defcnt[g], n);
+    if (old == n) {
         const uint32_t i = atomicAdd(&st->nzeroed, 1u);
         if (i < GM_ZEROED_INLINE) st->zeroed_ids[i] = g;
         if (i < d.ndefg) d.zlist[i] = g;
-        if (top_hit && g == top_grain) *top_hit = 1u;
-    } else if (ret.old < ret.n) {
+    } else if (old < n) {
         /* only a cell held by two records retires twice; the count wraps
          * as SCORE's uint32 does and the host re-reads them all */
         st->cwrap = 1u;

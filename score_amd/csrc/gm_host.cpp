@@ -191,6 +191,7 @@ struct score_gm_handle {
     std::vector<double> rho0_host;     /* mydefgpool[].rho0 (Michalak-Paxton recovery) */
     bool rho_changed = false;          /* recovery changed rho: upload and re-anchor */
     std::vector<uint32_t> rho_order;
+    std::vector<uint32_t> rho_pos;     /* each grain's place in it (staging for the device) */
     std::vector<uint8_t> alive;
     size_t rho_top = 0;
     std::vector<uint32_t> zbuf;
@@ -209,6 +210,7 @@ struct score_gm_handle {
     std::vector<GmRegion> reg;
     std::vector<uint32_t> lbase, lcap, lrcap, lrbase;
     uint32_t last_full = 0xFFFFFFFFu; /* most cells completed in one step of the last window */
+    uint32_t last_csz = 48;           /* parents per chunk after its last step */
 };
 
 namespace {
@@ -316,11 +318,11 @@ void dfree(score_gm_handle *h, void *p) {
 
 void free_device(score_gm_handle *h) {
     GmDev &d = h->d;
-    void *ptrs[] = {d.grid, d.claim, d.rlog, d.dmap, d.cstep, d.rec, d.pslot, d.dlist,
+    void *ptrs[] = {d.cell, d.pmA, d.gatt, d.rlog, d.dmap, d.cstep, d.rec, d.pslot, d.dlist,
                     d.par, d.recI, d.recB, d.mF, d.mR, d.pmI, d.pmB, d.bcnt, d.rho, d.defq,
                     d.rxq, d.defcnt, d.rxcnt, d.zlist, d.hkeys, d.hvals, d.pend_slot, d.pend_key, d.nflag, d.nI_, d.nB_,
                     d.scan_bsum, d.st, d.arr_ids, d.arr_off, d.nsite, d.nucP,
-                    d.win, d.wcnt, d.wpre, d.wwave, d.rcnt, d.rpre, d.rgone, d.rmrg, d.acnt, d.btot, d.ccnt,
+                    d.win, d.wcnt, d.wpre, d.wwave, d.rcnt, d.rpre, d.rgone, d.rmrg, d.acnt, d.btot, d.btop, d.ccnt, d.defsub, d.rorder, d.rpos,
                     d.reg, d.pmH, d.L.base, d.L.cap, d.L.rcap, d.L.rbase, d.L.n, d.L.nold, d.L.rlen,
                     d.L.win, d.L.occ, d.L.tile, d.L.tile_s, d.L.par, d.L.rst, d.L.rbuf, d.L.rs, d.L.bstart, d.L.breg,
                     d.L.hoff, d.plist};
@@ -834,14 +836,14 @@ int ensure_step_capacity(score_gm_handle *h) {
     if (parents > d.parentCap) {
         uint32_t nc = std::max<uint32_t>(parents, d.parentCap + d.parentCap / 2);
         dfree(h, d.pmI); dfree(h, d.pmB); dfree(h, d.pslot); dfree(h, d.par); dfree(h, d.pmH); dfree(h, d.plist);
-        dfree(h, d.ccnt);
-        d.pmI = d.pmB = d.pslot = d.pmH = d.plist = d.ccnt = nullptr;
+        dfree(h, d.ccnt); dfree(h, d.pmA);
+        d.pmA = d.pmI = d.pmB = d.pslot = d.pmH = d.plist = d.ccnt = nullptr;
         d.par = nullptr;
         d.parentCap = 0;
         int rc;
         if ((rc = dalloc(h, &d.pmI, nc)) || (rc = dalloc(h, &d.pmB, nc)) || (rc = dalloc(h, &d.pslot, nc)) ||
             (rc = dalloc(h, &d.par, (size_t)(d.nreg > 1 ? GM_PAR_PLANES : GM_PAR1_PLANES) * nc)) || (d.nreg > 1 && ((rc = dalloc(h, &d.pmH, nc)) || (rc = dalloc(h, &d.plist, nc)))) ||
-            (d.nreg <= 1 && (rc = dalloc(h, &d.ccnt, (size_t)nc / 64 + 1))))
+            (d.nreg <= 1 && ((rc = dalloc(h, &d.ccnt, (size_t)nc / 16 + 1)) || (rc = dalloc(h, &d.pmA, nc)))))
             return rc;
         d.parentCap = nc;
     }
@@ -982,6 +984,29 @@ int set_list_lengths(score_gm_handle *h, const std::vector<uint32_t> &n) {
     return 0;
 }
 
+/* one region: the grains' order of rho to the device */
+int upload_order(score_gm_handle *h) {
+    GmDev &d = h->d;
+    if (d.nreg > 1) return 0;
+    h->rho_pos.resize(d.ndefg);
+    for (uint32_t i = 0; i < d.ndefg; i++) h->rho_pos[h->rho_order[i]] = i;
+    HIPCHK(hipMemcpyAsync(d.rorder, h->rho_order.data(), sizeof(uint32_t) * d.ndefg, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(hipMemcpyAsync(d.rpos, h->rho_pos.data(), sizeof(uint32_t) * d.ndefg, hipMemcpyHostToDevice, h->stream));
+    return 0;
+}
+
+/* which deformed grains hold cells, from their counts on the device */
+int refresh_alive(score_gm_handle *h) {
+    GmDev &d = h->d;
+    std::vector<uint32_t> cnt(d.ndefg);
+    if (d.nreg <= 1) HIPCHK(gm_launch_fold_counts(d, h->stream));
+    HIPCHK(hipMemcpyAsync(cnt.data(), d.defcnt, sizeof(uint32_t) * d.ndefg, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(hipStreamSynchronize(h->stream));
+    for (uint32_t g = 0; g < d.ndefg; g++) h->alive[g] = cnt[g] > 0 ? 1 : 0;
+    h->rho_top = 0;
+    return 0;
+}
+
 /* ompshar_defragmentation (SCORE_Kernel.cpp:3877-3934) of the list whose slot
  * 0 is global slot `base`: capacity `cap`, nextSlotNeverActive `nnever`. */
 int defragment_list(score_gm_handle *h, uint32_t base, uint32_t cap, uint32_t &nnever) {
@@ -1118,6 +1143,7 @@ int log_grainevo(score_gm_handle *h, uint32_t sv) {
     GmDev &d = h->d;
     const size_t ng = (size_t)d.ndefg + d.nrxg;
     const size_t off = h->glog_counts.size();
+    if (d.nreg <= 1) HIPCHK(gm_launch_fold_counts(d, h->stream));
     h->glog_counts.resize(off + ng);
     HIPCHK(hipMemcpyAsync(h->glog_counts.data() + off, d.defcnt, sizeof(uint32_t) * d.ndefg, hipMemcpyDeviceToHost,
                           h->stream));
@@ -1183,6 +1209,7 @@ GmPart window_part(const score_gm_handle *h, uint32_t nI, uint32_t nB, uint32_t 
     const uint64_t slots = (uint64_t)nI + nB, est = std::min<uint64_t>(slots, 2ull * h->last_full + 1024u);
     P.nbp = (uint32_t)std::min<uint64_t>(GM_PB, est / 64 + 1);
     P.nbd = std::min<uint32_t>(GM_DB, P.nbp);
+    P.csz0 = h->last_csz;
     return P;
 }
 
@@ -1255,6 +1282,7 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
     memset(&w, 0, sizeof(w));
     w.xstop = window_xstop(h);
     w.top_grain = h->rho_top < h->rho_order.size() ? h->rho_order[h->rho_top] : 0xFFFFFFFFu;
+    w.top_pos = (uint32_t)std::min<size_t>(h->rho_top, d.ndefg);
     w.pend_limit = (uint32_t)std::min<uint64_t>(0xFFFFFFFFull, (uint64_t)d.hcap / 2 > h->hcount ? (uint64_t)d.hcap / 2 - h->hcount : 0ull);
     w.defer = W > 1 ? 1u : 0u;
     hipEvent_t *ev = prof ? h->ev : nullptr;
@@ -1270,7 +1298,7 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
     if (d.nreg > 1)
         e = gm_launch_window_begin(d, h->step, h->Xcells, h->stream);
     else
-        e = gm_launch_window(d, P, a, na != 0, h->Xcells, h->stream, ev);
+        e = gm_launch_window(d, P, a, w, na != 0, h->Xcells, h->stream, ev);
     if (e != hipSuccess) return h->err = hip_fail(e, "growth step");
     uint32_t launched = 0;
     for (uint32_t j = 0; j < W; j++) {
@@ -1289,7 +1317,7 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
             return h->err = hip_fail(e, "growth step");
     }
     e = d.nreg > 1 ? gm_launch_stats_out(d, h->hst_dev, h->stream)
-                   : gm_launch_window_end(d, P, launched, h->hst_dev, h->stream);
+                   : gm_launch_window_end(d, P, launched, w.top_pos, h->hst_dev, h->stream);
     if (e != hipSuccess || (e = hipStreamSynchronize(h->stream)) != hipSuccess)
         return h->err = hip_fail(e, "growth step");
     h->last_sp = sp;
@@ -1337,6 +1365,7 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
         const GmStepRow &last = st.rows[nexec - 1];
         h->nI = last.nI;
         h->nB = last.nB;
+        h->last_csz = gm_chunk_size(last.nfullI + last.nfullB, last.winI + last.winB);
         h->last_full = 0;
         for (uint32_t j = 0; j < nexec; j++) h->last_full = std::max(h->last_full, st.rows[j].nfullI + st.rows[j].nfullB);
     }
@@ -1397,7 +1426,7 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
         if (j + 1 == nexec) {
             /* grains that lost their last cell leave the rhomax search; before the
              * last step of a window none of them was the one that sets rhomax */
-            if (st.nzeroed) {
+            if (d.nreg > 1 && st.nzeroed) {
                 const uint32_t *ids = st.zeroed_ids;
                 if (st.nzeroed > GM_ZEROED_INLINE) {
                     h->zbuf.resize(st.nzeroed);
@@ -1409,24 +1438,23 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
                 }
                 for (uint32_t i = 0; i < std::min(st.nzeroed, d.ndefg); i++) h->alive[ids[i]] = 0;
             }
-            if (st.cwrap) {
-                /* a count went below zero and wrapped: cellcount > 0 again, as in SCORE */
-                std::vector<uint32_t> cnt(d.ndefg);
-                if ((e = hipMemcpyAsync(cnt.data(), d.defcnt, sizeof(uint32_t) * d.ndefg, hipMemcpyDeviceToHost,
-                                        h->stream)) != hipSuccess ||
-                    (e = hipStreamSynchronize(h->stream)) != hipSuccess)
-                    return h->err = hip_fail(e, "deformed grain counts");
-                for (uint32_t g = 0; g < d.ndefg; g++) h->alive[g] = cnt[g] > 0 ? 1 : 0;
-                h->rho_top = 0;
-            }
+            /* one region: those before the successor of the grain that set rhomax */
+            if (d.nreg <= 1 && st.top_hit)
+                for (uint32_t i = w.top_pos; i < std::min(st.top_next, d.ndefg); i++) h->alive[h->rho_order[i]] = 0;
+            /* a count went below zero and wrapped: cellcount > 0 again, as in SCORE */
+            if (st.cwrap && (rc = refresh_alive(h))) return h->err = rc;
         }
         if (h->p.recovery_mode != 0) {
             /* update_mydgoptimize_rho (SCORE_RecoveryModels.cpp:128-135): re-sorted by the
              * current rho; a stable sort leaves an ordered list as it is, so an
              * order that recovery kept (every rho scaled alike) is not sorted again */
             auto desc = [&](uint32_t a, uint32_t b) { return h->rho_host[a] > h->rho_host[b]; };
-            if (!std::is_sorted(h->rho_order.begin(), h->rho_order.end(), desc))
+            if (!std::is_sorted(h->rho_order.begin(), h->rho_order.end(), desc)) {
+                /* one region: only the first grain of the old order is known to hold cells */
+                if (d.nreg <= 1 && (rc = refresh_alive(h))) return h->err = rc;
                 std::stable_sort(h->rho_order.begin(), h->rho_order.end(), desc);
+                if ((rc = upload_order(h))) return h->err = rc;
+            }
             h->rho_top = 0;
         }
         update_rhomax(h);
@@ -1660,7 +1688,7 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
     if (multi)
         for (uint32_t r = 0; r < d.nreg; r++) capBsum += h->lcap[2 * r + 1];
     d.rlogCap = d.N + capBsum + 4096u;
-    if ((rc = dalloc(h, &d.grid, d.N)) || (rc = dalloc(h, &d.claim, d.N)) ||
+    if ((rc = dalloc(h, &d.cell, d.N)) ||
         (rc = dalloc(h, &d.rlog, d.rlogCap)) ||
         (rc = dalloc(h, &d.cstep, capTot)) ||
         (rc = dalloc(h, &d.rec, capTot)) ||
@@ -1683,12 +1711,17 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
     }
     if (!multi) {
         d.swb = sweep_block_rows(d);
+        d.gchunks = (uint32_t)std::min<uint64_t>(GM_GCHUNKS, d.N / 16 + 1);
         if ((rc = dalloc(h, &d.win, 1)) || (rc = dalloc(h, &d.wcnt, (size_t)(GM_WMAX + 1) * d.swb)) ||
             (rc = dalloc(h, &d.wpre, (size_t)(GM_WMAX + 1) * d.swb)) ||
             (rc = dalloc(h, &d.wwave, (size_t)GM_SW_WAVES * GM_WMAX * d.swb)) ||
             (rc = dalloc(h, &d.rcnt, 2 * (size_t)d.swb)) || (rc = dalloc(h, &d.rpre, 2 * (size_t)d.swb)) ||
             (rc = dalloc(h, &d.rgone, d.swb)) || (rc = dalloc(h, &d.rmrg, d.swb)) || (rc = dalloc(h, &d.acnt, 2 * GM_PB)) ||
-            (rc = dalloc(h, &d.btot, GM_DB)) || (rc = dalloc(h, &d.ccnt, (size_t)d.parentCap / 64 + 1))) {
+            (rc = dalloc(h, &d.btot, GM_DB)) || (rc = dalloc(h, &d.ccnt, (size_t)d.parentCap / 16 + 1)) ||
+            (rc = dalloc(h, &d.pmA, d.parentCap)) || (rc = dalloc(h, &d.btop, GM_DB)) ||
+            (rc = dalloc(h, &d.defsub, (size_t)GM_SUBS * d.ndefg)) || (rc = dalloc(h, &d.rorder, d.ndefg)) ||
+            (rc = dalloc(h, &d.rpos, d.ndefg)) ||
+            (rc = dalloc(h, &d.gatt, (size_t)GM_GATT * d.gchunks))) {
             free_device(h);
             delete h;
             return rc;
@@ -1729,11 +1762,13 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
     double *d_nucP = nullptr;
     auto setup = [&]() -> int {
         hipStream_t s = h->stream;
-        HIPCHK(hipMemcpyAsync(d.grid, dom->cellgrid, sizeof(uint32_t) * d.N, hipMemcpyHostToDevice, s));
-        HIPCHK(gm_launch_fill_u32(d.claim, GM_FREE_CLAIM, d.N, s));
+        /* the grid arrives in the record array, which nothing uses yet */
+        uint32_t *src = reinterpret_cast<uint32_t *>(d.rec);
+        HIPCHK(hipMemcpyAsync(src, dom->cellgrid, sizeof(uint32_t) * d.N, hipMemcpyHostToDevice, s));
         HIPCHK(gm_launch_fill_u32(d.defcnt, 0u, d.ndefg, s));
+        if (!multi) HIPCHK(gm_launch_fill_u32(d.defsub, 0u, (size_t)GM_SUBS * d.ndefg, s));
         HIPCHK(gm_launch_fill_u32((uint32_t *)d.st, 0u, sizeof(GmStats) / 4, s));
-        HIPCHK(gm_launch_grid_init(d, s));
+        HIPCHK(gm_launch_grid_init(d, src, s));
         HIPCHK(hipMemcpyAsync(defcnt.data(), d.defcnt, sizeof(uint32_t) * d.ndefg, hipMemcpyDeviceToHost, s));
         /* two INACTIVE codes per word (capTot is a multiple of 64) */
         HIPCHK(gm_launch_fill_u32((uint32_t *)d.cstep, 0xFFFFFFFFu, capTot / 2, s));
@@ -1792,6 +1827,11 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
     std::stable_sort(h->rho_order.begin(), h->rho_order.end(),
                      [&](uint32_t a, uint32_t b) { return h->rho_host[a] > h->rho_host[b]; });
     h->rho_top = 0;
+    if ((rc = upload_order(h))) {
+        free_device(h);
+        delete h;
+        return rc;
+    }
     update_rhomax(h);
     h->t = 0.0; h->X = 0.0; h->Xcells = 0.0; h->step = 0;
     update_temperature(h);
@@ -1875,7 +1915,6 @@ int score_gm_get_grainmap(score_gm_handle *h, uint32_t *out, int32_t encoding) {
     int rc = dalloc(h, &tmp, h->d.N);
     if (rc) return rc;
     auto copy = [&]() -> int {
-        HIPCHK(hipMemcpyAsync(tmp, h->d.grid, sizeof(uint32_t) * h->d.N, hipMemcpyDeviceToDevice, h->stream));
         HIPCHK(gm_launch_overlay_infected(h->d, h->nI, h->nB, h->step, tmp, h->stream));
         HIPCHK(hipMemcpyAsync(out, tmp, sizeof(uint32_t) * h->d.N, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
@@ -1892,6 +1931,7 @@ int score_gm_get_grainmap(score_gm_handle *h, uint32_t *out, int32_t encoding) {
 int score_gm_get_counts(score_gm_handle *h, uint32_t *defg_counts, uint32_t *rxg_counts) {
     if (!h) return fail(SCORE_GM_ERR_ARG, "null handle");
     HIPCHK(hipSetDevice(h->device));
+    if (defg_counts && h->d.nreg <= 1) HIPCHK(gm_launch_fold_counts(h->d, h->stream));
     if (defg_counts)
         HIPCHK(hipMemcpyAsync(defg_counts, h->d.defcnt, sizeof(uint32_t) * h->d.ndefg, hipMemcpyDeviceToHost, h->stream));
     if (rxg_counts && h->d.nrxg)
@@ -2124,7 +2164,9 @@ int score_gm_footprint(const score_gm_domain *dom, const score_gm_params *prm, u
     if (prm->n_regions <= 1) {
         /* the window sweep's tables */
         const uint64_t rows = std::max<uint64_t>(capTot / (GM_SW_CHUNK * GM_SW_WAVES * GM_SW_MAXCPW) + 67, GM_SW_BLOCKS);
-        b += sizeof(GmWin) + 4 * rows * (2 * (GM_WMAX + 1) + GM_SW_WAVES * GM_WMAX + 6) + 16 * GM_PB + front / 16 + 4;
+        b += sizeof(GmWin) + 4 * rows * (2 * (GM_WMAX + 1) + GM_SW_WAVES * GM_WMAX + 6) + 16 * GM_PB + 4 * (front + front / 16) +
+             (4ull * GM_SUBS + 8) * dom->n_defg +
+             4ull * GM_GATT * std::min<uint64_t>(GM_GCHUNKS, N / 16 + 1);
     }
     if (prm->n_regions > 1) {
         /* the lists of every region (build_regions), halo masks and tables */
@@ -2145,7 +2187,7 @@ int score_gm_footprint(const score_gm_domain *dom, const score_gm_params *prm, u
         b += 8 * (capTot / 64 + GM_SW_TPC); /* completed masks */
         b += 4 * front + (sizeof(GmRegion) + 4ull * (GM_RROWS + GM_NHALO + 26)) * (T + 1) + 16ull * GM_SW_TPC * 2 * T;
     }
-    b += 8 * N;                                   /* grid, claim */
+    b += 8 * N;                                   /* cells */
     b += 8 * (N + capB + 4096);                   /* retirement log */
     b += 32 * bricks;                             /* deformed bitmap */
     b += (sizeof(gm_cs_t) + sizeof(GmRec)) * capTot; /* completion steps, records */

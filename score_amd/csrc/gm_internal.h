@@ -2,16 +2,17 @@
  * gm_internal.h -- device layout and kernel launchers of the growth machine.
  *
  * One domain lives in HBM as:
- *   grid   uint32[N]   deformed-grain id (< ndefg); not written during the run: only
- *                      deformed cells' entries are ever read then, and a cell
- *                      that transforms is appended to the retirement log
+ *   cell   (claim, grain)[N]  the cell's infection claim key, 0xFFFFFFFF until
+ *                      claimed (a claimed cell is infected in the same step and never
+ *                      claimed again, so claims are never reset), beside its
+ *                      deformed-grain id (< ndefg), so that one scattered load gives
+ *                      both.  The id is not written during the run: only deformed
+ *                      cells' are read then, and a cell that transforms is appended
+ *                      to the retirement log
  *   rlog   (cell, ndefg+rxg) per retired cell in retirement order, written
  *                      coalesced with the step's parent data; the exported map
  *                      is the grid with the log applied and the front's cells
  *                      marked INFECTED
- *   claim  uint32[N]   per-cell infection claim key, 0xFFFFFFFF until claimed; a
- *                      claimed cell is infected in the same step and never
- *                      claimed again, so claims are never reset
  *   dmap   1 bit per cell, set while the cell is deformed (infectable), blocked so
  *          that one 128-byte line holds a 16x8x8 brick of cells: a 3x3x3
  *          neighbourhood usually lies in one or two lines
@@ -121,6 +122,9 @@ static inline __host__ __device__ uint32_t gm_tiles_inside(uint32_t nI) {
 #define GM_PB 2048u               /* blocks of the propose pass at most */
 #define GM_DB 1024u               /* blocks of the decide and commit passes at most */
 #define GM_GRID_BLOCKS 2048u      /* blocks of the pass over the cell grid at most */
+#define GM_SUBS 16u               /* parts of a deformed grain's count */
+#define GM_GATT 128u              /* attempts of a chunk whose targets' grains the decide pass hands on */
+#define GM_GCHUNKS 32768u         /* chunks it does that for */
 #define GM_RECYCLE_BLOCKS 2048u   /* blocks of the decide launch that write recycled slots */
 
 /* One front record: SCORE's `cell` (SCORE_Kernel.h:124-137) with rxFrac held as
@@ -194,8 +198,10 @@ struct alignas(8) GmStats {
     uint32_t pone;            /* set when a pair weight was short-circuited to 1.0 */
     uint32_t scan_tot[4];     /* totals written by the device-wide scans */
     uint32_t nattempt;        /* attempts that found a deformed target this step */
-    uint32_t nzeroed;         /* deformed grains that lost their last cell this step */
-    uint32_t cwrap;           /* a deformed-grain count was decremented past zero this step */
+    uint32_t nzeroed;         /* several regions: deformed grains that lost their last cell in the window */
+    uint32_t cwrap;           /* a deformed-grain count went past zero (one region: of a grain before the one that sets rhomax) */
+    uint32_t top_hit;         /* one region: the grain that sets rhomax lost its last cell, */
+    uint32_t top_next;        /* and the position of its successor in rorder (ndefg: none) */
     uint32_t dfirst;          /* defragmentation: first INACTIVE slot of the list */
     uint32_t dcount;          /* defragmentation: ACTIVE slots moved; status vector: entries */
     uint32_t novf;            /* weight lookups that found the cache full (their cells wait for a larger table) */
@@ -219,10 +225,19 @@ struct alignas(8) GmStats {
 struct GmWindow {
     double xstop;             /* Xcells at which the host must act (termination, defragmentation) */
     uint32_t top_grain;       /* the grain that sets rhomax (0xFFFFFFFF: none) */
+    uint32_t top_pos;         /* its position in rorder (ndefg: none) */
     uint32_t pend_limit;      /* new P-cache entries that keep the cache at most half full */
     uint32_t defer;           /* pending weights may wait for the end of the window */
-    uint32_t pad;
 };
+
+/* Parents per chunk of the decide and commit passes: a wave takes one chunk at a
+ * time, a lane per parent and then a lane per winner, so a chunk aims at 52
+ * winners (at 64 parents for 66 winners a second round for the last few cost as
+ * much as the first), by the ratio the step before had. */
+static inline __host__ __device__ uint32_t gm_chunk_size(uint32_t nfull, uint32_t nwin) {
+    const uint64_t c = nwin ? (uint64_t)nfull * 52u / nwin : 64u;
+    return c > 64u ? 64u : c < 16u ? 16u : (uint32_t)c;
+}
 
 /* How a window's passes are cut up, fixed over the window: sweep blocks of
  * GM_SW_WAVES waves with cpw chunks each, nbI of them over the Inside list's chI
@@ -230,6 +245,7 @@ struct GmWindow {
  * decide passes. */
 struct GmPart {
     uint32_t nbI, nb, cpw, chI, chB, W, nbp, nbd;
+    uint32_t csz0;              /* the first step's chunk size */
 };
 
 /* the front lists as a step of the window finds them */
@@ -237,6 +253,7 @@ struct GmWinStep {
     uint32_t nI, nB;            /* list lengths */
     uint32_t totRecI, totRecB;  /* INACTIVE slots */
     uint32_t recLenI, recLenB;  /* of which may be handed out */
+    uint32_t csz;               /* parents per chunk of the decide and commit passes, 16 .. 64 */
 };
 
 /* what the passes of a window share, all on the device */
@@ -244,7 +261,8 @@ struct GmWin {
     uint32_t full[GM_WMAX], fullI[GM_WMAX]; /* cells completing in each step, in all and of the Inside list */
     uint32_t off[GM_WMAX + 1];  /* completed cells before each step: its list starts at pslot[off[i]] */
     uint32_t npend0;            /* new weight-cache entries before the current step */
-    uint32_t top_hit;           /* the grain that sets rhomax lost its last cell */
+    uint32_t top_left;          /* cells of the grain that sets rhomax */
+    uint32_t top_hit;           /* it lost its last cell */
     GmWinStep step[GM_WMAX + 1];
     unsigned long long nret0;   /* retirements before the window */
     double xcells0;             /* Xcells before the window */
@@ -309,7 +327,7 @@ struct GmDev {
     uint32_t capI, capB;
     uint32_t recCapI, recCapB;
     /* state */
-    uint32_t *grid, *claim;
+    uint2 *cell;                /* (claim, deformed grain) per cell */
     uint2 *rlog;                /* retirement log, rlogCap entries */
     uint64_t rlogCap;
     uint32_t *dmap;
@@ -323,7 +341,9 @@ struct GmDev {
     uint4 *par;                 /* the same cells' parent data: GM_PAR_PLANES planes */
     uint32_t *recI, *recB;      /* recycled slots (list-relative), ascending, capped */
     uint64_t *mF, *mR;          /* per 64-slot tile: completed (several regions only) / INACTIVE masks */
-    uint32_t *pmI, *pmB;        /* per parent: winning ranks into Inside / Border */
+    uint32_t *pmA;              /* per parent: ranks of its attempts on deformed cells (one region) */
+    uint32_t *pmI, *pmB;        /* per parent: winning ranks into Inside / Border (several regions: pmI holds the
+                                 * attempts until they are decided) */
     /* pslot, par, pmI and pmB hold parentCap entries */
     uint32_t *bcnt;             /* per-block counts and offsets, 8 x GM_MAX_BLOCKS */
     uint32_t *dlist;            /* slots of the cells left DEFERRED in a window (dlistCap entries) */
@@ -339,10 +359,15 @@ struct GmDev {
     uint32_t *rgone, *rmrg;     /* slots the step before handed out; steps whose completed cells are in the block's masks */
     uint32_t *acnt;             /* attempts per propose block, two rows by the step's parity */
     uint2 *btot;                /* winners into Inside, Border per decide block */
-    uint32_t *ccnt;             /* the same per 64 parents, Inside << 16 | Border */
+    uint32_t *btop;             /* parents per decide block in the grain that sets rhomax */
+    uint32_t *ccnt;             /* the same per chunk of parents, Inside << 16 | Border */
+    uint32_t *gatt;             /* grains of the first GM_GATT attempts' targets of the first gchunks chunks */
+    uint32_t gchunks;           /* at most GM_GCHUNKS */
     /* grains */
     double *rho, *defq, *rxq;
     uint32_t *defcnt, *rxcnt;
+    uint32_t *defsub;           /* one region: GM_SUBS rows of ndefg, cells taken from defcnt since the last fold */
+    uint32_t *rorder, *rpos;    /* one region: the grains by descending rho, and each one's position */
     uint32_t *zlist;            /* ids of grains exhausted in the current step */
     /* mobility-weight cache: open addressing on key rxg*ndefg+defg+1 */
     unsigned long long *hkeys;
@@ -402,8 +427,10 @@ struct GmSweepArgs {
  * ev[i] is recorded before kernel i of the step and ev[GM_NK] after the last. */
 /* the start of a one-region window: re-anchoring (a.reanchor), the arrivals of
  * step a.k, and the window sweep */
-hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &a, bool arrivals, double xcells,
-                            hipStream_t s, hipEvent_t *ev);
+hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &a, const GmWindow &wd, bool arrivals,
+                            double xcells, hipStream_t s, hipEvent_t *ev);
+/* one region: d.defcnt brought up to date */
+hipError_t gm_launch_fold_counts(const GmDev &d, hipStream_t s);
 /* every active cell advanced to step a.k with its old increment and predicted again */
 hipError_t gm_launch_reanchor(const GmDev &d, const GmSweepArgs &a, hipStream_t s);
 /* the same two halves of a step with several regions (gm_regions.hip) */
@@ -419,7 +446,8 @@ hipError_t gm_launch_rg_place(const GmDev &d, const uint32_t *slots, const GmRec
 hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P,
                             const GmWindow &w, uint32_t j, hipStream_t s, hipEvent_t *ev);
 /* its end after `launched` steps: the last step's row, the stats into the host's mirror */
-hipError_t gm_launch_window_end(const GmDev &d, const GmPart &P, uint32_t launched, GmStats *out, hipStream_t s);
+hipError_t gm_launch_window_end(const GmDev &d, const GmPart &P, uint32_t launched, uint32_t top_pos, GmStats *out,
+                                hipStream_t s);
 /* start of a window with several regions: step index and Xcells; clears the window's accumulators */
 hipError_t gm_launch_window_begin(const GmDev &d, uint32_t k, double xcells, hipStream_t s);
 /* end of every step of a window with several regions: records the step's row, advances the step
@@ -439,9 +467,9 @@ struct GmFrontOut {
 };
 hipError_t gm_launch_materialize(const GmDev &d, uint32_t k, uint32_t base, uint32_t n, const GmFrontOut &o,
                                  hipStream_t s);
-/* the deformed-cell bitmap, the grains' cell counts (d.defcnt, zeroed before) and
+/* from the cell grid `src`: the cells' pairs, the deformed-cell bitmap, the grains' cell counts (d.defcnt, zeroed before) and
  * the check of the cell grid; raises GM_ERRF_GRID (d.st, zeroed before) */
-hipError_t gm_launch_grid_init(const GmDev &d, hipStream_t s);
+hipError_t gm_launch_grid_init(const GmDev &d, const uint32_t *src, hipStream_t s);
 /* ompshar_defragmentation on the list whose slot 0 is global slot `base`:
  * first_inactive leaves in st->dfirst the first INACTIVE slot in [lo, hi), or hi;
  * move compacts the ACTIVE slots of (first, nnever) to [first, first+count) through
@@ -456,7 +484,7 @@ hipError_t gm_launch_defrag_move(const GmDev &d, uint32_t base, uint32_t first, 
  * ixyz and gid hold nI+nB entries. */
 hipError_t gm_launch_status(const GmDev &d, uint32_t nI, uint32_t nB, uint32_t k, double thr, uint32_t *ixyz,
                             uint32_t *gid, hipStream_t s);
-/* the cell grid as SCORE holds it, from a copy of d.grid in `out`: every retired
+/* the cell grid as SCORE holds it into `out`: every retired
  * cell set to ndefg+rxg from the log, every cell held by an active front record
  * marked INFECTED */
 hipError_t gm_launch_overlay_infected(const GmDev &d, uint32_t nI, uint32_t nB, uint32_t k, uint32_t *out,

@@ -145,11 +145,38 @@ static __device__ __forceinline__ uint32_t code_at(const uint4 &cs, int q) {
     return (wd >> (16 * (q & 1))) & 0xFFFFu;
 }
 
+/* A grain's cells: the count at the last fold less the parts taken since.  Every
+ * lane of the wave takes part and gets the value. */
+static __device__ __forceinline__ uint32_t exact_count(const GmDev &d, uint32_t g) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t v = lane < GM_SUBS ? d.defsub[(size_t)lane * d.ndefg + g] : 0u;
+    for (int o = 32; o > 0; o >>= 1) v += (uint32_t)__shfl_xor((int)v, o, 64);
+    return d.defcnt[g] - v;
+}
+
+/* the parts into the counts */
+__global__ void k_fold_counts(GmDev d) {
+    for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < d.ndefg; g += gridDim.x * blockDim.x) {
+        uint32_t v = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < GM_SUBS; i++) {
+            v += d.defsub[(size_t)i * d.ndefg + g];
+            d.defsub[(size_t)i * d.ndefg + g] = 0;
+        }
+        d.defcnt[g] -= v;
+    }
+}
+
+hipError_t gm_launch_fold_counts(const GmDev &d, hipStream_t s) {
+    k_fold_counts<<<fill_blocks(d.ndefg), GM_BLOCK, 0, s>>>(d);
+    return hipGetLastError();
+}
+
 /* pass 1: per block, the cells that complete in each step of the window and the
  * INACTIVE slots (row GM_WMAX); per wave, the completing cells of each step.
  * Block 0 also clears the window's accumulators.  A slot without a prediction
  * (UNKNOWN) raises GM_ERRF_MISSED. */
-__global__ void __launch_bounds__(GM_BLOCK) k_sweep(GmDev d, GmPart P, uint32_t k0, double xcells) {
+__global__ void __launch_bounds__(GM_BLOCK) k_sweep(GmDev d, GmPart P, uint32_t k0, double xcells, uint32_t top_pos) {
     __shared__ uint32_t red[GM_SW_WAVES][GM_WMAX + 1];
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6, b = blockIdx.x;
     if (b == 0 && threadIdx.x == 0) {
@@ -159,13 +186,16 @@ __global__ void __launch_bounds__(GM_BLOCK) k_sweep(GmDev d, GmPart P, uint32_t 
         st->ndeferred = 0;
         st->npend = 0;
         st->pone = 0;
-        st->nzeroed = 0;
         st->cwrap = 0;
         st->novf = 0;
         d.win->nret0 = st->nret;
         d.win->xcells0 = xcells;
         d.win->npend0 = 0;
         d.win->top_hit = 0;
+    }
+    if (b == 0 && w == 1u && top_pos < d.ndefg) {
+        const uint32_t n = exact_count(d, d.rorder[top_pos]);
+        if (lane == 0) d.win->top_left = n;
     }
     const WaveChunks r = wave_chunks(d, P, b, w);
     const uint32_t kc = k0 & (GM_CS_MOD - 1u), horizon = d.horizon;
@@ -239,6 +269,7 @@ static __device__ void window_totals(const GmDev &d, const GmPart &P, const uint
     win->off[P.W] = off;
     if (err) atomicOr(&d.st->err, err);
     GmWinStep &s = win->step[0];
+    s.csz = P.csz0;
     s.nI = d.st->nI;
     s.nB = d.st->nB;
     s.totRecI = recI;
@@ -444,8 +475,8 @@ hipError_t gm_launch_reanchor(const GmDev &d, const GmSweepArgs &a, hipStream_t 
 
 __global__ void k_arrivals(GmDev d, GmSweepArgs A);
 
-hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &a, bool arrivals, double xcells,
-                            hipStream_t s, hipEvent_t *ev) {
+hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &a, const GmWindow &wd, bool arrivals,
+                            double xcells, hipStream_t s, hipEvent_t *ev) {
     hipError_t e;
     if ((e = mark(ev, 0, s)) != hipSuccess) return e;
     if (a.reanchor && (e = gm_launch_reanchor(d, a, s)) != hipSuccess) return e;
@@ -454,7 +485,7 @@ hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if ((e = mark(ev, 1, s)) != hipSuccess) return e;
-    k_sweep<<<P.nb, GM_BLOCK, 0, s>>>(d, P, a.k, xcells);
+    k_sweep<<<P.nb, GM_BLOCK, 0, s>>>(d, P, a.k, xcells, wd.top_pos);
     if ((e = mark(ev, 2, s)) != hipSuccess) return e;
     const bool fold = P.nb <= GM_SW_FOLD;
     if (!fold) k_sweep_scan<<<1, 1024, 0, s>>>(d, P);
@@ -466,7 +497,7 @@ hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &
 
 /* ----------------------------------------------------------------- infection */
 
-/* One pass over the cell grid as it arrived: every word of the bitmap (cells
+/* One pass over the cell grid as it arrived: the cells' (claim, grain) pairs, every word of the bitmap (cells
  * outside the domain stay 0), the cell count of every deformed grain, and whether
  * an id is no deformed grain's (GM_ERRF_GRID).  A thread takes a word, 2 x 16 cells.
  * A wave counts one grain at a time, every lane's cells of it together, and keeps
@@ -474,7 +505,7 @@ hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &
  * served one after another: a grain met in a long run of words costs few of them
  * (one grain in all: one per block).  The host's two loops over the grid that this
  * replaces took 123 ms at 512^3, the bitmap alone 0.58; the pass takes 0.26 (2 TB/s). */
-__global__ void __launch_bounds__(GM_BLOCK) k_grid_init(GmDev d, uint32_t nwords) {
+__global__ void __launch_bounds__(GM_BLOCK) k_grid_init(GmDev d, const uint32_t *src, uint32_t nwords) {
     __shared__ uint32_t sid[GM_BLOCK / 64], scnt[GM_BLOCK / 64];
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
     const bool vec = (d.nx & 3u) == 0u;
@@ -489,7 +520,9 @@ __global__ void __launch_bounds__(GM_BLOCK) k_grid_init(GmDev d, uint32_t nwords
 #pragma unroll
         for (uint32_t r = 0; r < 2u; r++) {
             const bool row = wd < nwords && y0 + r < d.ny && z < d.nz;
-            const uint32_t *g = d.grid + x0 + (size_t)(y0 + r) * d.nx + (size_t)z * d.nxy;
+            const size_t at = x0 + (size_t)(y0 + r) * d.nx + (size_t)z * d.nxy;
+            const uint32_t *g = src + at;
+            uint2 *c = d.cell + at;
 #pragma unroll
             for (uint32_t i = 0; i < 16u; i += 4u) {
                 uint4 q = make_uint4(0u, 0u, 0u, 0u);
@@ -500,6 +533,18 @@ __global__ void __launch_bounds__(GM_BLOCK) k_grid_init(GmDev d, uint32_t nwords
                     if (x0 + i + 1u < d.nx) q.y = g[i + 1u];
                     if (x0 + i + 2u < d.nx) q.z = g[i + 2u];
                     if (x0 + i + 3u < d.nx) q.w = g[i + 3u];
+                }
+                if (vec) {
+                    if (row && x0 + i < d.nx) {
+                        uint4 *o = reinterpret_cast<uint4 *>(c + i);
+                        o[0] = make_uint4(GM_FREE_CLAIM, q.x, GM_FREE_CLAIM, q.y);
+                        o[1] = make_uint4(GM_FREE_CLAIM, q.z, GM_FREE_CLAIM, q.w);
+                    }
+                } else if (row) {
+                    if (x0 + i < d.nx) c[i] = make_uint2(GM_FREE_CLAIM, q.x);
+                    if (x0 + i + 1u < d.nx) c[i + 1u] = make_uint2(GM_FREE_CLAIM, q.y);
+                    if (x0 + i + 2u < d.nx) c[i + 2u] = make_uint2(GM_FREE_CLAIM, q.z);
+                    if (x0 + i + 3u < d.nx) c[i + 3u] = make_uint2(GM_FREE_CLAIM, q.w);
                 }
                 const uint32_t k = 16u * r + i;
                 id[k] = q.x;
@@ -559,10 +604,10 @@ __global__ void __launch_bounds__(GM_BLOCK) k_grid_init(GmDev d, uint32_t nwords
     }
 }
 
-hipError_t gm_launch_grid_init(const GmDev &d, hipStream_t s) {
+hipError_t gm_launch_grid_init(const GmDev &d, const uint32_t *src, hipStream_t s) {
     const uint32_t nwords = d.dnbx * d.dnby * d.dnbz * 32u;
     const unsigned nb = fill_blocks(nwords);
-    k_grid_init<<<nb < GM_GRID_BLOCKS ? nb : GM_GRID_BLOCKS, GM_BLOCK, 0, s>>>(d, nwords);
+    k_grid_init<<<nb < GM_GRID_BLOCKS ? nb : GM_GRID_BLOCKS, GM_BLOCK, 0, s>>>(d, src, nwords);
     return hipGetLastError();
 }
 
@@ -710,7 +755,7 @@ static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, 
     r.winB = wB;
     r.npend = st->npend - win->npend0;
     r.nattempt = na;
-    r.nzeroed = st->nzeroed < d.ndefg ? st->nzeroed : d.ndefg;
+    r.nzeroed = 0;
     r.err = st->err;
     r.nplaced = st->nplaced;
     r.pone = st->pone;
@@ -726,6 +771,7 @@ static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, 
     st->nexec = js + 1u;
     if (next) {
         GmWinStep &s = win->step[js + 1u];
+        s.csz = gm_chunk_size(win->full[js], wI + wB);
         s.nI = r.nI;
         s.nB = r.nB;
         s.totRecI = (uint32_t)(carry >> 32);
@@ -840,7 +886,7 @@ static __device__ __forceinline__ uint32_t face_attempts(const GmDev &d, uint32_
  * goes to the dense parent planes (FullRX order), with its rxFrac after the
  * completing addition, replayed from the anchor.  Every attempt on a deformed cell
  * claims its target (the smallest key p*32+r is the serial winner); their mask
- * over the ranks is kept in pmI for the decide pass.  Few of the 26 neighbours are
+ * over the ranks is kept in pmA for the decide pass.  Few of the 26 neighbours are
  * still deformed (1.04 per parent on the 512^3 workload), so the cost is finding
  * them: a strictly interior parent reads its 3x3x3 bits with three 16-byte loads
  * (26 single tests before).  Wave w
@@ -894,10 +940,10 @@ __global__ void __launch_bounds__(GM_BLOCK) k_propose(GmDev d, GmPart P, GmWindo
                 attempt_target(d, true, x, y, z, (int)rk, tx, ty, tz, toB);
                 t = cell_of(d, tx, ty, tz);
             }
-            atomicMin(&d.claim[t], p * 32u + rk);
+            atomicMin(&d.cell[t].x, p * 32u + rk);
         }
         natt += (uint32_t)__popc(am);
-        d.pmI[p] = am;
+        d.pmA[p] = am;
         par_plane(d, GM_PAR1_CELL)[p] = make_uint4(x | y << 16, z | (fromB ? 1u << 16 : 0u), rc.defg, rxg);
         reinterpret_cast<double2 *>(par_plane(d, GM_PAR1_FP))[p] = make_double2(fin, rc.P);
         if (logged) d.rlog[nret + p] = make_uint2(cell, d.ndefg + rxg);
@@ -1006,18 +1052,17 @@ static __device__ void recycle_blocks(const GmDev &d, const GmPart &P, uint32_t 
     }
 }
 
-/* chunks of 64 parents that a block of the decide and commit passes takes */
-static __device__ __forceinline__ uint32_t chunks_per_block(uint32_t nfull, uint32_t nbd) {
-    return ((nfull + 63u) / 64u + nbd - 1u) / nbd;
-}
-
 /* The first nrec blocks write the recycled slots; the rest find which attempts
- * won.  A wave takes 64 parents at a time and flattens their attempts into a list,
- * a lane per attempt, so that all claims are loaded together (a loop over each
- * parent's attempts waits once per attempt of its busiest parent).  Winners as
- * 26-bit masks per destination list, their counts per 64 parents (Inside << 16 |
- * Border) and per block, from which the commit pass ranks them. */
-__global__ void __launch_bounds__(GM_BLOCK) k_decide(GmDev d, GmPart P, uint32_t j, uint32_t nrec) {
+ * won.  A wave takes a chunk of parents at a time and flattens their attempts into
+ * a list, a lane per attempt, so that all claims are loaded together (a loop over
+ * each parent's attempts waits once per attempt of its busiest parent).  A cell's
+ * claim and grain are one 8-byte load; the grains go to the commit pass in the
+ * attempts' order (the first GM_GATT of a chunk), which would wait for the same
+ * scattered lines again.  Winners as 26-bit masks per destination list, their
+ * counts per chunk (Inside << 16 | Border) and per block, from which the commit
+ * pass ranks them.  The parents retire here (updateFullRX*, SCORE_Kernel.cpp:
+ * 4640-4653), beside the waiting for the claims. */
+__global__ void __launch_bounds__(GM_BLOCK) k_decide(GmDev d, GmPart P, uint32_t j, uint32_t nrec, uint32_t top_pos) {
     extern __shared__ unsigned long long smask[];
     struct Wave {
         uint2 xyz[64];
@@ -1026,23 +1071,30 @@ __global__ void __launch_bounds__(GM_BLOCK) k_decide(GmDev d, GmPart P, uint32_t
     };
     __shared__ Wave sw[GM_BLOCK / 64];
     __shared__ uint32_t sh[GM_BLOCK / 64][3];
-    const uint32_t halt = d.st->halt, nfull = d.win->full[j];
+    const uint32_t halt = d.st->halt, nfull = d.win->full[j], csz = d.win->step[j].csz;
     if (halt) return;
     if (blockIdx.x < nrec) {
         recycle_blocks(d, P, j, blockIdx.x, nrec, smask);
         return;
     }
     const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u, blk = blockIdx.x - nrec;
-    const uint32_t nch = (nfull + 63u) / 64u;
-    const uint32_t cpd = chunks_per_block(nfull, P.nbd);
+    const uint32_t nch = (nfull + csz - 1u) / csz, cpd = (nch + P.nbd - 1u) / P.nbd;
     const uint32_t c0 = blk * cpd, c1 = c0 + cpd < nch ? c0 + cpd : nch;
     Wave &W = sw[w];
-    uint32_t tI = 0, tB = 0, dummy = 0;
+    uint32_t tI = 0, tB = 0, ntop = 0;
+    bool wrapped = false;
     for (uint32_t c = c0 + w; c < c1; c += GM_BLOCK / 64u) {
-        const uint32_t p = c * 64u + lane;
-        const bool valid = p < nfull;
-        const uint32_t am = valid ? d.pmI[p] : 0u;
-        W.xyz[lane] = valid ? *reinterpret_cast<const uint2 *>(par_plane(d, GM_PAR1_CELL) + p) : make_uint2(0u, 0u);
+        const uint32_t p = c * csz + lane;
+        const bool valid = lane < csz && p < nfull;
+        const uint32_t am = valid ? d.pmA[p] : 0u;
+        const uint4 q0 = valid ? par_plane(d, GM_PAR1_CELL)[p] : make_uint4(0u, 0u, 0u, 0u);
+        W.xyz[lane] = make_uint2(q0.x, q0.y);
+        retire(d, q0.z, q0.w, valid, blk & (GM_SUBS - 1u));
+        /* where the parent's grain stands in the order of rho: the one that sets
+         * rhomax is counted, one before it (all without cells) has its count wrap */
+        const uint32_t rp = valid ? d.rpos[q0.z] : 0xFFFFFFFFu;
+        ntop += rp == top_pos ? 1u : 0u;
+        wrapped |= rp < top_pos;
         W.mI[lane] = 0;
         W.mB[lane] = 0;
         const uint32_t na = (uint32_t)__popc(am), incl = wave_incl_scan(na);
@@ -1056,8 +1108,9 @@ __global__ void __launch_bounds__(GM_BLOCK) k_decide(GmDev d, GmPart P, uint32_t
             uint32_t tx, ty, tz;
             bool toB;
             attempt_target(d, (v.y >> 16) != 0u, v.x & 0xFFFFu, v.x >> 16, v.y & 0xFFFFu, (int)rk, tx, ty, tz, toB);
-            if (d.claim[cell_of(d, tx, ty, tz)] == (c * 64u + q) * 32u + rk)
-                atomicOr(toB ? &W.mB[q] : &W.mI[q], 1u << rk);
+            const uint2 t = d.cell[cell_of(d, tx, ty, tz)];
+            if (t.x == (c * csz + q) * 32u + rk) atomicOr(toB ? &W.mB[q] : &W.mI[q], 1u << rk);
+            if (i < GM_GATT && c < d.gchunks) d.gatt[(size_t)c * GM_GATT + i] = t.y;
         }
         wave_sync();
         const uint32_t mI = W.mI[lane], mB = W.mB[lane];
@@ -1074,24 +1127,26 @@ __global__ void __launch_bounds__(GM_BLOCK) k_decide(GmDev d, GmPart P, uint32_t
         }
         wave_sync();
     }
-    block_sum3(tI, tB, dummy, sh);
-    if (threadIdx.x == 0) d.btot[blk] = make_uint2(tI, tB);
+    if (__any(wrapped) && lane == 0) d.st->cwrap = 1u;
+    block_sum3(tI, tB, ntop, sh);
+    if (threadIdx.x == 0) {
+        d.btot[blk] = make_uint2(tI, tB);
+        d.btop[blk] = ntop;
+    }
 }
 
 /* New records as omp_infect_OutOfRXFront* write them (SCORE_Kernel.cpp:4281-4310,
- * :4402-4426), slots as omp_getNextFreeSlotIn* hand them out (:3757-3874); then
- * the parents retire as updateFullRX* does it (:4640-4653).  A wave takes 64
+ * :4402-4426), slots as omp_getNextFreeSlotIn* hand them out (:3757-3874).  A wave takes a chunk of
  * parents at a time; their winners are flattened into a list so that every lane
  * commits one infection.  Each lane loads its own parent's data with its winner
- * masks and shares it through LDS, and a winner issues its target's grid load and
- * its slot lookup together, so a wave waits on few dependent memory round trips.
+ * masks and shares it through LDS, and a winner issues its target's grain and its
+ * slot lookup together, so a wave waits on few dependent memory round trips.
  * A winner's rank in its list is the winners before it: the blocks of the decide
  * pass before its own (added up by the block), the chunks before its own in that
  * block, the parents before its own in the chunk. */
-__global__ void __launch_bounds__(GM_BLOCK) k_commit(GmDev d, GmPParams pp, GmSweepArgs A, GmPart P, uint32_t j,
-                                                     uint32_t top_grain) {
+__global__ void __launch_bounds__(GM_BLOCK, 4) k_commit(GmDev d, GmPParams pp, GmSweepArgs A, GmPart P, uint32_t j) {
     struct Wave {
-        uint32_t sI[64], sB[64], oI[64], oB[64];
+        uint32_t sA[64], sI[64], sB[64], oA[64], oI[64], oB[64];
         uint4 sq0[64];
         double sfin[64], sP[64];
         uint16_t wl[26 * 64];
@@ -1099,25 +1154,36 @@ __global__ void __launch_bounds__(GM_BLOCK) k_commit(GmDev d, GmPParams pp, GmSw
     __shared__ Wave sw[GM_BLOCK / 64];
     __shared__ uint32_t sh[GM_BLOCK / 64][3];
     GmStats *st = d.st;
-    const uint32_t halt = st->halt, nfull = d.win->full[j], nch = (nfull + 63u) / 64u;
+    const uint32_t halt = st->halt, nfull = d.win->full[j];
     const GmWinStep ws = d.win->step[j];
     if (halt) return;
-    const uint32_t k = A.k;
-    const uint32_t cpd = chunks_per_block(nfull, P.nbd), db = blockIdx.x;
+    const uint32_t k = A.k, csz = ws.csz;
+    const uint32_t nch = (nfull + csz - 1u) / csz, cpd = (nch + P.nbd - 1u) / P.nbd, db = blockIdx.x;
     const uint32_t c0 = db * cpd, c1 = c0 + cpd < nch ? c0 + cpd : nch;
+    if (db == 0) { /* the cells left of the grain that sets rhomax */
+        uint32_t n = 0, z0 = 0, z1 = 0;
+        for (uint32_t i = threadIdx.x; i < P.nbd; i += GM_BLOCK) n += d.btop[i];
+        block_sum3(n, z0, z1, sh);
+        if (threadIdx.x == 0 && n) {
+            const uint32_t left = d.win->top_left - n;
+            d.win->top_left = left;
+            if (left == 0u) d.win->top_hit = 1u;
+        }
+    }
     if (c0 >= nch) return;
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
     /* a lane's parent: winner masks | x | y, z | fromB, defg, rxg | fin, P; the
      * wave's first chunk is loaded before the winners of earlier blocks are added up */
-    uint32_t mI, mB;
+    uint32_t am, mI, mB;
     uint4 q0;
     double2 fp;
     auto load = [&](uint32_t c) {
-        const uint32_t pt = c * 64u + lane;
-        mI = mB = 0;
+        const uint32_t pt = c * csz + lane;
+        am = mI = mB = 0;
         q0 = make_uint4(0u, 0u, 0xFFFFFFFFu, 0xFFFFFFFFu);
         fp = make_double2(0.0, 0.0);
-        if (c < c1 && pt < nfull) {
+        if (c < c1 && lane < csz && pt < nfull) {
+            am = d.pmA[pt];
             mI = d.pmI[pt];
             mB = d.pmB[pt];
             q0 = par_plane(d, GM_PAR1_CELL)[pt];
@@ -1125,6 +1191,17 @@ __global__ void __launch_bounds__(GM_BLOCK) k_commit(GmDev d, GmPParams pp, GmSw
         }
     };
     load(c0 + wv);
+    /* winners of the block's chunks [a, b) */
+    auto count = [&](uint32_t a, uint32_t b, uint32_t &nI, uint32_t &nB) {
+        nI = nB = 0;
+        for (uint32_t i = a + lane; i < b; i += 64u) {
+            const uint32_t v = d.ccnt[i];
+            nI += v >> 16;
+            nB += v & 0xFFFFu;
+        }
+    };
+    uint32_t bI, bB;
+    count(c0, c0 + wv < c1 ? c0 + wv : c1, bI, bB);
     uint32_t runI = 0, runB = 0, dummy = 0;
     for (uint32_t i0 = threadIdx.x; i0 < db; i0 += 4u * GM_BLOCK) {
         uint2 v[4];
@@ -1140,20 +1217,12 @@ __global__ void __launch_bounds__(GM_BLOCK) k_commit(GmDev d, GmPParams pp, GmSw
         }
     }
     block_sum3(runI, runB, dummy, sh);
-    uint32_t cdone = c0; /* chunks of this block counted in runI, runB */
     Wave &W = sw[wv];
     for (uint32_t c = c0 + wv; c < c1; c += GM_BLOCK / 64u) {
-        if (c != c0 + wv) load(c);
-        const bool valid = c * 64u + lane < nfull;
-        uint32_t bI = 0, bB = 0;
-        for (uint32_t i = cdone + lane; i < c; i += 64u) {
-            const uint32_t v = d.ccnt[i];
-            bI += v >> 16;
-            bB += v & 0xFFFFu;
+        if (c != c0 + wv) {
+            load(c);
+            count(c - GM_BLOCK / 64u, c, bI, bB);
         }
-        cdone = c;
-        /* the parents' counts: issued here, looked at after the new records */
-        const Retired gone = retire_begin(d, q0, valid);
         for (int o = 32; o > 0; o >>= 1) {
             bI += __shfl_xor(bI, o, 64);
             bB += __shfl_xor(bB, o, 64);
@@ -1166,6 +1235,9 @@ __global__ void __launch_bounds__(GM_BLOCK) k_commit(GmDev d, GmPParams pp, GmSw
         const uint32_t incl = wave_incl_scan(packed);
         const uint32_t ex = incl - packed, tot = __shfl(incl, 63, 64);
         const uint32_t totI = tot >> 16, totB = tot & 0xFFFFu;
+        const uint32_t na = (uint32_t)__popc(am);
+        W.sA[lane] = am;
+        W.oA[lane] = wave_incl_scan(na) - na;
         W.oI[lane] = runI + (ex >> 16);
         W.oB[lane] = runB + (ex & 0xFFFFu);
         W.sI[lane] = mI;
@@ -1186,7 +1258,9 @@ __global__ void __launch_bounds__(GM_BLOCK) k_commit(GmDev d, GmPParams pp, GmSw
             attempt_target(d, (pq0.y >> 16) != 0u, pq0.x & 0xFFFFu, pq0.x >> 16, pq0.y & 0xFFFFu, (int)r, tx, ty, tz,
                            toB);
             const uint32_t t = cell_of(d, tx, ty, tz);
-            const uint32_t g = d.grid[t];
+            /* the target's grain, from the decide pass */
+            const uint32_t ia = W.oA[q] + (uint32_t)__popc(W.sA[q] & (bit - 1u));
+            const uint32_t g = ia < GM_GATT && c < d.gchunks ? d.gatt[(size_t)c * GM_GATT + ia] : d.cell[t].y;
             /* rank k into a list takes its k-th recycled slot, else appends */
             const uint32_t wI = W.sI[q];
             const bool intoI = (wI & bit) != 0u;
@@ -1195,14 +1269,13 @@ __global__ void __launch_bounds__(GM_BLOCK) k_commit(GmDev d, GmPParams pp, GmSw
             const uint32_t recLen = intoI ? ws.recLenI : ws.recLenB;
             const uint32_t *recl = intoI ? d.recI : d.recB;
             const uint32_t rel = rank < recLen ? recl[rank] : (intoI ? ws.nI : ws.nB) + (rank - recLen);
+            const NewCell nc = new_cell(d, pp, A, k, W.sfin[q], W.sP[q], pq0, r, g);
             if (rel >= (intoI ? d.capI : d.capB)) {
                 atomicOr(&st->err, intoI ? GM_ERRF_INSIDE_FULL : GM_ERRF_BORDER_FULL);
                 continue;
             }
-            const uint32_t gslot = intoI ? rel : d.capI + rel;
-            infect_one(d, pp, A, k, W.sfin[q], W.sP[q], pq0, r, t, g, tx, ty, tz, gslot);
+            put_cell(d, k, nc, pq0, t, g, tx, ty, tz, intoI ? rel : d.capI + rel);
         }
-        retire_end(d, q0.z, gone, top_grain, &d.win->top_hit);
         wave_sync();
     }
 }
@@ -1218,12 +1291,23 @@ hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepAr
     const uint32_t nrec = P.nb < GM_RECYCLE_BLOCKS ? P.nb : GM_RECYCLE_BLOCKS;
     /* a sweep block's INACTIVE masks and the offsets of its tiles */
     const size_t lds = (size_t)GM_SW_WAVES * P.cpw * GM_SW_TPC * (sizeof(unsigned long long) + sizeof(uint32_t));
-    k_decide<<<nrec + P.nbd, GM_BLOCK, lds, s>>>(d, P, j, nrec);
+    k_decide<<<nrec + P.nbd, GM_BLOCK, lds, s>>>(d, P, j, nrec, w.top_pos);
     for (int i = 6; i <= 8; i++)
         if ((e = mark(ev, i, s)) != hipSuccess) return e;
-    k_commit<<<P.nbd, GM_BLOCK, 0, s>>>(d, pp, A, P, j, w.top_grain);
+    k_commit<<<P.nbd, GM_BLOCK, 0, s>>>(d, pp, A, P, j);
     if ((e = mark(ev, 9, s)) != hipSuccess) return e;
     return hipGetLastError();
+}
+
+/* exported map: the grains the cells came with */
+__global__ void k_grid_out(GmDev d, uint32_t *out) {
+    const uint32_t n2 = (uint32_t)(d.N / 2u);
+    const uint4 *in = reinterpret_cast<const uint4 *>(d.cell);
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n2; i += gridDim.x * blockDim.x) {
+        const uint4 q = in[i];
+        reinterpret_cast<uint2 *>(out)[i] = make_uint2(q.y, q.w);
+    }
+    if ((d.N & 1u) && blockIdx.x == 0 && threadIdx.x == 0) out[d.N - 1u] = d.cell[d.N - 1u].y;
 }
 
 /* exported map: retired cells from the log, in retirement order (a cell retired
@@ -1248,6 +1332,7 @@ __global__ void k_overlay_infected(GmDev d, uint32_t nI, uint32_t nB, uint32_t k
 
 hipError_t gm_launch_overlay_infected(const GmDev &d, uint32_t nI, uint32_t nB, uint32_t k, uint32_t *out,
                                       hipStream_t s) {
+    k_grid_out<<<fill_blocks((d.N + 1u) / 2u), GM_BLOCK, 0, s>>>(d, out);
     k_apply_rlog<<<8192, GM_BLOCK, 0, s>>>(d, out);
     if (nI + nB == 0) return hipGetLastError();
     k_overlay_infected<<<fill_blocks(nI + nB), GM_BLOCK, 0, s>>>(d, nI, nB, k, out);
@@ -1365,7 +1450,7 @@ static __device__ __forceinline__ bool site_deformed(const GmDev &d, uint32_t w)
 __global__ void k_nuc_claim(GmDev d, const uint32_t *site, uint32_t n) {
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
         uint32_t w = site[k];
-        if (w != GM_NO_SITE && site_deformed(d, w)) atomicMin(&d.claim[w], k);
+        if (w != GM_NO_SITE && site_deformed(d, w)) atomicMin(&d.cell[w].x, k);
     }
 }
 
@@ -1377,7 +1462,7 @@ static __device__ __forceinline__ bool site_interior(const GmDev &d, uint32_t w)
 __global__ void k_nuc_flag(GmDev d, const uint32_t *site, uint32_t n) {
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
         uint32_t w = site[k];
-        bool win = w != GM_NO_SITE && site_deformed(d, w) && d.claim[w] == k;
+        bool win = w != GM_NO_SITE && site_deformed(d, w) && d.cell[w].x == k;
         bool in = win && site_interior(d, w);
         d.nI_[k] = (win && in) ? 1u : 0u;
         d.nB_[k] = (win && !in) ? 1u : 0u;
@@ -1399,7 +1484,7 @@ __global__ void k_nuc_commit(GmDev d, const uint32_t *site, const double *nucP, 
             if (rel >= d.capB) { atomicOr(&d.st->err, GM_ERRF_BORDER_FULL); continue; }
             gslot = d.capI + rel;
         }
-        uint32_t g = d.grid[w];
+        uint32_t g = d.cell[w].y;
         GmRec *r = d.rec + gslot;
         rec_set_a(r, 1.0, 0u, 26u);
         rec_set_b(r, 0.0);
@@ -1471,15 +1556,39 @@ hipError_t gm_launch_stats_out(const GmDev &d, GmStats *out, hipStream_t s) {
 
 /* The end of a window of `launched` steps: its last step is closed, unless the
  * window halted (the propose pass that halted it closed the step before), and
- * the stats go to the host's mirror. */
-__global__ void __launch_bounds__(GM_BLOCK) k_window_end(GmDev d, GmPart P, uint32_t launched, uint32_t *out) {
+ * the stats go to the host's mirror.  If the grain that sets rhomax lost its last
+ * cell, its successor is looked up. */
+__global__ void __launch_bounds__(GM_BLOCK) k_window_end(GmDev d, GmPart P, uint32_t launched, uint32_t top_pos,
+                                                         uint32_t *out) {
+    __shared__ uint32_t first;
+    const uint32_t hit = d.win->top_hit;
     if (!d.st->halt && d.st->nexec + 1u == launched) close_step(d, P, launched - 1u, false);
+    if (hit) { /* the next grain in the order of rho that holds cells */
+        if (threadIdx.x == 0) first = d.ndefg;
+        for (uint32_t i0 = top_pos; i0 < d.ndefg; i0 += GM_BLOCK) {
+            const uint32_t i = i0 + threadIdx.x;
+            __syncthreads();
+            if (first < d.ndefg) break;
+            __syncthreads();
+            if (i < d.ndefg) {
+                const uint32_t g = d.rorder[i];
+                uint32_t n = d.defcnt[g];
+#pragma unroll
+                for (uint32_t q = 0; q < GM_SUBS; q++) n -= d.defsub[(size_t)q * d.ndefg + g];
+                if (n) atomicMin(&first, i);
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) d.st->top_next = first;
+    }
+    if (threadIdx.x == 0) d.st->top_hit = hit;
     __syncthreads();
     copy_stats(d, out);
 }
 
-hipError_t gm_launch_window_end(const GmDev &d, const GmPart &P, uint32_t launched, GmStats *out, hipStream_t s) {
-    k_window_end<<<1, GM_BLOCK, 0, s>>>(d, P, launched, reinterpret_cast<uint32_t *>(out));
+hipError_t gm_launch_window_end(const GmDev &d, const GmPart &P, uint32_t launched, uint32_t top_pos, GmStats *out,
+                                hipStream_t s) {
+    k_window_end<<<1, GM_BLOCK, 0, s>>>(d, P, launched, top_pos, reinterpret_cast<uint32_t *>(out));
     return hipGetLastError();
 }
 
@@ -1754,7 +1863,7 @@ __global__ void __launch_bounds__(1024) k_arrivals(GmDev d, GmSweepArgs A) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
     for (uint32_t i = lo + tid; i < hi; i += 1024u) {
         const uint32_t id = d.arr_ids[i], c = d.nsite[id];
-        if (site_deformed(d, c)) atomicMin(&d.claim[c], id);
+        if (site_deformed(d, c)) atomicMin(&d.cell[c].x, id);
     }
     __syncthreads();
     uint32_t runI = st->nI, runB = st->nB, placed = 0;
@@ -1767,7 +1876,7 @@ __global__ void __launch_bounds__(1024) k_arrivals(GmDev d, GmSweepArgs A) {
             id = d.arr_ids[i];
             c = d.nsite[id];
             win = site_deformed(d, c) &&
-                  __hip_atomic_load(&d.claim[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == id;
+                  __hip_atomic_load(&d.cell[c].x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == id;
             in = win && site_interior(d, c);
         }
         const uint32_t vI = (win && in) ? 1u : 0u, vB = (win && !in) ? 1u : 0u;
@@ -1791,7 +1900,7 @@ __global__ void __launch_bounds__(1024) k_arrivals(GmDev d, GmSweepArgs A) {
                 atomicOr(&st->err, in ? GM_ERRF_INSIDE_FULL : GM_ERRF_BORDER_FULL);
             } else {
                 const uint32_t gslot = in ? rel : d.capI + rel;
-                const uint32_t g = d.grid[c];
+                const uint32_t g = d.cell[c].y;
                 const double P = d.nucP[id];
                 double inc = 0.0;
                 const gm_cs_t cs = cs_code(d, predict_values(d, A, k, 1.0, P, g, 26u, inc), k);

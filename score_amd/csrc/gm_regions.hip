@@ -579,7 +579,7 @@ __global__ void __launch_bounds__(GM_BLOCK) k_rg_propose(GmDev d) {
                 RgTarget o;
                 if (rg_target(d, box, q2.w, q2.x, q2.y, q2.z, (int)rk, o) && is_deformed(d, o.x, o.y, o.z)) {
                     att = true;
-                    atomicMin(&d.claim[cell_of(d, o.x, o.y, o.z)], o.khi | (p * 32u + rk));
+                    atomicMin(&d.cell[cell_of(d, o.x, o.y, o.z)].x, o.khi | (p * 32u + rk));
                 }
             }
             am |= (uint32_t)((__ballot(att) >> gsh) & ((1ull << GM_PG) - 1u)) << (GM_PG * i);
@@ -611,7 +611,7 @@ __global__ void __launch_bounds__(64) k_rg_decide(GmDev d) {
             const uint32_t rk = (uint32_t)__ffs(m) - 1u;
             RgTarget o;
             rg_target(d, box, q2.w, q2.x, q2.y, q2.z, (int)rk, o);
-            if (d.claim[cell_of(d, o.x, o.y, o.z)] != (o.khi | (p * 32u + rk))) continue;
+            if (d.cell[cell_of(d, o.x, o.y, o.z)].x != (o.khi | (p * 32u + rk))) continue;
             if (o.khi) {
                 mH |= 1u << rk;
 #pragma unroll
@@ -813,7 +813,7 @@ __global__ void __launch_bounds__(64) k_rg_commit(GmDev d, GmPParams pp, GmSweep
             RgTarget o;
             rg_target(d, box, pq2.w, pq2.x, pq2.y, pq2.z, (int)r, o);
             const uint32_t t = cell_of(d, o.x, o.y, o.z);
-            const uint32_t g = d.grid[t];
+            const uint32_t g = d.cell[t].y;
             /* the rank in the destination list, and that list's tables: the block's
              * own two lists' from LDS, a halo's receiving list's from memory */
             uint32_t rank, ix;
@@ -841,9 +841,9 @@ __global__ void __launch_bounds__(64) k_rg_commit(GmDev d, GmPParams pp, GmSweep
                 atomicOr(&st->err, (l & 1u) ? GM_ERRF_BORDER_FULL : GM_ERRF_INSIDE_FULL);
                 continue;
             }
-            infect_one(d, pp, A, k, sfin[j], sP[j], pq0, r, t, g, o.x, o.y, o.z, bs + rel, o.khi != 0u);
+            put_cell(d, k, new_cell(d, pp, A, k, sfin[j], sP[j], pq0, r, g, o.khi != 0u), pq0, t, g, o.x, o.y, o.z, bs + rel);
         }
-        retire_end(d, q0.z, retire_begin(d, q0, valid));
+        retire_batch(d, q0, valid);
 #pragma unroll
         for (int c = 0; c < GM_RROWS; c++) run[c] += bt[c];
         __syncthreads();
