@@ -671,7 +671,7 @@ static __device__ __forceinline__ uint32_t upper_index(const uint32_t *a, uint32
  * slot i, then Border slot i - nI; with several, region after region, each
  * Inside then Border (d.L.occ holds the lists' first occupied index). */
 static __device__ __forceinline__ uint32_t occ_slot(const GmDev &d, uint32_t nI, uint32_t i) {
-    if (d.nreg <= 1u) return i < nI ? i : d.capI + (i - nI);
+    if (d.nreg <= 1u) return i < nI ? d.baseI + i : i - nI;
     const uint32_t l = upper_index(d.L.occ, d.nlists, i);
     return d.L.base[l] + (i - d.L.occ[l]);
 }

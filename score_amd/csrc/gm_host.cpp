@@ -51,6 +51,7 @@ const double kRhoWellAnnealed = 1e8;
 const double kDefaultPmax = 0.0;
 const double kDefaultSmallNumber = 1e-6;
 const double kFullRecyclingAtt = 3.0;
+const uint64_t kMinFrontSlots = 1u << 20;      /* Inside slots a domain starts with, if it has as many cells */
 const int64_t kDefaultNmax = 1000000;          /* DEFAULT_NMAX, SCORE_Defs_Physics.h:133 */
 
 bool same_bits(double a, double b) { return memcmp(&a, &b, sizeof(double)) == 0; }
@@ -816,6 +817,92 @@ uint32_t arrivals_at(const score_gm_handle *h, uint32_t k) {
     return (k >= 1 && (size_t)k + 1 < h->arr_off.size()) ? h->arr_off[k + 1] - h->arr_off[k] : 0u;
 }
 
+/* the planes and masks of a step's parents, for at least `need` of them */
+int grow_parents(score_gm_handle *h, uint32_t need) {
+    GmDev &d = h->d;
+    const uint32_t nc = std::max<uint32_t>(need, d.parentCap + d.parentCap / 2);
+    dfree(h, d.pmI); dfree(h, d.pmB); dfree(h, d.par); dfree(h, d.pmH); dfree(h, d.plist);
+    dfree(h, d.ccnt); dfree(h, d.pmA);
+    d.pmA = d.pmI = d.pmB = d.pmH = d.plist = d.ccnt = nullptr;
+    d.par = nullptr;
+    d.parentCap = 0;
+    int rc;
+    if ((rc = dalloc(h, &d.pmI, nc)) || (rc = dalloc(h, &d.pmB, nc))) return rc;
+    if (d.nreg > 1) {
+        dfree(h, d.pslot);
+        d.pslot = nullptr;
+        if ((rc = dalloc(h, &d.pslot, nc)) || (rc = dalloc(h, &d.par, (size_t)GM_PAR_PLANES * nc)) ||
+            (rc = dalloc(h, &d.pmH, nc)) || (rc = dalloc(h, &d.plist, nc)))
+            return rc;
+    } else if ((rc = dalloc(h, &d.par, (size_t)GM_PAR1_PLANES * nc)) || (rc = dalloc(h, &d.pmA, nc)) ||
+               (rc = dalloc(h, &d.ccnt, (size_t)nc / 16 + 1))) {
+        return rc;
+    }
+    d.parentCap = nc;
+    return 0;
+}
+
+/* The Inside list grows by doubling, as SCORE's does, to at least `need` slots: it
+ * lies behind the Border list, so no slot changes its number.  New slots are
+ * INACTIVE.  Where both copies would hold more than a slot per cell the old one
+ * waits in host memory, so that a domain never needs more device memory than lists
+ * of full length (score_gm_footprint). */
+int grow_front(score_gm_handle *h, uint32_t need) {
+    GmDev &d = h->d;
+    uint64_t nc = (std::max<uint64_t>(need, 2ull * d.capI) + 63) / 64 * 64;
+    const bool staged = nc + d.capI > d.capImax;
+    if (staged) nc = d.capImax;
+    const size_t used = (size_t)d.baseI + d.capI, tot = (size_t)d.baseI + nc + GM_SW_CHUNK;
+    GmRec *rec = d.rec;
+    gm_cs_t *cs = d.cstep;
+    char *keep = nullptr;
+    if (staged) {
+        keep = static_cast<char *>(malloc(used * (sizeof(GmRec) + sizeof(gm_cs_t))));
+        if (!keep) return fail(SCORE_GM_ERR_OOM, "host memory for the front list");
+        hipError_t e;
+        if ((e = hipMemcpyAsync(keep, rec, sizeof(GmRec) * used, hipMemcpyDeviceToHost, h->stream)) != hipSuccess ||
+            (e = hipMemcpyAsync(keep + sizeof(GmRec) * used, cs, sizeof(gm_cs_t) * used, hipMemcpyDeviceToHost,
+                                h->stream)) != hipSuccess ||
+            (e = hipStreamSynchronize(h->stream)) != hipSuccess) {
+            free(keep);
+            return hip_fail(e, "growing the Inside list");
+        }
+        dfree(h, rec);
+        dfree(h, cs);
+        d.rec = nullptr;
+        d.cstep = nullptr;
+    }
+    GmRec *nrec = nullptr;
+    gm_cs_t *ncs = nullptr;
+    int rc;
+    if ((rc = dalloc(h, &nrec, tot)) || (rc = dalloc(h, &ncs, tot))) {
+        dfree(h, nrec);
+        free(keep);
+        return rc;
+    }
+    const hipMemcpyKind kind = staged ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
+    const void *from = staged ? (const void *)keep : (const void *)rec;
+    const void *fromcs = staged ? (const void *)(keep + sizeof(GmRec) * used) : (const void *)cs;
+    hipError_t e = gm_launch_fill_u32((uint32_t *)ncs, 0xFFFFFFFFu, tot / 2, h->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(nrec, from, sizeof(GmRec) * used, kind, h->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(ncs, fromcs, sizeof(gm_cs_t) * used, kind, h->stream);
+    if (e == hipSuccess && staged) e = hipStreamSynchronize(h->stream);
+    free(keep);
+    if (e != hipSuccess) {
+        dfree(h, nrec);
+        dfree(h, ncs);
+        return hip_fail(e, "growing the Inside list");
+    }
+    if (!staged) {
+        dfree(h, rec);
+        dfree(h, cs);
+    }
+    d.rec = nrec;
+    d.cstep = ncs;
+    d.capI = (uint32_t)nc;
+    return 0;
+}
+
 /* per-step lists, tile masks and per-parent masks sized for the current
  * occupancy and the next step's arrivals (to either list) */
 int ensure_step_capacity(score_gm_handle *h) {
@@ -832,22 +919,20 @@ int ensure_step_capacity(score_gm_handle *h) {
         if ((d.nreg > 1 && (rc = dalloc(h, &d.mF, nc))) || (rc = dalloc(h, &d.mR, nc))) return rc;
         d.tileCap = nc;
     }
-    const uint32_t parents = h->nI + h->nB + na;
-    if (parents > d.parentCap) {
-        uint32_t nc = std::max<uint32_t>(parents, d.parentCap + d.parentCap / 2);
-        dfree(h, d.pmI); dfree(h, d.pmB); dfree(h, d.pslot); dfree(h, d.par); dfree(h, d.pmH); dfree(h, d.plist);
-        dfree(h, d.ccnt); dfree(h, d.pmA);
-        d.pmA = d.pmI = d.pmB = d.pslot = d.pmH = d.plist = d.ccnt = nullptr;
-        d.par = nullptr;
-        d.parentCap = 0;
-        int rc;
-        if ((rc = dalloc(h, &d.pmI, nc)) || (rc = dalloc(h, &d.pmB, nc)) || (rc = dalloc(h, &d.pslot, nc)) ||
-            (rc = dalloc(h, &d.par, (size_t)(d.nreg > 1 ? GM_PAR_PLANES : GM_PAR1_PLANES) * nc)) || (d.nreg > 1 && ((rc = dalloc(h, &d.pmH, nc)) || (rc = dalloc(h, &d.plist, nc)))) ||
-            (d.nreg <= 1 && ((rc = dalloc(h, &d.ccnt, (size_t)nc / 16 + 1)) || (rc = dalloc(h, &d.pmA, nc)))))
-            return rc;
-        d.parentCap = nc;
+    int rc;
+    const uint32_t slots = h->nI + h->nB + na;
+    if (d.nreg > 1) return slots > d.parentCap ? grow_parents(h, slots) : 0;
+    if (slots > d.pslotCap) {
+        const uint32_t nc = std::max<uint32_t>(slots, d.pslotCap + d.pslotCap / 2);
+        dfree(h, d.pslot);
+        d.pslot = nullptr;
+        d.pslotCap = 0;
+        if ((rc = dalloc(h, &d.pslot, nc))) return rc;
+        d.pslotCap = nc;
     }
-    return 0;
+    /* the arrivals of the step may all go to the Inside list */
+    const uint64_t need = std::min<uint64_t>((uint64_t)h->nI + na, d.capImax);
+    return need > d.capI ? grow_front(h, (uint32_t)need) : 0;
 }
 
 /* Evaluate the pending pairs with glibc and store them in the device cache. */
@@ -906,8 +991,8 @@ int grow_pcache(score_gm_handle *h, uint64_t room = 0) {
         if (rc) return rc;
         for (uint32_t l = 0; l < d.nlists; l++) HIPCHK(gm_launch_materialize(d, h->step, h->lbase[l], ln[l], none, h->stream));
     } else {
-        HIPCHK(gm_launch_materialize(d, h->step, 0, h->nI, none, h->stream));
-        HIPCHK(gm_launch_materialize(d, h->step, d.capI, h->nB, none, h->stream));
+        HIPCHK(gm_launch_materialize(d, h->step, d.baseI, h->nI, none, h->stream));
+        HIPCHK(gm_launch_materialize(d, h->step, 0, h->nB, none, h->stream));
     }
     std::vector<unsigned long long> keys(d.hcap);
     std::vector<double> vals(d.hcap);
@@ -1215,7 +1300,7 @@ GmPart window_part(const score_gm_handle *h, uint32_t nI, uint32_t nB, uint32_t 
 
 /* entries of a row of sweep-block tables: enough for window_part of full lists */
 uint32_t sweep_block_rows(const GmDev &d) {
-    const uint64_t ch = ((uint64_t)d.capI + GM_SW_CHUNK - 1) / GM_SW_CHUNK + ((uint64_t)d.capB + GM_SW_CHUNK - 1) / GM_SW_CHUNK;
+    const uint64_t ch = ((uint64_t)d.capImax + GM_SW_CHUNK - 1) / GM_SW_CHUNK + ((uint64_t)d.capB + GM_SW_CHUNK - 1) / GM_SW_CHUNK;
     const uint64_t nb = ch / (GM_SW_WAVES * GM_SW_MAXCPW) + 2;
     return (uint32_t)((std::max<uint64_t>(nb, GM_SW_BLOCKS) + 63) / 64 * 64);
 }
@@ -1238,7 +1323,7 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
                 if ((rc = defragment_list(h, h->lbase[l], h->lcap[l], n[l]))) return h->err = rc;
             if ((rc = set_list_lengths(h, n))) return h->err = rc;
         } else {
-            if ((rc = defragment_list(h, 0u, d.capI, h->nI)) || (rc = defragment_list(h, d.capI, d.capB, h->nB)))
+            if ((rc = defragment_list(h, d.baseI, d.capI, h->nI)) || (rc = defragment_list(h, 0u, d.capB, h->nB)))
                 return h->err = rc;
             /* the device keeps the list lengths in its stats */
             hipError_t e2;
@@ -1320,6 +1405,23 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
                    : gm_launch_window_end(d, P, launched, w.top_pos, h->hst_dev, h->stream);
     if (e != hipSuccess || (e = hipStreamSynchronize(h->stream)) != hipSuccess)
         return h->err = hip_fail(e, "growth step");
+    /* a step that found too few Inside slots or parents' entries waits for them:
+     * step nexec runs on from its commit pass, or the first step from its start */
+    while (d.nreg <= 1 && !h->hst->err && (h->hst->grow || (h->hst->need_par && h->hst->nexec == 0))) {
+        const uint32_t j0 = h->hst->nexec, grow = h->hst->grow;
+        if ((rc = grow ? grow_front(h, grow) : grow_parents(h, h->hst->need_par))) return h->err = rc;
+        if ((e = gm_launch_fill_u32(&d.st->grow, 0u, 2, h->stream)) != hipSuccess ||
+            (e = gm_launch_fill_u32(&d.st->halt, 0u, 1, h->stream)) != hipSuccess ||
+            (grow && (e = gm_launch_commit(d, h->pp, a, P, j0, h->stream, ev)) != hipSuccess))
+            return h->err = hip_fail(e, "growth step");
+        for (uint32_t j = grow ? j0 + 1u : 0u; j < W; j++)
+            if ((e = gm_launch_infect(d, h->pp, a, P, w, j, h->stream, ev)) != hipSuccess)
+                return h->err = hip_fail(e, "growth step");
+        if ((e = gm_launch_window_end(d, P, W, w.top_pos, h->hst_dev, h->stream)) != hipSuccess ||
+            (e = hipStreamSynchronize(h->stream)) != hipSuccess)
+            return h->err = hip_fail(e, "growth step");
+    }
+    if (d.nreg <= 1 && !h->hst->err && h->hst->need_par && (rc = grow_parents(h, h->hst->need_par))) return h->err = rc;
     h->last_sp = sp;
     h->have_last_sp = true;
     h->force_reanchor = false;
@@ -1576,17 +1678,32 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
     d.N = (uint64_t)dom->nx * dom->ny * dom->nz;
     d.ndefg = dom->n_defg; d.nrxg = dom->n_rxg;
     /* list capacities (ompshar_init_myRXFrontInside/Border, SCORE_Kernel.cpp:3587-3710):
-     * the Inside list may grow up to N here (rounded up to whole 64-slot tiles, so
-     * that the Border slots start on a tile); the Border list and both recycling
-     * lists are fixed */
+     * the Inside list grows up to N here; the Border list, whose 64-slot tiles come
+     * first, and both recycling lists are fixed */
     d.nreg = 1;
     d.nlists = 2;
     if (prm->n_regions > 1) {
         /* several regions: per-region lists (build_regions); the one-region sizes stay 0 */
         build_regions(h, (uint32_t)prm->n_regions);
     } else {
-        d.capI = (uint32_t)((d.N + 63) / 64 * 64);
+        /* SCORE starts with a cache of rel_cell_caching*N cells and doubles it (0.2 in
+         * its decks; of the measured domains the front never took more than 0.4);
+         * small domains get every cell's slot */
+        const double frac = std::min(1.0, std::max(0.125, prm->rel_cell_caching));
+        uint64_t slots = std::max<uint64_t>((uint64_t)(frac * (double)d.N) + 1, std::max<uint64_t>(kMinFrontSlots, d.nrxg));
+        if (const char *ev = getenv("SCORE_GM_FRONT_SLOTS")) { /* tests make the list grow with it */
+            char *end = nullptr;
+            const long v = strtol(ev, &end, 10);
+            if (end == ev || *end != '\0' || v < 1) {
+                delete h;
+                return fail(SCORE_GM_ERR_ARG, "SCORE_GM_FRONT_SLOTS must be a positive integer");
+            }
+            slots = std::max<uint64_t>({(uint64_t)v, d.nrxg, d.N / 16});
+        }
+        d.capImax = (uint32_t)((d.N + 63) / 64 * 64);
+        d.capI = (uint32_t)(std::min<uint64_t>(slots + 63, d.capImax) / 64 * 64);
         d.capB = 2 * ((d.nx * d.ny) + (d.nx * d.nz) + (d.ny * d.nz));
+        d.baseI = (d.capB + 63) / 64 * 64;
         d.recCapI = (uint32_t)(prm->rel_cell_caching * (double)d.N * prm->maxfill * kFullRecyclingAtt);
         d.recCapB = (uint32_t)((double)d.capB * prm->maxfill * kFullRecyclingAtt);
     }
@@ -1652,7 +1769,7 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
     h->pp.fac = 1.0 / sqrt(2.0);
 
     /* slots plus a margin of one sweep chunk (512 slots) */
-    const size_t capTot = multi ? (size_t)h->lbase[d.nlists] + 512 : (size_t)d.capI + (d.capB + 63) / 64 * 64 + 512;
+    const size_t capTot = multi ? (size_t)h->lbase[d.nlists] + 512 : (size_t)d.baseI + d.capI + 512;
     d.hcap = pow2_at_least(std::max<uint64_t>(65536, 4ull * d.nrxg));
     d.dlistCap = (uint32_t)std::min<uint64_t>(d.N, 1u << 20);
     /* completion steps further ahead than the horizon are re-predicted at its
@@ -1671,7 +1788,8 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
     d.dnby = (d.ny + 7) / 8;
     d.dnbz = (d.nz + 7) / 8;
     d.tileCap = (uint32_t)std::max<uint64_t>(1024, (d.N / 16) / 64);
-    d.parentCap = (uint32_t)std::max<uint64_t>(65536, d.N / 16);
+    d.parentCap = (uint32_t)std::max<uint64_t>(65536, multi ? d.N / 16 : d.N / 64);
+    d.pslotCap = (uint32_t)std::max<uint64_t>(65536, d.N / 16);
     if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
         (void)hipGetLastError();
         delete h;
@@ -1693,7 +1811,7 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
         (rc = dalloc(h, &d.cstep, capTot)) ||
         (rc = dalloc(h, &d.rec, capTot)) ||
         (rc = dalloc(h, &d.dlist, d.dlistCap)) ||
-        (rc = dalloc(h, &d.dmap, (size_t)d.dnbx * d.dnby * d.dnbz * 32)) || (rc = dalloc(h, &d.pslot, d.parentCap)) ||
+        (rc = dalloc(h, &d.dmap, (size_t)d.dnbx * d.dnby * d.dnbz * 32)) || (rc = dalloc(h, &d.pslot, multi ? d.parentCap : d.pslotCap)) ||
         (rc = dalloc(h, &d.par, (size_t)(multi ? GM_PAR_PLANES : GM_PAR1_PLANES) * d.parentCap)) || (rc = dalloc(h, &d.recI, d.recCapI)) || (rc = dalloc(h, &d.recB, d.recCapB)) ||
         (multi && (rc = dalloc(h, &d.mF, d.tileCap))) || (rc = dalloc(h, &d.mR, d.tileCap)) || (rc = dalloc(h, &d.pmI, d.parentCap)) ||
         (rc = dalloc(h, &d.pmB, d.parentCap)) || (rc = dalloc(h, &d.bcnt, GM_BCNT_ROWS * GM_MAX_BLOCKS)) ||
@@ -1965,7 +2083,7 @@ int score_gm_get_front(score_gm_handle *h, int32_t list, uint32_t cap, uint32_t 
     if (list < 0 || (uint32_t)list >= h->d.nlists) return fail(SCORE_GM_ERR_ARG, "unknown list");
     HIPCHK(hipSetDevice(h->device));
     uint32_t cnt = list == SCORE_GM_LIST_INSIDE ? h->nI : h->nB;
-    uint32_t base = list == SCORE_GM_LIST_INSIDE ? 0u : h->d.capI;
+    uint32_t base = list == SCORE_GM_LIST_INSIDE ? h->d.baseI : 0u;
     if (h->d.nreg > 1) {
         std::vector<uint32_t> ln;
         int rc = list_lengths(h, ln);
@@ -2084,6 +2202,14 @@ int batch_one(score_gm_batch_item &it, int32_t device, BatchGate &gate) {
             seen = gate.finished;
         }
         rc = score_gm_create(it.domain, it.params, device, &h);
+        if (rc == SCORE_GM_OK) {
+            /* the front list may ask for more memory while the domain grows */
+            rc = score_gm_run(h, &it.result);
+            if (rc != SCORE_GM_ERR_OOM) break;
+            score_gm_destroy(h);
+            h = nullptr;
+            memset(&it.result, 0, sizeof(it.result));
+        }
         if (rc != SCORE_GM_ERR_OOM) break;
         /* wait for a running domain to give its memory back; with none running
          * besides the waiting ones, it does not fit */
@@ -2093,8 +2219,7 @@ int batch_one(score_gm_batch_item &it, int32_t device, BatchGate &gate) {
         gate.cv.wait(lk, [&] { return gate.finished != seen; });
         gate.waiting--;
     }
-    if (rc) return rc;
-    rc = score_gm_run(h, &it.result);
+    if (!h) return rc;
     if (!rc && (it.defg_counts || it.rxg_counts)) rc = score_gm_get_counts(h, it.defg_counts, it.rxg_counts);
     if (!rc && it.grainmap) rc = score_gm_get_grainmap(h, it.grainmap, it.map_encoding);
     score_gm_destroy(h);

@@ -16,7 +16,8 @@
  *   dmap   1 bit per cell, set while the cell is deformed (infectable), blocked so
  *          that one 128-byte line holds a 16x8x8 brick of cells: a 3x3x3
  *          neighbourhood usually lies in one or two lines
- *   front  capI+capB slots: Inside list slots [0,capI), Border list slots [capI,capI+capB)
+ *   front  Border list slots [0,capB), then from baseI on the Inside list's, which
+ *          starts with SCORE's initial cache of cells and grows
  *          cstep uint16[slots]   completion step (mod GM_CS_MOD) or a GM_CS_*
  *                                sentinel; the only array every step reads in full
  *          rec   GmRec[slots]    64-byte record, read and written only when a cell
@@ -200,6 +201,8 @@ struct alignas(8) GmStats {
     uint32_t nattempt;        /* attempts that found a deformed target this step */
     uint32_t nzeroed;         /* several regions: deformed grains that lost their last cell in the window */
     uint32_t cwrap;           /* a deformed-grain count went past zero (one region: of a grain before the one that sets rhomax) */
+    uint32_t grow;            /* one region: the Inside slots a step's commit pass asks for before it can run */
+    uint32_t need_par;        /* one region: the parents of a step that has more than the planes hold */
     uint32_t top_hit;         /* one region: the grain that sets rhomax lost its last cell, */
     uint32_t top_next;        /* and the position of its successor in rorder (ndefg: none) */
     uint32_t dfirst;          /* defragmentation: first INACTIVE slot of the list */
@@ -324,7 +327,9 @@ struct GmDev {
     uint32_t nx, ny, nz, nxy;
     uint64_t N;
     uint32_t ndefg, nrxg;
-    uint32_t capI, capB;
+    uint32_t capI, capB;        /* slots of the lists */
+    uint32_t baseI;             /* first Inside slot (the Border list's 64-slot tiles come first) */
+    uint32_t capImax;           /* what capI may grow to: every cell */
     uint32_t recCapI, recCapB;
     /* state */
     uint2 *cell;                /* (claim, deformed grain) per cell */
@@ -344,7 +349,9 @@ struct GmDev {
     uint32_t *pmA;              /* per parent: ranks of its attempts on deformed cells (one region) */
     uint32_t *pmI, *pmB;        /* per parent: winning ranks into Inside / Border (several regions: pmI holds the
                                  * attempts until they are decided) */
-    /* pslot, par, pmI and pmB hold parentCap entries */
+    /* par, pmA, pmI and pmB hold parentCap entries (the parents of one step), and with
+     * several regions pslot too; with one region it holds pslotCap (of a window) */
+    uint32_t pslotCap;
     uint32_t *bcnt;             /* per-block counts and offsets, 8 x GM_MAX_BLOCKS */
     uint32_t *dlist;            /* slots of the cells left DEFERRED in a window (dlistCap entries) */
     uint32_t dlistCap;
@@ -445,6 +452,9 @@ hipError_t gm_launch_rg_place(const GmDev &d, const uint32_t *slots, const GmRec
 /* step j of a one-region window: infections and retirements */
 hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P,
                             const GmWindow &w, uint32_t j, hipStream_t s, hipEvent_t *ev);
+/* its last pass alone, after the Inside list has grown for it */
+hipError_t gm_launch_commit(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P, uint32_t j,
+                            hipStream_t s, hipEvent_t *ev);
 /* its end after `launched` steps: the last step's row, the stats into the host's mirror */
 hipError_t gm_launch_window_end(const GmDev &d, const GmPart &P, uint32_t launched, uint32_t top_pos, GmStats *out,
                                 hipStream_t s);

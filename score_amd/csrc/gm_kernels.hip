@@ -124,7 +124,7 @@ static __device__ __forceinline__ WaveChunks wave_chunks(const GmDev &d, const G
     WaveChunks r;
     r.c0 = first < nch ? first : nch;
     r.c1 = first + P.cpw < nch ? first + P.cpw : nch;
-    r.slot0 = inB ? d.capI : 0u;
+    r.slot0 = inB ? 0u : d.baseI;
     r.n = inB ? d.st->nB : d.st->nI;
     r.tile0 = (inB ? P.chI : 0u) * GM_SW_TPC;
     return r;
@@ -188,6 +188,8 @@ __global__ void __launch_bounds__(GM_BLOCK) k_sweep(GmDev d, GmPart P, uint32_t 
         st->pone = 0;
         st->cwrap = 0;
         st->novf = 0;
+        st->grow = 0;
+        st->need_par = 0;
         d.win->nret0 = st->nret;
         d.win->xcells0 = xcells;
         d.win->npend0 = 0;
@@ -783,16 +785,18 @@ static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, 
 
 /* Whether step j of the window must not run: the host has to act on what step
  * j-1 left (an error, a count that wrapped, the exhaustion of the grain that
- * sets rhomax, Xcells at a threshold, weights the window cannot wait for).  Every
+ * sets rhomax, Xcells at a threshold, weights the window cannot wait for, a step
+ * that found too few slots), or step j has more parents than the planes hold.  Every
  * input was written by an earlier kernel, so all blocks of the propose pass find
  * the same; it records the answer in st->halt for the step's other passes. */
 static __device__ __forceinline__ bool must_halt(const GmDev &d, const GmWindow &w, uint32_t j) {
     const GmStats *st = d.st;
     const GmWin *win = d.win;
     /* every word loaded before the first test */
-    const uint32_t flags = st->err | st->cwrap | st->novf | win->top_hit, npend = st->npend;
+    const uint32_t flags = st->err | st->cwrap | st->novf | win->top_hit | st->grow, npend = st->npend;
     const double xc = win->xcells0 + (double)win->off[j];
-    return (flags != 0u) | ((npend != 0u) & !w.defer) | (npend > w.pend_limit) | ((j != 0u) & (xc >= w.xstop));
+    return (flags != 0u) | ((npend != 0u) & !w.defer) | (npend > w.pend_limit) | ((j != 0u) & (xc >= w.xstop)) |
+           (win->full[j] > d.parentCap);
 }
 
 /* The deformed bits around a cell: nine per plane, bit (dy+1)*3 + dx+1, for the
@@ -899,9 +903,12 @@ __global__ void __launch_bounds__(GM_BLOCK) k_propose(GmDev d, GmPart P, GmWindo
     const uint32_t nfull = win->full[j], off = win->off[j];
     const bool halt = must_halt(d, wd, j);
     if (blockIdx.x == 0) {
-        if (j) close_step(d, P, j - 1u, !halt);
+        /* a step whose commit pass found too few slots is not done */
+        const uint32_t undone = st->grow;
+        if (j && !undone) close_step(d, P, j - 1u, !halt);
         if (threadIdx.x == 0) {
             st->halt = halt ? 1u : 0u;
+            if (nfull > d.parentCap) st->need_par = nfull;
             if (d.prog)
                 __hip_atomic_store(d.prog, (j << 1) | (halt ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
@@ -924,7 +931,7 @@ __global__ void __launch_bounds__(GM_BLOCK) k_propose(GmDev d, GmPart P, GmWindo
         const double inc = r->inc;
         const uint32_t rxg = r->rxg, cell = rc.cell;
         const uint32_t z = cell / d.nxy, rem = cell - z * d.nxy, y = rem / d.nx, x = rem - y * d.nx;
-        const bool fromB = s >= d.capI;
+        const bool fromB = s < d.baseI;
         const bool interior = (x - 1u < d.nx - 2u) & (y - 1u < d.ny - 2u) & (z - 1u < d.nz - 2u);
         Neighbourhood nb;
         if (interior) nb.load(d, x, y, z);
@@ -1001,7 +1008,7 @@ static __device__ void recycle_blocks(const GmDev &d, const GmPart &P, uint32_t 
         const uint32_t nch = inB ? P.chB : P.chI, ch0 = (inB ? b - P.nbI : b) * GM_SW_WAVES * P.cpw;
         const uint32_t n = (ch0 + GM_SW_WAVES * P.cpw < nch ? GM_SW_WAVES * P.cpw : nch - ch0) * GM_SW_TPC;
         const uint32_t t0 = ((inB ? P.chI : 0u) + ch0) * GM_SW_TPC, merged = d.rmrg[b];
-        const uint32_t rel0 = ch0 * GM_SW_CHUNK, slot0 = (inB ? d.capI : 0u) + rel0;
+        const uint32_t rel0 = ch0 * GM_SW_CHUNK, slot0 = (inB ? 0u : d.baseI) + rel0;
         uint32_t run = 0;
         __syncthreads();
         for (uint32_t i0 = 0; i0 < n; i0 += GM_BLOCK) {
@@ -1160,16 +1167,6 @@ __global__ void __launch_bounds__(GM_BLOCK, 4) k_commit(GmDev d, GmPParams pp, G
     const uint32_t k = A.k, csz = ws.csz;
     const uint32_t nch = (nfull + csz - 1u) / csz, cpd = (nch + P.nbd - 1u) / P.nbd, db = blockIdx.x;
     const uint32_t c0 = db * cpd, c1 = c0 + cpd < nch ? c0 + cpd : nch;
-    if (db == 0) { /* the cells left of the grain that sets rhomax */
-        uint32_t n = 0, z0 = 0, z1 = 0;
-        for (uint32_t i = threadIdx.x; i < P.nbd; i += GM_BLOCK) n += d.btop[i];
-        block_sum3(n, z0, z1, sh);
-        if (threadIdx.x == 0 && n) {
-            const uint32_t left = d.win->top_left - n;
-            d.win->top_left = left;
-            if (left == 0u) d.win->top_hit = 1u;
-        }
-    }
     if (c0 >= nch) return;
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
     /* a lane's parent: winner masks | x | y, z | fromB, defg, rxg | fin, P; the
@@ -1202,21 +1199,42 @@ __global__ void __launch_bounds__(GM_BLOCK, 4) k_commit(GmDev d, GmPParams pp, G
     };
     uint32_t bI, bB;
     count(c0, c0 + wv < c1 ? c0 + wv : c1, bI, bB);
-    uint32_t runI = 0, runB = 0, dummy = 0;
-    for (uint32_t i0 = threadIdx.x; i0 < db; i0 += 4u * GM_BLOCK) {
+    uint32_t runI = 0, runB = 0, totI = 0;
+    for (uint32_t i0 = threadIdx.x; i0 < P.nbd; i0 += 4u * GM_BLOCK) {
         uint2 v[4];
 #pragma unroll
         for (uint32_t i = 0; i < 4u; i++) {
             v[i] = make_uint2(0u, 0u);
-            if (i0 + i * GM_BLOCK < db) v[i] = d.btot[i0 + i * GM_BLOCK];
+            if (i0 + i * GM_BLOCK < P.nbd) v[i] = d.btot[i0 + i * GM_BLOCK];
         }
 #pragma unroll
         for (uint32_t i = 0; i < 4u; i++) {
-            runI += v[i].x;
-            runB += v[i].y;
+            totI += v[i].x;
+            runI += i0 + i * GM_BLOCK < db ? v[i].x : 0u;
+            runB += i0 + i * GM_BLOCK < db ? v[i].y : 0u;
         }
     }
-    block_sum3(runI, runB, dummy, sh);
+    block_sum3(runI, runB, totI, sh);
+    /* every block finds the same: the Inside list must grow before the step's
+     * records go in, and the pass runs again */
+    const uint64_t need = (uint64_t)ws.nI + (totI > ws.recLenI ? totI - ws.recLenI : 0u);
+    if (need > d.capI && d.capI < d.capImax) {
+        if (db == 0 && threadIdx.x == 0) {
+            st->grow = need < d.capImax ? (uint32_t)need : d.capImax;
+            st->halt = 1u;
+        }
+        return;
+    }
+    if (db == 0) { /* the cells left of the grain that sets rhomax */
+        uint32_t n = 0, z0 = 0, z1 = 0;
+        for (uint32_t i = threadIdx.x; i < P.nbd; i += GM_BLOCK) n += d.btop[i];
+        block_sum3(n, z0, z1, sh);
+        if (threadIdx.x == 0 && n) {
+            const uint32_t left = d.win->top_left - n;
+            d.win->top_left = left;
+            if (left == 0u) d.win->top_hit = 1u;
+        }
+    }
     Wave &W = sw[wv];
     for (uint32_t c = c0 + wv; c < c1; c += GM_BLOCK / 64u) {
         if (c != c0 + wv) {
@@ -1274,7 +1292,7 @@ __global__ void __launch_bounds__(GM_BLOCK, 4) k_commit(GmDev d, GmPParams pp, G
                 atomicOr(&st->err, intoI ? GM_ERRF_INSIDE_FULL : GM_ERRF_BORDER_FULL);
                 continue;
             }
-            put_cell(d, k, nc, pq0, t, g, tx, ty, tz, intoI ? rel : d.capI + rel);
+            put_cell(d, k, nc, pq0, t, g, tx, ty, tz, intoI ? d.baseI + rel : rel);
         }
         wave_sync();
     }
@@ -1283,10 +1301,8 @@ __global__ void __launch_bounds__(GM_BLOCK, 4) k_commit(GmDev d, GmPParams pp, G
 hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P,
                             const GmWindow &w, uint32_t j, hipStream_t s, hipEvent_t *ev) {
     hipError_t e;
-    GmSweepArgs A = a;
-    A.k = a.k + j;
     if ((e = mark(ev, 4, s)) != hipSuccess) return e;
-    k_propose<<<P.nbp + 1u, GM_BLOCK, 0, s>>>(d, P, w, j, A.k);
+    k_propose<<<P.nbp + 1u, GM_BLOCK, 0, s>>>(d, P, w, j, a.k + j);
     if ((e = mark(ev, 5, s)) != hipSuccess) return e;
     const uint32_t nrec = P.nb < GM_RECYCLE_BLOCKS ? P.nb : GM_RECYCLE_BLOCKS;
     /* a sweep block's INACTIVE masks and the offsets of its tiles */
@@ -1294,6 +1310,14 @@ hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepAr
     k_decide<<<nrec + P.nbd, GM_BLOCK, lds, s>>>(d, P, j, nrec, w.top_pos);
     for (int i = 6; i <= 8; i++)
         if ((e = mark(ev, i, s)) != hipSuccess) return e;
+    return gm_launch_commit(d, pp, a, P, j, s, ev);
+}
+
+hipError_t gm_launch_commit(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P, uint32_t j,
+                            hipStream_t s, hipEvent_t *ev) {
+    hipError_t e;
+    GmSweepArgs A = a;
+    A.k = a.k + j;
     k_commit<<<P.nbd, GM_BLOCK, 0, s>>>(d, pp, A, P, j);
     if ((e = mark(ev, 9, s)) != hipSuccess) return e;
     return hipGetLastError();
@@ -1479,10 +1503,11 @@ __global__ void k_nuc_commit(GmDev d, const uint32_t *site, const double *nucP, 
         if (in) {
             gslot = d.nI_[k];
             if (gslot >= d.capI) { atomicOr(&d.st->err, GM_ERRF_INSIDE_FULL); continue; }
+            gslot += d.baseI;
         } else {
             uint32_t rel = d.nB_[k];
             if (rel >= d.capB) { atomicOr(&d.st->err, GM_ERRF_BORDER_FULL); continue; }
-            gslot = d.capI + rel;
+            gslot = rel;
         }
         uint32_t g = d.cell[w].y;
         GmRec *r = d.rec + gslot;
@@ -1899,7 +1924,7 @@ __global__ void __launch_bounds__(1024) k_arrivals(GmDev d, GmSweepArgs A) {
             if (rel >= (in ? d.capI : d.capB)) {
                 atomicOr(&st->err, in ? GM_ERRF_INSIDE_FULL : GM_ERRF_BORDER_FULL);
             } else {
-                const uint32_t gslot = in ? rel : d.capI + rel;
+                const uint32_t gslot = in ? d.baseI + rel : rel;
                 const uint32_t g = d.cell[c].y;
                 const double P = d.nucP[id];
                 double inc = 0.0;

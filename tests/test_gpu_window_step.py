@@ -68,3 +68,15 @@ def test_front_of_many_sweep_blocks(require_gpu):
         assert np.array_equal(fo[f][act], fg[f][act]), f
     assert np.array_equal(fo["activity"], fg["activity"])
     g.close()
+
+
+@pytest.mark.parametrize("slots,chunks", [(1, (9,)), (1, (2, 5)), (3000, (9, 1))])
+def test_inside_list_grows(require_gpu, monkeypatch, slots, chunks):
+    """The Inside list starts short, so that it has to grow before a commit pass (in
+    the first and in later steps of a window, twice in a row, and to a slot per cell
+    by way of host memory), with later arrivals and defragmentation between."""
+    monkeypatch.setenv("SCORE_GM_FRONT_SLOTS", str(slots))
+    dom = synth.make_voronoi_domain(34, 31, 29, n_grains=12, n_nuclei=400, seed=5)
+    _same(dom, ParamsSpec(defrag_at=(0.3 * dom.N, 0.6 * dom.N)), chunks)
+    sheet = synth.make_rolled_sheet_domain(48, 40, 16, n_grains=30, n_nuclei=600, arrival_steps=20, seed=3)
+    _same(sheet, ParamsSpec(rh_hagb_m0=2.0), chunks)
