@@ -127,7 +127,15 @@ double rh_omega_threshold(const score_gm_params &p) {
     /* margin of 0.2 degree: the weight's deficit falls by a large factor over it */
     const double theta_hi = hi + 0.2 / 180.0 * kPi;
     if (theta_hi >= 2.0 * acos(0.85)) return -1.0; /* beyond the largest cubic disorientation */
-    for (int i = 0; i <= 200000; i++) {
+    /* The weight is 1.0 - x with x = cut * exp(-trans * (theta / 15 deg)^n), which falls
+     * with theta, and rounds to 1.0 once x <= 2^-54.  The computed x is off by at most
+     * a factor 1 + arg * (n + 4) * 2^-52 (arg = trans * (theta / 15 deg)^n), which the
+     * margin of 2 below covers at theta_hi and, since x falls faster than arg grows,
+     * at every larger angle, while n and arg are moderate.  Other settings are checked
+     * at 200,001 angles (7 of the 8 ms a handle took to create). */
+    const double arg = p.rh_trans * pow((theta_hi / kLagbHagb), p.rh_exponent);
+    const bool sure = p.rh_exponent <= 1000.0 && arg >= 2.0 && arg <= 700.0 && p.rh_cut * exp(-1.0 * arg) <= 0x1p-55;
+    for (int i = 0; !sure && i <= 200000; i++) {
         double th = theta_hi + (kPi - theta_hi) * (double)i / 200000.0;
         if (rh_weight_of_theta(p, th) != 1.0) return -1.0;
     }
@@ -210,6 +218,16 @@ struct score_gm_handle {
      * capacities (2T lists, region r's Inside list 2r and Border list 2r+1) */
     std::vector<GmRegion> reg;
     std::vector<uint32_t> lbase, lcap, lrcap, lrbase;
+    char *stage = nullptr; /* pinned buffers of copy_staged; null: plain copies */
+    /* arena of the arrays made at creation */
+    struct Planned {
+        void **p;
+        size_t off;
+    };
+    std::vector<Planned> plan;
+    bool planning = false;
+    char *arena = nullptr;
+    size_t arena_bytes = 0;
     uint32_t last_full = 0xFFFFFFFFu; /* most cells completed in one step of the last window */
     uint32_t last_csz = 48;           /* parents per chunk after its last step */
 };
@@ -295,6 +313,88 @@ int pinned_mapped(score_gm_handle *h, void **host, void **dev, size_t bytes) {
     return 0;
 }
 
+/* Large copies between device and pageable host memory, in chunks through pinned
+ * buffers: worker k takes chunks k, k + T, ... and keeps two in flight, so that the
+ * host side of the copy (one core moves ~17 GB/s, and writes into fresh memory at
+ * 4 to 8 because it is mapped page by page on the way) runs on several cores beside
+ * the bus.  512 MiB: 17 -> 11 ms to the device, 63 (huge pages) to 125 -> 25 ms from
+ * it into fresh memory; below 16 MiB the runtime's own copy is as good.  Returns
+ * when the copy is done; `stream` orders it on the device. */
+constexpr size_t kStageChunk = 2u << 20, kStageMin = 16u << 20;
+constexpr unsigned kStageWorkers = 8;
+
+hipError_t copy_plain(void *dev, void *host, size_t bytes, bool to_host, hipStream_t s) {
+    const hipError_t e = to_host ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s)
+                                 : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+    return e != hipSuccess ? e : hipStreamSynchronize(s);
+}
+
+unsigned stage_workers() { return std::min(kStageWorkers, std::max(1u, std::thread::hardware_concurrency() / 2)); }
+
+/* `pin`: 2 chunks for each worker, or null (the plain copy) */
+hipError_t copy_staged(int device, char *pin, void *dev, void *host, size_t bytes, bool to_host, hipStream_t s) {
+    const size_t chunks = (bytes + kStageChunk - 1) / kStageChunk;
+    const unsigned T = stage_workers();
+    if (!pin || bytes < kStageMin) return copy_plain(dev, host, bytes, to_host, s);
+    std::atomic<int> err{hipSuccess};
+    auto work = [&](unsigned k) {
+        hipEvent_t ev[2] = {};
+        hipError_t e = hipSetDevice(device);
+        for (hipEvent_t &x : ev)
+            if (e == hipSuccess) e = hipEventCreateWithFlags(&x, hipEventDisableTiming);
+        char *buf[2] = {pin + 2 * kStageChunk * k, pin + 2 * kStageChunk * k + kStageChunk};
+        auto part = [&](size_t c, size_t &off) {
+            off = c * kStageChunk;
+            return std::min(kStageChunk, bytes - off);
+        };
+        size_t before = 0; /* the chunk before, still on the bus */
+        unsigned i = 0;
+        for (size_t c = k; c < chunks && e == hipSuccess && err.load() == hipSuccess; c += T, i++) {
+            size_t off, n = part(c, off);
+            if (to_host) {
+                e = hipMemcpyAsync(buf[i & 1u], (char *)dev + off, n, hipMemcpyDeviceToHost, s);
+                if (e == hipSuccess) e = hipEventRecord(ev[i & 1u], s);
+                if (i && e == hipSuccess && (e = hipEventSynchronize(ev[(i - 1u) & 1u])) == hipSuccess) {
+                    size_t o, m = part(before, o);
+                    memcpy((char *)host + o, buf[(i - 1u) & 1u], m);
+                }
+                before = c;
+            } else {
+                if (i >= 2) e = hipEventSynchronize(ev[i & 1u]);
+                if (e != hipSuccess) break;
+                memcpy(buf[i & 1u], (char *)host + off, n);
+                e = hipMemcpyAsync((char *)dev + off, buf[i & 1u], n, hipMemcpyHostToDevice, s);
+                if (e == hipSuccess) e = hipEventRecord(ev[i & 1u], s);
+            }
+        }
+        if (to_host && i && e == hipSuccess && (e = hipEventSynchronize(ev[(i - 1u) & 1u])) == hipSuccess) {
+            size_t o, m = part(before, o);
+            memcpy((char *)host + o, buf[(i - 1u) & 1u], m);
+        }
+        if (e != hipSuccess) err.store(e);
+        /* the buffers must be idle before they are given back */
+        for (hipEvent_t x : ev)
+            if (x) {
+                (void)hipEventSynchronize(x);
+                (void)hipEventDestroy(x);
+            }
+    };
+    std::thread th[kStageWorkers];
+    unsigned started = 0;
+    try {
+        for (; started + 1 < T; started++) th[started] = std::thread(work, started + 1);
+    } catch (...) {
+        /* fewer threads than asked: their chunks are this thread's */
+    }
+    work(0);
+    for (unsigned k = started + 1; k < T; k++) work(k);
+    for (unsigned t = 0; t < started; t++) th[t].join();
+    hipError_t e = (hipError_t)err.load();
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    else (void)hipStreamSynchronize(s);
+    return e;
+}
+
 /* Device memory comes from the device's stream-ordered pool on the handle's
  * stream: a free does not wait for the whole device (as hipFree does), so
  * handles created and destroyed next to running ones do not stall them, and
@@ -303,6 +403,12 @@ template <typename T>
 int dalloc(score_gm_handle *h, T **p, size_t n) {
     *p = nullptr;
     if (n == 0) n = 1;
+    if (h->planning) {
+        /* an array of the handle's arena: placed when all are known (arena_place) */
+        h->plan.push_back({reinterpret_cast<void **>(p), h->arena_bytes});
+        h->arena_bytes += (n * sizeof(T) + 255) / 256 * 256;
+        return 0;
+    }
     hipError_t e = hipMallocFromPoolAsync((void **)p, n * sizeof(T), h->pool, h->stream);
     if (e != hipSuccess) {
         *p = nullptr;
@@ -314,7 +420,24 @@ int dalloc(score_gm_handle *h, T **p, size_t n) {
 }
 
 void dfree(score_gm_handle *h, void *p) {
+    /* what lies in the arena goes with it */
+    const char *c = static_cast<const char *>(p);
+    if (h->arena && c >= h->arena && c < h->arena + h->arena_bytes) return;
     if (p) (void)hipFreeAsync(p, h->stream);
+}
+
+/* The arrays a handle is created with, in one block: some 50 allocations and frees
+ * cost 0.3 to 3 ms a handle, and 24 domains of a batch 235 ms instead of 200.  An
+ * array that is replaced by a longer one leaves its place in the block unused. */
+int arena_place(score_gm_handle *h) {
+    h->planning = false;
+    char *block = nullptr;
+    const int rc = dalloc(h, &block, h->arena_bytes);
+    if (rc) return rc;
+    h->arena = block;
+    for (const score_gm_handle::Planned &q : h->plan) *q.p = block + q.off;
+    h->plan.clear();
+    return 0;
 }
 
 void free_device(score_gm_handle *h) {
@@ -328,7 +451,12 @@ void free_device(score_gm_handle *h) {
                     d.L.win, d.L.occ, d.L.tile, d.L.tile_s, d.L.par, d.L.rst, d.L.rbuf, d.L.rs, d.L.bstart, d.L.breg,
                     d.L.hoff, d.plist};
     for (void *q : ptrs) dfree(h, q);
+    if (h->arena) (void)hipFreeAsync(h->arena, h->stream);
+    h->arena = nullptr;
+    h->arena_bytes = 0;
     memset(&h->d, 0, sizeof(h->d));
+    if (h->stage) (void)hipHostFree(h->stage);
+    h->stage = nullptr;
     if (h->hst) (void)hipHostFree(h->hst);
     h->hst = nullptr;
     h->hst_dev = nullptr;
@@ -1720,6 +1848,10 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
      * counted on the device */
     std::vector<uint32_t> defcnt(d.ndefg, 0u);
 
+    h->pp.model = prm->mobility_model;
+    h->pp.omega_hi = rh_omega_threshold(h->p);
+    h->pp.fac = 1.0 / sqrt(2.0);
+
     /* nucleus weights with glibc (calc_mobilityweight, SCORE_GrowthMachine.cpp:152); a
      * nucleus keeps the deformed grain of its site until it arrives, since a cell
      * changes its grain only by transforming, which rejects the nucleus.  The
@@ -1732,13 +1864,17 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
         std::vector<uint64_t> seen((d.N + 63) / 64, 0ull);
         uint32_t last = 0;
         for (uint32_t k = 0; k < d.nrxg; k++) {
+            if (k + 16u < d.nrxg) __builtin_prefetch(&dom->cellgrid[dom->rxg_site[k + 16u]]);
             const uint32_t w = dom->rxg_site[k];
             const uint32_t g = dom->cellgrid[w];
             if (g >= d.ndefg) {
                 delete h;
                 return fail(SCORE_GM_ERR_ARG, kBadGrid);
             }
-            nucP[k] = mobility_weight(h->p, &h->rxq[4 * (size_t)k], &h->defq[4 * (size_t)g]);
+            /* as the device: 1.0 exactly far above the LAGB/HAGB transition */
+            const double *qr = &h->rxq[4 * (size_t)k], *qd = &h->defq[4 * (size_t)g];
+            nucP[k] = h->pp.omega_hi >= 0.0 && score_orient::disori_omega(qr, qd) <= h->pp.omega_hi
+                          ? 1.0 : mobility_weight(h->p, qr, qd);
             const uint32_t ks = dom->rxg_step ? dom->rxg_step[k] : 0u;
             if (ks > last) last = ks;
             if (ks != 0) continue;
@@ -1763,10 +1899,6 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
             d.arr_last = last;
         }
     }
-
-    h->pp.model = prm->mobility_model;
-    h->pp.omega_hi = rh_omega_threshold(h->p);
-    h->pp.fac = 1.0 / sqrt(2.0);
 
     /* slots plus a margin of one sweep chunk (512 slots) */
     const size_t capTot = multi ? (size_t)h->lbase[d.nlists] + 512 : (size_t)d.baseI + d.capI + 512;
@@ -1806,10 +1938,15 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
     if (multi)
         for (uint32_t r = 0; r < d.nreg; r++) capBsum += h->lcap[2 * r + 1];
     d.rlogCap = d.N + capBsum + 4096u;
+    /* the front lists may be replaced by longer ones, so they stand by themselves */
+    if ((rc = dalloc(h, &d.cstep, capTot)) || (rc = dalloc(h, &d.rec, capTot))) {
+        free_device(h);
+        delete h;
+        return rc;
+    }
+    h->planning = true;
     if ((rc = dalloc(h, &d.cell, d.N)) ||
         (rc = dalloc(h, &d.rlog, d.rlogCap)) ||
-        (rc = dalloc(h, &d.cstep, capTot)) ||
-        (rc = dalloc(h, &d.rec, capTot)) ||
         (rc = dalloc(h, &d.dlist, d.dlistCap)) ||
         (rc = dalloc(h, &d.dmap, (size_t)d.dnbx * d.dnby * d.dnbz * 32)) || (rc = dalloc(h, &d.pslot, multi ? d.parentCap : d.pslotCap)) ||
         (rc = dalloc(h, &d.par, (size_t)(multi ? GM_PAR_PLANES : GM_PAR1_PLANES) * d.parentCap)) || (rc = dalloc(h, &d.recI, d.recCapI)) || (rc = dalloc(h, &d.recB, d.recCapB)) ||
@@ -1869,7 +2006,7 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
         delete h;
         return rc;
     }
-    if ((rc = pinned_mapped(h, (void **)&h->hst, (void **)&h->hst_dev, sizeof(GmStats))) ||
+    if ((rc = arena_place(h)) || (rc = pinned_mapped(h, (void **)&h->hst, (void **)&h->hst_dev, sizeof(GmStats))) ||
         (rc = pinned_mapped(h, (void **)&h->hprog, (void **)&h->hprog_dev, 64))) {
         free_device(h);
         delete h;
@@ -1880,9 +2017,15 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
     double *d_nucP = nullptr;
     auto setup = [&]() -> int {
         hipStream_t s = h->stream;
+        /* without them (no pinned memory left) the grid and the maps are copied plainly */
+        if (sizeof(uint32_t) * d.N >= kStageMin && stage_workers() > 1 &&
+            hipHostMalloc((void **)&h->stage, 2 * kStageChunk * stage_workers(), hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            h->stage = nullptr;
+        }
         /* the grid arrives in the record array, which nothing uses yet */
         uint32_t *src = reinterpret_cast<uint32_t *>(d.rec);
-        HIPCHK(hipMemcpyAsync(src, dom->cellgrid, sizeof(uint32_t) * d.N, hipMemcpyHostToDevice, s));
+        HIPCHK(copy_staged(device, h->stage, src, const_cast<uint32_t *>(dom->cellgrid), sizeof(uint32_t) * d.N, false, s));
         HIPCHK(gm_launch_fill_u32(d.defcnt, 0u, d.ndefg, s));
         if (!multi) HIPCHK(gm_launch_fill_u32(d.defsub, 0u, (size_t)GM_SUBS * d.ndefg, s));
         HIPCHK(gm_launch_fill_u32((uint32_t *)d.st, 0u, sizeof(GmStats) / 4, s));
@@ -2034,16 +2177,13 @@ int score_gm_get_grainmap(score_gm_handle *h, uint32_t *out, int32_t encoding) {
     if (rc) return rc;
     auto copy = [&]() -> int {
         HIPCHK(gm_launch_overlay_infected(h->d, h->nI, h->nB, h->step, tmp, h->stream));
-        HIPCHK(hipMemcpyAsync(out, tmp, sizeof(uint32_t) * h->d.N, hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(hipStreamSynchronize(h->stream));
+        if (encoding == SCORE_GM_MAP_RAW2GID) HIPCHK(gm_launch_raw2gid(tmp, h->d.N, h->stream));
+        HIPCHK(copy_staged(h->device, h->stage, tmp, out, sizeof(uint32_t) * h->d.N, true, h->stream));
         return 0;
     };
     rc = copy();
     dfree(h, tmp);
-    if (rc) return rc;
-    if (encoding == SCORE_GM_MAP_RAW2GID)
-        for (uint64_t i = 0; i < h->d.N; i++) out[i] = out[i] == GM_INFECTED ? 1u : 2u + out[i];
-    return 0;
+    return rc;
 }
 
 int score_gm_get_counts(score_gm_handle *h, uint32_t *defg_counts, uint32_t *rxg_counts) {

@@ -1323,6 +1323,17 @@ hipError_t gm_launch_commit(const GmDev &d, const GmPParams &pp, const GmSweepAr
     return hipGetLastError();
 }
 
+/* exported map, SCORE's raw file encoding: 1 for an infected cell, else 2 + id */
+__global__ void k_raw2gid(uint32_t *m, uint64_t n) {
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+        m[i] = m[i] == GM_INFECTED ? 1u : 2u + m[i];
+}
+
+hipError_t gm_launch_raw2gid(uint32_t *m, uint64_t n, hipStream_t s) {
+    k_raw2gid<<<fill_blocks(n), GM_BLOCK, 0, s>>>(m, n);
+    return hipGetLastError();
+}
+
 /* exported map: the grains the cells came with */
 __global__ void k_grid_out(GmDev d, uint32_t *out) {
     const uint32_t n2 = (uint32_t)(d.N / 2u);

@@ -39,8 +39,8 @@ inline void grimmer(const double *r, double (*c)[4]) {
     c[5][0] = a; c[5][1] = b; c[5][2] = cc; c[5][3] = d;
 }
 
-/* disori_angle_oriquat_cubic_imm (SCORE_Math.cpp:558-622), radians */
-inline double disori_angle(const double *p, const double *q) {
+/* the largest |component| over the Grimmer candidates (SCORE_Math.cpp:604-608) */
+inline double disori_omega(const double *p, const double *q) {
     double r[4], c[6][4];
     misorientation(p, q, r);
     grimmer(r, c);
@@ -48,6 +48,12 @@ inline double disori_angle(const double *p, const double *q) {
     for (int i = 0; i < 6; i++)
         for (int j = 0; j < 4; j++)
             if (fabs(c[i][j]) > omega) omega = fabs(c[i][j]);
+    return omega;
+}
+
+/* disori_angle_oriquat_cubic_imm (SCORE_Math.cpp:558-622), radians */
+inline double disori_angle(const double *p, const double *q) {
+    const double omega = disori_omega(p, q);
     if (omega < (1.0 - kDoubleAccuracy)) return 2.0 * acos(omega);
     return 0.0;
 }
