@@ -234,7 +234,7 @@ static __device__ __forceinline__ bool cell_increment(const GmDev &d, const GmSw
  * when none up to the step cap does).  Sets the increment (0.0 for a cell SCORE
  * does not advance).  The value after the completing addition, whose excess
  * over 1.0 the infection carries on, is replayed from the anchor when the cell
- * completes and wins a target (parent_fin). */
+ * completes (the propose passes). */
 static __device__ __forceinline__ uint32_t predict_values(const GmDev &d, const GmSweepArgs &A, uint32_t k, double f,
                                                           double P, uint32_t defg, uint32_t inf, double &inc) {
     uint32_t cs = GM_STEP_NONE;
@@ -256,15 +256,6 @@ static __device__ __forceinline__ uint32_t predict_values(const GmDev &d, const 
 /* f after n >= 1 additions of inc */
 static __device__ __forceinline__ double advanced(double f, double inc, uint32_t n) {
     return n == 1u ? f + inc : gm_radd_n(f, inc, n);
-}
-
-/* rxFrac of a parent after its completing addition in step k: n = k - s0 + 1
- * additions of its increment to the value it was anchored with before step s0 */
-static __device__ __forceinline__ double parent_fin(const GmDev &d, uint32_t slot, uint32_t k) {
-    const GmRec *r = d.rec + slot;
-    const RecA a = rec_a(r);
-    const double inc = r->inc;
-    return advanced(a.frac0, inc, k - a.s0 + 1u);
 }
 
 /* the stored code of completion step cs predicted at step kp */
@@ -403,6 +394,93 @@ static __device__ __forceinline__ void clear_deformed(const GmDev &d, uint32_t x
 }
 
 
+/* The deformed bits around a cell: nine per plane, bit (dy+1)*3 + dx+1, for the
+ * cell's own plane, the one below and the one above, in the order of the attempts'
+ * ranks (SCORE_Kernel.cpp:4611-4638: the own plane without the cell itself, the
+ * lower plane with its row y+1 first, the upper plane). */
+static __device__ __forceinline__ uint32_t rank_mask(uint32_t m, uint32_t dn, uint32_t up) {
+    const uint32_t lower = (dn >> 6 & 7u) | (dn & 7u) << 3 | (dn >> 3 & 7u) << 6;
+    return (m & 0xFu) | (m >> 1 & 0xF0u) | lower << 8 | up << 17;
+}
+
+/* A strictly interior cell's neighbourhood in the bitmap.  A brick holds 16 x 8
+ * cells of a plane in 16 bytes, a row of 16 cells in 16 bits, so one 16-byte load
+ * a plane usually covers the nine cells; a cell at a brick's edge also loads from
+ * the bricks beside it.  The loads of all planes are issued together (load), so
+ * that the caller can work until it needs them (mask). */
+struct Neighbourhood {
+    uint4 c[3], cx[3];          /* planes z, z-1, z+1: the cell's brick, the one beside it along x */
+    uint32_t ry[3], rxy[3];     /* the word with the adjacent row of the bricks beside along y */
+    uint32_t xi, yi;
+    __device__ __forceinline__ void load(const GmDev &d, uint32_t x, uint32_t y, uint32_t z) {
+        const uint4 *D = reinterpret_cast<const uint4 *>(d.dmap);
+        xi = x & 15u;
+        yi = y & 7u;
+        const uint32_t row = (x >> 4) + d.dnbx * (y >> 3), layer = d.dnbx * d.dnby;
+        uint32_t at[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const uint32_t zi = i == 0 ? z : i == 1 ? z - 1u : z + 1u;
+            at[i] = (row + layer * (zi >> 3)) * 8u + (zi & 7u);
+            c[i] = D[at[i]];
+            cx[i] = make_uint4(0u, 0u, 0u, 0u);
+            ry[i] = rxy[i] = 0;
+        }
+        const bool ex = xi == 0u || xi == 15u, ey = yi == 0u || yi == 7u;
+        const uint32_t sx = xi ? 8u : 0u - 8u, sy = (yi ? 8u : 0u - 8u) * d.dnbx, yw = yi ? 0u : 3u;
+        if (ex) {
+#pragma unroll
+            for (int i = 0; i < 3; i++) cx[i] = D[at[i] + sx];
+        }
+        if (ey) {
+#pragma unroll
+            for (int i = 0; i < 3; i++) ry[i] = d.dmap[(at[i] + sy) * 4u + yw];
+        }
+        if (ex && ey) {
+#pragma unroll
+            for (int i = 0; i < 3; i++) rxy[i] = d.dmap[(at[i] + sx + sy) * 4u + yw];
+        }
+    }
+    /* three rows of 16 bits, y-1 first */
+    __device__ __forceinline__ unsigned long long rows(const uint4 &q, uint32_t r) const {
+        const unsigned long long lo = (unsigned long long)q.y << 32 | q.x, hi = (unsigned long long)q.w << 32 | q.z;
+        const uint32_t s = 16u * (yi - 1u);
+        unsigned long long v = s < 64u ? lo >> (s & 63u) : hi >> (s & 63u);
+        if (s != 0u && s < 64u) v |= hi << (64u - s);
+        if (yi == 0u) v = lo << 16 | r >> 16;
+        if (yi == 7u) v = hi >> 32 | (unsigned long long)(r & 0xFFFFu) << 32;
+        return v;
+    }
+    __device__ __forceinline__ uint32_t plane(int i) const {
+        const unsigned long long one = 0x0000000100010001ull;
+        const unsigned long long T = rows(c[i], ry[i]), TX = rows(cx[i], rxy[i]);
+        unsigned long long U = T >> ((xi - 1u) & 63u);
+        if (xi == 0u) U = (T & 3u * one) << 1 | (TX >> 15 & one);
+        if (xi == 15u) U = (T >> 14 & 3u * one) | (TX & one) << 2;
+        return (uint32_t)(U & 7u) | (uint32_t)(U >> 13 & 0x38u) | (uint32_t)(U >> 26 & 0x1C0u);
+    }
+    __device__ __forceinline__ uint32_t mask() const { return rank_mask(plane(0), plane(1), plane(2)); }
+};
+
+/* The attempts of a Border cell on a face of the domain: x and y wrap, planes
+ * outside z have none.  27 single words, all loaded together. */
+static __device__ __forceinline__ uint32_t face_attempts(const GmDev &d, uint32_t x, uint32_t y, uint32_t z) {
+    const uint32_t xs[3] = {x ? x - 1u : d.nx - 1u, x, x + 1u < d.nx ? x + 1u : 0u};
+    const uint32_t ys[3] = {y ? y - 1u : d.ny - 1u, y, y + 1u < d.ny ? y + 1u : 0u};
+    uint32_t wd[27];
+#pragma unroll
+    for (int i = 0; i < 27; i++) {
+        const uint32_t zz = i < 9 ? z : i < 18 ? (z ? z - 1u : z) : (z + 1u < d.nz ? z + 1u : z);
+        const uint32_t yy = ys[i / 3 % 3], xx = xs[i % 3];
+        wd[i] = d.dmap[((xx >> 4) + d.dnbx * ((yy >> 3) + d.dnby * (zz >> 3))) * 32u + (zz & 7u) * 4u + ((yy & 7u) >> 1)];
+    }
+    uint32_t m[3] = {0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 27; i++)
+        m[i / 9] |= (wd[i] >> ((xs[i % 3] & 15u) + 16u * (ys[i / 3 % 3] & 1u)) & 1u) << (i % 9);
+    return rank_mask(m[0], z ? m[1] : 0u, z + 1u < d.nz ? m[2] : 0u);
+}
+
 /* plane GM_PAR_* of the parent array */
 static __device__ __forceinline__ uint4 *par_plane(const GmDev &d, uint32_t plane) {
     return d.par + (size_t)plane * d.parentCap;
@@ -416,11 +494,6 @@ static __device__ __forceinline__ uint32_t cell_of(const GmDev &d, uint32_t x, u
 /* Parents are cut into chunks of GM_PCHUNK for the decide and commit passes, so
  * that a 64-lane wave takes a whole chunk. */
 #define GM_PCHUNK 64
-#ifndef GM_PG
-#define GM_PG 4                       /* lanes per parent in the propose pass (4, 8 or 16) */
-#endif
-#define GM_PG_ITERS ((26 + GM_PG - 1) / GM_PG)
-static_assert(GM_PG == 4 || GM_PG == 8 || GM_PG == 16, "lanes per parent");
 
 /* The new record of a won attempt of rank r on target t = (tx, ty, tz) in slot
  * gslot: the carry of the parent's overshoot by the direction's class
@@ -617,6 +690,16 @@ static __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+/* The lanes' bits as a list in lane and bit order, lane | bit << 8 each, in wl (26 per
+ * lane at most); their number.  Every lane of the wave takes part. */
+static __device__ __forceinline__ uint32_t list_attempts(uint32_t mask, uint16_t *wl) {
+    const uint32_t n = (uint32_t)__popc(mask), incl = wave_incl_scan(n);
+    uint32_t pos = incl - n;
+    for (uint32_t m = mask; m; m &= m - 1u) wl[pos++] = (uint16_t)((threadIdx.x & 63u) | ((uint32_t)__ffs(m) - 1u) << 8);
+    wave_sync();
+    return (uint32_t)__shfl((int)incl, 63, 64);
 }
 
 /* Classifies a lane's eight slots of a sweep chunk (2-byte codes in cs, the

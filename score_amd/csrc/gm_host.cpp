@@ -1513,6 +1513,10 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
     else
         e = gm_launch_window(d, P, a, w, na != 0, h->Xcells, h->stream, ev);
     if (e != hipSuccess) return h->err = hip_fail(e, "growth step");
+    /* several regions: twice the last window's largest step sizes the infection passes'
+     * grids (which cover any number), not the occupied slots: at 8500 parents of 400,000
+     * slots most of 8192 blocks had nothing to do */
+    const uint32_t rg_parents = (uint32_t)std::min<uint64_t>(std::max(slots0, nIe + nBe), 2ull * h->last_full + 1024u);
     uint32_t launched = 0;
     for (uint32_t j = 0; j < W; j++) {
         if (paced && j > GM_LEAD && !wait_steps(h, j - GM_LEAD)) break;
@@ -1520,8 +1524,8 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
         if (d.nreg > 1) {
             GmSweepArgs aj = a;
             if (j) aj.reanchor = 0;
-            if ((e = gm_launch_rg_sweep(d, aj, std::max(slots0, nIe + nBe), h->stream, ev)) != hipSuccess ||
-                (e = gm_launch_rg_infect(d, h->pp, aj, std::max(slots0, nIe + nBe), h->stream, ev)) != hipSuccess ||
+            if ((e = gm_launch_rg_sweep(d, aj, rg_parents, h->stream, ev)) != hipSuccess ||
+                (e = gm_launch_rg_infect(d, h->pp, aj, rg_parents, h->stream, ev)) != hipSuccess ||
                 (e = gm_launch_step_tail(d, w, h->stream)) != hipSuccess)
                 return h->err = hip_fail(e, "growth step");
             continue;

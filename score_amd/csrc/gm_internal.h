@@ -282,10 +282,10 @@ struct GmHalo {
 };
 static_assert(sizeof(GmHalo) == 16, "GmHalo is 16 bytes");
 
-struct GmRegion {
+struct alignas(16) GmRegion {
+    GmHalo halo[27];            /* halo towards each neighbour; [0] unused */
     uint32_t lo[3], hi[3];      /* inclusive box */
     uint32_t nbor[27];          /* mynborregions ids: myself, faces, edges, corners */
-    GmHalo halo[27];            /* halo towards each neighbour; [0] unused */
 };
 
 /* halos an infection can be parked in (the other 18 are dummies or always

@@ -799,93 +799,6 @@ static __device__ __forceinline__ bool must_halt(const GmDev &d, const GmWindow 
            (win->full[j] > d.parentCap);
 }
 
-/* The deformed bits around a cell: nine per plane, bit (dy+1)*3 + dx+1, for the
- * cell's own plane, the one below and the one above, in the order of the attempts'
- * ranks (SCORE_Kernel.cpp:4611-4638: the own plane without the cell itself, the
- * lower plane with its row y+1 first, the upper plane). */
-static __device__ __forceinline__ uint32_t rank_mask(uint32_t m, uint32_t dn, uint32_t up) {
-    const uint32_t lower = (dn >> 6 & 7u) | (dn & 7u) << 3 | (dn >> 3 & 7u) << 6;
-    return (m & 0xFu) | (m >> 1 & 0xF0u) | lower << 8 | up << 17;
-}
-
-/* A strictly interior cell's neighbourhood in the bitmap.  A brick holds 16 x 8
- * cells of a plane in 16 bytes, a row of 16 cells in 16 bits, so one 16-byte load
- * a plane usually covers the nine cells; a cell at a brick's edge also loads from
- * the bricks beside it.  The loads of all planes are issued together (load), so
- * that the caller can work until it needs them (mask). */
-struct Neighbourhood {
-    uint4 c[3], cx[3];          /* planes z, z-1, z+1: the cell's brick, the one beside it along x */
-    uint32_t ry[3], rxy[3];     /* the word with the adjacent row of the bricks beside along y */
-    uint32_t xi, yi;
-    __device__ __forceinline__ void load(const GmDev &d, uint32_t x, uint32_t y, uint32_t z) {
-        const uint4 *D = reinterpret_cast<const uint4 *>(d.dmap);
-        xi = x & 15u;
-        yi = y & 7u;
-        const uint32_t row = (x >> 4) + d.dnbx * (y >> 3), layer = d.dnbx * d.dnby;
-        uint32_t at[3];
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-            const uint32_t zi = i == 0 ? z : i == 1 ? z - 1u : z + 1u;
-            at[i] = (row + layer * (zi >> 3)) * 8u + (zi & 7u);
-            c[i] = D[at[i]];
-            cx[i] = make_uint4(0u, 0u, 0u, 0u);
-            ry[i] = rxy[i] = 0;
-        }
-        const bool ex = xi == 0u || xi == 15u, ey = yi == 0u || yi == 7u;
-        const uint32_t sx = xi ? 8u : 0u - 8u, sy = (yi ? 8u : 0u - 8u) * d.dnbx, yw = yi ? 0u : 3u;
-        if (ex) {
-#pragma unroll
-            for (int i = 0; i < 3; i++) cx[i] = D[at[i] + sx];
-        }
-        if (ey) {
-#pragma unroll
-            for (int i = 0; i < 3; i++) ry[i] = d.dmap[(at[i] + sy) * 4u + yw];
-        }
-        if (ex && ey) {
-#pragma unroll
-            for (int i = 0; i < 3; i++) rxy[i] = d.dmap[(at[i] + sx + sy) * 4u + yw];
-        }
-    }
-    /* three rows of 16 bits, y-1 first */
-    __device__ __forceinline__ unsigned long long rows(const uint4 &q, uint32_t r) const {
-        const unsigned long long lo = (unsigned long long)q.y << 32 | q.x, hi = (unsigned long long)q.w << 32 | q.z;
-        const uint32_t s = 16u * (yi - 1u);
-        unsigned long long v = s < 64u ? lo >> (s & 63u) : hi >> (s & 63u);
-        if (s != 0u && s < 64u) v |= hi << (64u - s);
-        if (yi == 0u) v = lo << 16 | r >> 16;
-        if (yi == 7u) v = hi >> 32 | (unsigned long long)(r & 0xFFFFu) << 32;
-        return v;
-    }
-    __device__ __forceinline__ uint32_t plane(int i) const {
-        const unsigned long long one = 0x0000000100010001ull;
-        const unsigned long long T = rows(c[i], ry[i]), TX = rows(cx[i], rxy[i]);
-        unsigned long long U = T >> ((xi - 1u) & 63u);
-        if (xi == 0u) U = (T & 3u * one) << 1 | (TX >> 15 & one);
-        if (xi == 15u) U = (T >> 14 & 3u * one) | (TX & one) << 2;
-        return (uint32_t)(U & 7u) | (uint32_t)(U >> 13 & 0x38u) | (uint32_t)(U >> 26 & 0x1C0u);
-    }
-    __device__ __forceinline__ uint32_t mask() const { return rank_mask(plane(0), plane(1), plane(2)); }
-};
-
-/* The attempts of a Border cell on a face of the domain: x and y wrap, planes
- * outside z have none.  27 single words, all loaded together. */
-static __device__ __forceinline__ uint32_t face_attempts(const GmDev &d, uint32_t x, uint32_t y, uint32_t z) {
-    const uint32_t xs[3] = {x ? x - 1u : d.nx - 1u, x, x + 1u < d.nx ? x + 1u : 0u};
-    const uint32_t ys[3] = {y ? y - 1u : d.ny - 1u, y, y + 1u < d.ny ? y + 1u : 0u};
-    uint32_t wd[27];
-#pragma unroll
-    for (int i = 0; i < 27; i++) {
-        const uint32_t zz = i < 9 ? z : i < 18 ? (z ? z - 1u : z) : (z + 1u < d.nz ? z + 1u : z);
-        const uint32_t yy = ys[i / 3 % 3], xx = xs[i % 3];
-        wd[i] = d.dmap[((xx >> 4) + d.dnbx * ((yy >> 3) + d.dnby * (zz >> 3))) * 32u + (zz & 7u) * 4u + ((yy & 7u) >> 1)];
-    }
-    uint32_t m[3] = {0u, 0u, 0u};
-#pragma unroll
-    for (int i = 0; i < 27; i++)
-        m[i / 9] |= (wd[i] >> ((xs[i % 3] & 15u) + 16u * (ys[i / 3 % 3] & 1u)) & 1u) << (i % 9);
-    return rank_mask(m[0], z ? m[1] : 0u, z + 1u < d.nz ? m[2] : 0u);
-}
-
 /* Step j's attempts, one lane per parent.  What the infection needs of the parent
  * goes to the dense parent planes (FullRX order), with its rxFrac after the
  * completing addition, replayed from the anchor.  Every attempt on a deformed cell

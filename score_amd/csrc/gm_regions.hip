@@ -35,6 +35,10 @@
  * infection passes give each block the parents of one region only, so that
  * count is the offset of the region's first block.
  *
+ * At 160^3 in eight regions (477 steps of 8500 parents) a step of these passes went
+ * from 135 to 77 us: propose 25 to 10, decide 23 to 12 with the retirement, commit 25
+ * to 14, the two scans 27 to 15.
+ *
  * Per step, in the profiling slots of the one-region kernels:
  *   k_reanchor (shared)   k_rg_sweep   k_rg_sweep_scan (+ per-list starts)
  *   k_rg_compact   k_rg_propose   k_rg_decide
@@ -50,6 +54,9 @@ static __constant__ uint8_t c_opp[27] = {0, 2, 1, 4, 3, 6, 5, 10, 9, 8, 7, 14, 1
                                          26, 25, 24, 23, 22, 21, 20, 19};
 /* the halos an infection can be parked in, and each direction's index among them */
 static __constant__ uint8_t c_hdir[GM_NHALO] = {3, 4, 5, 6, 15, 16, 17, 18};
+static __device__ __forceinline__ constexpr uint32_t h_dir(int i) { return i < 4 ? 3u + i : 11u + i; }
+/* the index among them of the opposite direction: 3 4 5 6 15 16 17 18 have 4 3 6 5 18 17 16 15 */
+static __device__ __forceinline__ uint32_t h_opp(uint32_t i) { return i < 4u ? i ^ 1u : 11u - i; }
 /* neighbour index of the direction (0, sy, sz), at [(sy+1)*3 + sz+1] */
 static __constant__ uint8_t c_ydir_nb[9] = {15, 3, 16, 5, 0, 6, 17, 4, 18};
 static __constant__ uint8_t c_hidx[27] = {0xFF, 0xFF, 0xFF, 0, 1, 2, 3, 0xFF, 0xFF, 0xFF, 0xFF, 0xFF, 0xFF, 0xFF,
@@ -68,54 +75,37 @@ static __device__ __forceinline__ uint32_t part_per(uint32_t n, uint32_t nb, uin
     return (per + q - 1u) / q * q;
 }
 
-/* Exclusive scan, in place, of `rows` rows of nb <= GM_MAX_BLOCKS per-block
- * counts by one block of 1024 threads, as scan_block_counts does but one row
- * at a time, reading each thread's eight entries again (and scanning them
- * across the wave again) for the offsets, so that few registers stay live and
- * no private array is indexed at run time: a kernel that spills to scratch pays
- * for its scratch set-up at every launch.  tot (shared) receives the totals. */
-static __device__ uint32_t sum8(const uint32_t *row, uint32_t i0, uint32_t nb) {
-    if (i0 >= nb) return 0u;
-    const uint4 *p = reinterpret_cast<const uint4 *>(row + i0);
-    const uint4 a = p[0], b = p[1];
-    const uint32_t v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    uint32_t s = 0;
+/* Exclusive scan, in place, of `rows` <= 16 rows of nb <= GM_MAX_BLOCKS per-block
+ * counts by one block of 1024 threads, a wave per row, eight consecutive entries per
+ * lane; tot (shared) receives the totals.  (The whole block on one row after another
+ * waited for memory twice a row: 17.6 us a step for eleven rows.) */
+static __device__ void scan_rows(uint32_t *bcnt, uint32_t rows, uint32_t nb, uint32_t *tot) {
+    const uint32_t lane = threadIdx.x & 63u, c = threadIdx.x >> 6;
+    if (c < rows) {
+        uint32_t carry = 0;
+        for (uint32_t b0 = 0; b0 < nb; b0 += 512u) {
+            const uint32_t i0 = b0 + 8u * lane;
+            uint4 *q = reinterpret_cast<uint4 *>(bcnt + (size_t)c * GM_MAX_BLOCKS + i0);
+            uint4 a = make_uint4(0u, 0u, 0u, 0u), b = a;
+            if (i0 < nb) {
+                a = q[0];
+                b = q[1];
+            }
+            uint32_t v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}, sum = 0;
 #pragma unroll
-    for (uint32_t j = 0; j < 8; j++) s += i0 + j < nb ? v[j] : 0u;
-    return s;
-}
-
-static __device__ void scan_rows_lean(uint32_t *bcnt, uint32_t rows, uint32_t nb, uint32_t *tot) {
-    __shared__ uint32_t ws[16][16];
-    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint32_t i0 = threadIdx.x * 8u;
-    for (uint32_t c = 0; c < rows; c++) {
-        const uint32_t incl = wave_incl_scan(sum8(bcnt + c * GM_MAX_BLOCKS, i0, nb));
-        if (lane == 63) ws[w][c] = incl;
-    }
-    __syncthreads();
-    for (uint32_t c = 0; c < rows; c++) {
-        uint32_t pre = 0, t = 0;
-        for (uint32_t i = 0; i < 16; i++) {
-            if (i < w) pre += ws[i][c];
-            t += ws[i][c];
+            for (uint32_t j = 0; j < 8; j++) {
+                const uint32_t x = i0 + j < nb ? v[j] : 0u;
+                v[j] = sum;
+                sum += x;
+            }
+            const uint32_t incl = wave_incl_scan(sum), run = carry + incl - sum;
+            if (i0 < nb) {
+                q[0] = make_uint4(run + v[0], run + v[1], run + v[2], run + v[3]);
+                q[1] = make_uint4(run + v[4], run + v[5], run + v[6], run + v[7]);
+            }
+            carry += __shfl(incl, 63, 64);
         }
-        if (threadIdx.x == 0) tot[c] = t;
-        uint32_t *row = bcnt + c * GM_MAX_BLOCKS;
-        const uint32_t sum = sum8(row, i0, nb);
-        const uint32_t incl = wave_incl_scan(sum);
-        if (i0 >= nb) continue;
-        uint4 *q = reinterpret_cast<uint4 *>(row + i0);
-        const uint4 a = q[0], b = q[1];
-        const uint32_t v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        uint32_t run = pre + incl - sum, o[8];
-#pragma unroll
-        for (uint32_t j = 0; j < 8; j++) {
-            o[j] = run;
-            run += i0 + j < nb ? v[j] : 0u;
-        }
-        q[0] = make_uint4(o[0], o[1], o[2], o[3]);
-        q[1] = make_uint4(o[4], o[5], o[6], o[7]);
+        if (lane == 0) tot[c] = carry;
     }
     __syncthreads();
 }
@@ -212,24 +202,28 @@ static __device__ __forceinline__ bool rg_target(const GmDev &d, const RgBox &B,
             if (q == r) {
                 o.dl = 2u * r + 1u;
             } else {
-                uint32_t h = 0;
-                for (uint32_t c = 1; c < 27; c++) {
-                    const GmHalo &H = R.halo[c];
-                    if (H.inregion != q || H.ext[0] == 0) continue;
-                    if (tx >= (int)H.org[0] && tx <= (int)H.org[0] + (int)H.ext[0] && ty >= (int)H.org[1] &&
-                        ty <= (int)H.org[1] + (int)H.ext[1] && tz >= (int)H.org[2] && tz <= (int)H.org[2] + (int)H.ext[2]) {
-                        h = c;
-                        break;
-                    }
+                /* the eight halos that can be, loaded together: a wave with one such
+                 * attempt waits once, not once per halo (27 of them one after another
+                 * made the propose, decide and commit passes 25, 23 and 25 us at 8500
+                 * parents in eight regions) */
+                uint4 hv[GM_NHALO];
+#pragma unroll
+                for (int i = 0; i < GM_NHALO; i++) hv[i] = *reinterpret_cast<const uint4 *>(&R.halo[h_dir(i)]);
+                uint32_t hx = GM_NHALO;
+#pragma unroll
+                for (int i = GM_NHALO - 1; i >= 0; i--) {
+                    const int ox = (int)(hv[i].y & 0xFFFFu), oy = (int)(hv[i].y >> 16), oz = (int)(hv[i].z & 0xFFFFu);
+                    const int ex = (int)(hv[i].z >> 16), ey = (int)(hv[i].w & 0xFFFFu), ez = (int)(hv[i].w >> 16);
+                    const bool in = tx >= ox && tx <= ox + ex && ty >= oy && ty <= oy + ey && tz >= oz && tz <= oz + ez;
+                    if (hv[i].x == q && ex != 0 && in) hx = (uint32_t)i;
                 }
-                const uint32_t hx = c_hidx[h];
                 if (hx >= GM_NHALO) {
                     atomicOr(&d.st->err, GM_ERRF_HALO);
                     return false;
                 }
                 o.hidx = hx;
                 o.dl = 2u * q + 1u;
-                o.khi = (1u << 31) | ((uint32_t)c_hidx[c_opp[h]] << 28);
+                o.khi = (1u << 31) | (h_opp(hx) << 28);
             }
         }
     }
@@ -365,50 +359,53 @@ __global__ void __launch_bounds__(GM_BLOCK) k_rg_sweep(GmDev d, GmSweepArgs A0) 
 /* One block: per-block offsets; then each list's first completed and first
  * INACTIVE position (the block offset of the tile where the list starts plus
  * the block's tiles before it), the per-list counts, and their sums over the
- * Inside and the Border lists. */
+ * Inside and the Border lists.  The tiles are read beside the scan, and what the
+ * lists' threads hand to each other stays in LDS. */
 __global__ void __launch_bounds__(1024) k_rg_sweep_scan(GmDev d, uint32_t nb, uint32_t nbd) {
-    __shared__ uint32_t acc[6];
-    __shared__ uint32_t ws[16];
+    __shared__ uint32_t acc[6], tot[3], ws[16], sF[2049], sR[2049], sS[1025];
     GmStats *st = d.st;
     if (st->halt) return;
-    uint32_t tot[3];
-    scan_block_counts<3>(d.bcnt, nb, tot);
-    if (threadIdx.x < 6) acc[threadIdx.x] = 0;
-    if (threadIdx.x == 0) {
-        if (tot[RS_UN]) st->err |= GM_ERRF_MISSED;
-        /* infection keys are (halo, neighbour, p, rank) in 32 bits, p < 2^23 */
-        if ((uint64_t)tot[RS_F] > (1ull << 23)) st->err |= GM_ERRF_KEYS;
-    }
-    __syncthreads();
     const uint32_t T = d.L.tile[d.nlists];
     const uint32_t per = T ? part_per(T, nb, GM_SW_TPC) : 1u;
-    /* one wave per list, the lanes sharing the block's tiles before the list's first */
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    if (threadIdx.x < 6) acc[threadIdx.x] = 0;
+    /* one wave per list, the lanes sharing the block's tiles before the list's first */
     for (uint32_t l = wv; l <= d.nlists; l += 1024u / 64u) {
         const uint32_t t0 = d.L.tile[l];
-        uint32_t ef = 0, er = 0, b = 0;
-        if (t0 < T) {
-            b = t0 / per;
-            for (uint32_t t = b * per + lane; t < t0; t += 64) {
+        uint32_t ef = 0, er = 0;
+        if (t0 < T)
+            for (uint32_t t = t0 / per * per + lane; t < t0; t += 64) {
                 ef += (uint32_t)__popcll(d.mF[t]);
                 er += (uint32_t)__popcll(d.mR[t]);
             }
-        }
         for (int o = 32; o > 0; o >>= 1) {
             ef += __shfl_down(ef, o, 64);
             er += __shfl_down(er, o, 64);
         }
         if (lane == 0) {
             d.L.tile_s[l] = t0; /* this step's tiles, for the recycling pass after the lengths change */
-            d.L.par[l] = t0 < T ? d.bcnt[RS_F * GM_MAX_BLOCKS + b] + ef : tot[RS_F];
-            d.L.rst[l] = t0 < T ? d.bcnt[RS_R * GM_MAX_BLOCKS + b] + er : tot[RS_R];
+            sF[l] = ef;
+            sR[l] = er;
         }
+    }
+    scan_rows(d.bcnt, 3u, nb, tot);
+    if (threadIdx.x == 0) {
+        if (tot[RS_UN]) st->err |= GM_ERRF_MISSED;
+        /* infection keys are (halo, neighbour, p, rank) in 32 bits, p < 2^23 */
+        if ((uint64_t)tot[RS_F] > (1ull << 23)) st->err |= GM_ERRF_KEYS;
+    }
+    for (uint32_t l = threadIdx.x; l <= d.nlists; l += 1024) {
+        const uint32_t t0 = d.L.tile[l], b = t0 / per;
+        const uint32_t f = t0 < T ? d.bcnt[RS_F * GM_MAX_BLOCKS + b] + sF[l] : tot[RS_F];
+        const uint32_t r = t0 < T ? d.bcnt[RS_R * GM_MAX_BLOCKS + b] + sR[l] : tot[RS_R];
+        d.L.par[l] = sF[l] = f;
+        d.L.rst[l] = sR[l] = r;
     }
     __syncthreads();
     uint32_t a[6] = {0, 0, 0, 0, 0, 0};
     for (uint32_t l = threadIdx.x; l < d.nlists; l += 1024) {
-        const uint32_t nf = d.L.par[l + 1] - d.L.par[l], nr = d.L.rst[l + 1] - d.L.rst[l];
-        const uint32_t rl = nr < d.L.rcap[l] ? nr : d.L.rcap[l];
+        const uint32_t nf = sF[l + 1] - sF[l], nr = sR[l + 1] - sR[l], rc = d.L.rcap[l];
+        const uint32_t rl = nr < rc ? nr : rc;
         d.L.rlen[l] = rl;
         const uint32_t k = (l & 1u) * 3u;
         a[k] += nf;
@@ -424,7 +421,7 @@ __global__ void __launch_bounds__(1024) k_rg_sweep_scan(GmDev d, uint32_t nb, ui
     uint32_t pper = (nfull + (nbd - d.nreg) - 1u) / (nbd - d.nreg);
     pper = pper ? (pper + GM_PCHUNK - 1u) / GM_PCHUNK * GM_PCHUNK : GM_PCHUNK;
     const uint32_t r = threadIdx.x;
-    const uint32_t nr = r < d.nreg ? d.L.par[2u * r + 2u] - d.L.par[2u * r] : 0u;
+    const uint32_t nr = r < d.nreg ? sF[2u * r + 2u] - sF[2u * r] : 0u;
     const uint32_t blk = (nr + pper - 1u) / pper;
     const uint32_t incl = wave_incl_scan(blk);
     if (lane == 63u) ws[wv] = incl;
@@ -434,12 +431,12 @@ __global__ void __launch_bounds__(1024) k_rg_sweep_scan(GmDev d, uint32_t nb, ui
         if (i < wv) pre += ws[i];
         totb += ws[i];
     }
-    if (r < d.nreg) d.L.bstart[r] = pre + incl - blk;
-    if (threadIdx.x == 0) d.L.bstart[d.nreg] = totb;
+    if (r < d.nreg) d.L.bstart[r] = sS[r] = pre + incl - blk;
+    if (threadIdx.x == 0) d.L.bstart[d.nreg] = sS[d.nreg] = totb;
     __syncthreads();
     /* each block's region; blocks past the ones in use find none */
     for (uint32_t b = threadIdx.x; b < nbd; b += 1024)
-        d.L.breg[b] = b < totb ? upper_index(d.L.bstart, d.nreg, b) : 0xFFFFFFFFu;
+        d.L.breg[b] = b < totb ? upper_index(sS, d.nreg, b) : 0xFFFFFFFFu;
     if (threadIdx.x == 0) {
         st->rg_per = pper;
         st->nfullI = acc[0];
@@ -536,121 +533,124 @@ hipError_t gm_launch_rg_sweep(const GmDev &d, const GmSweepArgs &a, uint32_t par
 
 /* --------------------------------------------------------------- infection */
 
-/* GM_PG lanes per parent, as the one-region propose pass: the parent's data
- * into the dense array (with its list in place of the Border flag), its
- * retirement into the log, and every attempt on a deformed cell claims it with
- * its 64-bit key. */
+/* One lane per parent, as the one-region propose pass: the parent's data into the
+ * dense array (with its list in place of the Border flag), its value after the
+ * completing addition, its retirement into the log; its deformed neighbours come from
+ * three 16-byte loads of the bitmap.  Every attempt on one of them, routed to the
+ * region it lies in, claims it: 64 parents' attempts are flattened into a list, a
+ * lane per attempt, so that a wave waits for its attempts' halos at once. */
 __global__ void __launch_bounds__(GM_BLOCK) k_rg_propose(GmDev d) {
+    struct Wave {
+        uint4 q2[64];
+        uint32_t bad[64];
+        uint16_t wl[26 * 64];
+    };
+    __shared__ Wave sw[GM_BLOCK / 64];
     if (d.st->halt) return;
-    const uint32_t nfull = d.st->nfullI + d.st->nfullB;
+    const uint32_t nfull = d.st->nfullI + d.st->nfullB, k = d.st->kcur;
     const unsigned long long nret = d.st->nret;
     const bool logged = nret + nfull <= d.rlogCap;
     if (!logged && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&d.st->err, GM_ERRF_RLOG_FULL);
-    const uint32_t lg = threadIdx.x & (GM_PG - 1);
-    const uint32_t ngroups = gridDim.x * (GM_BLOCK / GM_PG);
-    for (uint32_t p = blockIdx.x * (GM_BLOCK / GM_PG) + threadIdx.x / GM_PG; p < nfull; p += ngroups) {
-        uint4 q2 = make_uint4(0u, 0u, 0u, 0u);
-        if (lg == 0) {
-            const uint32_t s = d.pslot[p];
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    Wave &W = sw[w];
+    for (uint32_t c = w * gridDim.x + blockIdx.x; c * 64u < nfull; c += gridDim.x * (GM_BLOCK / 64u)) {
+        const uint32_t p = c * 64u + lane;
+        uint32_t am = 0;
+        if (p < nfull) {
+            const uint32_t s = d.pslot[p], l = d.plist[p];
             const GmRec *r = d.rec + s;
-            const RecC c = rec_c(r);
-            const uint32_t rxg = r->rxg;
-            const uint32_t cell = c.cell;
+            const RecC rc = rec_c(r);
+            const RecA ra = rec_a(r);
+            const double inc = r->inc;
+            const uint32_t rxg = r->rxg, cell = rc.cell;
             const uint32_t z = cell / d.nxy, rem = cell - z * d.nxy, y = rem / d.nx, x = rem - y * d.nx;
-            q2 = make_uint4(x, y, z, d.plist[p]);
-            par_plane(d, GM_PAR_IDS)[p] = make_uint4(s, cell, c.defg, rxg);
-            /* the value after the completing addition follows in k_rg_decide */
-            reinterpret_cast<double2 *>(par_plane(d, GM_PAR_FP))[p] = make_double2(0.0, c.P);
+            const bool interior = (x - 1u < d.nx - 2u) & (y - 1u < d.ny - 2u) & (z - 1u < d.nz - 2u);
+            Neighbourhood nb;
+            if (interior) nb.load(d, x, y, z);
+            const double fin = advanced(ra.frac0, inc, k - ra.s0 + 1u);
+            am = interior ? nb.mask() : face_attempts(d, x, y, z);
+            const uint4 q2 = make_uint4(x, y, z, l);
+            W.q2[lane] = q2;
+            par_plane(d, GM_PAR_IDS)[p] = make_uint4(s, cell, rc.defg, rxg);
+            reinterpret_cast<double2 *>(par_plane(d, GM_PAR_FP))[p] = make_double2(fin, rc.P);
             par_plane(d, GM_PAR_XYZ)[p] = q2;
             if (logged) d.rlog[nret + p] = make_uint2(cell, d.ndefg + rxg);
         }
-        q2.x = (uint32_t)__shfl((int)q2.x, 0, GM_PG);
-        q2.y = (uint32_t)__shfl((int)q2.y, 0, GM_PG);
-        q2.z = (uint32_t)__shfl((int)q2.z, 0, GM_PG);
-        q2.w = (uint32_t)__shfl((int)q2.w, 0, GM_PG);
-        const uint32_t gsh = (threadIdx.x & 63) & ~(GM_PG - 1);
-        const RgBox box = rg_box(d, q2.w >> 1);
-        uint32_t am = 0;
-#pragma unroll
-        for (uint32_t i = 0; i < GM_PG_ITERS; i++) {
-            const uint32_t rk = lg + GM_PG * i;
-            bool att = false;
-            if (rk < 26) {
-                RgTarget o;
-                if (rg_target(d, box, q2.w, q2.x, q2.y, q2.z, (int)rk, o) && is_deformed(d, o.x, o.y, o.z)) {
-                    att = true;
-                    atomicMin(&d.cell[cell_of(d, o.x, o.y, o.z)].x, o.khi | (p * 32u + rk));
-                }
-            }
-            am |= (uint32_t)((__ballot(att) >> gsh) & ((1ull << GM_PG) - 1u)) << (GM_PG * i);
+        W.bad[lane] = 0;
+        const uint32_t n = list_attempts(am, W.wl);
+        for (uint32_t i = lane; i < n; i += 64u) {
+            const uint32_t e = W.wl[i], q = e & 0xFFu, rk = e >> 8;
+            const uint4 q2 = W.q2[q];
+            RgTarget o;
+            if (rg_target(d, rg_box(d, q2.w >> 1), q2.w, q2.x, q2.y, q2.z, (int)rk, o))
+                atomicMin(&d.cell[cell_of(d, o.x, o.y, o.z)].x, o.khi | ((c * 64u + q) * 32u + rk));
+            else
+                atomicOr(&W.bad[q], 1u << rk);
         }
-        if (lg == 0) d.pmI[p] = am;
+        wave_sync();
+        if (p < nfull) d.pmI[p] = am & ~W.bad[lane];
+        wave_sync();
     }
 }
 
-/* One lane per parent: the attempts that hold their target's smallest key, as
- * masks by destination (own Inside, own Border, a halo), counted per block by
- * row (GM_RW_*); a parent that won a target gets its value after the completing
- * addition in the parent array.  The partition into blocks (one region per
- * block) is the commit pass's. */
+/* The attempts that hold their target's smallest key, as masks by destination (own
+ * Inside, own Border, a halo), counted per block by row (GM_RW_*).  64 parents'
+ * attempts are flattened into a list, a lane per attempt, so that all claims are
+ * loaded together.  The parents retire here, beside the waiting for the claims.  The
+ * partition into blocks (one region per block) is the commit pass's. */
 __global__ void __launch_bounds__(64) k_rg_decide(GmDev d) {
+    __shared__ uint4 sq2[64];
+    __shared__ uint32_t sI[64], sB[64], sH[64], scnt[GM_RROWS];
+    __shared__ uint16_t wl[26 * 64];
     if (d.st->halt) return;
-    const uint32_t k = d.st->kcur;
+    const uint32_t lane = threadIdx.x;
     uint32_t lo, hi, reg;
     rg_part(d, lo, hi, reg);
     const RgBox box = rg_box(d, reg);
-    uint32_t cnt[GM_RROWS];
-#pragma unroll
-    for (int c = 0; c < GM_RROWS; c++) cnt[c] = 0;
-    for (uint32_t p = lo + threadIdx.x; p < hi; p += 64) {
-        const uint4 q2 = par_plane(d, GM_PAR_XYZ)[p];
-        const uint32_t am = d.pmI[p];
-        const uint32_t ps = d.pslot[p]; /* loaded with the rest, used if the parent wins */
-        uint32_t mI = 0, mB = 0, mH = 0;
-        for (uint32_t m = am; m; m &= m - 1u) {
-            const uint32_t rk = (uint32_t)__ffs(m) - 1u;
+    if (lane < GM_RROWS) scnt[lane] = 0;
+    uint32_t nI = 0, nB = 0, nA = 0;
+    for (uint32_t batch = lo; batch < hi; batch += 64) {
+        const uint32_t p = batch + lane;
+        const bool valid = p < hi;
+        const uint32_t am = valid ? d.pmI[p] : 0u;
+        sq2[lane] = valid ? par_plane(d, GM_PAR_XYZ)[p] : make_uint4(0u, 0u, 0u, 0u);
+        sI[lane] = sB[lane] = sH[lane] = 0;
+        retire_batch(d, valid ? par_plane(d, GM_PAR_IDS)[p] : make_uint4(0u, 0u, 0xFFFFFFFFu, 0xFFFFFFFFu), valid);
+        const uint32_t n = list_attempts(am, wl);
+        for (uint32_t i = lane; i < n; i += 64u) {
+            const uint32_t e = wl[i], q = e & 0xFFu, rk = e >> 8;
+            const uint4 q2 = sq2[q];
             RgTarget o;
             rg_target(d, box, q2.w, q2.x, q2.y, q2.z, (int)rk, o);
-            if (d.cell[cell_of(d, o.x, o.y, o.z)].x != (o.khi | (p * 32u + rk))) continue;
+            if (d.cell[cell_of(d, o.x, o.y, o.z)].x != (o.khi | ((batch + q) * 32u + rk))) continue;
             if (o.khi) {
-                mH |= 1u << rk;
-#pragma unroll
-                for (uint32_t j = 0; j < GM_NHALO; j++) cnt[GM_RW_H0 + j] += o.hidx == j ? 1u : 0u;
-            } else if (o.dl & 1u) {
-                mB |= 1u << rk;
+                atomicOr(&sH[q], 1u << rk);
+                atomicAdd(&scnt[GM_RW_H0 + o.hidx], 1u);
             } else {
-                mI |= 1u << rk;
+                atomicOr((o.dl & 1u) ? &sB[q] : &sI[q], 1u << rk);
             }
         }
-        d.pmI[p] = mI;
-        d.pmB[p] = mB;
-        d.pmH[p] = mH;
-        if (mI | mB | mH) reinterpret_cast<double *>(par_plane(d, GM_PAR_FP))[2 * (size_t)p] = parent_fin(d, ps, k);
-        cnt[GM_RW_I] += (uint32_t)__popc(mI);
-        cnt[GM_RW_B] += (uint32_t)__popc(mB);
-        cnt[GM_RW_A] += (uint32_t)__popc(am);
+        wave_sync();
+        const uint32_t mI = sI[lane], mB = sB[lane];
+        if (valid) {
+            d.pmI[p] = mI;
+            d.pmB[p] = mB;
+            d.pmH[p] = sH[lane];
+        }
+        nI += (uint32_t)__popc(mI);
+        nB += (uint32_t)__popc(mB);
+        nA += (uint32_t)__popc(am);
+        wave_sync();
     }
-#pragma unroll
-    for (int c = 0; c < GM_RROWS; c++) {
-        uint32_t v = cnt[c];
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-        if (threadIdx.x == 0) d.bcnt[(RW_ROW0 + c) * GM_MAX_BLOCKS + blockIdx.x] = v;
+    for (int o = 32; o > 0; o >>= 1) {
+        nI += __shfl_xor(nI, o, 64);
+        nB += __shfl_xor(nB, o, 64);
+        nA += __shfl_xor(nA, o, 64);
     }
-}
-
-/* the halo index of every parked winner of parent p (whose data is q2), as
- * GM_NHALO masks */
-static __device__ __forceinline__ void halo_masks(const GmDev &d, const RgBox &box, const uint4 &q2, uint32_t mH,
-                                                  uint32_t *mh) {
-#pragma unroll
-    for (uint32_t j = 0; j < GM_NHALO; j++) mh[j] = 0;
-    for (uint32_t m = mH; m; m &= m - 1u) {
-        const uint32_t rk = (uint32_t)__ffs(m) - 1u;
-        RgTarget o;
-        rg_target(d, box, q2.w, q2.x, q2.y, q2.z, (int)rk, o);
-#pragma unroll
-        for (uint32_t j = 0; j < GM_NHALO; j++) mh[j] |= o.hidx == j ? 1u << rk : 0u;
-    }
+    wave_sync();
+    if (lane < GM_RROWS)
+        d.bcnt[(RW_ROW0 + lane) * GM_MAX_BLOCKS + blockIdx.x] =
+            lane == GM_RW_I ? nI : lane == GM_RW_B ? nB : lane == GM_RW_A ? nA : scnt[lane];
 }
 
 /* One block: per-block offsets of every row; then, per region, the counts of
@@ -667,7 +667,7 @@ __global__ void __launch_bounds__(1024) k_rg_decide_scan(GmDev d, uint32_t nb) {
     /* only the blocks in use hold counts */
     const uint32_t nused = d.L.bstart[d.nreg];
     __shared__ uint32_t tot[GM_RROWS];
-    scan_rows_lean(d.bcnt + RW_ROW0 * GM_MAX_BLOCKS, GM_RROWS, nused < nb ? nused : nb, tot);
+    scan_rows(d.bcnt + RW_ROW0 * GM_MAX_BLOCKS, GM_RROWS, nused < nb ? nused : nb, tot);
     if (threadIdx.x < 2) acc[threadIdx.x] = 0;
     if (threadIdx.x == 0) st->nattempt = tot[GM_RW_A];
     /* each region's counts at its first parent: the offset of its first block
@@ -719,7 +719,7 @@ __global__ void __launch_bounds__(1024) k_rg_decide_scan(GmDev d, uint32_t nb) {
     rg_prefix_block(d);
 }
 
-/* New records and retiring parents as the one-region commit pass writes them;
+/* New records as the one-region commit pass writes them;
  * a winner's slot is its rank in its list: own Inside and own Border winners
  * by the parents' prefix counts less the count at the region's first parent,
  * halo winners after the receiving region's own, by neighbour, then by the
@@ -727,7 +727,6 @@ __global__ void __launch_bounds__(1024) k_rg_decide_scan(GmDev d, uint32_t nb) {
  * looked up again whatever its deformed grain (SCORE_Kernel.cpp:4853). */
 __global__ void __launch_bounds__(64) k_rg_commit(GmDev d, GmPParams pp, GmSweepArgs A) {
     __shared__ uint32_t sI[64], sB[64], oI[64], oB[64];
-    __shared__ uint32_t sH[GM_NHALO][64], oH[GM_NHALO][64];
     __shared__ uint4 sq0[64], sq2[64];
     __shared__ double sfin[64], sP[64];
     __shared__ uint16_t wl[26 * 64];
@@ -764,36 +763,11 @@ __global__ void __launch_bounds__(64) k_rg_commit(GmDev d, GmPParams pp, GmSweep
             fp = reinterpret_cast<const double2 *>(par_plane(d, GM_PAR_FP))[pt];
             q2 = par_plane(d, GM_PAR_XYZ)[pt];
         }
-        uint32_t mh[GM_NHALO];
-        halo_masks(d, box, q2, mH, mh);
-        /* exclusive prefixes within the batch, two 16-bit counts per scan
-         * (a batch holds at most 64*26 winners of a row) */
-        uint32_t cnt[GM_RROWS], ex[GM_RROWS], bt[GM_RROWS];
-        cnt[GM_RW_I] = (uint32_t)__popc(mI);
-        cnt[GM_RW_B] = (uint32_t)__popc(mB);
-        cnt[GM_RW_A] = 0u;
-#pragma unroll
-        for (uint32_t j = 0; j < GM_NHALO; j++) cnt[GM_RW_H0 + j] = (uint32_t)__popc(mh[j]);
-#pragma unroll
-        for (int c = 0; c < GM_RROWS; c += 2) {
-            const uint32_t hi16 = c + 1 < GM_RROWS ? cnt[c + 1] : 0u;
-            const uint32_t packed = (cnt[c] << 16) | hi16;
-            const uint32_t incl = wave_incl_scan(packed);
-            const uint32_t e = incl - packed, t = __shfl(incl, 63, 64);
-            ex[c] = e >> 16;
-            bt[c] = t >> 16;
-            if (c + 1 < GM_RROWS) {
-                ex[c + 1] = e & 0xFFFFu;
-                bt[c + 1] = t & 0xFFFFu;
-            }
-        }
-        oI[lane] = run[GM_RW_I] + ex[GM_RW_I];
-        oB[lane] = run[GM_RW_B] + ex[GM_RW_B];
-#pragma unroll
-        for (uint32_t j = 0; j < GM_NHALO; j++) {
-            oH[j][lane] = run[GM_RW_H0 + j] + ex[GM_RW_H0 + j];
-            sH[j][lane] = mh[j];
-        }
+        /* one scan of both own lists' counts (a batch holds at most 64*26 of each) */
+        const uint32_t packed = (uint32_t)__popc(mI) << 16 | (uint32_t)__popc(mB);
+        const uint32_t inclIB = wave_incl_scan(packed), ex = inclIB - packed, bt = __shfl(inclIB, 63, 64);
+        oI[lane] = run[GM_RW_I] + (ex >> 16);
+        oB[lane] = run[GM_RW_B] + (ex & 0xFFFFu);
         sI[lane] = mI;
         sB[lane] = mB;
         sq0[lane] = q0;
@@ -801,17 +775,28 @@ __global__ void __launch_bounds__(64) k_rg_commit(GmDev d, GmPParams pp, GmSweep
         sfin[lane] = fp.x;
         sP[lane] = fp.y;
         /* this parent's winners at their place in the flat list, by rank */
-        const uint32_t mall = mI | mB | mH, call = (uint32_t)__popc(mall);
-        const uint32_t inc = wave_incl_scan(call);
-        const uint32_t nw = __shfl(inc, 63, 64);
-        uint32_t pos = inc - call;
-        for (uint32_t m = mall; m; m &= m - 1u) wl[pos++] = (uint16_t)(lane | ((uint32_t)__ffs(m) - 1u) << 8);
-        __syncthreads();
-        for (uint32_t w = lane; w < nw; w += 64) {
-            const uint32_t e = wl[w], j = e & 0xFFu, r = e >> 8, bit = 1u << r;
+        const uint32_t nw = list_attempts(mI | mB | mH, wl);
+        for (uint32_t w0 = 0; w0 < nw; w0 += 64) {
+            const uint32_t w = w0 + lane;
+            const bool on = w < nw;
+            const uint32_t e = on ? wl[w] : 0u, j = e & 0xFFu, r = e >> 8, bit = 1u << r;
             const uint4 pq0 = sq0[j], pq2 = sq2[j];
             RgTarget o;
-            rg_target(d, box, pq2.w, pq2.x, pq2.y, pq2.z, (int)r, o);
+            o.khi = 0u;
+            o.hidx = GM_NHALO;
+            if (on) rg_target(d, box, pq2.w, pq2.x, pq2.y, pq2.z, (int)r, o);
+            /* the list is in the order of the parents and ranks: a parked winner's rank
+             * in its halo is those of the halo before it */
+            uint32_t hrank = 0;
+            if (__any(o.hidx < GM_NHALO)) {
+#pragma unroll
+                for (uint32_t h = 0; h < GM_NHALO; h++) {
+                    const uint64_t m = __ballot(o.hidx == h);
+                    if (o.hidx == h) hrank = run[GM_RW_H0 + h] + lanemask_lt_count(m);
+                    run[GM_RW_H0 + h] += (uint32_t)__popcll(m);
+                }
+            }
+            if (!on) continue;
             const uint32_t t = cell_of(d, o.x, o.y, o.z);
             const uint32_t g = d.cell[t].y;
             /* the rank in the destination list, and that list's tables: the block's
@@ -819,8 +804,7 @@ __global__ void __launch_bounds__(64) k_rg_commit(GmDev d, GmPParams pp, GmSweep
             uint32_t rank, ix;
             if (o.khi) {
                 const uint32_t q = o.dl >> 1, nbi = (o.khi >> 28) & 7u;
-                rank = d.L.hoff[q * GM_NHALO + nbi] + (oH[o.hidx][j] - srs[GM_RW_H0 + o.hidx]) +
-                       (uint32_t)__popc(sH[o.hidx][j] & (bit - 1u));
+                rank = d.L.hoff[q * GM_NHALO + nbi] + (hrank - srs[GM_RW_H0 + o.hidx]);
                 ix = 2u;
             } else if (o.dl & 1u) {
                 rank = oB[j] - srs[GM_RW_B] + (uint32_t)__popc(sB[j] & (bit - 1u));
@@ -843,9 +827,8 @@ __global__ void __launch_bounds__(64) k_rg_commit(GmDev d, GmPParams pp, GmSweep
             }
             put_cell(d, k, new_cell(d, pp, A, k, sfin[j], sP[j], pq0, r, g, o.khi != 0u), pq0, t, g, o.x, o.y, o.z, bs + rel);
         }
-        retire_batch(d, q0, valid);
-#pragma unroll
-        for (int c = 0; c < GM_RROWS; c++) run[c] += bt[c];
+        run[GM_RW_I] += bt >> 16;
+        run[GM_RW_B] += bt & 0xFFFFu;
         __syncthreads();
     }
 }
@@ -854,7 +837,7 @@ hipError_t gm_launch_rg_infect(const GmDev &d, const GmPParams &pp, const GmSwee
                                hipStream_t s, hipEvent_t *ev) {
     hipError_t e;
     if ((e = mark(ev, 4, s)) != hipSuccess) return e;
-    k_rg_propose<<<grid_for(parents_upper, GM_BLOCK / GM_PG), GM_BLOCK, 0, s>>>(d);
+    k_rg_propose<<<grid_for(parents_upper, 64u), GM_BLOCK, 0, s>>>(d);
     const uint32_t nb = rg_infect_blocks(d, parents_upper);
     if ((e = mark(ev, 5, s)) != hipSuccess) return e;
     k_rg_decide<<<nb, 64, 0, s>>>(d);
