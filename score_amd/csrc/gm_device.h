@@ -66,6 +66,14 @@ static __device__ __forceinline__ uint64_t rdlane64(uint64_t v, uint32_t j) {
     return ((uint64_t)rdlane((uint32_t)(v >> 32), j) << 32) | (uint64_t)rdlane((uint32_t)v, j);
 }
 
+/* a word that other blocks of the same launch change, by atomics */
+static __device__ __forceinline__ uint32_t agent_load(const uint32_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+static __device__ __forceinline__ void agent_store(uint32_t *p, uint32_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 static __device__ __forceinline__ bool is_pending(double v) {
     return ((unsigned long long)__double_as_longlong(v) & GM_PENDING_MASK) == GM_PENDING_TAG;
 }
@@ -111,12 +119,12 @@ static __device__ __forceinline__ double grimmer_omega(const double *p, const do
  * disorientation is far above the LAGB/HAGB transition have P == 1.0 exactly in
  * glibc arithmetic (threshold set and checked by the host); every other pair is
  * looked up in the cache, and a miss inserts a pending entry the host resolves
- * with glibc before the next sweep reads it. */
-static __device__ double pair_weight(const GmDev &d, const GmPParams &pp, uint32_t rxg, uint32_t g) {
+ * with glibc before the next sweep reads it.  one: set for a pair of the first kind. */
+static __device__ double pair_weight(const GmDev &d, const GmPParams &pp, uint32_t rxg, uint32_t g, bool &one) {
     if (pp.model == GM_RH && pp.omega_hi >= 0.0) {
         double om = grimmer_omega(&d.rxq[4 * (size_t)rxg], &d.defq[4 * (size_t)g], pp.fac);
         if (om <= pp.omega_hi) {
-            d.st->pone = 1u;
+            one = true;
             return 1.0;
         }
     }
@@ -131,7 +139,9 @@ static __device__ double pair_weight(const GmDev &d, const GmPParams &pp, uint32
                 uint32_t i = atomicAdd(&d.st->npend, 1u);
                 d.pend_slot[i] = h;
                 d.pend_key[i] = key;
-                if (i < GM_PEND_INLINE) d.st->pend_keys[i] = key;
+                /* (read by the commit pass's last block, which may be another) */
+                if (i < GM_PEND_INLINE)
+                    __hip_atomic_store(&d.st->pend_keys[i], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 return pending_box(h);
             }
             k = old;
@@ -510,6 +520,7 @@ struct NewCell {
     double carry, P, inc;
     uint32_t inf;
     gm_cs_t cs;
+    bool one;                   /* the pair's weight was short-circuited to 1.0 */
 };
 static __device__ __forceinline__ NewCell new_cell(const GmDev &d, const GmPParams &pp, const GmSweepArgs &A, uint32_t k,
                                                    double pfin, double pP, const uint4 &pq0, uint32_t r, uint32_t g,
@@ -519,7 +530,8 @@ static __device__ __forceinline__ NewCell new_cell(const GmDev &d, const GmPPara
     NewCell n;
     n.carry = cls == 1 ? overshoot * 0.0682 : (cls == 2 ? overshoot * 0.0542 : overshoot * 0.0484);
     n.P = pP;
-    if (fresh_weight || pq0.z != g) n.P = pair_weight(d, pp, pq0.w, g);
+    n.one = false;
+    if (fresh_weight || pq0.z != g) n.P = pair_weight(d, pp, pq0.w, g, n.one);
     n.inf = dir_code(r);
     n.inc = 0.0;
     n.cs = (gm_cs_t)GM_CS_DEFERRED;

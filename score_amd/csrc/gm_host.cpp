@@ -442,6 +442,8 @@ int arena_place(score_gm_handle *h) {
 
 void free_device(score_gm_handle *h) {
     GmDev &d = h->d;
+    /* the last window's kernels may still be ending: pinned memory goes back below */
+    if (h->stream) (void)hipStreamSynchronize(h->stream);
     void *ptrs[] = {d.cell, d.pmA, d.gatt, d.rlog, d.dmap, d.cstep, d.rec, d.pslot, d.dlist,
                     d.par, d.recI, d.recB, d.mF, d.mR, d.pmI, d.pmB, d.bcnt, d.rho, d.defq,
                     d.rxq, d.defcnt, d.rxcnt, d.zlist, d.hkeys, d.hvals, d.pend_slot, d.pend_key, d.nflag, d.nI_, d.nB_,
@@ -1402,6 +1404,21 @@ bool wait_steps(score_gm_handle *h, uint32_t need) {
     }
 }
 
+/* Waits until the window's stats are in the host's mirror: the word the device sets
+ * after them (copy_stats), or, after a second without it, whatever the stream says. */
+hipError_t wait_window(score_gm_handle *h) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (uint32_t it = 1; !__atomic_load_n(h->hprog + 1, __ATOMIC_ACQUIRE); it++) {
+        if ((it & 63u) == 0u) {
+            std::this_thread::yield();
+            if (std::chrono::steady_clock::now() - t0 > std::chrono::seconds(1)) return hipStreamSynchronize(h->stream);
+        } else {
+            __builtin_ia32_pause();
+        }
+    }
+    return hipSuccess;
+}
+
 /* Cuts the window's passes into blocks for lists of at most nI and nB slots: one
  * 512-slot chunk per wave of a sweep block while GM_SW_BLOCKS blocks (8 on every
  * CU) cover the lists, then more chunks per wave, and beyond GM_SW_MAXCPW (the
@@ -1498,6 +1515,7 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
     w.top_pos = (uint32_t)std::min<size_t>(h->rho_top, d.ndefg);
     w.pend_limit = (uint32_t)std::min<uint64_t>(0xFFFFFFFFull, (uint64_t)d.hcap / 2 > h->hcount ? (uint64_t)d.hcap / 2 - h->hcount : 0ull);
     w.defer = W > 1 ? 1u : 0u;
+    w.need_one = h->regPmax < 1.0 ? 1u : 0u;
     hipEvent_t *ev = prof ? h->ev : nullptr;
     const auto th0 = std::chrono::steady_clock::now();
     hipError_t e;
@@ -1508,6 +1526,7 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
      * nothing, whatever the host sees in time. */
     const bool paced = !prof && W > GM_LEAD + 1;
     if (paced) __atomic_store_n(h->hprog, 0u, __ATOMIC_RELAXED);
+    __atomic_store_n(h->hprog + 1, 0u, __ATOMIC_RELAXED);
     if (d.nreg > 1)
         e = gm_launch_window_begin(d, h->step, h->Xcells, h->stream);
     else
@@ -1530,12 +1549,12 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
                 return h->err = hip_fail(e, "growth step");
             continue;
         }
-        if ((e = gm_launch_infect(d, h->pp, a, P, w, j, h->stream, ev)) != hipSuccess)
+        if ((e = gm_launch_infect(d, h->pp, a, P, w, j, j + 1 == W && !prof ? h->hst_dev : nullptr, h->stream, ev)) != hipSuccess)
             return h->err = hip_fail(e, "growth step");
     }
-    e = d.nreg > 1 ? gm_launch_stats_out(d, h->hst_dev, h->stream)
-                   : gm_launch_window_end(d, P, launched, w.top_pos, h->hst_dev, h->stream);
-    if (e != hipSuccess || (e = hipStreamSynchronize(h->stream)) != hipSuccess)
+    if (d.nreg > 1) e = gm_launch_stats_out(d, h->hst_dev, h->stream);
+    else if (launched < W || prof) e = gm_launch_window_end(d, P, launched, w.top_pos, h->hst_dev, h->stream);
+    if (e != hipSuccess || (e = prof ? hipStreamSynchronize(h->stream) : wait_window(h)) != hipSuccess)
         return h->err = hip_fail(e, "growth step");
     /* a step that found too few Inside slots or parents' entries waits for them:
      * step nexec runs on from its commit pass, or the first step from its start */
@@ -1544,10 +1563,10 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
         if ((rc = grow ? grow_front(h, grow) : grow_parents(h, h->hst->need_par))) return h->err = rc;
         if ((e = gm_launch_fill_u32(&d.st->grow, 0u, 2, h->stream)) != hipSuccess ||
             (e = gm_launch_fill_u32(&d.st->halt, 0u, 1, h->stream)) != hipSuccess ||
-            (grow && (e = gm_launch_commit(d, h->pp, a, P, j0, h->stream, ev)) != hipSuccess))
+            (grow && (e = gm_launch_commit(d, h->pp, a, P, w, j0, nullptr, h->stream, ev)) != hipSuccess))
             return h->err = hip_fail(e, "growth step");
         for (uint32_t j = grow ? j0 + 1u : 0u; j < W; j++)
-            if ((e = gm_launch_infect(d, h->pp, a, P, w, j, h->stream, ev)) != hipSuccess)
+            if ((e = gm_launch_infect(d, h->pp, a, P, w, j, nullptr, h->stream, ev)) != hipSuccess)
                 return h->err = hip_fail(e, "growth step");
         if ((e = gm_launch_window_end(d, P, W, w.top_pos, h->hst_dev, h->stream)) != hipSuccess ||
             (e = hipStreamSynchronize(h->stream)) != hipSuccess)

@@ -201,6 +201,7 @@ struct alignas(8) GmStats {
     uint32_t nattempt;        /* attempts that found a deformed target this step */
     uint32_t nzeroed;         /* several regions: deformed grains that lost their last cell in the window */
     uint32_t cwrap;           /* a deformed-grain count went past zero (one region: of a grain before the one that sets rhomax) */
+    uint32_t ticket;          /* one region: blocks of the window's last commit pass that are done */
     uint32_t grow;            /* one region: the Inside slots a step's commit pass asks for before it can run */
     uint32_t need_par;        /* one region: the parents of a step that has more than the planes hold */
     uint32_t top_hit;         /* one region: the grain that sets rhomax lost its last cell, */
@@ -231,6 +232,7 @@ struct GmWindow {
     uint32_t top_pos;         /* its position in rorder (ndefg: none) */
     uint32_t pend_limit;      /* new P-cache entries that keep the cache at most half full */
     uint32_t defer;           /* pending weights may wait for the end of the window */
+    uint32_t need_one;        /* a weight of 1.0 would be the largest so far (one region: GmStepRow::pone is only kept then) */
 };
 
 /* Parents per chunk of the decide and commit passes: a wave takes one chunk at a
@@ -393,7 +395,8 @@ struct GmDev {
     uint32_t *nflag, *nI_, *nB_;
     uint32_t *scan_bsum;        /* 2*GM_SCAN_BLOCKS */
     GmStats *st;
-    uint32_t *prog;             /* mapped host word: (steps the window has finished << 1) | halt */
+    uint32_t *prog;             /* mapped host words: (steps the window has finished << 1) | halt, and whether the
+                                 * stats of the window's end are in the host's mirror */
     /* several memory regions (nreg > 1); with one region none of this is used */
     uint32_t nreg, nlists;      /* T and 2T */
     uint32_t npy, npz, nry, nrz;/* region grid and slab thickness along y and z */
@@ -449,13 +452,14 @@ hipError_t gm_launch_rg_infect(const GmDev &d, const GmPParams &pp, const GmSwee
 hipError_t gm_launch_rg_prefix(const GmDev &d, hipStream_t s);
 /* with several regions: nuclei the host placed, records scattered to their slots */
 hipError_t gm_launch_rg_place(const GmDev &d, const uint32_t *slots, const GmRec *recs, uint32_t n, hipStream_t s);
-/* step j of a one-region window: infections and retirements */
+/* step j of a one-region window: infections and retirements; with `out` the window
+ * ends with it (once a window): the last step's row, the stats into the host's mirror */
 hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P,
-                            const GmWindow &w, uint32_t j, hipStream_t s, hipEvent_t *ev);
+                            const GmWindow &w, uint32_t j, GmStats *out, hipStream_t s, hipEvent_t *ev);
 /* its last pass alone, after the Inside list has grown for it */
-hipError_t gm_launch_commit(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P, uint32_t j,
-                            hipStream_t s, hipEvent_t *ev);
-/* its end after `launched` steps: the last step's row, the stats into the host's mirror */
+hipError_t gm_launch_commit(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P,
+                            const GmWindow &w, uint32_t j, GmStats *out, hipStream_t s, hipEvent_t *ev);
+/* the end of a window whose last step was launched without it, after `launched` steps: the last step's row, the stats into the host's mirror */
 hipError_t gm_launch_window_end(const GmDev &d, const GmPart &P, uint32_t launched, uint32_t top_pos, GmStats *out,
                                 hipStream_t s);
 /* start of a window with several regions: step index and Xcells; clears the window's accumulators */

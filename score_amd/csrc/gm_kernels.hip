@@ -190,6 +190,7 @@ __global__ void __launch_bounds__(GM_BLOCK) k_sweep(GmDev d, GmPart P, uint32_t 
         st->novf = 0;
         st->grow = 0;
         st->need_par = 0;
+        st->ticket = 0;
         d.win->nret0 = st->nret;
         d.win->xcells0 = xcells;
         d.win->npend0 = 0;
@@ -755,18 +756,19 @@ static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, 
     r.recLenB = o.recLenB;
     r.winI = wI;
     r.winB = wB;
-    r.npend = st->npend - win->npend0;
+    const uint32_t npend = agent_load(&st->npend);
+    r.npend = npend - win->npend0;
     r.nattempt = na;
     r.nzeroed = 0;
-    r.err = st->err;
+    r.err = agent_load(&st->err);
     r.nplaced = st->nplaced;
-    r.pone = st->pone;
+    r.pone = agent_load(&st->pone);
     r.pkey = st->arr_pkey;
     st->rows[js] = r;
     st->nplaced = 0;
     st->pone = 0;
     st->arr_pkey = 0ull;
-    win->npend0 = st->npend;
+    win->npend0 = npend;
     st->nI = r.nI;
     st->nB = r.nB;
     st->nret += (unsigned long long)win->full[js];
@@ -1064,7 +1066,8 @@ __global__ void __launch_bounds__(GM_BLOCK) k_decide(GmDev d, GmPart P, uint32_t
  * A winner's rank in its list is the winners before it: the blocks of the decide
  * pass before its own (added up by the block), the chunks before its own in that
  * block, the parents before its own in the chunk. */
-__global__ void __launch_bounds__(GM_BLOCK, 4) k_commit(GmDev d, GmPParams pp, GmSweepArgs A, GmPart P, uint32_t j) {
+static __device__ __forceinline__ void commit_step(const GmDev &d, const GmPParams &pp, const GmSweepArgs &A, const GmPart &P,
+                                                   uint32_t j, uint32_t need_one) {
     struct Wave {
         uint32_t sA[64], sI[64], sB[64], oA[64], oI[64], oB[64];
         uint4 sq0[64];
@@ -1133,8 +1136,8 @@ __global__ void __launch_bounds__(GM_BLOCK, 4) k_commit(GmDev d, GmPParams pp, G
     const uint64_t need = (uint64_t)ws.nI + (totI > ws.recLenI ? totI - ws.recLenI : 0u);
     if (need > d.capI && d.capI < d.capImax) {
         if (db == 0 && threadIdx.x == 0) {
-            st->grow = need < d.capImax ? (uint32_t)need : d.capImax;
-            st->halt = 1u;
+            agent_store(&st->grow, need < d.capImax ? (uint32_t)need : d.capImax);
+            agent_store(&st->halt, 1u);
         }
         return;
     }
@@ -1145,10 +1148,11 @@ __global__ void __launch_bounds__(GM_BLOCK, 4) k_commit(GmDev d, GmPParams pp, G
         if (threadIdx.x == 0 && n) {
             const uint32_t left = d.win->top_left - n;
             d.win->top_left = left;
-            if (left == 0u) d.win->top_hit = 1u;
+            if (left == 0u) agent_store(&d.win->top_hit, 1u);
         }
     }
     Wave &W = sw[wv];
+    bool one = false;
     for (uint32_t c = c0 + wv; c < c1; c += GM_BLOCK / 64u) {
         if (c != c0 + wv) {
             load(c);
@@ -1201,6 +1205,7 @@ __global__ void __launch_bounds__(GM_BLOCK, 4) k_commit(GmDev d, GmPParams pp, G
             const uint32_t *recl = intoI ? d.recI : d.recB;
             const uint32_t rel = rank < recLen ? recl[rank] : (intoI ? ws.nI : ws.nB) + (rank - recLen);
             const NewCell nc = new_cell(d, pp, A, k, W.sfin[q], W.sP[q], pq0, r, g);
+            one |= nc.one;
             if (rel >= (intoI ? d.capI : d.capB)) {
                 atomicOr(&st->err, intoI ? GM_ERRF_INSIDE_FULL : GM_ERRF_BORDER_FULL);
                 continue;
@@ -1209,10 +1214,32 @@ __global__ void __launch_bounds__(GM_BLOCK, 4) k_commit(GmDev d, GmPParams pp, G
         }
         wave_sync();
     }
+    /* (stores to one address are served one after another: only where it matters) */
+    if (need_one && __any(one) && lane == 0) agent_store(&st->pone, 1u);
+}
+
+static __device__ void window_end(const GmDev &d, const GmPart &P, uint32_t launched, uint32_t top_pos, uint32_t *out);
+
+/* With `out` the pass is the window's last: the block that finds all others done closes
+ * the window (window_end), where a launch of its own took 6 us a window: a tenth of a
+ * step where the scalars change in every one.  What it needs of the other
+ * blocks they change by device atomics alone (counters, flags, the new pairs' keys),
+ * so no block has to write its XCD's cache back; each waits until its own have
+ * arrived before it takes its ticket. */
+__global__ void __launch_bounds__(GM_BLOCK, 4) k_commit(GmDev d, GmPParams pp, GmSweepArgs A, GmPart P, uint32_t j,
+                                                       uint32_t need_one, uint32_t top_pos, uint32_t *out) {
+    __shared__ uint32_t last;
+    commit_step(d, pp, A, P, j, need_one);
+    if (!out) return;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0) last = atomicAdd(&d.st->ticket, 1u) == gridDim.x - 1u ? 1u : 0u;
+    __syncthreads();
+    if (last) window_end(d, P, j + 1u, top_pos, out);
 }
 
 hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P,
-                            const GmWindow &w, uint32_t j, hipStream_t s, hipEvent_t *ev) {
+                            const GmWindow &w, uint32_t j, GmStats *out, hipStream_t s, hipEvent_t *ev) {
     hipError_t e;
     if ((e = mark(ev, 4, s)) != hipSuccess) return e;
     k_propose<<<P.nbp + 1u, GM_BLOCK, 0, s>>>(d, P, w, j, a.k + j);
@@ -1223,15 +1250,15 @@ hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepAr
     k_decide<<<nrec + P.nbd, GM_BLOCK, lds, s>>>(d, P, j, nrec, w.top_pos);
     for (int i = 6; i <= 8; i++)
         if ((e = mark(ev, i, s)) != hipSuccess) return e;
-    return gm_launch_commit(d, pp, a, P, j, s, ev);
+    return gm_launch_commit(d, pp, a, P, w, j, out, s, ev);
 }
 
-hipError_t gm_launch_commit(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P, uint32_t j,
-                            hipStream_t s, hipEvent_t *ev) {
+hipError_t gm_launch_commit(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P,
+                            const GmWindow &w, uint32_t j, GmStats *out, hipStream_t s, hipEvent_t *ev) {
     hipError_t e;
     GmSweepArgs A = a;
     A.k = a.k + j;
-    k_commit<<<P.nbd, GM_BLOCK, 0, s>>>(d, pp, A, P, j);
+    k_commit<<<P.nbd, GM_BLOCK, 0, s>>>(d, pp, A, P, j, w.need_one, w.top_pos, reinterpret_cast<uint32_t *>(out));
     if ((e = mark(ev, 9, s)) != hipSuccess) return e;
     return hipGetLastError();
 }
@@ -1480,20 +1507,27 @@ hipError_t gm_launch_resolve_pending(const GmDev &d, const double *vals, uint32_
     return hipGetLastError();
 }
 
-/* the stats into the host's pinned mirror (mapped, coherent), word by word:
- * cheaper than a copy command at the end of every window.  Only the filled part
- * of the inline id and key arrays crosses the bus; the host reads no more. */
+/* The stats into the host's pinned mirror (mapped, coherent), word by word, by one
+ * block: cheaper than a copy command at the end of every window.  Only the filled part
+ * of the inline id and key arrays crosses the bus; the host reads no more.  When every
+ * word has arrived the host is told by the word behind the progress word, which it
+ * waits for instead of the kernel's end (the launch's own completion reaches it 8 us
+ * later). */
 static __device__ __forceinline__ void copy_stats(const GmDev &d, uint32_t *out) {
     const uint32_t *in = reinterpret_cast<const uint32_t *>(d.st);
     const GmStats *st = d.st;
-    const uint32_t nz = st->nzeroed < GM_ZEROED_INLINE ? st->nzeroed : GM_ZEROED_INLINE;
-    const uint32_t np = st->npend < GM_PEND_INLINE ? st->npend : GM_PEND_INLINE;
+    const uint32_t nzd = agent_load(&st->nzeroed), npd = agent_load(&st->npend);
+    const uint32_t nz = nzd < GM_ZEROED_INLINE ? nzd : GM_ZEROED_INLINE;
+    const uint32_t np = npd < GM_PEND_INLINE ? npd : GM_PEND_INLINE;
     const uint32_t z0 = offsetof(GmStats, zeroed_ids) / 4, p0 = offsetof(GmStats, pend_keys) / 4;
     const uint32_t t0 = offsetof(GmStats, kcur) / 4, end = sizeof(GmStats) / 4;
     for (uint32_t i = threadIdx.x; i < end; i += GM_BLOCK) {
         const bool skip = (i >= z0 + nz && i < p0) || (i >= p0 + 2u * np && i < t0);
-        if (!skip) out[i] = in[i];
+        if (!skip) __hip_atomic_store(out + i, agent_load(in + i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0 && d.prog) __hip_atomic_store(d.prog + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ void __launch_bounds__(GM_BLOCK) k_stats_out(GmDev d, uint32_t *out) { copy_stats(d, out); }
@@ -1503,15 +1537,14 @@ hipError_t gm_launch_stats_out(const GmDev &d, GmStats *out, hipStream_t s) {
     return hipGetLastError();
 }
 
-/* The end of a window of `launched` steps: its last step is closed, unless the
- * window halted (the propose pass that halted it closed the step before), and
- * the stats go to the host's mirror.  If the grain that sets rhomax lost its last
+/* The end of a window of `launched` steps, by one block: its last step is closed,
+ * unless the window halted (the propose pass that halted it closed the step before),
+ * and the stats go to the host's mirror.  If the grain that sets rhomax lost its last
  * cell, its successor is looked up. */
-__global__ void __launch_bounds__(GM_BLOCK) k_window_end(GmDev d, GmPart P, uint32_t launched, uint32_t top_pos,
-                                                         uint32_t *out) {
+static __device__ void window_end(const GmDev &d, const GmPart &P, uint32_t launched, uint32_t top_pos, uint32_t *out) {
     __shared__ uint32_t first;
-    const uint32_t hit = d.win->top_hit;
-    if (!d.st->halt && d.st->nexec + 1u == launched) close_step(d, P, launched - 1u, false);
+    const uint32_t hit = agent_load(&d.win->top_hit);
+    if (!agent_load(&d.st->halt) && d.st->nexec + 1u == launched) close_step(d, P, launched - 1u, false);
     if (hit) { /* the next grain in the order of rho that holds cells */
         if (threadIdx.x == 0) first = d.ndefg;
         for (uint32_t i0 = top_pos; i0 < d.ndefg; i0 += GM_BLOCK) {
@@ -1531,8 +1564,14 @@ __global__ void __launch_bounds__(GM_BLOCK) k_window_end(GmDev d, GmPart P, uint
         if (threadIdx.x == 0) d.st->top_next = first;
     }
     if (threadIdx.x == 0) d.st->top_hit = hit;
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     copy_stats(d, out);
+}
+
+__global__ void __launch_bounds__(GM_BLOCK) k_window_end(GmDev d, GmPart P, uint32_t launched, uint32_t top_pos,
+                                                         uint32_t *out) {
+    window_end(d, P, launched, top_pos, out);
 }
 
 hipError_t gm_launch_window_end(const GmDev &d, const GmPart &P, uint32_t launched, uint32_t top_pos, GmStats *out,
@@ -1912,10 +1951,7 @@ hipError_t gm_launch_window_begin(const GmDev &d, uint32_t k, double xcells, hip
 
 
 /* One wave after the commit pass: the step's row and whether the next step of
- * the window may run.  (A separate kernel: the kernel boundary is the grid-wide
- * barrier, where a last-block handoff inside the commit pass would need a
- * device-scope release per block, which on this GPU writes back the L2 of the
- * block's XCD.) */
+ * the window may run. */
 __global__ void __launch_bounds__(64) k_step_tail(GmDev d, GmWindow w) {
     if (d.st->halt) return;
     step_tail(d, w);
@@ -1980,7 +2016,8 @@ __global__ void __launch_bounds__(GM_BLOCK) k_reinsert_spilled(GmDev d, GmPParam
         if (d.cstep[s] != GM_CS_DEFERRED) continue;
         GmRec *r = d.rec + s;
         if (!is_spilled(r->P)) continue;
-        r->P = pair_weight(d, pp, r->rxg, r->defg);
+        bool one = false;
+        r->P = pair_weight(d, pp, r->rxg, r->defg, one);
     }
 }
 

@@ -825,7 +825,9 @@ __global__ void __launch_bounds__(64) k_rg_commit(GmDev d, GmPParams pp, GmSweep
                 atomicOr(&st->err, (l & 1u) ? GM_ERRF_BORDER_FULL : GM_ERRF_INSIDE_FULL);
                 continue;
             }
-            put_cell(d, k, new_cell(d, pp, A, k, sfin[j], sP[j], pq0, r, g, o.khi != 0u), pq0, t, g, o.x, o.y, o.z, bs + rel);
+            const NewCell nc = new_cell(d, pp, A, k, sfin[j], sP[j], pq0, r, g, o.khi != 0u);
+            if (nc.one) st->pone = 1u;
+            put_cell(d, k, nc, pq0, t, g, o.x, o.y, o.z, bs + rel);
         }
         run[GM_RW_I] += bt >> 16;
         run[GM_RW_B] += bt & 0xFFFFu;
