@@ -1065,8 +1065,9 @@ int ensure_step_capacity(score_gm_handle *h) {
     return need > d.capI ? grow_front(h, (uint32_t)need) : 0;
 }
 
-/* Evaluate the pending pairs with glibc and store them in the device cache. */
-int resolve_pending(score_gm_handle *h, const GmStats &st) {
+/* Evaluate the pending pairs with glibc and store them in the device cache (store
+ * false: the caller does that). */
+int resolve_pending(score_gm_handle *h, const GmStats &st, bool store = true) {
     const uint32_t npend = st.npend;
     if (npend == 0) return 0;
     GmDev &d = h->d;
@@ -1100,7 +1101,7 @@ int resolve_pending(score_gm_handle *h, const GmStats &st) {
     /* stream-ordered: the kernel reads the values from the mapped buffer and
      * stores them into the cache before the next step's kernels read it; the
      * buffer is not rewritten before the next window's sync */
-    HIPCHK(gm_launch_resolve_pending(d, h->hpend_dev, npend, h->stream));
+    if (store) HIPCHK(gm_launch_resolve_pending(d, h->hpend_dev, npend, h->stream));
     h->hcount += npend;
     return 0;
 }
@@ -1613,7 +1614,9 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
         pf.pending_resolved += r0.npend;
     }
     /* the window's new pairs, evaluated with glibc and stored in the device cache */
-    if ((rc = resolve_pending(h, st))) return h->err = rc;
+    const bool fused = st.npend && st.npend <= GM_RP_MAX && st.ndeferred && st.ndeferred <= std::min(GM_RP_MAX, d.dlistCap) &&
+                       !st.novf && ((uint64_t)h->hcount + st.npend) * 2 <= d.hcap;
+    if ((rc = resolve_pending(h, st, !fused))) return h->err = rc;
     {
         const GmStepRow &last = st.rows[nexec - 1];
         h->nI = last.nI;
@@ -1639,7 +1642,9 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
         ad.k = h->step + nexec;
         ad.nI = h->nI;
         ad.nB = h->nB;
-        if ((e = gm_launch_predict_deferred(d, ad, st.ndeferred, h->stream)) != hipSuccess)
+        e = fused ? gm_launch_resolve_predict(d, ad, h->hpend_dev, st.npend, h->stream)
+                  : gm_launch_predict_deferred(d, ad, st.ndeferred, h->stream);
+        if (e != hipSuccess)
             return h->err = hip_fail(e, "deferred predictions");
     }
     /* master section of every step (SCORE_Kernel.cpp:6688-6742) */

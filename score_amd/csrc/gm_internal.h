@@ -119,7 +119,9 @@ static inline __host__ __device__ uint32_t gm_tiles_inside(uint32_t nI) {
 #define GM_SW_BLOCKS 2048u        /* sweep blocks up to GM_SW_MAXCPW chunks per wave */
 #define GM_SW_MAXCPW 32u
 #define GM_SW_PACK 31u            /* chunks whose per-lane counts fit a byte */
-#define GM_SW_FOLD 256u           /* sweep blocks up to which no scan pass runs between counting and compaction */
+#define GM_SW_FOLD 256u           /* sweep blocks up to which no scan pass runs between counting and compaction; more
+                                   * in a window of few steps, while a compaction block has at most ten rows of 256
+                                   * counts to add up (a scan pass takes 5 us) */
 #define GM_PB 2048u               /* blocks of the propose pass at most */
 #define GM_DB 1024u               /* blocks of the decide and commit passes at most */
 #define GM_GRID_BLOCKS 2048u      /* blocks of the pass over the cell grid at most */
@@ -472,6 +474,9 @@ hipError_t gm_launch_step_tail(const GmDev &d, const GmWindow &w, hipStream_t s)
 hipError_t gm_launch_predict_deferred(const GmDev &d, const GmSweepArgs &a, uint32_t ndeferred, hipStream_t s);
 hipError_t gm_launch_nucleate(const GmDev &d, const uint32_t *site, const double *nucP, uint32_t nrxg, hipStream_t s);
 hipError_t gm_launch_resolve_pending(const GmDev &d, const double *vals, uint32_t npend, hipStream_t s);
+/* gm_launch_resolve_pending and gm_launch_predict_deferred in one, for GM_RP_MAX of each at most */
+#define GM_RP_MAX 2048u
+hipError_t gm_launch_resolve_predict(const GmDev &d, const GmSweepArgs &a, const double *vals, uint32_t npend, hipStream_t s);
 hipError_t gm_launch_stats_out(const GmDev &d, GmStats *out, hipStream_t s);
 /* SCORE's view of slots [base, base+n) before step k, unpacked into per-field arrays */
 struct GmFrontOut {

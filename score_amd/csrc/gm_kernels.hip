@@ -281,7 +281,7 @@ static __device__ void window_totals(const GmDev &d, const GmPart &P, const uint
     s.recLenB = recB < d.recCapB ? recB : d.recCapB;
 }
 
-/* pass 2, where the window has more than GM_SW_FOLD blocks: one block, a wave
+/* pass 2, where the window has many blocks (GM_SW_FOLD): one block, a wave
  * per row of counts, 32 consecutive entries per lane; exclusive prefixes over
  * the blocks.  The INACTIVE counts and their prefixes within each list go to the
  * recycling tables of step 0.  (With fewer blocks each block of pass 3 adds up
@@ -353,7 +353,7 @@ __global__ void __launch_bounds__(1024) k_sweep_scan(GmDev d, GmPart P) {
  * every step as ordered compaction: step i's completed slots ascending, Inside
  * then Border, at pslot[win->off[i]...]; and the INACTIVE mask of every 64-slot
  * tile, from which the steps hand out recycled slots.  FOLD: the block adds up
- * the counts of at most GM_SW_FOLD blocks itself. */
+ * the counts of the blocks itself. */
 template <bool FOLD>
 __global__ void __launch_bounds__(GM_BLOCK) k_compact(GmDev d, GmPart P, uint32_t k0) {
     __shared__ uint32_t stot[GM_WMAX + 1], spre[GM_WMAX + 1], stotI[GM_WMAX + 1], base[GM_WMAX];
@@ -366,17 +366,17 @@ __global__ void __launch_bounds__(GM_BLOCK) k_compact(GmDev d, GmPart P, uint32_
         for (uint32_t row = w; row <= P.W; row += GM_SW_WAVES) {
             const bool rec = row == P.W;
             const uint32_t *cnt = d.wcnt + (size_t)(rec ? (uint32_t)GM_WMAX : row) * d.swb;
-            const uint32_t i0 = 4u * lane;
-            uint4 q = make_uint4(0u, 0u, 0u, 0u);
-            if (i0 < P.nb) q = *reinterpret_cast<const uint4 *>(cnt + i0);
-            const uint32_t v[4] = {q.x, q.y, q.z, q.w};
             uint32_t a = 0, p = 0, pI = 0;
+            for (uint32_t i0 = 4u * lane; i0 < P.nb; i0 += 256u) {
+                const uint4 q = *reinterpret_cast<const uint4 *>(cnt + i0);
+                const uint32_t v[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-            for (uint32_t i = 0; i < 4; i++) {
-                const uint32_t x = i0 + i < P.nb ? v[i] : 0u;
-                a += x;
-                p += i0 + i < b ? x : 0u;
-                pI += i0 + i < P.nbI ? x : 0u;
+                for (uint32_t i = 0; i < 4; i++) {
+                    const uint32_t x = i0 + i < P.nb ? v[i] : 0u;
+                    a += x;
+                    p += i0 + i < b ? x : 0u;
+                    pI += i0 + i < P.nbI ? x : 0u;
+                }
             }
             for (int o = 32; o > 0; o >>= 1) {
                 a += __shfl_xor(a, o, 64);
@@ -490,7 +490,7 @@ hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &
     if ((e = mark(ev, 1, s)) != hipSuccess) return e;
     k_sweep<<<P.nb, GM_BLOCK, 0, s>>>(d, P, a.k, xcells, wd.top_pos);
     if ((e = mark(ev, 2, s)) != hipSuccess) return e;
-    const bool fold = P.nb <= GM_SW_FOLD;
+    const bool fold = P.nb <= GM_SW_FOLD || (P.W + 1u) * P.nb <= GM_SW_FOLD * 10u;
     if (!fold) k_sweep_scan<<<1, 1024, 0, s>>>(d, P);
     if ((e = mark(ev, 3, s)) != hipSuccess) return e;
     if (fold) k_compact<true><<<P.nb, GM_BLOCK, 0, s>>>(d, P, a.k);
@@ -1967,11 +1967,11 @@ hipError_t gm_launch_step_tail(const GmDev &d, const GmWindow &w, hipStream_t s)
  * value before step a.k is replayed from the anchor, then predicted.  The cells
  * come from the deferred list, or from a scan of every occupied slot when the
  * list overflowed. */
-__global__ void __launch_bounds__(GM_BLOCK) k_predict_deferred(GmDev d, GmSweepArgs A) {
+static __device__ __forceinline__ void predict_deferred(const GmDev &d, const GmSweepArgs &A, uint32_t i0, uint32_t stride) {
     const uint32_t nd = d.st->ndeferred;
     const bool listed = nd <= d.dlistCap;
     const uint32_t nI = d.st->nI, n = listed ? nd : nI + d.st->nB;
-    for (uint32_t i = blockIdx.x * GM_BLOCK + threadIdx.x; i < n; i += gridDim.x * GM_BLOCK) {
+    for (uint32_t i = i0; i < n; i += stride) {
         const uint32_t s = listed ? d.dlist[i] : occ_slot(d, nI, i);
         if (d.cstep[s] != GM_CS_DEFERRED) continue;
         GmRec *r = d.rec + s;
@@ -1987,6 +1987,24 @@ __global__ void __launch_bounds__(GM_BLOCK) k_predict_deferred(GmDev d, GmSweepA
         if (cell_increment(d, A.sp, P, c.defg, a.inf, inc)) f = gm_radd_n(f, inc, A.k - a.s0);
         predict_slot(d, A, s, f, A.k, P, c.defg, a.inf);
     }
+}
+
+__global__ void __launch_bounds__(GM_BLOCK) k_predict_deferred(GmDev d, GmSweepArgs A) {
+    predict_deferred(d, A, blockIdx.x * GM_BLOCK + threadIdx.x, gridDim.x * GM_BLOCK);
+}
+
+/* A window's new weights into the cache and the cells that wait for them predicted, by
+ * one block: few of both is the ordinary case, and two launches with a gap took 8 us
+ * of it, in three steps of four on the rolled sheet. */
+__global__ void __launch_bounds__(1024) k_resolve_predict(GmDev d, GmSweepArgs A, const double *vals, uint32_t npend) {
+    for (uint32_t i = threadIdx.x; i < npend; i += 1024u) d.hvals[d.pend_slot[i]] = vals[i];
+    __syncthreads();
+    predict_deferred(d, A, threadIdx.x, 1024u);
+}
+
+hipError_t gm_launch_resolve_predict(const GmDev &d, const GmSweepArgs &a, const double *vals, uint32_t npend, hipStream_t s) {
+    k_resolve_predict<<<1, 1024, 0, s>>>(d, a, vals, npend);
+    return hipGetLastError();
 }
 
 hipError_t gm_launch_predict_deferred(const GmDev &d, const GmSweepArgs &a, uint32_t ndeferred, hipStream_t s) {

@@ -56,3 +56,19 @@ def test_blocks_of_the_last_pass(require_gpu, nuclei, model):
     e = 70 if nuclei == 5000 else 36
     dom = synth.make_voronoi_domain(e + 5, e + 2, e - 1, n_grains=9, n_nuclei=nuclei, seed=nuclei)
     _same(dom, ParamsSpec(mobility_model=model, xmax=0.3 if nuclei == 1 else 0.99), 7)
+
+
+def test_one_step_windows_of_a_long_front(require_gpu):
+    """Windows of one step whose compaction adds up more than 256 blocks' counts, and
+    new pairs beyond and below the number one block resolves."""
+    dom = synth.make_voronoi_domain(150, 140, 130, n_grains=6000, n_nuclei=9000, seed=4)
+    prm = ParamsSpec(mobility_model=abi.MOB_SEBALDGOTTSTEIN, xmax=0.6)
+    o, g = Oracle(dom, prm), GrowthMachine(dom, prm)
+    o.solve_rxgrowth()
+    g.solve_rxgrowth()
+    to, tg = o.trajectory(), g.trajectory()
+    assert same_trajectory(to, tg)
+    assert np.array_equal(o.grainmap(), g.grainmap())
+    assert (tg["nslots_inside"] + tg["nslots_border"]).max() > 256 * 2048
+    assert tg["npending"].max() > 2048 and ((tg["npending"] > 0) & (tg["npending"] <= 2048)).any()
+    g.close()
