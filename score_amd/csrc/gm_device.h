@@ -596,34 +596,16 @@ static __device__ __forceinline__ uint32_t retire_runs(const GmDev &d, uint32_t 
     return (nxt ? (uint32_t)__ffsll((long long)nxt) - 1u : 64u) - lane;
 }
 
-/* One region: the deformed grains' counts are taken down in GM_SUBS parts each,
+/* The deformed grains' counts are taken down in GM_SUBS parts each,
  * part `sub` by this block.  Atomics on one address are served one after another,
  * and a step takes some 30 to 50 cells from every grain: with one counter a grain,
  * whose old value told when the grain was exhausted, the commit pass took 21.6 us
  * at 320^3 and 11.8 at 100^3, without it 13.5 and 8.8.  Which grains are exhausted
  * is only asked of the one that sets rhomax: it is counted per step
- * (k_decide, k_commit), and its successor found when it is gone (k_window_end). */
+ * (the decide passes), and its successor found when it is gone (find_successor). */
 static __device__ __forceinline__ void retire(const GmDev &d, uint32_t g, uint32_t r, bool valid, uint32_t sub) {
     const uint32_t n = retire_runs(d, g, r, valid);
     if (n) atomicAdd(&d.defsub[(size_t)sub * d.ndefg + g], n);
-}
-
-/* Several regions: a deformed grain losing its last cell is reported so the host
- * can update rhomax (update_myrhomax, SCORE_RecoveryModels.cpp:146-165). */
-static __device__ __forceinline__ void retire_batch(const GmDev &d, const uint4 &q0, bool valid) {
-    GmStats *st = d.st;
-    const uint32_t g = q0.z, n = retire_runs(d, g, q0.w, valid);
-    if (!n) return;
-    const uint32_t old = atomicSub(&d.defcnt[g], n);
-    if (old == n) {
-        const uint32_t i = atomicAdd(&st->nzeroed, 1u);
-        if (i < GM_ZEROED_INLINE) st->zeroed_ids[i] = g;
-        if (i < d.ndefg) d.zlist[i] = g;
-    } else if (old < n) {
-        /* only a cell held by two records retires twice; the count wraps
-         * as SCORE's uint32 does and the host re-reads them all */
-        st->cwrap = 1u;
-    }
 }
 
 /* With several regions: the row of the step just done, and whether the next one may run without the
@@ -653,23 +635,13 @@ static __device__ void step_finish(const GmDev &d, const GmWindow &w, const GmSt
     st->halt = halt ? 1u : 0u;
 }
 
-/* whether one of the grains exhausted in this step (zlist[z0, z1)) sets rhomax;
- * every lane of the calling wave takes part */
-static __device__ __forceinline__ bool top_exhausted(const GmDev &d, const GmWindow &w, uint32_t z0, uint32_t z1) {
-    bool top = false;
-    for (uint32_t i = z0 + (threadIdx.x & 63u); i < z1; i += 64) top |= d.zlist[i] == w.top_grain;
-    return __ballot(top) != 0ull;
-}
-
-/* The end of a step, run by one wave after the commit pass: the step's row and
- * whether the next step may run; the window's progress, (steps finished << 1) |
- * halt, goes to the host's mapped word, which paces the launches (gm_host.cpp,
- * step_window). */
+/* The end of a step with several regions, run by the commit pass's last block (one
+ * wave): the step's row and whether the next step may run; the window's progress,
+ * (steps finished << 1) | halt, goes to the host's mapped word, which paces the
+ * launches (gm_host.cpp, step_window).  What the pass's other blocks changed, they
+ * changed by device atomics. */
 static __device__ void step_tail(const GmDev &d, const GmWindow &w) {
     GmStats *st = d.st;
-    const uint32_t j = st->nexec;
-    const uint32_t z0 = j ? st->rows[j - 1].nzeroed : 0u, z1 = st->nzeroed < d.ndefg ? st->nzeroed : d.ndefg;
-    const bool any_top = top_exhausted(d, w, z0, z1);
     if (threadIdx.x != 0) return;
     GmStepRow r;
     r.nI = st->nI;
@@ -682,18 +654,78 @@ static __device__ void step_tail(const GmDev &d, const GmWindow &w) {
     r.recLenB = st->recLenB;
     r.winI = st->winI;
     r.winB = st->winB;
-    r.npend = st->npend - st->npend0;
+    r.npend = agent_load(&st->npend) - st->npend0;
     r.nattempt = st->nattempt;
-    r.nzeroed = z1;
-    r.err = st->err;
+    r.err = agent_load(&st->err);
     r.nplaced = st->nplaced;
-    r.pone = st->pone;
+    r.pone = agent_load(&st->pone);
     r.pkey = st->arr_pkey;
     st->nplaced = 0;
     st->pone = 0;
     st->arr_pkey = 0ull;
-    step_finish(d, w, r, any_top);
+    step_finish(d, w, r, d.win->top_hit != 0u);
     if (d.prog) __hip_atomic_store(d.prog, (st->nexec << 1) | st->halt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+/* a grain's cells: the count at the last fold less the parts taken since; every lane of
+ * the wave takes part and gets the value */
+static __device__ __forceinline__ uint32_t exact_count(const GmDev &d, uint32_t g) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t v = lane < GM_SUBS ? d.defsub[(size_t)lane * d.ndefg + g] : 0u;
+    for (int o = 32; o > 0; o >>= 1) v += (uint32_t)__shfl_xor((int)v, o, 64);
+    return d.defcnt[g] - v;
+}
+
+/* The grain that sets rhomax lost its last cell: the position in the order of rho of
+ * the next one that holds cells (ndefg: none) into st->top_next, by one block. */
+static __device__ void find_successor(const GmDev &d, uint32_t top_pos) {
+    __shared__ uint32_t first;
+    if (threadIdx.x == 0) first = d.ndefg;
+    for (uint32_t i0 = top_pos; i0 < d.ndefg; i0 += blockDim.x) {
+        const uint32_t i = i0 + threadIdx.x;
+        __syncthreads();
+        if (first < d.ndefg) break;
+        __syncthreads();
+        if (i < d.ndefg) {
+            const uint32_t g = d.rorder[i];
+            uint32_t n = d.defcnt[g];
+#pragma unroll
+            for (uint32_t q = 0; q < GM_SUBS; q++) n -= d.defsub[(size_t)q * d.ndefg + g];
+            if (n) atomicMin(&first, i);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) d.st->top_next = first;
+}
+
+/* The stats into the host's pinned mirror (mapped, coherent), word by word, by one
+ * block: cheaper than a copy command at the end of every window.  Only the filled part
+ * of the inline key array crosses the bus; the host reads no more.  When every
+ * word has arrived the host is told by the word behind the progress word, which it
+ * waits for instead of the kernel's end (the launch's own completion reaches it 8 us
+ * later). */
+static __device__ __forceinline__ void copy_stats(const GmDev &d, uint32_t *out) {
+    const uint32_t *in = reinterpret_cast<const uint32_t *>(d.st);
+    const uint32_t npd = agent_load(&d.st->npend), np = npd < GM_PEND_INLINE ? npd : GM_PEND_INLINE;
+    const uint32_t p0 = offsetof(GmStats, pend_keys) / 4, t0 = offsetof(GmStats, kcur) / 4, end = sizeof(GmStats) / 4;
+    for (uint32_t i = threadIdx.x; i < end; i += blockDim.x) {
+        const bool skip = i >= p0 + 2u * np && i < t0;
+        if (!skip) __hip_atomic_store(out + i, agent_load(in + i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0 && d.prog) __hip_atomic_store(d.prog + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+/* the end of a window, by one block: the successor of the grain that sets rhomax, if it
+ * lost its last cell, and the stats to the host */
+static __device__ __forceinline__ void stats_to_host(const GmDev &d, uint32_t top_pos, uint32_t *out) {
+    const uint32_t hit = agent_load(&d.win->top_hit);
+    if (hit) find_successor(d, top_pos);
+    if (threadIdx.x == 0) d.st->top_hit = hit;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    copy_stats(d, out);
 }
 
 /* orders a wave's LDS writes before its later LDS reads (the lanes of a wave

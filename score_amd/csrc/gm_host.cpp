@@ -203,7 +203,6 @@ struct score_gm_handle {
     std::vector<uint32_t> rho_pos;     /* each grain's place in it (staging for the device) */
     std::vector<uint8_t> alive;
     size_t rho_top = 0;
-    std::vector<uint32_t> zbuf;
     /* weights of the window's new pairs, in insertion order (steps in order; a
      * spilled step's re-inserted pairs last) */
     std::vector<double> pend_P;
@@ -446,7 +445,7 @@ void free_device(score_gm_handle *h) {
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     void *ptrs[] = {d.cell, d.pmA, d.gatt, d.rlog, d.dmap, d.cstep, d.rec, d.pslot, d.dlist,
                     d.par, d.recI, d.recB, d.mF, d.mR, d.pmI, d.pmB, d.bcnt, d.rho, d.defq,
-                    d.rxq, d.defcnt, d.rxcnt, d.zlist, d.hkeys, d.hvals, d.pend_slot, d.pend_key, d.nflag, d.nI_, d.nB_,
+                    d.rxq, d.defcnt, d.rxcnt, d.hkeys, d.hvals, d.pend_slot, d.pend_key, d.nflag, d.nI_, d.nB_,
                     d.scan_bsum, d.st, d.arr_ids, d.arr_off, d.nsite, d.nucP,
                     d.win, d.wcnt, d.wpre, d.wwave, d.rcnt, d.rpre, d.rgone, d.rmrg, d.acnt, d.btot, d.btop, d.ccnt, d.defsub, d.rorder, d.rpos,
                     d.reg, d.pmH, d.L.base, d.L.cap, d.L.rcap, d.L.rbase, d.L.n, d.L.nold, d.L.rlen,
@@ -1200,10 +1199,9 @@ int set_list_lengths(score_gm_handle *h, const std::vector<uint32_t> &n) {
     return 0;
 }
 
-/* one region: the grains' order of rho to the device */
+/* the grains' order of rho to the device */
 int upload_order(score_gm_handle *h) {
     GmDev &d = h->d;
-    if (d.nreg > 1) return 0;
     h->rho_pos.resize(d.ndefg);
     for (uint32_t i = 0; i < d.ndefg; i++) h->rho_pos[h->rho_order[i]] = i;
     HIPCHK(hipMemcpyAsync(d.rorder, h->rho_order.data(), sizeof(uint32_t) * d.ndefg, hipMemcpyHostToDevice, h->stream));
@@ -1215,7 +1213,7 @@ int upload_order(score_gm_handle *h) {
 int refresh_alive(score_gm_handle *h) {
     GmDev &d = h->d;
     std::vector<uint32_t> cnt(d.ndefg);
-    if (d.nreg <= 1) HIPCHK(gm_launch_fold_counts(d, h->stream));
+    HIPCHK(gm_launch_fold_counts(d, h->stream));
     HIPCHK(hipMemcpyAsync(cnt.data(), d.defcnt, sizeof(uint32_t) * d.ndefg, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
     for (uint32_t g = 0; g < d.ndefg; g++) h->alive[g] = cnt[g] > 0 ? 1 : 0;
@@ -1359,7 +1357,7 @@ int log_grainevo(score_gm_handle *h, uint32_t sv) {
     GmDev &d = h->d;
     const size_t ng = (size_t)d.ndefg + d.nrxg;
     const size_t off = h->glog_counts.size();
-    if (d.nreg <= 1) HIPCHK(gm_launch_fold_counts(d, h->stream));
+    HIPCHK(gm_launch_fold_counts(d, h->stream));
     h->glog_counts.resize(off + ng);
     HIPCHK(hipMemcpyAsync(h->glog_counts.data() + off, d.defcnt, sizeof(uint32_t) * d.ndefg, hipMemcpyDeviceToHost,
                           h->stream));
@@ -1512,7 +1510,6 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
     GmWindow w;
     memset(&w, 0, sizeof(w));
     w.xstop = window_xstop(h);
-    w.top_grain = h->rho_top < h->rho_order.size() ? h->rho_order[h->rho_top] : 0xFFFFFFFFu;
     w.top_pos = (uint32_t)std::min<size_t>(h->rho_top, d.ndefg);
     w.pend_limit = (uint32_t)std::min<uint64_t>(0xFFFFFFFFull, (uint64_t)d.hcap / 2 > h->hcount ? (uint64_t)d.hcap / 2 - h->hcount : 0ull);
     w.defer = W > 1 ? 1u : 0u;
@@ -1529,7 +1526,7 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
     if (paced) __atomic_store_n(h->hprog, 0u, __ATOMIC_RELAXED);
     __atomic_store_n(h->hprog + 1, 0u, __ATOMIC_RELAXED);
     if (d.nreg > 1)
-        e = gm_launch_window_begin(d, h->step, h->Xcells, h->stream);
+        e = gm_launch_window_begin(d, h->step, h->Xcells, w.top_pos, h->stream);
     else
         e = gm_launch_window(d, P, a, w, na != 0, h->Xcells, h->stream, ev);
     if (e != hipSuccess) return h->err = hip_fail(e, "growth step");
@@ -1541,20 +1538,21 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
     for (uint32_t j = 0; j < W; j++) {
         if (paced && j > GM_LEAD && !wait_steps(h, j - GM_LEAD)) break;
         launched = j + 1;
+        GmStats *end = launched == W && !prof ? h->hst_dev : nullptr;
         if (d.nreg > 1) {
             GmSweepArgs aj = a;
             if (j) aj.reanchor = 0;
             if ((e = gm_launch_rg_sweep(d, aj, rg_parents, h->stream, ev)) != hipSuccess ||
-                (e = gm_launch_rg_infect(d, h->pp, aj, rg_parents, h->stream, ev)) != hipSuccess ||
-                (e = gm_launch_step_tail(d, w, h->stream)) != hipSuccess)
+                (e = gm_launch_rg_infect(d, h->pp, aj, rg_parents, w, end, h->stream, ev)) != hipSuccess)
                 return h->err = hip_fail(e, "growth step");
             continue;
         }
-        if ((e = gm_launch_infect(d, h->pp, a, P, w, j, j + 1 == W && !prof ? h->hst_dev : nullptr, h->stream, ev)) != hipSuccess)
+        if ((e = gm_launch_infect(d, h->pp, a, P, w, j, end, h->stream, ev)) != hipSuccess)
             return h->err = hip_fail(e, "growth step");
     }
-    if (d.nreg > 1) e = gm_launch_stats_out(d, h->hst_dev, h->stream);
-    else if (launched < W || prof) e = gm_launch_window_end(d, P, launched, w.top_pos, h->hst_dev, h->stream);
+    if (launched < W || prof)
+        e = d.nreg > 1 ? gm_launch_rg_window_end(d, w, h->hst_dev, h->stream)
+                       : gm_launch_window_end(d, P, launched, w.top_pos, h->hst_dev, h->stream);
     if (e != hipSuccess || (e = prof ? hipStreamSynchronize(h->stream) : wait_window(h)) != hipSuccess)
         return h->err = hip_fail(e, "growth step");
     /* a step that found too few Inside slots or parents' entries waits for them:
@@ -1682,22 +1680,9 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
         h->X = (h->Xcells / ((double)d.N));
         h->sum_sv += sv;
         if (j + 1 == nexec) {
-            /* grains that lost their last cell leave the rhomax search; before the
-             * last step of a window none of them was the one that sets rhomax */
-            if (d.nreg > 1 && st.nzeroed) {
-                const uint32_t *ids = st.zeroed_ids;
-                if (st.nzeroed > GM_ZEROED_INLINE) {
-                    h->zbuf.resize(st.nzeroed);
-                    if ((e = hipMemcpyAsync(h->zbuf.data(), d.zlist, sizeof(uint32_t) * std::min(st.nzeroed, d.ndefg),
-                                            hipMemcpyDeviceToHost, h->stream)) != hipSuccess ||
-                        (e = hipStreamSynchronize(h->stream)) != hipSuccess)
-                        return h->err = hip_fail(e, "exhausted grains");
-                    ids = h->zbuf.data();
-                }
-                for (uint32_t i = 0; i < std::min(st.nzeroed, d.ndefg); i++) h->alive[ids[i]] = 0;
-            }
-            /* one region: those before the successor of the grain that set rhomax */
-            if (d.nreg <= 1 && st.top_hit)
+            /* the grain that set rhomax and those after it that hold no cells leave the
+             * search; before the last step of a window it was not gone */
+            if (st.top_hit)
                 for (uint32_t i = w.top_pos; i < std::min(st.top_next, d.ndefg); i++) h->alive[h->rho_order[i]] = 0;
             /* a count went below zero and wrapped: cellcount > 0 again, as in SCORE */
             if (st.cwrap && (rc = refresh_alive(h))) return h->err = rc;
@@ -1708,8 +1693,8 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
              * order that recovery kept (every rho scaled alike) is not sorted again */
             auto desc = [&](uint32_t a, uint32_t b) { return h->rho_host[a] > h->rho_host[b]; };
             if (!std::is_sorted(h->rho_order.begin(), h->rho_order.end(), desc)) {
-                /* one region: only the first grain of the old order is known to hold cells */
-                if (d.nreg <= 1 && (rc = refresh_alive(h))) return h->err = rc;
+                /* only the first grain of the old order is known to hold cells */
+                if ((rc = refresh_alive(h))) return h->err = rc;
                 std::stable_sort(h->rho_order.begin(), h->rho_order.end(), desc);
                 if ((rc = upload_order(h))) return h->err = rc;
             }
@@ -1982,7 +1967,9 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
         (rc = dalloc(h, &d.pmB, d.parentCap)) || (rc = dalloc(h, &d.bcnt, GM_BCNT_ROWS * GM_MAX_BLOCKS)) ||
         (rc = dalloc(h, &d.rho, d.ndefg)) || (rc = dalloc(h, &d.defq, 4 * (size_t)d.ndefg)) ||
         (rc = dalloc(h, &d.rxq, 4 * (size_t)d.nrxg + 4)) || (rc = dalloc(h, &d.defcnt, d.ndefg)) ||
-        (rc = dalloc(h, &d.rxcnt, (size_t)d.nrxg + 1)) || (rc = dalloc(h, &d.zlist, d.ndefg)) ||
+        (rc = dalloc(h, &d.rxcnt, (size_t)d.nrxg + 1)) || (rc = dalloc(h, &d.win, 1)) || (rc = dalloc(h, &d.acnt, 2 * GM_PB)) ||
+        (rc = dalloc(h, &d.defsub, (size_t)GM_SUBS * d.ndefg)) || (rc = dalloc(h, &d.rorder, d.ndefg)) ||
+        (rc = dalloc(h, &d.rpos, d.ndefg)) ||
         (rc = dalloc(h, &d.hkeys, d.hcap)) ||
         (rc = dalloc(h, &d.hvals, d.hcap)) || (rc = dalloc(h, &d.pend_slot, d.hcap)) || (rc = dalloc(h, &d.pend_key, d.hcap)) ||
         (rc = dalloc(h, &d.nflag, (size_t)d.nrxg + 1)) || (rc = dalloc(h, &d.nI_, (size_t)d.nrxg + 1)) ||
@@ -1995,15 +1982,13 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
     if (!multi) {
         d.swb = sweep_block_rows(d);
         d.gchunks = (uint32_t)std::min<uint64_t>(GM_GCHUNKS, d.N / 16 + 1);
-        if ((rc = dalloc(h, &d.win, 1)) || (rc = dalloc(h, &d.wcnt, (size_t)(GM_WMAX + 1) * d.swb)) ||
+        if ((rc = dalloc(h, &d.wcnt, (size_t)(GM_WMAX + 1) * d.swb)) ||
             (rc = dalloc(h, &d.wpre, (size_t)(GM_WMAX + 1) * d.swb)) ||
             (rc = dalloc(h, &d.wwave, (size_t)GM_SW_WAVES * GM_WMAX * d.swb)) ||
             (rc = dalloc(h, &d.rcnt, 2 * (size_t)d.swb)) || (rc = dalloc(h, &d.rpre, 2 * (size_t)d.swb)) ||
-            (rc = dalloc(h, &d.rgone, d.swb)) || (rc = dalloc(h, &d.rmrg, d.swb)) || (rc = dalloc(h, &d.acnt, 2 * GM_PB)) ||
+            (rc = dalloc(h, &d.rgone, d.swb)) || (rc = dalloc(h, &d.rmrg, d.swb)) ||
             (rc = dalloc(h, &d.btot, GM_DB)) || (rc = dalloc(h, &d.ccnt, (size_t)d.parentCap / 16 + 1)) ||
             (rc = dalloc(h, &d.pmA, d.parentCap)) || (rc = dalloc(h, &d.btop, GM_DB)) ||
-            (rc = dalloc(h, &d.defsub, (size_t)GM_SUBS * d.ndefg)) || (rc = dalloc(h, &d.rorder, d.ndefg)) ||
-            (rc = dalloc(h, &d.rpos, d.ndefg)) ||
             (rc = dalloc(h, &d.gatt, (size_t)GM_GATT * d.gchunks))) {
             free_device(h);
             delete h;
@@ -2055,7 +2040,7 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
         uint32_t *src = reinterpret_cast<uint32_t *>(d.rec);
         HIPCHK(copy_staged(device, h->stage, src, const_cast<uint32_t *>(dom->cellgrid), sizeof(uint32_t) * d.N, false, s));
         HIPCHK(gm_launch_fill_u32(d.defcnt, 0u, d.ndefg, s));
-        if (!multi) HIPCHK(gm_launch_fill_u32(d.defsub, 0u, (size_t)GM_SUBS * d.ndefg, s));
+        HIPCHK(gm_launch_fill_u32(d.defsub, 0u, (size_t)GM_SUBS * d.ndefg, s));
         HIPCHK(gm_launch_fill_u32((uint32_t *)d.st, 0u, sizeof(GmStats) / 4, s));
         HIPCHK(gm_launch_grid_init(d, src, s));
         HIPCHK(hipMemcpyAsync(defcnt.data(), d.defcnt, sizeof(uint32_t) * d.ndefg, hipMemcpyDeviceToHost, s));
@@ -2217,7 +2202,7 @@ int score_gm_get_grainmap(score_gm_handle *h, uint32_t *out, int32_t encoding) {
 int score_gm_get_counts(score_gm_handle *h, uint32_t *defg_counts, uint32_t *rxg_counts) {
     if (!h) return fail(SCORE_GM_ERR_ARG, "null handle");
     HIPCHK(hipSetDevice(h->device));
-    if (defg_counts && h->d.nreg <= 1) HIPCHK(gm_launch_fold_counts(h->d, h->stream));
+    if (defg_counts) HIPCHK(gm_launch_fold_counts(h->d, h->stream));
     if (defg_counts)
         HIPCHK(hipMemcpyAsync(defg_counts, h->d.defcnt, sizeof(uint32_t) * h->d.ndefg, hipMemcpyDeviceToHost, h->stream));
     if (rxg_counts && h->d.nrxg)
@@ -2457,8 +2442,7 @@ int score_gm_footprint(const score_gm_domain *dom, const score_gm_params *prm, u
     if (prm->n_regions <= 1) {
         /* the window sweep's tables */
         const uint64_t rows = std::max<uint64_t>(capTot / (GM_SW_CHUNK * GM_SW_WAVES * GM_SW_MAXCPW) + 67, GM_SW_BLOCKS);
-        b += sizeof(GmWin) + 4 * rows * (2 * (GM_WMAX + 1) + GM_SW_WAVES * GM_WMAX + 6) + 16 * GM_PB + 4 * (front + front / 16) +
-             (4ull * GM_SUBS + 8) * dom->n_defg +
+        b += 4 * rows * (2 * (GM_WMAX + 1) + GM_SW_WAVES * GM_WMAX + 6) + 8 * GM_PB + 4 * (front + front / 16) +
              4ull * GM_GATT * std::min<uint64_t>(GM_GCHUNKS, N / 16 + 1);
     }
     if (prm->n_regions > 1) {
@@ -2489,6 +2473,7 @@ int score_gm_footprint(const score_gm_domain *dom, const score_gm_params *prm, u
     b += 8 * (capTot / 64 + GM_SW_TPC);           /* tile masks */
     b += 4 * rbuf;                                /* recycled slots */
     b += 4 * GM_BCNT_ROWS * GM_MAX_BLOCKS;
+    b += sizeof(GmWin) + 8 * GM_PB + (4ull * GM_SUBS + 8) * dom->n_defg; /* counts in parts, order of rho */
     b += 52ull * dom->n_defg + 52ull * (dom->n_rxg + 1);
     if (dom->rxg_step) b += 20ull * dom->n_rxg;   /* arrivals: ids, sites, weights */
     b += 28 * hcap;                               /* weight cache: keys, values, pending slots and keys */

@@ -109,7 +109,6 @@ static inline __host__ __device__ uint32_t gm_tiles_inside(uint32_t nI) {
 }
 #define GM_MAX_BLOCKS 8192        /* grid of the partitioned passes (scanned by one 1024-thread block) */
 #define GM_SCAN_BLOCKS 1024       /* fixed grid of the device-wide scans (nucleation) */
-#define GM_ZEROED_INLINE 1022     /* exhausted grain ids returned with the per-step stats */
 #define GM_PEND_INLINE 2048       /* new P-cache keys returned with the per-step stats */
 #define GM_NK 9                   /* kernels per step (SCORE_GM_K_* order) */
 #define GM_WMAX 16                /* steps per launch window at most (also below imin - 1) */
@@ -180,7 +179,6 @@ struct GmStepRow {
     uint32_t winI, winB;
     uint32_t npend;           /* P-cache entries the step inserted */
     uint32_t nattempt;
-    uint32_t nzeroed;         /* exhausted grains so far in the window */
     uint32_t err;
     uint32_t nplaced;         /* nuclei placed at the start of the step */
     uint32_t pone;            /* a new pair's weight was short-circuited to 1.0 in the step */
@@ -201,12 +199,11 @@ struct alignas(8) GmStats {
     uint32_t pone;            /* set when a pair weight was short-circuited to 1.0 */
     uint32_t scan_tot[4];     /* totals written by the device-wide scans */
     uint32_t nattempt;        /* attempts that found a deformed target this step */
-    uint32_t nzeroed;         /* several regions: deformed grains that lost their last cell in the window */
-    uint32_t cwrap;           /* a deformed-grain count went past zero (one region: of a grain before the one that sets rhomax) */
-    uint32_t ticket;          /* one region: blocks of the window's last commit pass that are done */
+    uint32_t cwrap;           /* the count of a grain before the one that sets rhomax went past zero */
+    uint32_t ticket;          /* blocks of the commit pass that are done (one region: of the window's last one) */
     uint32_t grow;            /* one region: the Inside slots a step's commit pass asks for before it can run */
     uint32_t need_par;        /* one region: the parents of a step that has more than the planes hold */
-    uint32_t top_hit;         /* one region: the grain that sets rhomax lost its last cell, */
+    uint32_t top_hit;         /* the grain that sets rhomax lost its last cell, */
     uint32_t top_next;        /* and the position of its successor in rorder (ndefg: none) */
     uint32_t dfirst;          /* defragmentation: first INACTIVE slot of the list */
     uint32_t dcount;          /* defragmentation: ACTIVE slots moved; status vector: entries */
@@ -215,7 +212,6 @@ struct alignas(8) GmStats {
     uint32_t nplaced;         /* nuclei placed at the start of the current step */
     unsigned long long arr_pkey; /* largest weight of those nuclei (gm_pkey order) */
     unsigned long long nret;  /* entries of the retirement log (cells retired so far) */
-    uint32_t zeroed_ids[GM_ZEROED_INLINE]; /* the first of them; all are in GmDev::zlist */
     unsigned long long pend_keys[GM_PEND_INLINE]; /* the first new P-cache keys; all are in GmDev::pend_key */
     /* launch windows: several steps run back to back; the host reads the rows at the end */
     uint32_t kcur;            /* index of the next step */
@@ -230,11 +226,10 @@ struct alignas(8) GmStats {
 /* stop conditions of a window, checked after every step */
 struct GmWindow {
     double xstop;             /* Xcells at which the host must act (termination, defragmentation) */
-    uint32_t top_grain;       /* the grain that sets rhomax (0xFFFFFFFF: none) */
-    uint32_t top_pos;         /* its position in rorder (ndefg: none) */
+    uint32_t top_pos;         /* position in rorder of the grain that sets rhomax (ndefg: none) */
     uint32_t pend_limit;      /* new P-cache entries that keep the cache at most half full */
     uint32_t defer;           /* pending weights may wait for the end of the window */
-    uint32_t need_one;        /* a weight of 1.0 would be the largest so far (one region: GmStepRow::pone is only kept then) */
+    uint32_t need_one;        /* a weight of 1.0 would be the largest so far (GmStepRow::pone is only kept then) */
 };
 
 /* Parents per chunk of the decide and commit passes: a wave takes one chunk at a
@@ -368,7 +363,7 @@ struct GmDev {
     uint32_t *wwave;            /* GM_WMAX counts per wave of each block */
     uint32_t *rcnt, *rpre;      /* INACTIVE slots of each block and before it in its list; two rows, by the step's parity */
     uint32_t *rgone, *rmrg;     /* slots the step before handed out; steps whose completed cells are in the block's masks */
-    uint32_t *acnt;             /* attempts per propose block, two rows by the step's parity */
+    uint32_t *acnt;             /* attempts per propose block, two rows by the step's parity (several regions: one) */
     uint2 *btot;                /* winners into Inside, Border per decide block */
     uint32_t *btop;             /* parents per decide block in the grain that sets rhomax */
     uint32_t *ccnt;             /* the same per chunk of parents, Inside << 16 | Border */
@@ -377,9 +372,8 @@ struct GmDev {
     /* grains */
     double *rho, *defq, *rxq;
     uint32_t *defcnt, *rxcnt;
-    uint32_t *defsub;           /* one region: GM_SUBS rows of ndefg, cells taken from defcnt since the last fold */
-    uint32_t *rorder, *rpos;    /* one region: the grains by descending rho, and each one's position */
-    uint32_t *zlist;            /* ids of grains exhausted in the current step */
+    uint32_t *defsub;           /* GM_SUBS rows of ndefg, cells taken from defcnt since the last fold */
+    uint32_t *rorder, *rpos;    /* the grains by descending rho, and each one's position */
     /* mobility-weight cache: open addressing on key rxg*ndefg+defg+1 */
     unsigned long long *hkeys;
     double *hvals;
@@ -441,7 +435,7 @@ struct GmSweepArgs {
  * step a.k, and the window sweep */
 hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &a, const GmWindow &wd, bool arrivals,
                             double xcells, hipStream_t s, hipEvent_t *ev);
-/* one region: d.defcnt brought up to date */
+/* d.defcnt brought up to date */
 hipError_t gm_launch_fold_counts(const GmDev &d, hipStream_t s);
 /* every active cell advanced to step a.k with its old increment and predicted again */
 hipError_t gm_launch_reanchor(const GmDev &d, const GmSweepArgs &a, hipStream_t s);
@@ -449,7 +443,9 @@ hipError_t gm_launch_reanchor(const GmDev &d, const GmSweepArgs &a, hipStream_t 
 hipError_t gm_launch_rg_sweep(const GmDev &d, const GmSweepArgs &a, uint32_t parents_upper, hipStream_t s,
                               hipEvent_t *ev);
 hipError_t gm_launch_rg_infect(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, uint32_t parents_upper,
-                               hipStream_t s, hipEvent_t *ev);
+                               const GmWindow &w, GmStats *out, hipStream_t s, hipEvent_t *ev);
+/* the end of a window with several regions whose last step was launched without `out` or not at all */
+hipError_t gm_launch_rg_window_end(const GmDev &d, const GmWindow &w, GmStats *out, hipStream_t s);
 /* with several regions: the lists' prefixes and summed lengths from d.L.n */
 hipError_t gm_launch_rg_prefix(const GmDev &d, hipStream_t s);
 /* with several regions: nuclei the host placed, records scattered to their slots */
@@ -465,10 +461,7 @@ hipError_t gm_launch_commit(const GmDev &d, const GmPParams &pp, const GmSweepAr
 hipError_t gm_launch_window_end(const GmDev &d, const GmPart &P, uint32_t launched, uint32_t top_pos, GmStats *out,
                                 hipStream_t s);
 /* start of a window with several regions: step index and Xcells; clears the window's accumulators */
-hipError_t gm_launch_window_begin(const GmDev &d, uint32_t k, double xcells, hipStream_t s);
-/* end of every step of a window with several regions: records the step's row, advances the step
- * index, and sets halt when the host must act before the next step */
-hipError_t gm_launch_step_tail(const GmDev &d, const GmWindow &w, hipStream_t s);
+hipError_t gm_launch_window_begin(const GmDev &d, uint32_t k, double xcells, uint32_t top_pos, hipStream_t s);
 /* cells left DEFERRED in a window, with their weights now resolved: replayed to
  * step a.k under the window's scalars and predicted */
 hipError_t gm_launch_predict_deferred(const GmDev &d, const GmSweepArgs &a, uint32_t ndeferred, hipStream_t s);

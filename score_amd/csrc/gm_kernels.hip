@@ -145,15 +145,6 @@ static __device__ __forceinline__ uint32_t code_at(const uint4 &cs, int q) {
     return (wd >> (16 * (q & 1))) & 0xFFFFu;
 }
 
-/* A grain's cells: the count at the last fold less the parts taken since.  Every
- * lane of the wave takes part and gets the value. */
-static __device__ __forceinline__ uint32_t exact_count(const GmDev &d, uint32_t g) {
-    const uint32_t lane = threadIdx.x & 63u;
-    uint32_t v = lane < GM_SUBS ? d.defsub[(size_t)lane * d.ndefg + g] : 0u;
-    for (int o = 32; o > 0; o >>= 1) v += (uint32_t)__shfl_xor((int)v, o, 64);
-    return d.defcnt[g] - v;
-}
-
 /* the parts into the counts */
 __global__ void k_fold_counts(GmDev d) {
     for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < d.ndefg; g += gridDim.x * blockDim.x) {
@@ -759,7 +750,6 @@ static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, 
     const uint32_t npend = agent_load(&st->npend);
     r.npend = npend - win->npend0;
     r.nattempt = na;
-    r.nzeroed = 0;
     r.err = agent_load(&st->err);
     r.nplaced = st->nplaced;
     r.pone = agent_load(&st->pone);
@@ -1507,29 +1497,6 @@ hipError_t gm_launch_resolve_pending(const GmDev &d, const double *vals, uint32_
     return hipGetLastError();
 }
 
-/* The stats into the host's pinned mirror (mapped, coherent), word by word, by one
- * block: cheaper than a copy command at the end of every window.  Only the filled part
- * of the inline id and key arrays crosses the bus; the host reads no more.  When every
- * word has arrived the host is told by the word behind the progress word, which it
- * waits for instead of the kernel's end (the launch's own completion reaches it 8 us
- * later). */
-static __device__ __forceinline__ void copy_stats(const GmDev &d, uint32_t *out) {
-    const uint32_t *in = reinterpret_cast<const uint32_t *>(d.st);
-    const GmStats *st = d.st;
-    const uint32_t nzd = agent_load(&st->nzeroed), npd = agent_load(&st->npend);
-    const uint32_t nz = nzd < GM_ZEROED_INLINE ? nzd : GM_ZEROED_INLINE;
-    const uint32_t np = npd < GM_PEND_INLINE ? npd : GM_PEND_INLINE;
-    const uint32_t z0 = offsetof(GmStats, zeroed_ids) / 4, p0 = offsetof(GmStats, pend_keys) / 4;
-    const uint32_t t0 = offsetof(GmStats, kcur) / 4, end = sizeof(GmStats) / 4;
-    for (uint32_t i = threadIdx.x; i < end; i += GM_BLOCK) {
-        const bool skip = (i >= z0 + nz && i < p0) || (i >= p0 + 2u * np && i < t0);
-        if (!skip) __hip_atomic_store(out + i, agent_load(in + i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0 && d.prog) __hip_atomic_store(d.prog + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 __global__ void __launch_bounds__(GM_BLOCK) k_stats_out(GmDev d, uint32_t *out) { copy_stats(d, out); }
 
 hipError_t gm_launch_stats_out(const GmDev &d, GmStats *out, hipStream_t s) {
@@ -1539,34 +1506,10 @@ hipError_t gm_launch_stats_out(const GmDev &d, GmStats *out, hipStream_t s) {
 
 /* The end of a window of `launched` steps, by one block: its last step is closed,
  * unless the window halted (the propose pass that halted it closed the step before),
- * and the stats go to the host's mirror.  If the grain that sets rhomax lost its last
- * cell, its successor is looked up. */
+ * and the stats go to the host. */
 static __device__ void window_end(const GmDev &d, const GmPart &P, uint32_t launched, uint32_t top_pos, uint32_t *out) {
-    __shared__ uint32_t first;
-    const uint32_t hit = agent_load(&d.win->top_hit);
     if (!agent_load(&d.st->halt) && d.st->nexec + 1u == launched) close_step(d, P, launched - 1u, false);
-    if (hit) { /* the next grain in the order of rho that holds cells */
-        if (threadIdx.x == 0) first = d.ndefg;
-        for (uint32_t i0 = top_pos; i0 < d.ndefg; i0 += GM_BLOCK) {
-            const uint32_t i = i0 + threadIdx.x;
-            __syncthreads();
-            if (first < d.ndefg) break;
-            __syncthreads();
-            if (i < d.ndefg) {
-                const uint32_t g = d.rorder[i];
-                uint32_t n = d.defcnt[g];
-#pragma unroll
-                for (uint32_t q = 0; q < GM_SUBS; q++) n -= d.defsub[(size_t)q * d.ndefg + g];
-                if (n) atomicMin(&first, i);
-            }
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) d.st->top_next = first;
-    }
-    if (threadIdx.x == 0) d.st->top_hit = hit;
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    copy_stats(d, out);
+    stats_to_host(d, top_pos, out);
 }
 
 __global__ void __launch_bounds__(GM_BLOCK) k_window_end(GmDev d, GmPart P, uint32_t launched, uint32_t top_pos,
@@ -1927,8 +1870,15 @@ __global__ void __launch_bounds__(1024) k_arrivals(GmDev d, GmSweepArgs A) {
  * the step index and list lengths from the stats and returns at once once a
  * step has set `halt`, so that the host takes over at the step after it. */
 
-__global__ void k_window_begin(GmDev d, uint32_t k, double xcells) {
+__global__ void __launch_bounds__(64) k_window_begin(GmDev d, uint32_t k, double xcells, uint32_t top_pos) {
     GmStats *st = d.st;
+    if (top_pos < d.ndefg) {
+        const uint32_t n = exact_count(d, d.rorder[top_pos]);
+        if (threadIdx.x == 0) d.win->top_left = n;
+    }
+    if (threadIdx.x != 0) return;
+    d.win->top_hit = 0;
+    st->ticket = 0;
     st->kcur = k;
     st->halt = 0;
     st->nexec = 0;
@@ -1936,7 +1886,6 @@ __global__ void k_window_begin(GmDev d, uint32_t k, double xcells) {
     st->npend = 0;
     st->npend0 = 0;
     st->pone = 0;
-    st->nzeroed = 0;
     st->cwrap = 0;
     st->novf = 0;
     st->nplaced = 0;
@@ -1944,23 +1893,11 @@ __global__ void k_window_begin(GmDev d, uint32_t k, double xcells) {
     st->xcells = xcells;
 }
 
-hipError_t gm_launch_window_begin(const GmDev &d, uint32_t k, double xcells, hipStream_t s) {
-    k_window_begin<<<1, 1, 0, s>>>(d, k, xcells);
+hipError_t gm_launch_window_begin(const GmDev &d, uint32_t k, double xcells, uint32_t top_pos, hipStream_t s) {
+    k_window_begin<<<1, 64, 0, s>>>(d, k, xcells, top_pos);
     return hipGetLastError();
 }
 
-
-/* One wave after the commit pass: the step's row and whether the next step of
- * the window may run. */
-__global__ void __launch_bounds__(64) k_step_tail(GmDev d, GmWindow w) {
-    if (d.st->halt) return;
-    step_tail(d, w);
-}
-
-hipError_t gm_launch_step_tail(const GmDev &d, const GmWindow &w, hipStream_t s) {
-    k_step_tail<<<1, 64, 0, s>>>(d, w);
-    return hipGetLastError();
-}
 
 /* DEFERRED cells: anchored at the step after their infection with their carry;
  * every step since then added the increment of the window's scalars, so the

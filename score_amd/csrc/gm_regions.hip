@@ -36,13 +36,13 @@
  * count is the offset of the region's first block.
  *
  * At 160^3 in eight regions (477 steps of 8500 parents) a step of these passes went
- * from 135 to 77 us: propose 25 to 10, decide 23 to 12 with the retirement, commit 25
- * to 14, the two scans 27 to 15.
+ * from 135 to 67 us: propose 25 to 10, decide with the retirement and the recycled
+ * slots 28 to 9.5, commit with the step's end 29 to 17, the two scans 27 to 14.5.
  *
  * Per step, in the profiling slots of the one-region kernels:
  *   k_reanchor (shared)   k_rg_sweep   k_rg_sweep_scan (+ per-list starts)
- *   k_rg_compact   k_rg_propose   k_rg_decide
- *   k_rg_decide_scan (+ per-region starts, list lengths)   k_rg_recycle   k_rg_commit
+ *   k_rg_compact   k_rg_propose   k_rg_decide (+ recycled slots)
+ *   k_rg_decide_scan (+ per-region starts, list lengths)   k_rg_commit (+ the step's end)
  */
 #include <algorithm>
 
@@ -68,6 +68,8 @@ static __constant__ uint8_t c_hidx[27] = {0xFF, 0xFF, 0xFF, 0, 1, 2, 3, 0xFF, 0x
 #define RS_R 1
 #define RS_UN 2
 #define RW_ROW0 3
+/* and, after its own, the row of its parents in the grain that sets rhomax */
+#define RW_TOP (RW_ROW0 + GM_RROWS)
 
 /* the part_of block size for a grid of nb blocks, from any thread */
 static __device__ __forceinline__ uint32_t part_per(uint32_t n, uint32_t nb, uint32_t q) {
@@ -120,8 +122,7 @@ static uint32_t rg_infect_blocks(const GmDev &d, uint32_t parents_upper) {
 /* The parents of infection-pass block b: blocks are handed out region by region
  * (L.bstart[r] is region r's first block, st->rg_per parents each), so a block
  * holds one region's parents only; r is that region. */
-static __device__ __forceinline__ void rg_part(const GmDev &d, uint32_t &lo, uint32_t &hi, uint32_t &r) {
-    const uint32_t b = blockIdx.x;
+static __device__ __forceinline__ void rg_part(const GmDev &d, uint32_t b, uint32_t &lo, uint32_t &hi, uint32_t &r) {
     lo = hi = r = 0;
     r = d.L.breg[b];
     if (r >= d.nreg) return; /* a block past the ones in use */
@@ -477,16 +478,18 @@ __global__ void __launch_bounds__(64) k_rg_compact(GmDev d) {
 }
 
 /* Each list's INACTIVE slots in ascending order (append_to_recycling_*_list,
- * SCORE_Kernel.cpp:4037-4041, :4175-4179), written once the step's new records
- * per list are known and only as far as they are handed out: the first
- * min(new records, recycled slots) of each list.  The sweep's partition and
- * offsets; one wave per sweep block. */
-__global__ void __launch_bounds__(64) k_rg_recycle(GmDev d) {
-    if (d.st->halt) return;
-    const uint32_t lane = threadIdx.x;
-    uint32_t lo, hi;
-    part_of(d.L.tile_s[d.nlists], GM_SW_TPC, lo, hi);
-    uint32_t runR = d.bcnt[RS_R * GM_MAX_BLOCKS + blockIdx.x];
+ * SCORE_Kernel.cpp:4037-4041, :4175-4179), as far as they can be handed out: at most
+ * the recycled slots, and no more than the step's attempts.  Runs beside the decide
+ * pass, before the new records per list are known (a pass of its own after that took
+ * 5 us and a gap).  The sweep's partition and offsets; one wave per sweep block. */
+static __device__ __forceinline__ void rg_recycle(const GmDev &d, uint32_t blk, uint32_t nblk, uint32_t nbp) {
+    const uint32_t lane = threadIdx.x, T = d.L.tile_s[d.nlists], per = part_per(T, nblk, GM_SW_TPC);
+    uint32_t lo = blk * per, hi = lo + per, na = 0;
+    if (lo > T) lo = T;
+    if (hi > T) hi = T;
+    for (uint32_t i = lane; i < nbp; i += 64u) na += d.acnt[i];
+    for (int o = 32; o > 0; o >>= 1) na += (uint32_t)__shfl_xor((int)na, o, 64);
+    uint32_t runR = d.bcnt[RS_R * GM_MAX_BLOCKS + blk];
     for (uint32_t batch = lo; batch < hi; batch += 64) {
         const uint32_t t = batch + lane;
         const uint64_t br = t < hi ? d.mR[t] : 0ull;
@@ -496,8 +499,7 @@ __global__ void __launch_bounds__(64) k_rg_recycle(GmDev d) {
         runR += __shfl(incr, 63, 64);
         if (br) {
             const uint32_t l = upper_index(d.L.tile_s, d.nlists, t);
-            const uint32_t w = d.L.win[l], rl = d.L.rlen[l];
-            const uint32_t lim = w < rl ? w : rl;
+            const uint32_t rl = d.L.rlen[l], lim = na < rl ? na : rl;
             uint32_t k = orr - d.L.rst[l];
             if (k < lim) {
                 const uint32_t rel0 = (t - d.L.tile_s[l]) * 64u;
@@ -546,6 +548,7 @@ __global__ void __launch_bounds__(GM_BLOCK) k_rg_propose(GmDev d) {
         uint16_t wl[26 * 64];
     };
     __shared__ Wave sw[GM_BLOCK / 64];
+    __shared__ uint32_t satt[GM_BLOCK / 64];
     if (d.st->halt) return;
     const uint32_t nfull = d.st->nfullI + d.st->nfullB, k = d.st->kcur;
     const unsigned long long nret = d.st->nret;
@@ -553,6 +556,7 @@ __global__ void __launch_bounds__(GM_BLOCK) k_rg_propose(GmDev d) {
     if (!logged && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&d.st->err, GM_ERRF_RLOG_FULL);
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
     Wave &W = sw[w];
+    uint32_t natt = 0;
     for (uint32_t c = w * gridDim.x + blockIdx.x; c * 64u < nfull; c += gridDim.x * (GM_BLOCK / 64u)) {
         const uint32_t p = c * 64u + lane;
         uint32_t am = 0;
@@ -578,6 +582,7 @@ __global__ void __launch_bounds__(GM_BLOCK) k_rg_propose(GmDev d) {
         }
         W.bad[lane] = 0;
         const uint32_t n = list_attempts(am, W.wl);
+        natt += n;
         for (uint32_t i = lane; i < n; i += 64u) {
             const uint32_t e = W.wl[i], q = e & 0xFFu, rk = e >> 8;
             const uint4 q2 = W.q2[q];
@@ -591,31 +596,44 @@ __global__ void __launch_bounds__(GM_BLOCK) k_rg_propose(GmDev d) {
         if (p < nfull) d.pmI[p] = am & ~W.bad[lane];
         wave_sync();
     }
+    if (lane == 0) satt[w] = natt;
+    __syncthreads();
+    if (threadIdx.x == 0) d.acnt[blockIdx.x] = satt[0] + satt[1] + satt[2] + satt[3];
 }
 
 /* The attempts that hold their target's smallest key, as masks by destination (own
  * Inside, own Border, a halo), counted per block by row (GM_RW_*).  64 parents'
  * attempts are flattened into a list, a lane per attempt, so that all claims are
  * loaded together.  The parents retire here, beside the waiting for the claims.  The
- * partition into blocks (one region per block) is the commit pass's. */
-__global__ void __launch_bounds__(64) k_rg_decide(GmDev d) {
+ * partition into blocks (one region per block) is the commit pass's.  The launch's
+ * first nrec blocks write the recycled slots. */
+__global__ void __launch_bounds__(64) k_rg_decide(GmDev d, uint32_t nrec, uint32_t nbp, uint32_t top_pos) {
     __shared__ uint4 sq2[64];
     __shared__ uint32_t sI[64], sB[64], sH[64], scnt[GM_RROWS];
     __shared__ uint16_t wl[26 * 64];
     if (d.st->halt) return;
-    const uint32_t lane = threadIdx.x;
+    if (blockIdx.x < nrec) {
+        rg_recycle(d, blockIdx.x, nrec, nbp);
+        return;
+    }
+    const uint32_t lane = threadIdx.x, blk = blockIdx.x - nrec;
     uint32_t lo, hi, reg;
-    rg_part(d, lo, hi, reg);
+    rg_part(d, blk, lo, hi, reg);
     const RgBox box = rg_box(d, reg);
     if (lane < GM_RROWS) scnt[lane] = 0;
-    uint32_t nI = 0, nB = 0, nA = 0;
+    uint32_t nI = 0, nB = 0, nA = 0, ntop = 0;
+    bool wrapped = false;
     for (uint32_t batch = lo; batch < hi; batch += 64) {
         const uint32_t p = batch + lane;
         const bool valid = p < hi;
         const uint32_t am = valid ? d.pmI[p] : 0u;
         sq2[lane] = valid ? par_plane(d, GM_PAR_XYZ)[p] : make_uint4(0u, 0u, 0u, 0u);
         sI[lane] = sB[lane] = sH[lane] = 0;
-        retire_batch(d, valid ? par_plane(d, GM_PAR_IDS)[p] : make_uint4(0u, 0u, 0xFFFFFFFFu, 0xFFFFFFFFu), valid);
+        const uint4 q0 = valid ? par_plane(d, GM_PAR_IDS)[p] : make_uint4(0u, 0u, 0xFFFFFFFFu, 0xFFFFFFFFu);
+        retire(d, q0.z, q0.w, valid, blk & (GM_SUBS - 1u));
+        const uint32_t rp = valid ? d.rpos[q0.z] : 0xFFFFFFFFu;
+        ntop += rp == top_pos ? 1u : 0u;
+        wrapped |= rp < top_pos;
         const uint32_t n = list_attempts(am, wl);
         for (uint32_t i = lane; i < n; i += 64u) {
             const uint32_t e = wl[i], q = e & 0xFFu, rk = e >> 8;
@@ -646,10 +664,13 @@ __global__ void __launch_bounds__(64) k_rg_decide(GmDev d) {
         nI += __shfl_xor(nI, o, 64);
         nB += __shfl_xor(nB, o, 64);
         nA += __shfl_xor(nA, o, 64);
+        ntop += __shfl_xor(ntop, o, 64);
     }
     wave_sync();
+    if (__any(wrapped) && lane == 0) d.st->cwrap = 1u;
+    if (lane == GM_RROWS) d.bcnt[RW_TOP * GM_MAX_BLOCKS + blk] = ntop;
     if (lane < GM_RROWS)
-        d.bcnt[(RW_ROW0 + lane) * GM_MAX_BLOCKS + blockIdx.x] =
+        d.bcnt[(RW_ROW0 + lane) * GM_MAX_BLOCKS + blk] =
             lane == GM_RW_I ? nI : lane == GM_RW_B ? nB : lane == GM_RW_A ? nA : scnt[lane];
 }
 
@@ -666,10 +687,17 @@ __global__ void __launch_bounds__(1024) k_rg_decide_scan(GmDev d, uint32_t nb) {
     if (st->halt) return;
     /* only the blocks in use hold counts */
     const uint32_t nused = d.L.bstart[d.nreg];
-    __shared__ uint32_t tot[GM_RROWS];
-    scan_rows(d.bcnt + RW_ROW0 * GM_MAX_BLOCKS, GM_RROWS, nused < nb ? nused : nb, tot);
+    __shared__ uint32_t tot[GM_RROWS + 1];
+    scan_rows(d.bcnt + RW_ROW0 * GM_MAX_BLOCKS, GM_RROWS + 1, nused < nb ? nused : nb, tot);
     if (threadIdx.x < 2) acc[threadIdx.x] = 0;
-    if (threadIdx.x == 0) st->nattempt = tot[GM_RW_A];
+    if (threadIdx.x == 0) {
+        st->nattempt = tot[GM_RW_A];
+        if (tot[GM_RROWS]) { /* the cells left of the grain that sets rhomax */
+            const uint32_t left = d.win->top_left - tot[GM_RROWS];
+            d.win->top_left = left;
+            if (left == 0u) d.win->top_hit = 1u;
+        }
+    }
     /* each region's counts at its first parent: the offset of its first block
      * (the next region's, or the totals, for a region without parents) */
     for (uint32_t r = threadIdx.x; r <= d.nreg; r += 1024) {
@@ -725,18 +753,18 @@ __global__ void __launch_bounds__(1024) k_rg_decide_scan(GmDev d, uint32_t nb) {
  * halo winners after the receiving region's own, by neighbour, then by the
  * infecting region's prefix count of that halo.  A halo winner's weight is
  * looked up again whatever its deformed grain (SCORE_Kernel.cpp:4853). */
-__global__ void __launch_bounds__(64) k_rg_commit(GmDev d, GmPParams pp, GmSweepArgs A) {
+static __device__ __forceinline__ void rg_commit_step(const GmDev &d, const GmPParams &pp, const GmSweepArgs &A, uint32_t need_one) {
     __shared__ uint32_t sI[64], sB[64], oI[64], oB[64];
     __shared__ uint4 sq0[64], sq2[64];
     __shared__ double sfin[64], sP[64];
     __shared__ uint16_t wl[26 * 64];
     GmStats *st = d.st;
-    if (st->halt) return;
     const uint32_t k = st->kcur;
+    bool one = false;
     const uint32_t lane = threadIdx.x;
     __shared__ uint32_t srs[GM_RROWS], sL[2][5];
     uint32_t lo, hi, reg;
-    rg_part(d, lo, hi, reg);
+    rg_part(d, blockIdx.x, lo, hi, reg);
     if (lo >= hi) return; /* no parents: nothing to commit */
     const RgBox box = rg_box(d, reg);
     /* the block's region: its counts at its first parent, and its two lists' tables */
@@ -826,31 +854,61 @@ __global__ void __launch_bounds__(64) k_rg_commit(GmDev d, GmPParams pp, GmSweep
                 continue;
             }
             const NewCell nc = new_cell(d, pp, A, k, sfin[j], sP[j], pq0, r, g, o.khi != 0u);
-            if (nc.one) st->pone = 1u;
+            one |= nc.one;
             put_cell(d, k, nc, pq0, t, g, o.x, o.y, o.z, bs + rel);
         }
         run[GM_RW_I] += bt >> 16;
         run[GM_RW_B] += bt & 0xFFFFu;
         __syncthreads();
     }
+    if (need_one && __any(one) && lane == 0) agent_store(&st->pone, 1u);
+}
+
+/* The block that finds the others in use done ends the step (step_tail), where a launch
+ * of its own took 4 us and a gap, and with `out` the window.  What it needs of the
+ * other blocks they change by device atomics alone. */
+__global__ void __launch_bounds__(64) k_rg_commit(GmDev d, GmPParams pp, GmSweepArgs A, GmWindow w, uint32_t *out) {
+    if (d.st->halt) {
+        if (out && blockIdx.x == 0) stats_to_host(d, w.top_pos, out);
+        return;
+    }
+    const uint32_t used = d.L.bstart[d.nreg], n = used ? used : 1u;
+    if (blockIdx.x >= n) return;
+    rg_commit_step(d, pp, A, w.need_one);
+    __builtin_amdgcn_s_waitcnt(0);
+    uint32_t t = 0;
+    if (threadIdx.x == 0) t = atomicAdd(&d.st->ticket, 1u);
+    if (rdlane(t, 0u) != n - 1u) return;
+    if (threadIdx.x == 0) agent_store(&d.st->ticket, 0u);
+    step_tail(d, w);
+    if (!out) return;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    stats_to_host(d, w.top_pos, out);
+}
+
+__global__ void __launch_bounds__(64) k_rg_window_end(GmDev d, uint32_t top_pos, uint32_t *out) { stats_to_host(d, top_pos, out); }
+
+hipError_t gm_launch_rg_window_end(const GmDev &d, const GmWindow &w, GmStats *out, hipStream_t s) {
+    k_rg_window_end<<<1, 64, 0, s>>>(d, w.top_pos, reinterpret_cast<uint32_t *>(out));
+    return hipGetLastError();
 }
 
 hipError_t gm_launch_rg_infect(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, uint32_t parents_upper,
-                               hipStream_t s, hipEvent_t *ev) {
+                               const GmWindow &w, GmStats *out, hipStream_t s, hipEvent_t *ev) {
     hipError_t e;
     if ((e = mark(ev, 4, s)) != hipSuccess) return e;
-    k_rg_propose<<<grid_for(parents_upper, 64u), GM_BLOCK, 0, s>>>(d);
-    const uint32_t nb = rg_infect_blocks(d, parents_upper);
+    const uint32_t nbp = std::min(GM_PB, grid_for(parents_upper, 64u));
+    k_rg_propose<<<nbp, GM_BLOCK, 0, s>>>(d);
+    const uint32_t nb = rg_infect_blocks(d, parents_upper), nrec = rg_sweep_blocks(d, a);
     if ((e = mark(ev, 5, s)) != hipSuccess) return e;
-    k_rg_decide<<<nb, 64, 0, s>>>(d);
+    k_rg_decide<<<nrec + nb, 64, 0, s>>>(d, nrec, nbp, w.top_pos);
     if ((e = mark(ev, 6, s)) != hipSuccess) return e;
     k_rg_decide_scan<<<1, 1024, 0, s>>>(d, nb);
-    if ((e = mark(ev, 7, s)) != hipSuccess) return e;
-    k_rg_recycle<<<rg_sweep_blocks(d, a), 64, 0, s>>>(d);
-    if ((e = mark(ev, 8, s)) != hipSuccess) return e;
+    if ((e = mark(ev, 7, s)) != hipSuccess || (e = mark(ev, 8, s)) != hipSuccess) return e;
     GmSweepArgs A = a;
     A.reanchor = 0;
-    k_rg_commit<<<nb, 64, 0, s>>>(d, pp, A);
+    k_rg_commit<<<nb, 64, 0, s>>>(d, pp, A, w, reinterpret_cast<uint32_t *>(out));
     if ((e = mark(ev, 9, s)) != hipSuccess) return e;
     return hipGetLastError();
 }
