@@ -1126,8 +1126,9 @@ static __device__ __forceinline__ void commit_step(const GmDev &d, const GmPPara
     const uint64_t need = (uint64_t)ws.nI + (totI > ws.recLenI ? totI - ws.recLenI : 0u);
     if (need > d.capI && d.capI < d.capImax) {
         if (db == 0 && threadIdx.x == 0) {
+            /* not st->halt, which the pass's other blocks read: two waves of one must
+             * not see different values of it; the next propose pass halts on this */
             agent_store(&st->grow, need < d.capImax ? (uint32_t)need : d.capImax);
-            agent_store(&st->halt, 1u);
         }
         return;
     }
@@ -1508,7 +1509,7 @@ hipError_t gm_launch_stats_out(const GmDev &d, GmStats *out, hipStream_t s) {
  * unless the window halted (the propose pass that halted it closed the step before),
  * and the stats go to the host. */
 static __device__ void window_end(const GmDev &d, const GmPart &P, uint32_t launched, uint32_t top_pos, uint32_t *out) {
-    if (!agent_load(&d.st->halt) && d.st->nexec + 1u == launched) close_step(d, P, launched - 1u, false);
+    if (!d.st->halt && !agent_load(&d.st->grow) && d.st->nexec + 1u == launched) close_step(d, P, launched - 1u, false);
     stats_to_host(d, top_pos, out);
 }
 
