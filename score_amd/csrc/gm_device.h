@@ -225,13 +225,13 @@ static __device__ __forceinline__ double resolved(const GmDev &d, double P) {
 /* rxFrac increment of one cell: SCORE's v = m*p; v *= shape; rxFrac += (v*dt)*inv_dx
  * (SCORE_Kernel.cpp:4077-4092, :5459-5470); returns false when p <= DOUBLE_ACCURACY
  * (the cell is not advanced) */
-static __device__ __forceinline__ bool cell_increment(const GmDev &d, const GmSweepParams &sp, double P, uint32_t defg,
-                                                      uint32_t inf, double &inc) {
+static __device__ __forceinline__ bool cell_increment(const GmSweepParams &sp, double P, double rho, uint32_t inf,
+                                                      double &inc) {
     double m;
     if (sp.model == GM_RH) m = P * sp.mRH;
     else if (P < 0.0) m = sp.mLAGB;
     else m = (P * sp.mGS) + ((1.0 - P) * sp.mHAGB);
-    double p = (sp.Gbhalfsq * (d.rho[defg] - GM_RHO_RX)) - sp.zener;
+    double p = (sp.Gbhalfsq * (rho - GM_RHO_RX)) - sp.zener;
     if (!(p > GM_DOUBLE_ACCURACY)) return false;
     double v = m * p;
     v *= c_shape[inf];
@@ -245,10 +245,10 @@ static __device__ __forceinline__ bool cell_increment(const GmDev &d, const GmSw
  * does not advance).  The value after the completing addition, whose excess
  * over 1.0 the infection carries on, is replayed from the anchor when the cell
  * completes (the propose passes). */
-static __device__ __forceinline__ uint32_t predict_values(const GmDev &d, const GmSweepArgs &A, uint32_t k, double f,
-                                                          double P, uint32_t defg, uint32_t inf, double &inc) {
+static __device__ __forceinline__ uint32_t predict_values(const GmSweepArgs &A, uint32_t k, double f, double P, double rho,
+                                                          uint32_t inf, double &inc) {
     uint32_t cs = GM_STEP_NONE;
-    if (cell_increment(d, A.sp, P, defg, inf, inc)) {
+    if (cell_increment(A.sp, P, rho, inf, inc)) {
         if (k <= A.stepcap && A.next_only) {
             /* the step's one addition; a cell it leaves below 1.0 is re-anchored
              * and predicted again before the next step (GM_STEP_FAR_NEXT) */
@@ -294,7 +294,7 @@ static __device__ __forceinline__ bool cs_inactive(uint32_t cs, uint32_t kc, uin
 static __device__ __forceinline__ void predict_slot(const GmDev &d, const GmSweepArgs &A, uint32_t s, double f,
                                                     uint32_t s0, double P, uint32_t defg, uint32_t inf) {
     double inc;
-    const uint32_t cs = predict_values(d, A, A.k, f, P, defg, inf, inc);
+    const uint32_t cs = predict_values(A, A.k, f, P, d.rho[defg], inf, inc);
     rec_set_a(d.rec + s, f, s0, inf);
     rec_set_b(d.rec + s, inc);
     d.cstep[s] = cs_code(d, cs, A.k);
@@ -531,12 +531,14 @@ static __device__ __forceinline__ NewCell new_cell(const GmDev &d, const GmPPara
     n.carry = cls == 1 ? overshoot * 0.0682 : (cls == 2 ? overshoot * 0.0542 : overshoot * 0.0484);
     n.P = pP;
     n.one = false;
+    /* on its way beside the orientations of a new pair */
+    const double rho = d.rho[g];
     if (fresh_weight || pq0.z != g) n.P = pair_weight(d, pp, pq0.w, g, n.one);
     n.inf = dir_code(r);
     n.inc = 0.0;
     n.cs = (gm_cs_t)GM_CS_DEFERRED;
     if (!is_pending(n.P)) {
-        const uint32_t step = predict_values(d, A, k + 1u, n.carry, n.P, g, n.inf, n.inc);
+        const uint32_t step = predict_values(A, k + 1u, n.carry, n.P, rho, n.inf, n.inc);
         /* the window's lists of completed cells were made at its start */
         if (step < A.wend) atomicOr(&d.st->err, GM_ERRF_MISSED);
         n.cs = cs_code(d, step, k + 1u);

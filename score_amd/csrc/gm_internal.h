@@ -263,7 +263,8 @@ struct GmWin {
     uint32_t full[GM_WMAX], fullI[GM_WMAX]; /* cells completing in each step, in all and of the Inside list */
     uint32_t off[GM_WMAX + 1];  /* completed cells before each step: its list starts at pslot[off[i]] */
     uint32_t npend0;            /* new weight-cache entries before the current step */
-    uint32_t top_left;          /* cells of the grain that sets rhomax */
+    uint32_t left[GM_WMAX + 1]; /* cells of the grain that sets rhomax before each step (several regions: [0], moved on;
+                                 * a commit pass that runs again finds what it found) */
     uint32_t top_hit;           /* it lost its last cell */
     GmWinStep step[GM_WMAX + 1];
     unsigned long long nret0;   /* retirements before the window */

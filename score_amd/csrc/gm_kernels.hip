@@ -189,7 +189,7 @@ __global__ void __launch_bounds__(GM_BLOCK) k_sweep(GmDev d, GmPart P, uint32_t 
     }
     if (b == 0 && w == 1u && top_pos < d.ndefg) {
         const uint32_t n = exact_count(d, d.rorder[top_pos]);
-        if (lane == 0) d.win->top_left = n;
+        if (lane == 0) d.win->left[0] = n;
     }
     const WaveChunks r = wave_chunks(d, P, b, w);
     const uint32_t kc = k0 & (GM_CS_MOD - 1u), horizon = d.horizon;
@@ -670,33 +670,50 @@ static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, 
     GmStats *st = d.st;
     GmWin *win = d.win;
     const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
-    uint32_t wI = 0, wB = 0, na = 0;
-    for (uint32_t i = t; i < P.nbd; i += GM_BLOCK) {
-        const uint2 v = d.btot[i];
-        wI += v.x;
-        wB += v.y;
-    }
-    for (uint32_t i = t; i < P.nbp; i += GM_BLOCK) na += d.acnt[(js & 1u) * GM_PB + i];
-    block_sum3(wI, wB, na, sh);
-    const GmWinStep o = win->step[js];
-    const uint32_t limI = wI < o.recLenI ? wI : o.recLenI, limB = wB < o.recLenB ? wB : o.recLenB;
     const uint32_t rp = (js & 1u) * d.swb, rn = ((js + 1u) & 1u) * d.swb;
+    /* every load that needs no other's result is issued before the first is waited for:
+     * with six round trips in a row this block, not the parents', was the propose
+     * pass's longest */
+    static_assert(GM_DB <= 4 * GM_BLOCK && GM_PB <= 8 * GM_BLOCK, "one round of loads each");
+    uint2 bt[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; i++) bt[i] = t + i * GM_BLOCK < P.nbd ? d.btot[t + i * GM_BLOCK] : make_uint2(0u, 0u);
+    uint32_t ac[8];
+    const uint32_t *acnt = d.acnt + (js & 1u) * GM_PB;
+#pragma unroll
+    for (uint32_t i = 0; i < 8u; i++) ac[i] = t + i * GM_BLOCK < P.nbp ? acnt[t + i * GM_BLOCK] : 0u;
+    uint32_t R[8], pre[8], full[8];
+    auto tables = [&](uint32_t i0) {
+        if (i0 >= P.nb) return;
+        const uint4 *q = reinterpret_cast<const uint4 *>(d.rcnt + rp + i0);
+        const uint4 *u = reinterpret_cast<const uint4 *>(d.rpre + rp + i0);
+        const uint4 *f = reinterpret_cast<const uint4 *>(d.wcnt + (size_t)js * d.swb + i0);
+        const uint4 q0 = q[0], q1 = q[1], u0 = u[0], u1 = u[1], f0 = f[0], f1 = f[1];
+        R[0] = q0.x; R[1] = q0.y; R[2] = q0.z; R[3] = q0.w; R[4] = q1.x; R[5] = q1.y; R[6] = q1.z; R[7] = q1.w;
+        pre[0] = u0.x; pre[1] = u0.y; pre[2] = u0.z; pre[3] = u0.w;
+        pre[4] = u1.x; pre[5] = u1.y; pre[6] = u1.z; pre[7] = u1.w;
+        full[0] = f0.x; full[1] = f0.y; full[2] = f0.z; full[3] = f0.w;
+        full[4] = f1.x; full[5] = f1.y; full[6] = f1.z; full[7] = f1.w;
+    };
+    if (next) tables(8u * t);
+    const GmWinStep o = win->step[js];
+    GmStepRow r;
+    r.nfullI = win->fullI[js];
+    const uint32_t nfull = win->full[js], npend = agent_load(&st->npend), npend0 = win->npend0;
+    r.err = agent_load(&st->err);
+    r.pone = agent_load(&st->pone);
+    r.nplaced = st->nplaced;
+    r.pkey = st->arr_pkey;
+    const unsigned long long nret = st->nret;
+    uint32_t wI = bt[0].x + bt[1].x + bt[2].x + bt[3].x, wB = bt[0].y + bt[1].y + bt[2].y + bt[3].y;
+    uint32_t na = ac[0] + ac[1] + ac[2] + ac[3] + ac[4] + ac[5] + ac[6] + ac[7];
+    block_sum3(wI, wB, na, sh);
+    const uint32_t limI = wI < o.recLenI ? wI : o.recLenI, limB = wB < o.recLenB ? wB : o.recLenB;
     unsigned long long carry = 0ull; /* Inside | Border totals */
     if (next) {
         for (uint32_t b0 = 0; b0 < P.nb; b0 += 8u * GM_BLOCK) {
             const uint32_t i0 = b0 + 8u * t;
-            uint32_t R[8], pre[8], full[8];
-            if (i0 < P.nb) {
-                const uint4 *q = reinterpret_cast<const uint4 *>(d.rcnt + rp + i0);
-                const uint4 *u = reinterpret_cast<const uint4 *>(d.rpre + rp + i0);
-                const uint4 *f = reinterpret_cast<const uint4 *>(d.wcnt + (size_t)js * d.swb + i0);
-                const uint4 q0 = q[0], q1 = q[1], u0 = u[0], u1 = u[1], f0 = f[0], f1 = f[1];
-                R[0] = q0.x; R[1] = q0.y; R[2] = q0.z; R[3] = q0.w; R[4] = q1.x; R[5] = q1.y; R[6] = q1.z; R[7] = q1.w;
-                pre[0] = u0.x; pre[1] = u0.y; pre[2] = u0.z; pre[3] = u0.w;
-                pre[4] = u1.x; pre[5] = u1.y; pre[6] = u1.z; pre[7] = u1.w;
-                full[0] = f0.x; full[1] = f0.y; full[2] = f0.z; full[3] = f0.w;
-                full[4] = f1.x; full[5] = f1.y; full[6] = f1.z; full[7] = f1.w;
-            }
+            if (b0) tables(i0);
             unsigned long long sum = 0ull;
 #pragma unroll
             for (int i = 0; i < 8; i++) {
@@ -736,24 +753,17 @@ static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, 
         }
     }
     if (t != 0) return;
-    GmStepRow r;
     r.nI = o.nI + (wI - limI);
     r.nB = o.nB + (wB - limB);
-    r.nfullI = win->fullI[js];
-    r.nfullB = win->full[js] - win->fullI[js];
+    r.nfullB = nfull - r.nfullI;
     r.totRecI = o.totRecI;
     r.totRecB = o.totRecB;
     r.recLenI = o.recLenI;
     r.recLenB = o.recLenB;
     r.winI = wI;
     r.winB = wB;
-    const uint32_t npend = agent_load(&st->npend);
-    r.npend = npend - win->npend0;
+    r.npend = npend - npend0;
     r.nattempt = na;
-    r.err = agent_load(&st->err);
-    r.nplaced = st->nplaced;
-    r.pone = agent_load(&st->pone);
-    r.pkey = st->arr_pkey;
     st->rows[js] = r;
     st->nplaced = 0;
     st->pone = 0;
@@ -761,11 +771,11 @@ static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, 
     win->npend0 = npend;
     st->nI = r.nI;
     st->nB = r.nB;
-    st->nret += (unsigned long long)win->full[js];
+    st->nret = nret + (unsigned long long)nfull;
     st->nexec = js + 1u;
     if (next) {
         GmWinStep &s = win->step[js + 1u];
-        s.csz = gm_chunk_size(win->full[js], wI + wB);
+        s.csz = gm_chunk_size(nfull, wI + wB);
         s.nI = r.nI;
         s.nB = r.nB;
         s.totRecI = (uint32_t)(carry >> 32);
@@ -893,32 +903,57 @@ static __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t 
  * blocks beyond it are left alone and catch up when they are reached. */
 static __device__ void recycle_blocks(const GmDev &d, const GmPart &P, uint32_t j, uint32_t r, uint32_t nrec,
                                       unsigned long long *sm) {
-    __shared__ uint32_t sh[GM_BLOCK / 64], sn[GM_BLOCK / 64][3];
+    __shared__ uint32_t sh[GM_BLOCK / 64], sn[GM_BLOCK / 64][3], sfull[GM_WMAX], slist[GM_WMAX];
     const GmWin *win = d.win;
     const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
     const uint32_t rp = (j & 1u) * d.swb, nt = GM_SW_WAVES * P.cpw * GM_SW_TPC;
     uint32_t *so = reinterpret_cast<uint32_t *>(sm + nt);
     const uint32_t recI = win->step[j].recLenI, recB = win->step[j].recLenB;
+    const uint32_t halt = d.st->halt;
     uint32_t na = 0, z0 = 0, z1 = 0;
-    for (uint32_t i = 4u * t; i < P.nbp; i += 4u * GM_BLOCK) {
-        const uint4 q = *reinterpret_cast<const uint4 *>(d.acnt + (j & 1u) * GM_PB + i);
-        na += q.x + (i + 1u < P.nbp ? q.y : 0u) + (i + 2u < P.nbp ? q.z : 0u) + (i + 3u < P.nbp ? q.w : 0u);
+    uint4 ac[2];
+    static_assert(GM_PB <= 8 * GM_BLOCK, "one round of loads");
+#pragma unroll
+    for (uint32_t i = 0; i < 2u; i++) {
+        ac[i] = make_uint4(0u, 0u, 0u, 0u);
+        const uint32_t at = 4u * (t + i * GM_BLOCK);
+        if (at < P.nbp) ac[i] = *reinterpret_cast<const uint4 *>(d.acnt + (j & 1u) * GM_PB + at);
     }
-    block_sum3(na, z0, z1, sn);
     for (uint32_t b = r; b < P.nb; b += nrec) {
+        /* everything a block may need is loaded before its first use: its masks, what the
+         * step before handed out, where each step's completed cells are listed */
         const bool inB = b >= P.nbI;
-        const uint32_t pre = d.rpre[rp + b], gone = j ? d.rgone[b] : 0u, rec = inB ? recB : recI;
-        const uint32_t bound = na < rec ? na : rec;
-        if (gone == 0u && pre >= bound) continue;
         const uint32_t nch = inB ? P.chB : P.chI, ch0 = (inB ? b - P.nbI : b) * GM_SW_WAVES * P.cpw;
         const uint32_t n = (ch0 + GM_SW_WAVES * P.cpw < nch ? GM_SW_WAVES * P.cpw : nch - ch0) * GM_SW_TPC;
-        const uint32_t t0 = ((inB ? P.chI : 0u) + ch0) * GM_SW_TPC, merged = d.rmrg[b];
+        const uint32_t t0 = ((inB ? P.chI : 0u) + ch0) * GM_SW_TPC;
+        const unsigned long long m0 = t < n ? d.mR[t0 + t] : 0ull;
+        const uint32_t merged = d.rmrg[b], pre = d.rpre[rp + b], gone = j ? d.rgone[b] : 0u, rec = inB ? recB : recI;
+        uint32_t lf = 0, lo = 0;
+        if (t < j) {
+            lf = d.wcnt[(size_t)t * d.swb + b];
+            lo = win->off[t] + d.wpre[(size_t)t * d.swb + b];
+        }
+        if (b == r) {
+#pragma unroll
+            for (uint32_t i = 0; i < 2u; i++) {
+                const uint32_t at = 4u * (t + i * GM_BLOCK);
+                na += ac[i].x + (at + 1u < P.nbp ? ac[i].y : 0u) + (at + 2u < P.nbp ? ac[i].z : 0u) + (at + 3u < P.nbp ? ac[i].w : 0u);
+            }
+            block_sum3(na, z0, z1, sn);
+            if (halt) return;
+        }
+        const uint32_t bound = na < rec ? na : rec;
+        if (gone == 0u && pre >= bound) continue;
         const uint32_t rel0 = ch0 * GM_SW_CHUNK, slot0 = (inB ? 0u : d.baseI) + rel0;
         uint32_t run = 0;
         __syncthreads();
+        if (t < j) {
+            sfull[t] = lf;
+            slist[t] = lo;
+        }
         for (uint32_t i0 = 0; i0 < n; i0 += GM_BLOCK) {
             const uint32_t i = i0 + t;
-            unsigned long long m = i < n ? d.mR[t0 + i] : 0ull;
+            unsigned long long m = i0 == 0u ? m0 : i < n ? d.mR[t0 + i] : 0ull;
             if (run < gone) {
                 const uint32_t c = (uint32_t)__popcll(m);
                 uint32_t tot;
@@ -932,8 +967,8 @@ static __device__ void recycle_blocks(const GmDev &d, const GmPart &P, uint32_t 
         }
         __syncthreads();
         for (uint32_t i = merged; i < j; i++) {
-            const uint32_t nf = d.wcnt[(size_t)i * d.swb + b];
-            const uint32_t *list = d.pslot + win->off[i] + d.wpre[(size_t)i * d.swb + b];
+            const uint32_t nf = sfull[i];
+            const uint32_t *list = d.pslot + slist[i];
             for (uint32_t q = t; q < nf; q += GM_BLOCK) {
                 const uint32_t s = list[q] - slot0;
                 atomicOr(&sm[s >> 6], 1ull << (s & 63u));
@@ -983,12 +1018,12 @@ __global__ void __launch_bounds__(GM_BLOCK) k_decide(GmDev d, GmPart P, uint32_t
     };
     __shared__ Wave sw[GM_BLOCK / 64];
     __shared__ uint32_t sh[GM_BLOCK / 64][3];
-    const uint32_t halt = d.st->halt, nfull = d.win->full[j], csz = d.win->step[j].csz;
-    if (halt) return;
     if (blockIdx.x < nrec) {
         recycle_blocks(d, P, j, blockIdx.x, nrec, smask);
         return;
     }
+    const uint32_t halt = d.st->halt, nfull = d.win->full[j], csz = d.win->step[j].csz;
+    if (halt) return;
     const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u, blk = blockIdx.x - nrec;
     const uint32_t nch = (nfull + csz - 1u) / csz, cpd = (nch + P.nbd - 1u) / P.nbd;
     const uint32_t c0 = blk * cpd, c1 = c0 + cpd < nch ? c0 + cpd : nch;
@@ -1005,8 +1040,6 @@ __global__ void __launch_bounds__(GM_BLOCK) k_decide(GmDev d, GmPart P, uint32_t
         /* where the parent's grain stands in the order of rho: the one that sets
          * rhomax is counted, one before it (all without cells) has its count wrap */
         const uint32_t rp = valid ? d.rpos[q0.z] : 0xFFFFFFFFu;
-        ntop += rp == top_pos ? 1u : 0u;
-        wrapped |= rp < top_pos;
         W.mI[lane] = 0;
         W.mB[lane] = 0;
         const uint32_t na = (uint32_t)__popc(am), incl = wave_incl_scan(na);
@@ -1024,6 +1057,8 @@ __global__ void __launch_bounds__(GM_BLOCK) k_decide(GmDev d, GmPart P, uint32_t
             if (t.x == (c * csz + q) * 32u + rk) atomicOr(toB ? &W.mB[q] : &W.mI[q], 1u << rk);
             if (i < GM_GATT && c < d.gchunks) d.gatt[(size_t)c * GM_GATT + i] = t.y;
         }
+        ntop += rp == top_pos ? 1u : 0u;
+        wrapped |= rp < top_pos;
         wave_sync();
         const uint32_t mI = W.mI[lane], mB = W.mB[lane];
         if (valid) {
@@ -1103,22 +1138,22 @@ static __device__ __forceinline__ void commit_step(const GmDev &d, const GmPPara
             nB += v & 0xFFFFu;
         }
     };
+    uint32_t runI = 0, runB = 0, totI = 0;
+    uint2 bt[4];
+    static_assert(GM_DB <= 4 * GM_BLOCK, "one round of loads");
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; i++) {
+        const uint32_t at = threadIdx.x + i * GM_BLOCK;
+        bt[i] = at < P.nbd ? d.btot[at] : make_uint2(0u, 0u);
+    }
     uint32_t bI, bB;
     count(c0, c0 + wv < c1 ? c0 + wv : c1, bI, bB);
-    uint32_t runI = 0, runB = 0, totI = 0;
-    for (uint32_t i0 = threadIdx.x; i0 < P.nbd; i0 += 4u * GM_BLOCK) {
-        uint2 v[4];
 #pragma unroll
-        for (uint32_t i = 0; i < 4u; i++) {
-            v[i] = make_uint2(0u, 0u);
-            if (i0 + i * GM_BLOCK < P.nbd) v[i] = d.btot[i0 + i * GM_BLOCK];
-        }
-#pragma unroll
-        for (uint32_t i = 0; i < 4u; i++) {
-            totI += v[i].x;
-            runI += i0 + i * GM_BLOCK < db ? v[i].x : 0u;
-            runB += i0 + i * GM_BLOCK < db ? v[i].y : 0u;
-        }
+    for (uint32_t i = 0; i < 4u; i++) {
+        const bool before = threadIdx.x + i * GM_BLOCK < db;
+        totI += bt[i].x;
+        runI += before ? bt[i].x : 0u;
+        runB += before ? bt[i].y : 0u;
     }
     block_sum3(runI, runB, totI, sh);
     /* every block finds the same: the Inside list must grow before the step's
@@ -1131,16 +1166,6 @@ static __device__ __forceinline__ void commit_step(const GmDev &d, const GmPPara
             agent_store(&st->grow, need < d.capImax ? (uint32_t)need : d.capImax);
         }
         return;
-    }
-    if (db == 0) { /* the cells left of the grain that sets rhomax */
-        uint32_t n = 0, z0 = 0, z1 = 0;
-        for (uint32_t i = threadIdx.x; i < P.nbd; i += GM_BLOCK) n += d.btop[i];
-        block_sum3(n, z0, z1, sh);
-        if (threadIdx.x == 0 && n) {
-            const uint32_t left = d.win->top_left - n;
-            d.win->top_left = left;
-            if (left == 0u) agent_store(&d.win->top_hit, 1u);
-        }
     }
     Wave &W = sw[wv];
     bool one = false;
@@ -1211,6 +1236,21 @@ static __device__ __forceinline__ void commit_step(const GmDev &d, const GmPPara
 
 static __device__ void window_end(const GmDev &d, const GmPart &P, uint32_t launched, uint32_t top_pos, uint32_t *out);
 
+/* the cells left of the grain that sets rhomax after step j, by the pass's last block,
+ * which most often has no parents (and in a pass that runs again finds the same) */
+static __device__ __forceinline__ void count_top(const GmDev &d, const GmPart &P, uint32_t j) {
+    __shared__ uint32_t sh[GM_BLOCK / 64][3];
+    const uint32_t halt = d.st->halt, had = d.win->left[j];
+    uint32_t n = 0, z0 = 0, z1 = 0;
+    for (uint32_t i = threadIdx.x; i < P.nbd; i += GM_BLOCK) n += d.btop[i];
+    if (halt) return;
+    block_sum3(n, z0, z1, sh);
+    if (threadIdx.x == 0) {
+        d.win->left[j + 1u] = had - n;
+        if (n && had == n) agent_store(&d.win->top_hit, 1u);
+    }
+}
+
 /* With `out` the pass is the window's last: the block that finds all others done closes
  * the window (window_end), where a launch of its own took 6 us a window: a tenth of a
  * step where the scalars change in every one.  What it needs of the other
@@ -1221,6 +1261,7 @@ __global__ void __launch_bounds__(GM_BLOCK, 4) k_commit(GmDev d, GmPParams pp, G
                                                        uint32_t need_one, uint32_t top_pos, uint32_t *out) {
     __shared__ uint32_t last;
     commit_step(d, pp, A, P, j, need_one);
+    if (blockIdx.x == gridDim.x - 1u) count_top(d, P, j);
     if (!out) return;
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -1835,7 +1876,7 @@ __global__ void __launch_bounds__(1024) k_arrivals(GmDev d, GmSweepArgs A) {
                 const uint32_t g = d.cell[c].y;
                 const double P = d.nucP[id];
                 double inc = 0.0;
-                const gm_cs_t cs = cs_code(d, predict_values(d, A, k, 1.0, P, g, 26u, inc), k);
+                const gm_cs_t cs = cs_code(d, predict_values(A, k, 1.0, P, d.rho[g], 26u, inc), k);
                 GmRec *r = d.rec + gslot;
                 rec_set_a(r, 1.0, k, 26u);
                 rec_set_b(r, inc);
@@ -1875,7 +1916,7 @@ __global__ void __launch_bounds__(64) k_window_begin(GmDev d, uint32_t k, double
     GmStats *st = d.st;
     if (top_pos < d.ndefg) {
         const uint32_t n = exact_count(d, d.rorder[top_pos]);
-        if (threadIdx.x == 0) d.win->top_left = n;
+        if (threadIdx.x == 0) d.win->left[0] = n;
     }
     if (threadIdx.x != 0) return;
     d.win->top_hit = 0;
@@ -1922,7 +1963,7 @@ static __device__ __forceinline__ void predict_deferred(const GmDev &d, const Gm
         }
         r->P = P;
         double inc, f = a.frac0;
-        if (cell_increment(d, A.sp, P, c.defg, a.inf, inc)) f = gm_radd_n(f, inc, A.k - a.s0);
+        if (cell_increment(A.sp, P, d.rho[c.defg], a.inf, inc)) f = gm_radd_n(f, inc, A.k - a.s0);
         predict_slot(d, A, s, f, A.k, P, c.defg, a.inf);
     }
 }

@@ -632,8 +632,6 @@ __global__ void __launch_bounds__(64) k_rg_decide(GmDev d, uint32_t nrec, uint32
         const uint4 q0 = valid ? par_plane(d, GM_PAR_IDS)[p] : make_uint4(0u, 0u, 0xFFFFFFFFu, 0xFFFFFFFFu);
         retire(d, q0.z, q0.w, valid, blk & (GM_SUBS - 1u));
         const uint32_t rp = valid ? d.rpos[q0.z] : 0xFFFFFFFFu;
-        ntop += rp == top_pos ? 1u : 0u;
-        wrapped |= rp < top_pos;
         const uint32_t n = list_attempts(am, wl);
         for (uint32_t i = lane; i < n; i += 64u) {
             const uint32_t e = wl[i], q = e & 0xFFu, rk = e >> 8;
@@ -649,6 +647,8 @@ __global__ void __launch_bounds__(64) k_rg_decide(GmDev d, uint32_t nrec, uint32
             }
         }
         wave_sync();
+        ntop += rp == top_pos ? 1u : 0u;
+        wrapped |= rp < top_pos;
         const uint32_t mI = sI[lane], mB = sB[lane];
         if (valid) {
             d.pmI[p] = mI;
@@ -693,8 +693,8 @@ __global__ void __launch_bounds__(1024) k_rg_decide_scan(GmDev d, uint32_t nb) {
     if (threadIdx.x == 0) {
         st->nattempt = tot[GM_RW_A];
         if (tot[GM_RROWS]) { /* the cells left of the grain that sets rhomax */
-            const uint32_t left = d.win->top_left - tot[GM_RROWS];
-            d.win->top_left = left;
+            const uint32_t left = d.win->left[0] - tot[GM_RROWS];
+            d.win->left[0] = left;
             if (left == 0u) d.win->top_hit = 1u;
         }
     }
