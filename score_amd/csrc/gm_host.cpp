@@ -1439,6 +1439,7 @@ GmPart window_part(const score_gm_handle *h, uint32_t nI, uint32_t nB, uint32_t 
     P.nbp = (uint32_t)std::min<uint64_t>(GM_PB, est / 64 + 1);
     P.nbd = std::min<uint32_t>(GM_DB, P.nbp);
     P.csz0 = h->last_csz;
+    P.fused = h->d.nreg <= 1 && !h->prof && gm_fold(P) && P.nb <= GM_PB ? 1u : 0u;
     return P;
 }
 
@@ -1505,7 +1506,7 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
     a.nB = nBe;
     a.wend = d.nreg > 1 ? 0u : h->step + W;
     const uint32_t na = arrivals_at(h, h->step);
-    const GmPart P = window_part(h, (uint32_t)std::min<uint64_t>(d.capI, (uint64_t)h->nI + na),
+    GmPart P = window_part(h, (uint32_t)std::min<uint64_t>(d.capI, (uint64_t)h->nI + na),
                                  (uint32_t)std::min<uint64_t>(d.capB, (uint64_t)h->nB + na), W);
     GmWindow w;
     memset(&w, 0, sizeof(w));
@@ -1564,6 +1565,9 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
             (e = gm_launch_fill_u32(&d.st->halt, 0u, 1, h->stream)) != hipSuccess ||
             (grow && (e = gm_launch_commit(d, h->pp, a, P, w, j0, nullptr, h->stream, ev)) != hipSuccess))
             return h->err = hip_fail(e, "growth step");
+        /* (a first step that is run again has its propose pass to itself; its attempts'
+         * counts are then the only ones) */
+        if (!grow) P.fused = 0;
         for (uint32_t j = grow ? j0 + 1u : 0u; j < W; j++)
             if ((e = gm_launch_infect(d, h->pp, a, P, w, j, nullptr, h->stream, ev)) != hipSuccess)
                 return h->err = hip_fail(e, "growth step");

@@ -248,7 +248,11 @@ static inline __host__ __device__ uint32_t gm_chunk_size(uint32_t nfull, uint32_
 struct GmPart {
     uint32_t nbI, nb, cpw, chI, chB, W, nbp, nbd;
     uint32_t csz0;              /* the first step's chunk size */
+    uint32_t fused;             /* the compaction does the first step's propose pass */
 };
+
+/* whether compaction blocks add up the sweep blocks' counts themselves */
+static inline bool gm_fold(const GmPart &P) { return P.nb <= GM_SW_FOLD || (P.W + 1u) * P.nb <= GM_SW_FOLD * 10u; }
 
 /* the front lists as a step of the window finds them */
 struct GmWinStep {

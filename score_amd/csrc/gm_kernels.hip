@@ -19,7 +19,8 @@
  *   k_sweep_scan   one block scans the per-block counts into offsets (short fronts:
  *                  each block of the next pass adds up what it needs).
  *   k_compact      the completed slots of every step in FullRX order (Inside list,
- *                  then Border), and the INACTIVE slots as masks.
+ *                  then Border), and the INACTIVE slots as masks.  Short fronts: the
+ *                  first step's propose pass too.
  *   k_window_end   closes the last step and hands the stats to the host.
  * per step
  *   k_propose      block 0 closes the step before (its row, list lengths, recycling
@@ -340,152 +341,8 @@ __global__ void __launch_bounds__(1024) k_sweep_scan(GmDev d, GmPart P) {
     if (threadIdx.x == 0) window_totals(d, P, stot, stotI[P.W], stot[P.W] - stotI[P.W], stotI);
 }
 
-/* pass 3: append_to_fullrx_*_list (SCORE_Kernel.cpp:3994-4042, :4133-4180) of
- * every step as ordered compaction: step i's completed slots ascending, Inside
- * then Border, at pslot[win->off[i]...]; and the INACTIVE mask of every 64-slot
- * tile, from which the steps hand out recycled slots.  FOLD: the block adds up
- * the counts of the blocks itself. */
-template <bool FOLD>
-__global__ void __launch_bounds__(GM_BLOCK) k_compact(GmDev d, GmPart P, uint32_t k0) {
-    __shared__ uint32_t stot[GM_WMAX + 1], spre[GM_WMAX + 1], stotI[GM_WMAX + 1], base[GM_WMAX];
-    __shared__ uint32_t run[GM_SW_WAVES][GM_WMAX];
-    __shared__ uint64_t sR[GM_SW_WAVES][8];
-    /* per lane 16 counters of 16 bits, rows of 40 bytes against bank conflicts */
-    __shared__ __align__(8) uint32_t sl[GM_SW_WAVES][64][10];
-    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6, b = blockIdx.x, t = threadIdx.x;
-    if (FOLD) {
-        for (uint32_t row = w; row <= P.W; row += GM_SW_WAVES) {
-            const bool rec = row == P.W;
-            const uint32_t *cnt = d.wcnt + (size_t)(rec ? (uint32_t)GM_WMAX : row) * d.swb;
-            uint32_t a = 0, p = 0, pI = 0;
-            for (uint32_t i0 = 4u * lane; i0 < P.nb; i0 += 256u) {
-                const uint4 q = *reinterpret_cast<const uint4 *>(cnt + i0);
-                const uint32_t v[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-                for (uint32_t i = 0; i < 4; i++) {
-                    const uint32_t x = i0 + i < P.nb ? v[i] : 0u;
-                    a += x;
-                    p += i0 + i < b ? x : 0u;
-                    pI += i0 + i < P.nbI ? x : 0u;
-                }
-            }
-            for (int o = 32; o > 0; o >>= 1) {
-                a += __shfl_xor(a, o, 64);
-                p += __shfl_xor(p, o, 64);
-                pI += __shfl_xor(pI, o, 64);
-            }
-            if (lane == 0) {
-                stot[row] = a;
-                spre[row] = p;
-                stotI[row] = pI;
-            }
-        }
-        __syncthreads();
-        if (t < P.W) {
-            uint32_t o = spre[t];
-            d.wpre[(size_t)t * d.swb + b] = o;
-            for (uint32_t i = 0; i < t; i++) o += stot[i];
-            base[t] = o;
-        }
-        if (t == GM_WMAX) {
-            d.rcnt[b] = d.wcnt[(size_t)GM_WMAX * d.swb + b];
-            d.rpre[b] = spre[P.W] - (b >= P.nbI ? stotI[P.W] : 0u);
-            d.rgone[b] = 0;
-            d.rmrg[b] = 0;
-        }
-        if (b == 0 && t == 64u) window_totals(d, P, stot, stotI[P.W], stot[P.W] - stotI[P.W], stotI);
-    } else if (t < P.W) {
-        base[t] = d.win->off[t] + d.wpre[(size_t)t * d.swb + b];
-    }
-    __syncthreads();
-    if (lane < P.W) {
-        uint32_t o = base[lane];
-        const uint32_t *ww = d.wwave + (size_t)b * GM_SW_WAVES * GM_WMAX + lane;
-        for (uint32_t q = 0; q < w; q++) o += ww[q * GM_WMAX];
-        run[w][lane] = o;
-    }
-    wave_sync();
-    const WaveChunks r = wave_chunks(d, P, b, w);
-    const uint32_t kc = k0 & (GM_CS_MOD - 1u), horizon = d.horizon;
-    for (uint32_t c = r.c0; c < r.c1; c++) {
-        uint32_t nocc;
-        const uint4 cs = chunk_codes(d, r, c, lane, nocc);
-        unsigned long long cnt = 0ull; /* 16 counters of 4 bits (at most 8 each) */
-        uint32_t full = 0, rec = 0;
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const uint32_t x = code_at(cs, q);
-            const bool in = (uint32_t)q < nocc;
-            const uint32_t di = (x - kc) & (GM_CS_MOD - 1u);
-            const bool f = in && x < GM_CS_MOD && di < P.W;
-            cnt += f ? 1ull << (4u * (di & 15u)) : 0ull;
-            full |= f ? 1u << q : 0u;
-            rec |= in && cs_inactive(x, kc, horizon) ? 1u << q : 0u;
-        }
-        reinterpret_cast<uint8_t *>(sR[w])[lane] = (uint8_t)rec;
-        wave_sync();
-        if (lane < GM_SW_TPC) d.mR[r.tile0 + c * GM_SW_TPC + lane] = sR[w][lane];
-        if (!__any(full != 0u)) {
-            wave_sync();
-            continue;
-        }
-        uint32_t incl[GM_WMAX / 2];
-#pragma unroll
-        for (int i = 0; i < GM_WMAX / 2; i++) {
-            if (2u * i >= P.W) break;
-            const uint32_t f = (uint32_t)(cnt >> (8 * i));
-            const uint32_t v = (f & 0xFu) | (f & 0xF0u) << 12;
-            incl[i] = wave_incl_scan(v);
-            sl[w][lane][i] = incl[i] - v;
-        }
-        wave_sync();
-        uint16_t *mineRow = reinterpret_cast<uint16_t *>(sl[w][lane]);
-        const uint32_t slot = r.slot0 + c * GM_SW_CHUNK + 8u * lane;
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            if (!((full >> q) & 1u)) continue;
-            const uint32_t di = (code_at(cs, q) - kc) & (GM_CS_MOD - 1u);
-            const uint32_t o = mineRow[di];
-            mineRow[di] = (uint16_t)(o + 1u);
-            d.pslot[run[w][di] + o] = slot + (uint32_t)q;
-        }
-        wave_sync();
-        if (lane == 63u) {
-#pragma unroll
-            for (int i = 0; i < GM_WMAX / 2; i++) {
-                if (2u * i >= P.W) break;
-                run[w][2 * i] += incl[i] & 0xFFFFu;
-                run[w][2 * i + 1] += incl[i] >> 16;
-            }
-        }
-        wave_sync();
-    }
-}
-
 hipError_t gm_launch_reanchor(const GmDev &d, const GmSweepArgs &a, hipStream_t s) {
     k_reanchor<<<grid_for(a.nI + a.nB, GM_BLOCK), GM_BLOCK, 0, s>>>(d, a);
-    return hipGetLastError();
-}
-
-__global__ void k_arrivals(GmDev d, GmSweepArgs A);
-
-hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &a, const GmWindow &wd, bool arrivals,
-                            double xcells, hipStream_t s, hipEvent_t *ev) {
-    hipError_t e;
-    if ((e = mark(ev, 0, s)) != hipSuccess) return e;
-    if (a.reanchor && (e = gm_launch_reanchor(d, a, s)) != hipSuccess) return e;
-    if (arrivals) {
-        k_arrivals<<<1, 1024, 0, s>>>(d, a);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
-    if ((e = mark(ev, 1, s)) != hipSuccess) return e;
-    k_sweep<<<P.nb, GM_BLOCK, 0, s>>>(d, P, a.k, xcells, wd.top_pos);
-    if ((e = mark(ev, 2, s)) != hipSuccess) return e;
-    const bool fold = P.nb <= GM_SW_FOLD || (P.W + 1u) * P.nb <= GM_SW_FOLD * 10u;
-    if (!fold) k_sweep_scan<<<1, 1024, 0, s>>>(d, P);
-    if ((e = mark(ev, 3, s)) != hipSuccess) return e;
-    if (fold) k_compact<true><<<P.nb, GM_BLOCK, 0, s>>>(d, P, a.k);
-    else k_compact<false><<<P.nb, GM_BLOCK, 0, s>>>(d, P, a.k);
     return hipGetLastError();
 }
 
@@ -658,6 +515,11 @@ static __device__ __forceinline__ void block_sum3(uint32_t &a, uint32_t &b, uint
     }
 }
 
+/* blocks that counted step j's attempts */
+static __device__ __forceinline__ uint32_t attempt_blocks(const GmPart &P, uint32_t j) {
+    return j == 0u && P.fused ? P.nb : P.nbp;
+}
+
 /* Closes step js of the window, by one block after the step's commit pass: its
  * row for the host's master section, the lists' lengths and, with `next`, the
  * recycling tables of step js+1: per sweep block, how many of its INACTIVE slots
@@ -679,9 +541,9 @@ static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, 
 #pragma unroll
     for (uint32_t i = 0; i < 4u; i++) bt[i] = t + i * GM_BLOCK < P.nbd ? d.btot[t + i * GM_BLOCK] : make_uint2(0u, 0u);
     uint32_t ac[8];
-    const uint32_t *acnt = d.acnt + (js & 1u) * GM_PB;
+    const uint32_t *acnt = d.acnt + (js & 1u) * GM_PB, nba = attempt_blocks(P, js);
 #pragma unroll
-    for (uint32_t i = 0; i < 8u; i++) ac[i] = t + i * GM_BLOCK < P.nbp ? acnt[t + i * GM_BLOCK] : 0u;
+    for (uint32_t i = 0; i < 8u; i++) ac[i] = t + i * GM_BLOCK < nba ? acnt[t + i * GM_BLOCK] : 0u;
     uint32_t R[8], pre[8], full[8];
     auto tables = [&](uint32_t i0) {
         if (i0 >= P.nb) return;
@@ -791,14 +653,49 @@ static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, 
  * that found too few slots), or step j has more parents than the planes hold.  Every
  * input was written by an earlier kernel, so all blocks of the propose pass find
  * the same; it records the answer in st->halt for the step's other passes. */
-static __device__ __forceinline__ bool must_halt(const GmDev &d, const GmWindow &w, uint32_t j) {
+static __device__ __forceinline__ bool must_halt_at(const GmDev &d, const GmWindow &w, uint32_t nfull) {
     const GmStats *st = d.st;
-    const GmWin *win = d.win;
     /* every word loaded before the first test */
-    const uint32_t flags = st->err | st->cwrap | st->novf | win->top_hit | st->grow, npend = st->npend;
-    const double xc = win->xcells0 + (double)win->off[j];
-    return (flags != 0u) | ((npend != 0u) & !w.defer) | (npend > w.pend_limit) | ((j != 0u) & (xc >= w.xstop)) |
-           (win->full[j] > d.parentCap);
+    const uint32_t flags = st->err | st->cwrap | st->novf | d.win->top_hit | st->grow, npend = st->npend;
+    return (flags != 0u) | ((npend != 0u) & !w.defer) | (npend > w.pend_limit) | (nfull > d.parentCap);
+}
+static __device__ __forceinline__ bool must_halt(const GmDev &d, const GmWindow &w, uint32_t j) {
+    const double xc = d.win->xcells0 + (double)d.win->off[j];
+    return must_halt_at(d, w, d.win->full[j]) | ((j != 0u) & (xc >= w.xstop));
+}
+
+/* Step k's parent p, in slot s: see k_propose; returns its attempts.  rlog: where the
+ * step's retirements go in the log (null: they do not fit). */
+static __device__ __forceinline__ uint32_t propose_parent(const GmDev &d, uint32_t s, uint32_t p, uint32_t k, uint2 *rlog) {
+    const GmRec *r = d.rec + s;
+    const RecC rc = rec_c(r);
+    const RecA ra = rec_a(r);
+    const double inc = r->inc;
+    const uint32_t rxg = r->rxg, cell = rc.cell;
+    const uint32_t z = cell / d.nxy, rem = cell - z * d.nxy, y = rem / d.nx, x = rem - y * d.nx;
+    const bool fromB = s < d.baseI;
+    const bool interior = (x - 1u < d.nx - 2u) & (y - 1u < d.ny - 2u) & (z - 1u < d.nz - 2u);
+    Neighbourhood nb;
+    if (interior) nb.load(d, x, y, z);
+    /* rxFrac after the completing addition, while the bits are on their way */
+    const double fin = advanced(ra.frac0, inc, k - ra.s0 + 1u);
+    const uint32_t am = interior ? nb.mask() : face_attempts(d, x, y, z);
+    for (uint32_t m = am; m; m &= m - 1u) {
+        const uint32_t rk = (uint32_t)__ffs(m) - 1u;
+        uint32_t t = cell + (uint32_t)(dir_dx(rk) + dir_dy(rk) * (int)d.nx + dir_dz(rk) * (int)d.nxy);
+        if (!interior) {
+            uint32_t tx, ty, tz;
+            bool toB;
+            attempt_target(d, true, x, y, z, (int)rk, tx, ty, tz, toB);
+            t = cell_of(d, tx, ty, tz);
+        }
+        atomicMin(&d.cell[t].x, p * 32u + rk);
+    }
+    d.pmA[p] = am;
+    par_plane(d, GM_PAR1_CELL)[p] = make_uint4(x | y << 16, z | (fromB ? 1u << 16 : 0u), rc.defg, rxg);
+    reinterpret_cast<double2 *>(par_plane(d, GM_PAR1_FP))[p] = make_double2(fin, rc.P);
+    if (rlog) rlog[p] = make_uint2(cell, d.ndefg + rxg);
+    return (uint32_t)__popc(am);
 }
 
 /* Step j's attempts, one lane per parent.  What the infection needs of the parent
@@ -839,41 +736,181 @@ __global__ void __launch_bounds__(GM_BLOCK) k_propose(GmDev d, GmPart P, GmWindo
     for (uint32_t c = w * P.nbp + blk; c * 64u < nfull; c += P.nbp * (GM_BLOCK / 64u)) {
         const uint32_t p = c * 64u + lane;
         if (p >= nfull) break;
-        const uint32_t s = d.pslot[off + p];
-        const GmRec *r = d.rec + s;
-        const RecC rc = rec_c(r);
-        const RecA ra = rec_a(r);
-        const double inc = r->inc;
-        const uint32_t rxg = r->rxg, cell = rc.cell;
-        const uint32_t z = cell / d.nxy, rem = cell - z * d.nxy, y = rem / d.nx, x = rem - y * d.nx;
-        const bool fromB = s < d.baseI;
-        const bool interior = (x - 1u < d.nx - 2u) & (y - 1u < d.ny - 2u) & (z - 1u < d.nz - 2u);
-        Neighbourhood nb;
-        if (interior) nb.load(d, x, y, z);
-        /* rxFrac after the completing addition, while the bits are on their way */
-        const double fin = advanced(ra.frac0, inc, k - ra.s0 + 1u);
-        const uint32_t am = interior ? nb.mask() : face_attempts(d, x, y, z);
-        for (uint32_t m = am; m; m &= m - 1u) {
-            const uint32_t rk = (uint32_t)__ffs(m) - 1u;
-            uint32_t t = cell + (uint32_t)(dir_dx(rk) + dir_dy(rk) * (int)d.nx + dir_dz(rk) * (int)d.nxy);
-            if (!interior) {
-                uint32_t tx, ty, tz;
-                bool toB;
-                attempt_target(d, true, x, y, z, (int)rk, tx, ty, tz, toB);
-                t = cell_of(d, tx, ty, tz);
-            }
-            atomicMin(&d.cell[t].x, p * 32u + rk);
-        }
-        natt += (uint32_t)__popc(am);
-        d.pmA[p] = am;
-        par_plane(d, GM_PAR1_CELL)[p] = make_uint4(x | y << 16, z | (fromB ? 1u << 16 : 0u), rc.defg, rxg);
-        reinterpret_cast<double2 *>(par_plane(d, GM_PAR1_FP))[p] = make_double2(fin, rc.P);
-        if (logged) d.rlog[nret + p] = make_uint2(cell, d.ndefg + rxg);
+        natt += propose_parent(d, d.pslot[off + p], p, k, logged ? d.rlog + nret : nullptr);
     }
     for (int o = 32; o > 0; o >>= 1) natt += __shfl_xor(natt, o, 64);
     if (lane == 0) satt[w] = natt;
     __syncthreads();
     if (threadIdx.x == 0) d.acnt[(j & 1u) * GM_PB + blk] = satt[0] + satt[1] + satt[2] + satt[3];
+}
+
+/* pass 3: append_to_fullrx_*_list (SCORE_Kernel.cpp:3994-4042, :4133-4180) of
+ * every step as ordered compaction: step i's completed slots ascending, Inside
+ * then Border, at pslot[win->off[i]...]; and the INACTIVE mask of every 64-slot
+ * tile, from which the steps hand out recycled slots.  FOLD: the block adds up
+ * the counts of the blocks itself.  PROPOSE: the blocks then take the first step's
+ * parents they have listed through the propose pass, which saves a launch a window: 5 us
+ * of every step where the scalars change in each. */
+template <bool FOLD, bool PROPOSE>
+__global__ void __launch_bounds__(GM_BLOCK) k_compact(GmDev d, GmPart P, GmWindow wd, uint32_t k0) {
+    __shared__ uint32_t stot[GM_WMAX + 1], spre[GM_WMAX + 1], stotI[GM_WMAX + 1], base[GM_WMAX];
+    __shared__ uint32_t run[GM_SW_WAVES][GM_WMAX];
+    __shared__ uint64_t sR[GM_SW_WAVES][8];
+    /* per lane 16 counters of 16 bits, rows of 40 bytes against bank conflicts */
+    __shared__ __align__(8) uint32_t sl[GM_SW_WAVES][64][10];
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6, b = blockIdx.x, t = threadIdx.x;
+    if (FOLD) {
+        for (uint32_t row = w; row <= P.W; row += GM_SW_WAVES) {
+            const bool rec = row == P.W;
+            const uint32_t *cnt = d.wcnt + (size_t)(rec ? (uint32_t)GM_WMAX : row) * d.swb;
+            uint32_t a = 0, p = 0, pI = 0;
+            for (uint32_t i0 = 4u * lane; i0 < P.nb; i0 += 256u) {
+                const uint4 q = *reinterpret_cast<const uint4 *>(cnt + i0);
+                const uint32_t v[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+                for (uint32_t i = 0; i < 4; i++) {
+                    const uint32_t x = i0 + i < P.nb ? v[i] : 0u;
+                    a += x;
+                    p += i0 + i < b ? x : 0u;
+                    pI += i0 + i < P.nbI ? x : 0u;
+                }
+            }
+            for (int o = 32; o > 0; o >>= 1) {
+                a += __shfl_xor(a, o, 64);
+                p += __shfl_xor(p, o, 64);
+                pI += __shfl_xor(pI, o, 64);
+            }
+            if (lane == 0) {
+                stot[row] = a;
+                spre[row] = p;
+                stotI[row] = pI;
+            }
+        }
+        __syncthreads();
+        if (t < P.W) {
+            uint32_t o = spre[t];
+            d.wpre[(size_t)t * d.swb + b] = o;
+            for (uint32_t i = 0; i < t; i++) o += stot[i];
+            base[t] = o;
+        }
+        if (t == GM_WMAX) {
+            d.rcnt[b] = d.wcnt[(size_t)GM_WMAX * d.swb + b];
+            d.rpre[b] = spre[P.W] - (b >= P.nbI ? stotI[P.W] : 0u);
+            d.rgone[b] = 0;
+            d.rmrg[b] = 0;
+        }
+        if (b == 0 && t == 64u) window_totals(d, P, stot, stotI[P.W], stot[P.W] - stotI[P.W], stotI);
+    } else if (t < P.W) {
+        base[t] = d.win->off[t] + d.wpre[(size_t)t * d.swb + b];
+    }
+    __syncthreads();
+    if (lane < P.W) {
+        uint32_t o = base[lane];
+        const uint32_t *ww = d.wwave + (size_t)b * GM_SW_WAVES * GM_WMAX + lane;
+        for (uint32_t q = 0; q < w; q++) o += ww[q * GM_WMAX];
+        run[w][lane] = o;
+    }
+    wave_sync();
+    const WaveChunks r = wave_chunks(d, P, b, w);
+    const uint32_t kc = k0 & (GM_CS_MOD - 1u), horizon = d.horizon;
+    for (uint32_t c = r.c0; c < r.c1; c++) {
+        uint32_t nocc;
+        const uint4 cs = chunk_codes(d, r, c, lane, nocc);
+        unsigned long long cnt = 0ull; /* 16 counters of 4 bits (at most 8 each) */
+        uint32_t full = 0, rec = 0;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const uint32_t x = code_at(cs, q);
+            const bool in = (uint32_t)q < nocc;
+            const uint32_t di = (x - kc) & (GM_CS_MOD - 1u);
+            const bool f = in && x < GM_CS_MOD && di < P.W;
+            cnt += f ? 1ull << (4u * (di & 15u)) : 0ull;
+            full |= f ? 1u << q : 0u;
+            rec |= in && cs_inactive(x, kc, horizon) ? 1u << q : 0u;
+        }
+        reinterpret_cast<uint8_t *>(sR[w])[lane] = (uint8_t)rec;
+        wave_sync();
+        if (lane < GM_SW_TPC) d.mR[r.tile0 + c * GM_SW_TPC + lane] = sR[w][lane];
+        if (!__any(full != 0u)) {
+            wave_sync();
+            continue;
+        }
+        uint32_t incl[GM_WMAX / 2];
+#pragma unroll
+        for (int i = 0; i < GM_WMAX / 2; i++) {
+            if (2u * i >= P.W) break;
+            const uint32_t f = (uint32_t)(cnt >> (8 * i));
+            const uint32_t v = (f & 0xFu) | (f & 0xF0u) << 12;
+            incl[i] = wave_incl_scan(v);
+            sl[w][lane][i] = incl[i] - v;
+        }
+        wave_sync();
+        uint16_t *mineRow = reinterpret_cast<uint16_t *>(sl[w][lane]);
+        const uint32_t slot = r.slot0 + c * GM_SW_CHUNK + 8u * lane;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            if (!((full >> q) & 1u)) continue;
+            const uint32_t di = (code_at(cs, q) - kc) & (GM_CS_MOD - 1u);
+            const uint32_t o = mineRow[di];
+            mineRow[di] = (uint16_t)(o + 1u);
+            d.pslot[run[w][di] + o] = slot + (uint32_t)q;
+        }
+        wave_sync();
+        if (lane == 63u) {
+#pragma unroll
+            for (int i = 0; i < GM_WMAX / 2; i++) {
+                if (2u * i >= P.W) break;
+                run[w][2 * i] += incl[i] & 0xFFFFu;
+                run[w][2 * i + 1] += incl[i] >> 16;
+            }
+        }
+        wave_sync();
+    }
+    if (!PROPOSE) return;
+    /* the first step's attempts by the blocks that list its parents */
+    const uint32_t nfull = stot[0], first = spre[0], cnt = d.wcnt[b];
+    GmStats *st = d.st;
+    const bool halt = must_halt_at(d, wd, nfull);
+    const unsigned long long nret = st->nret;
+    const bool logged = nret + nfull <= d.rlogCap;
+    if (b == 0 && t == 0) {
+        st->halt = halt ? 1u : 0u;
+        if (nfull > d.parentCap) st->need_par = nfull;
+        if (d.prog) __hip_atomic_store(d.prog, halt ? 1u : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (!halt && !logged) atomicOr(&st->err, GM_ERRF_RLOG_FULL);
+    }
+    if (halt) return;
+    __syncthreads();
+    uint32_t natt = 0;
+    for (uint32_t i = t; i < cnt; i += GM_BLOCK)
+        natt += propose_parent(d, d.pslot[first + i], first + i, k0, logged ? d.rlog + nret : nullptr);
+    for (int o = 32; o > 0; o >>= 1) natt += __shfl_xor(natt, o, 64);
+    if (lane == 0) run[w][0] = natt;
+    __syncthreads();
+    if (t == 0) d.acnt[b] = run[0][0] + run[1][0] + run[2][0] + run[3][0];
+}
+
+__global__ void k_arrivals(GmDev d, GmSweepArgs A);
+
+hipError_t gm_launch_window(const GmDev &d, const GmPart &P, const GmSweepArgs &a, const GmWindow &wd, bool arrivals,
+                            double xcells, hipStream_t s, hipEvent_t *ev) {
+    hipError_t e;
+    if ((e = mark(ev, 0, s)) != hipSuccess) return e;
+    if (a.reanchor && (e = gm_launch_reanchor(d, a, s)) != hipSuccess) return e;
+    if (arrivals) {
+        k_arrivals<<<1, 1024, 0, s>>>(d, a);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    if ((e = mark(ev, 1, s)) != hipSuccess) return e;
+    k_sweep<<<P.nb, GM_BLOCK, 0, s>>>(d, P, a.k, xcells, wd.top_pos);
+    if ((e = mark(ev, 2, s)) != hipSuccess) return e;
+    const bool fold = gm_fold(P);
+    if (!fold) k_sweep_scan<<<1, 1024, 0, s>>>(d, P);
+    if ((e = mark(ev, 3, s)) != hipSuccess) return e;
+    if (P.fused) k_compact<true, true><<<P.nb, GM_BLOCK, 0, s>>>(d, P, wd, a.k);
+    else if (fold) k_compact<true, false><<<P.nb, GM_BLOCK, 0, s>>>(d, P, wd, a.k);
+    else k_compact<false, false><<<P.nb, GM_BLOCK, 0, s>>>(d, P, wd, a.k);
+    return hipGetLastError();
 }
 
 /* exclusive prefix of v over the block (GM_BLOCK threads) and the total */
@@ -909,7 +946,7 @@ static __device__ void recycle_blocks(const GmDev &d, const GmPart &P, uint32_t 
     const uint32_t rp = (j & 1u) * d.swb, nt = GM_SW_WAVES * P.cpw * GM_SW_TPC;
     uint32_t *so = reinterpret_cast<uint32_t *>(sm + nt);
     const uint32_t recI = win->step[j].recLenI, recB = win->step[j].recLenB;
-    const uint32_t halt = d.st->halt;
+    const uint32_t halt = d.st->halt, nba = attempt_blocks(P, j);
     uint32_t na = 0, z0 = 0, z1 = 0;
     uint4 ac[2];
     static_assert(GM_PB <= 8 * GM_BLOCK, "one round of loads");
@@ -917,7 +954,7 @@ static __device__ void recycle_blocks(const GmDev &d, const GmPart &P, uint32_t 
     for (uint32_t i = 0; i < 2u; i++) {
         ac[i] = make_uint4(0u, 0u, 0u, 0u);
         const uint32_t at = 4u * (t + i * GM_BLOCK);
-        if (at < P.nbp) ac[i] = *reinterpret_cast<const uint4 *>(d.acnt + (j & 1u) * GM_PB + at);
+        if (at < nba) ac[i] = *reinterpret_cast<const uint4 *>(d.acnt + (j & 1u) * GM_PB + at);
     }
     for (uint32_t b = r; b < P.nb; b += nrec) {
         /* everything a block may need is loaded before its first use: its masks, what the
@@ -937,7 +974,7 @@ static __device__ void recycle_blocks(const GmDev &d, const GmPart &P, uint32_t 
 #pragma unroll
             for (uint32_t i = 0; i < 2u; i++) {
                 const uint32_t at = 4u * (t + i * GM_BLOCK);
-                na += ac[i].x + (at + 1u < P.nbp ? ac[i].y : 0u) + (at + 2u < P.nbp ? ac[i].z : 0u) + (at + 3u < P.nbp ? ac[i].w : 0u);
+                na += ac[i].x + (at + 1u < nba ? ac[i].y : 0u) + (at + 2u < nba ? ac[i].z : 0u) + (at + 3u < nba ? ac[i].w : 0u);
             }
             block_sum3(na, z0, z1, sn);
             if (halt) return;
@@ -1274,7 +1311,7 @@ hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepAr
                             const GmWindow &w, uint32_t j, GmStats *out, hipStream_t s, hipEvent_t *ev) {
     hipError_t e;
     if ((e = mark(ev, 4, s)) != hipSuccess) return e;
-    k_propose<<<P.nbp + 1u, GM_BLOCK, 0, s>>>(d, P, w, j, a.k + j);
+    if (j || !P.fused) k_propose<<<P.nbp + 1u, GM_BLOCK, 0, s>>>(d, P, w, j, a.k + j);
     if ((e = mark(ev, 5, s)) != hipSuccess) return e;
     const uint32_t nrec = P.nb < GM_RECYCLE_BLOCKS ? P.nb : GM_RECYCLE_BLOCKS;
     /* a sweep block's INACTIVE masks and the offsets of its tiles */

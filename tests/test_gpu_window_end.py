@@ -72,3 +72,24 @@ def test_one_step_windows_of_a_long_front(require_gpu):
     assert (tg["nslots_inside"] + tg["nslots_border"]).max() > 256 * 2048
     assert tg["npending"].max() > 2048 and ((tg["npending"] > 0) & (tg["npending"] <= 2048)).any()
     g.close()
+
+
+@pytest.mark.parametrize("nuclei", [64, 80000])
+def test_first_step_beyond_the_parents_entries(require_gpu, nuclei):
+    """More parents in the first step than there is room for at first (65536): the step
+    is run again with its own propose pass."""
+    dom = synth.make_voronoi_domain(64, 64, 64, n_grains=30, n_nuclei=nuclei, seed=3)
+    # strictly interior sites, all different: the Border list has little room
+    i = np.random.default_rng(1).choice(60 ** 3, nuclei, replace=False)
+    dom.rxg_site[:] = (i % 60 + 2) + 64 * (i // 60 % 60 + 2) + 4096 * (i // 3600 + 2)
+    prm = ParamsSpec(xmax=0.4 if nuclei > 64 else 0.9)
+    o, g = Oracle(dom, prm), GrowthMachine(dom, prm)
+    o.solve_rxgrowth()
+    g.solve_rxgrowth()
+    to, tg = o.trajectory(), g.trajectory()
+    assert same_trajectory(to, tg)
+    assert np.array_equal(o.grainmap(), g.grainmap())
+    for a, b in zip(o.counts(), g.counts()):
+        assert np.array_equal(a, b)
+    assert (tg["nfull_inside"][0] + tg["nfull_border"][0] > 65536) == (nuclei == 80000)
+    g.close()
