@@ -449,7 +449,7 @@ void free_device(score_gm_handle *h) {
                     d.scan_bsum, d.st, d.arr_ids, d.arr_off, d.nsite, d.nucP,
                     d.win, d.wcnt, d.wpre, d.wwave, d.rcnt, d.rpre, d.rgone, d.rmrg, d.acnt, d.btot, d.btop, d.ccnt, d.defsub, d.rorder, d.rpos,
                     d.reg, d.pmH, d.L.base, d.L.cap, d.L.rcap, d.L.rbase, d.L.n, d.L.nold, d.L.rlen,
-                    d.L.win, d.L.occ, d.L.tile, d.L.tile_s, d.L.par, d.L.rst, d.L.rbuf, d.L.rs, d.L.bstart, d.L.breg,
+                    d.L.occ, d.L.tile, d.L.tile_s, d.L.par, d.L.rst, d.L.rbuf, d.L.rs, d.L.bstart, d.L.breg,
                     d.L.hoff, d.plist};
     for (void *q : ptrs) dfree(h, q);
     if (h->arena) (void)hipFreeAsync(h->arena, h->stream);
@@ -1971,7 +1971,7 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
         (rc = dalloc(h, &d.pmB, d.parentCap)) || (rc = dalloc(h, &d.bcnt, GM_BCNT_ROWS * GM_MAX_BLOCKS)) ||
         (rc = dalloc(h, &d.rho, d.ndefg)) || (rc = dalloc(h, &d.defq, 4 * (size_t)d.ndefg)) ||
         (rc = dalloc(h, &d.rxq, 4 * (size_t)d.nrxg + 4)) || (rc = dalloc(h, &d.defcnt, d.ndefg)) ||
-        (rc = dalloc(h, &d.rxcnt, (size_t)d.nrxg + 1)) || (rc = dalloc(h, &d.win, 1)) || (rc = dalloc(h, &d.acnt, 2 * GM_PB)) ||
+        (rc = dalloc(h, &d.rxcnt, (size_t)d.nrxg + 1)) || (rc = dalloc(h, &d.win, 1)) ||
         (rc = dalloc(h, &d.defsub, (size_t)GM_SUBS * d.ndefg)) || (rc = dalloc(h, &d.rorder, d.ndefg)) ||
         (rc = dalloc(h, &d.rpos, d.ndefg)) ||
         (rc = dalloc(h, &d.hkeys, d.hcap)) ||
@@ -1990,7 +1990,7 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
             (rc = dalloc(h, &d.wpre, (size_t)(GM_WMAX + 1) * d.swb)) ||
             (rc = dalloc(h, &d.wwave, (size_t)GM_SW_WAVES * GM_WMAX * d.swb)) ||
             (rc = dalloc(h, &d.rcnt, 2 * (size_t)d.swb)) || (rc = dalloc(h, &d.rpre, 2 * (size_t)d.swb)) ||
-            (rc = dalloc(h, &d.rgone, d.swb)) || (rc = dalloc(h, &d.rmrg, d.swb)) ||
+            (rc = dalloc(h, &d.rgone, d.swb)) || (rc = dalloc(h, &d.rmrg, d.swb)) || (rc = dalloc(h, &d.acnt, 2 * GM_PB)) ||
             (rc = dalloc(h, &d.btot, GM_DB)) || (rc = dalloc(h, &d.ccnt, (size_t)d.parentCap / 16 + 1)) ||
             (rc = dalloc(h, &d.pmA, d.parentCap)) || (rc = dalloc(h, &d.btop, GM_DB)) ||
             (rc = dalloc(h, &d.gatt, (size_t)GM_GATT * d.gchunks))) {
@@ -2006,7 +2006,7 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
             (rc = dalloc(h, &d.L.breg, GM_MAX_BLOCKS)) ||
             (rc = dalloc(h, &d.L.base, L + 1)) || (rc = dalloc(h, &d.L.cap, L)) || (rc = dalloc(h, &d.L.rcap, L)) ||
             (rc = dalloc(h, &d.L.rbase, L + 1)) || (rc = dalloc(h, &d.L.n, L)) || (rc = dalloc(h, &d.L.nold, L)) ||
-            (rc = dalloc(h, &d.L.rlen, L)) || (rc = dalloc(h, &d.L.win, L)) || (rc = dalloc(h, &d.L.occ, L + 1)) ||
+            (rc = dalloc(h, &d.L.rlen, L)) || (rc = dalloc(h, &d.L.occ, L + 1)) ||
             (rc = dalloc(h, &d.L.tile, L + 1)) || (rc = dalloc(h, &d.L.tile_s, L + 1)) ||
             (rc = dalloc(h, &d.L.par, L + 1)) || (rc = dalloc(h, &d.L.rst, L + 1)) ||
             (rc = dalloc(h, &d.L.rbuf, h->lrbase[L])) || (rc = dalloc(h, &d.L.rs, (size_t)(d.nreg + 1) * GM_RROWS)) ||
@@ -2446,7 +2446,7 @@ int score_gm_footprint(const score_gm_domain *dom, const score_gm_params *prm, u
     if (prm->n_regions <= 1) {
         /* the window sweep's tables */
         const uint64_t rows = std::max<uint64_t>(capTot / (GM_SW_CHUNK * GM_SW_WAVES * GM_SW_MAXCPW) + 67, GM_SW_BLOCKS);
-        b += 4 * rows * (2 * (GM_WMAX + 1) + GM_SW_WAVES * GM_WMAX + 6) + 8 * GM_PB + 4 * (front + front / 16) +
+        b += 4 * rows * (2 * (GM_WMAX + 1) + GM_SW_WAVES * GM_WMAX + 6) + 16 * GM_PB + 4 * (front + front / 16) +
              4ull * GM_GATT * std::min<uint64_t>(GM_GCHUNKS, N / 16 + 1);
     }
     if (prm->n_regions > 1) {
@@ -2466,7 +2466,8 @@ int score_gm_footprint(const score_gm_domain *dom, const score_gm_params *prm, u
                         (uint64_t)((double)cb * prm->maxfill * kFullRecyclingAtt);
             }
         b += 8 * (capTot / 64 + GM_SW_TPC); /* completed masks */
-        b += 4 * front + (sizeof(GmRegion) + 4ull * (GM_RROWS + GM_NHALO + 26)) * (T + 1) + 16ull * GM_SW_TPC * 2 * T;
+        b += 4 * front + (sizeof(GmRegion) + 4ull * (GM_RROWS + GM_NHALO + 26)) * (T + 1) + 16ull * GM_SW_TPC * 2 * T +
+             16ull * GM_MAX_BLOCKS;
     }
     b += 8 * N;                                   /* cells */
     b += 8 * (N + capB + 4096);                   /* retirement log */
@@ -2477,7 +2478,7 @@ int score_gm_footprint(const score_gm_domain *dom, const score_gm_params *prm, u
     b += 8 * (capTot / 64 + GM_SW_TPC);           /* tile masks */
     b += 4 * rbuf;                                /* recycled slots */
     b += 4 * GM_BCNT_ROWS * GM_MAX_BLOCKS;
-    b += sizeof(GmWin) + 8 * GM_PB + (4ull * GM_SUBS + 8) * dom->n_defg; /* counts in parts, order of rho */
+    b += sizeof(GmWin) + (4ull * GM_SUBS + 8) * dom->n_defg; /* counts in parts, order of rho */
     b += 52ull * dom->n_defg + 52ull * (dom->n_rxg + 1);
     if (dom->rxg_step) b += 20ull * dom->n_rxg;   /* arrivals: ids, sites, weights */
     b += 28 * hcap;                               /* weight cache: keys, values, pending slots and keys */

@@ -208,7 +208,7 @@ struct alignas(8) GmStats {
     uint32_t dfirst;          /* defragmentation: first INACTIVE slot of the list */
     uint32_t dcount;          /* defragmentation: ACTIVE slots moved; status vector: entries */
     uint32_t novf;            /* weight lookups that found the cache full (their cells wait for a larger table) */
-    uint32_t rg_per;          /* with several regions: parents per block of the infection passes */
+    uint32_t ntried;          /* with several regions: the step's attempts on deformed cells, before they are decided */
     uint32_t nplaced;         /* nuclei placed at the start of the current step */
     unsigned long long arr_pkey; /* largest weight of those nuclei (gm_pkey order) */
     unsigned long long nret;  /* entries of the retirement log (cells retired so far) */
@@ -313,7 +313,6 @@ struct GmLists {
     uint32_t *n;                /* nextSlotNeverActive */
     uint32_t *nold;             /* the same before the current step's appends */
     uint32_t *rlen;             /* recycled slots that may be handed out this step */
-    uint32_t *win;              /* this step's new records into each list */
     uint32_t *occ;              /* exclusive prefix of n: occupied slot i lies in list l iff occ[l] <= i < occ[l+1] */
     uint32_t *tile;             /* exclusive prefix of the sweep's tiles per list (whole 8-tile chunks) */
     uint32_t *tile_s;           /* the same as the current step's sweep saw it (tile moves on with the lengths) */
@@ -322,7 +321,7 @@ struct GmLists {
     uint32_t *rbuf;             /* recycled slots (list-relative), ascending per list */
     uint32_t *rs;               /* per region r (and r = T: totals), GM_RROWS prefix counts at its first parent */
     uint32_t *bstart;           /* first block of each region in the infection passes (nreg+1: blocks in use) */
-    uint32_t *breg;             /* region of each block of the infection passes (GM_MAX_BLOCKS; ~0u past those in use) */
+    uint4 *breg;                /* each block of the infection passes (GM_MAX_BLOCKS): its parents [x, y) and region z */
     uint32_t *hoff;             /* per region, GM_NHALO offsets of the halo winners in its Border list */
 };
 
@@ -368,7 +367,7 @@ struct GmDev {
     uint32_t *wwave;            /* GM_WMAX counts per wave of each block */
     uint32_t *rcnt, *rpre;      /* INACTIVE slots of each block and before it in its list; two rows, by the step's parity */
     uint32_t *rgone, *rmrg;     /* slots the step before handed out; steps whose completed cells are in the block's masks */
-    uint32_t *acnt;             /* attempts per propose block, two rows by the step's parity (several regions: one) */
+    uint32_t *acnt;             /* attempts per propose block, two rows by the step's parity */
     uint2 *btot;                /* winners into Inside, Border per decide block */
     uint32_t *btop;             /* parents per decide block in the grain that sets rhomax */
     uint32_t *ccnt;             /* the same per chunk of parents, Inside << 16 | Border */

@@ -36,12 +36,12 @@
  * count is the offset of the region's first block.
  *
  * At 160^3 in eight regions (477 steps of 8500 parents) a step of these passes went
- * from 135 to 67 us: propose 25 to 10, decide with the retirement and the recycled
+ * from 135 to 63 us: compaction and propose pass 30 to 11, decide with the retirement and the recycled
  * slots 28 to 9.5, commit with the step's end 29 to 17, the two scans 27 to 14.5.
  *
  * Per step, in the profiling slots of the one-region kernels:
  *   k_reanchor (shared)   k_rg_sweep   k_rg_sweep_scan (+ per-list starts)
- *   k_rg_compact   k_rg_propose   k_rg_decide (+ recycled slots)
+ *   k_rg_compact (+ the propose pass)   k_rg_decide (+ recycled slots)
  *   k_rg_decide_scan (+ per-region starts, list lengths)   k_rg_commit (+ the step's end)
  */
 #include <algorithm>
@@ -120,15 +120,13 @@ static uint32_t rg_infect_blocks(const GmDev &d, uint32_t parents_upper) {
 }
 
 /* The parents of infection-pass block b: blocks are handed out region by region
- * (L.bstart[r] is region r's first block, st->rg_per parents each), so a block
- * holds one region's parents only; r is that region. */
+ * (L.bstart[r] is region r's first block), so a block holds one region's parents
+ * only; r is that region (k_rg_sweep_scan; past the blocks in use: none). */
 static __device__ __forceinline__ void rg_part(const GmDev &d, uint32_t b, uint32_t &lo, uint32_t &hi, uint32_t &r) {
-    lo = hi = r = 0;
-    r = d.L.breg[b];
-    if (r >= d.nreg) return; /* a block past the ones in use */
-    const uint32_t per = d.st->rg_per, end = d.L.par[2u * r + 2u];
-    lo = d.L.par[2u * r] + (b - d.L.bstart[r]) * per;
-    hi = lo + per < end ? lo + per : end;
+    const uint4 v = d.L.breg[b];
+    lo = v.x;
+    hi = v.y;
+    r = v.z;
 }
 
 /* sweep tiles of a list of n occupied slots: whole 8-tile chunks */
@@ -238,12 +236,12 @@ static __device__ __forceinline__ bool rg_target(const GmDev &d, const RgBox &B,
 
 /* One block of 1024 threads: the lists' occupied and tile prefixes from their
  * lengths, and the lengths summed over Inside and Border lists; thread t takes
- * region t's two lists (at most 1024 regions). */
-static __device__ void rg_prefix_block(const GmDev &d) {
+ * region t's two lists, of lengths nI and nB (at most 1024 regions). */
+static __device__ __forceinline__ void rg_prefix_block(const GmDev &d, uint32_t nI, uint32_t nB) {
     __shared__ uint32_t ws[16][4];
     const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
     const bool v = t < d.nreg;
-    const uint32_t nI = v ? d.L.n[2u * t] : 0u, nB = v ? d.L.n[2u * t + 1u] : 0u;
+    if (!v) nI = nB = 0;
     const uint32_t tI = list_tiles(nI), tB = list_tiles(nB);
     const uint32_t val[4] = {nI + nB, tI + tB, nI, nB};
     uint32_t incl[4];
@@ -276,7 +274,10 @@ static __device__ void rg_prefix_block(const GmDev &d) {
     __syncthreads();
 }
 
-__global__ void __launch_bounds__(1024) k_rg_prefix(GmDev d) { rg_prefix_block(d); }
+__global__ void __launch_bounds__(1024) k_rg_prefix(GmDev d) {
+    const uint32_t t = threadIdx.x < d.nreg ? threadIdx.x : 0u;
+    rg_prefix_block(d, d.L.n[2u * t], d.L.n[2u * t + 1u]);
+}
 
 hipError_t gm_launch_rg_prefix(const GmDev &d, hipStream_t s) {
     k_rg_prefix<<<1, 1024, 0, s>>>(d);
@@ -371,7 +372,11 @@ __global__ void __launch_bounds__(1024) k_rg_sweep_scan(GmDev d, uint32_t nb, ui
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
     if (threadIdx.x < 6) acc[threadIdx.x] = 0;
     /* one wave per list, the lanes sharing the block's tiles before the list's first */
-    for (uint32_t l = wv; l <= d.nlists; l += 1024u / 64u) {
+    if (threadIdx.x == 0) {
+        d.L.tile_s[d.nlists] = T;
+        sF[d.nlists] = sR[d.nlists] = 0;
+    }
+    for (uint32_t l = wv; l < d.nlists; l += 1024u / 64u) {
         const uint32_t t0 = d.L.tile[l];
         uint32_t ef = 0, er = 0;
         if (t0 < T)
@@ -416,7 +421,7 @@ __global__ void __launch_bounds__(1024) k_rg_sweep_scan(GmDev d, uint32_t nb, ui
 #pragma unroll
     for (int c = 0; c < 6; c++)
         if (a[c]) atomicAdd(&acc[c], a[c]);
-    /* the infection passes' blocks, region by region: rg_per parents each (a
+    /* the infection passes' blocks, region by region: pper parents each (a
      * multiple of GM_PCHUNK), few enough that all regions fit in nbd blocks */
     const uint32_t nfull = tot[RS_F];
     uint32_t pper = (nfull + (nbd - d.nreg) - 1u) / (nbd - d.nreg);
@@ -435,11 +440,17 @@ __global__ void __launch_bounds__(1024) k_rg_sweep_scan(GmDev d, uint32_t nb, ui
     if (r < d.nreg) d.L.bstart[r] = sS[r] = pre + incl - blk;
     if (threadIdx.x == 0) d.L.bstart[d.nreg] = sS[d.nreg] = totb;
     __syncthreads();
-    /* each block's region; blocks past the ones in use find none */
-    for (uint32_t b = threadIdx.x; b < nbd; b += 1024)
-        d.L.breg[b] = b < totb ? upper_index(sS, d.nreg, b) : 0xFFFFFFFFu;
+    /* each block's parents and region; blocks past the ones in use have none */
+    for (uint32_t b = threadIdx.x; b < nbd; b += 1024) {
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (b < totb) {
+            const uint32_t q = upper_index(sS, d.nreg, b), lo = sF[2u * q] + (b - sS[q]) * pper, end = sF[2u * q + 2u];
+            v = make_uint4(lo, lo + pper < end ? lo + pper : end, q, 0u);
+        }
+        d.L.breg[b] = v;
+    }
     if (threadIdx.x == 0) {
-        st->rg_per = pper;
+        st->ntried = 0;
         st->nfullI = acc[0];
         st->totRecI = acc[1];
         st->recLenI = acc[2];
@@ -449,32 +460,105 @@ __global__ void __launch_bounds__(1024) k_rg_sweep_scan(GmDev d, uint32_t nb, ui
     }
 }
 
-/* One wave per sweep block, one lane per tile: the completed slots in FullRX
- * order (append_to_fullrx_*_list, SCORE_Kernel.cpp:3994-4042, :4133-4180), the
- * lists one after another. */
-__global__ void __launch_bounds__(64) k_rg_compact(GmDev d) {
-    if (d.st->halt) return;
-    const uint32_t lane = threadIdx.x;
-    const uint32_t T = d.L.tile[d.nlists];
+struct RgWave {
+    uint4 q2[64];
+    uint32_t bad[64];
+    uint16_t wl[26 * 64];
+};
+
+/* Parents p0 .. p0+n-1 (n <= 64) by a wave, a lane each, as the one-region propose
+ * pass: the parent's data into the dense array (with its list in place of the Border
+ * flag), its value after the completing addition, its retirement into the log (rlog;
+ * null: it does not fit); its deformed neighbours come from three 16-byte loads of the
+ * bitmap.  Every attempt on one of them, routed to the region it lies in, claims it:
+ * the parents' attempts are flattened into a list, a lane per attempt, so that a wave
+ * waits for its attempts' halos at once.  Returns the attempts. */
+static __device__ __forceinline__ uint32_t rg_propose(const GmDev &d, RgWave &W, uint32_t p0, uint32_t n, uint32_t k,
+                                                      uint2 *rlog) {
+    const uint32_t lane = threadIdx.x & 63u, p = p0 + lane;
+    uint32_t am = 0;
+    if (lane < n) {
+        const uint32_t s = d.pslot[p], l = d.plist[p];
+        const GmRec *r = d.rec + s;
+        const RecC rc = rec_c(r);
+        const RecA ra = rec_a(r);
+        const double inc = r->inc;
+        const uint32_t rxg = r->rxg, cell = rc.cell;
+        const uint32_t z = cell / d.nxy, rem = cell - z * d.nxy, y = rem / d.nx, x = rem - y * d.nx;
+        const bool interior = (x - 1u < d.nx - 2u) & (y - 1u < d.ny - 2u) & (z - 1u < d.nz - 2u);
+        Neighbourhood nb;
+        if (interior) nb.load(d, x, y, z);
+        const double fin = advanced(ra.frac0, inc, k - ra.s0 + 1u);
+        am = interior ? nb.mask() : face_attempts(d, x, y, z);
+        const uint4 q2 = make_uint4(x, y, z, l);
+        W.q2[lane] = q2;
+        par_plane(d, GM_PAR_IDS)[p] = make_uint4(s, cell, rc.defg, rxg);
+        reinterpret_cast<double2 *>(par_plane(d, GM_PAR_FP))[p] = make_double2(fin, rc.P);
+        par_plane(d, GM_PAR_XYZ)[p] = q2;
+        if (rlog) rlog[p] = make_uint2(cell, d.ndefg + rxg);
+    }
+    W.bad[lane] = 0;
+    const uint32_t na = list_attempts(am, W.wl);
+    for (uint32_t i = lane; i < na; i += 64u) {
+        const uint32_t e = W.wl[i], q = e & 0xFFu, rk = e >> 8;
+        const uint4 q2 = W.q2[q];
+        RgTarget o;
+        if (rg_target(d, rg_box(d, q2.w >> 1), q2.w, q2.x, q2.y, q2.z, (int)rk, o))
+            atomicMin(&d.cell[cell_of(d, o.x, o.y, o.z)].x, o.khi | ((p0 + q) * 32u + rk));
+        else
+            atomicOr(&W.bad[q], 1u << rk);
+    }
+    wave_sync();
+    if (lane < n) d.pmI[p] = am & ~W.bad[lane];
+    wave_sync();
+    return na;
+}
+
+/* The sweep's partition: a block's first wave, one lane per tile, lists its completed
+ * slots in FullRX order (append_to_fullrx_*_list, SCORE_Kernel.cpp:3994-4042,
+ * :4133-4180), the lists one after another; then all its waves take these parents
+ * through the propose pass, which in a launch of its own read them back (5 us a step). */
+__global__ void __launch_bounds__(GM_BLOCK) k_rg_compact(GmDev d) {
+    __shared__ RgWave sw[GM_BLOCK / 64];
+    __shared__ uint32_t send, satt[GM_BLOCK / 64];
+    GmStats *st = d.st;
+    if (st->halt) return;
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    const uint32_t T = d.L.tile[d.nlists], nfull = st->nfullI + st->nfullB, k = st->kcur;
+    const unsigned long long nret = st->nret;
     uint32_t lo, hi;
     part_of(T, GM_SW_TPC, lo, hi);
-    uint32_t runF = d.bcnt[RS_F * GM_MAX_BLOCKS + blockIdx.x];
-    for (uint32_t batch = lo; batch < hi; batch += 64) {
-        const uint32_t t = batch + lane;
-        const uint64_t bf = t < hi ? d.mF[t] : 0ull;
-        const uint32_t cf = (uint32_t)__popcll(bf);
-        const uint32_t incf = wave_incl_scan(cf);
-        uint32_t of = runF + incf - cf;
-        runF += __shfl(incf, 63, 64);
-        if (bf) {
-            const uint32_t l = upper_index(d.L.tile, d.nlists, t);
-            const uint32_t s0 = d.L.base[l] + (t - d.L.tile[l]) * 64u;
-            for (uint64_t m = bf; m; m &= m - 1ull) {
-                d.plist[of] = l;
-                d.pslot[of++] = s0 + (uint32_t)__ffsll((long long)m) - 1u;
+    const uint32_t first = d.bcnt[RS_F * GM_MAX_BLOCKS + blockIdx.x];
+    const bool logged = nret + nfull <= d.rlogCap;
+    if (!logged && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&st->err, GM_ERRF_RLOG_FULL);
+    if (w == 0) {
+        uint32_t runF = first;
+        for (uint32_t batch = lo; batch < hi; batch += 64) {
+            const uint32_t t = batch + lane;
+            const uint64_t bf = t < hi ? d.mF[t] : 0ull;
+            const uint32_t cf = (uint32_t)__popcll(bf);
+            const uint32_t incf = wave_incl_scan(cf);
+            uint32_t of = runF + incf - cf;
+            runF += __shfl(incf, 63, 64);
+            if (bf) {
+                const uint32_t l = upper_index(d.L.tile, d.nlists, t);
+                const uint32_t s0 = d.L.base[l] + (t - d.L.tile[l]) * 64u;
+                for (uint64_t m = bf; m; m &= m - 1ull) {
+                    d.plist[of] = l;
+                    d.pslot[of++] = s0 + (uint32_t)__ffsll((long long)m) - 1u;
+                }
             }
         }
+        if (lane == 0) send = runF;
     }
+    __syncthreads();
+    uint32_t natt = 0;
+    for (uint32_t p = first + w * 64u; p < send; p += GM_BLOCK)
+        natt += rg_propose(d, sw[w], p, send - p < 64u ? send - p : 64u, k, logged ? d.rlog + nret : nullptr);
+    if (lane == 0) satt[w] = natt;
+    __syncthreads();
+    natt = satt[0] + satt[1] + satt[2] + satt[3];
+    if (threadIdx.x == 0 && natt) atomicAdd(&st->ntried, natt);
 }
 
 /* Each list's INACTIVE slots in ascending order (append_to_recycling_*_list,
@@ -482,13 +566,12 @@ __global__ void __launch_bounds__(64) k_rg_compact(GmDev d) {
  * the recycled slots, and no more than the step's attempts.  Runs beside the decide
  * pass, before the new records per list are known (a pass of its own after that took
  * 5 us and a gap).  The sweep's partition and offsets; one wave per sweep block. */
-static __device__ __forceinline__ void rg_recycle(const GmDev &d, uint32_t blk, uint32_t nblk, uint32_t nbp) {
+static __device__ __forceinline__ void rg_recycle(const GmDev &d, uint32_t blk, uint32_t nblk) {
     const uint32_t lane = threadIdx.x, T = d.L.tile_s[d.nlists], per = part_per(T, nblk, GM_SW_TPC);
-    uint32_t lo = blk * per, hi = lo + per, na = 0;
+    uint32_t lo = blk * per, hi = lo + per;
+    const uint32_t na = d.st->ntried;
     if (lo > T) lo = T;
     if (hi > T) hi = T;
-    for (uint32_t i = lane; i < nbp; i += 64u) na += d.acnt[i];
-    for (int o = 32; o > 0; o >>= 1) na += (uint32_t)__shfl_xor((int)na, o, 64);
     uint32_t runR = d.bcnt[RS_R * GM_MAX_BLOCKS + blk];
     for (uint32_t batch = lo; batch < hi; batch += 64) {
         const uint32_t t = batch + lane;
@@ -529,77 +612,11 @@ hipError_t gm_launch_rg_sweep(const GmDev &d, const GmSweepArgs &a, uint32_t par
     if ((e = mark(ev, 2, s)) != hipSuccess) return e;
     k_rg_sweep_scan<<<1, 1024, 0, s>>>(d, nb, rg_infect_blocks(d, parents_upper));
     if ((e = mark(ev, 3, s)) != hipSuccess) return e;
-    k_rg_compact<<<nb, 64, 0, s>>>(d);
+    k_rg_compact<<<nb, GM_BLOCK, 0, s>>>(d);
     return hipGetLastError();
 }
 
 /* --------------------------------------------------------------- infection */
-
-/* One lane per parent, as the one-region propose pass: the parent's data into the
- * dense array (with its list in place of the Border flag), its value after the
- * completing addition, its retirement into the log; its deformed neighbours come from
- * three 16-byte loads of the bitmap.  Every attempt on one of them, routed to the
- * region it lies in, claims it: 64 parents' attempts are flattened into a list, a
- * lane per attempt, so that a wave waits for its attempts' halos at once. */
-__global__ void __launch_bounds__(GM_BLOCK) k_rg_propose(GmDev d) {
-    struct Wave {
-        uint4 q2[64];
-        uint32_t bad[64];
-        uint16_t wl[26 * 64];
-    };
-    __shared__ Wave sw[GM_BLOCK / 64];
-    __shared__ uint32_t satt[GM_BLOCK / 64];
-    if (d.st->halt) return;
-    const uint32_t nfull = d.st->nfullI + d.st->nfullB, k = d.st->kcur;
-    const unsigned long long nret = d.st->nret;
-    const bool logged = nret + nfull <= d.rlogCap;
-    if (!logged && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&d.st->err, GM_ERRF_RLOG_FULL);
-    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-    Wave &W = sw[w];
-    uint32_t natt = 0;
-    for (uint32_t c = w * gridDim.x + blockIdx.x; c * 64u < nfull; c += gridDim.x * (GM_BLOCK / 64u)) {
-        const uint32_t p = c * 64u + lane;
-        uint32_t am = 0;
-        if (p < nfull) {
-            const uint32_t s = d.pslot[p], l = d.plist[p];
-            const GmRec *r = d.rec + s;
-            const RecC rc = rec_c(r);
-            const RecA ra = rec_a(r);
-            const double inc = r->inc;
-            const uint32_t rxg = r->rxg, cell = rc.cell;
-            const uint32_t z = cell / d.nxy, rem = cell - z * d.nxy, y = rem / d.nx, x = rem - y * d.nx;
-            const bool interior = (x - 1u < d.nx - 2u) & (y - 1u < d.ny - 2u) & (z - 1u < d.nz - 2u);
-            Neighbourhood nb;
-            if (interior) nb.load(d, x, y, z);
-            const double fin = advanced(ra.frac0, inc, k - ra.s0 + 1u);
-            am = interior ? nb.mask() : face_attempts(d, x, y, z);
-            const uint4 q2 = make_uint4(x, y, z, l);
-            W.q2[lane] = q2;
-            par_plane(d, GM_PAR_IDS)[p] = make_uint4(s, cell, rc.defg, rxg);
-            reinterpret_cast<double2 *>(par_plane(d, GM_PAR_FP))[p] = make_double2(fin, rc.P);
-            par_plane(d, GM_PAR_XYZ)[p] = q2;
-            if (logged) d.rlog[nret + p] = make_uint2(cell, d.ndefg + rxg);
-        }
-        W.bad[lane] = 0;
-        const uint32_t n = list_attempts(am, W.wl);
-        natt += n;
-        for (uint32_t i = lane; i < n; i += 64u) {
-            const uint32_t e = W.wl[i], q = e & 0xFFu, rk = e >> 8;
-            const uint4 q2 = W.q2[q];
-            RgTarget o;
-            if (rg_target(d, rg_box(d, q2.w >> 1), q2.w, q2.x, q2.y, q2.z, (int)rk, o))
-                atomicMin(&d.cell[cell_of(d, o.x, o.y, o.z)].x, o.khi | ((c * 64u + q) * 32u + rk));
-            else
-                atomicOr(&W.bad[q], 1u << rk);
-        }
-        wave_sync();
-        if (p < nfull) d.pmI[p] = am & ~W.bad[lane];
-        wave_sync();
-    }
-    if (lane == 0) satt[w] = natt;
-    __syncthreads();
-    if (threadIdx.x == 0) d.acnt[blockIdx.x] = satt[0] + satt[1] + satt[2] + satt[3];
-}
 
 /* The attempts that hold their target's smallest key, as masks by destination (own
  * Inside, own Border, a halo), counted per block by row (GM_RW_*).  64 parents'
@@ -607,13 +624,13 @@ __global__ void __launch_bounds__(GM_BLOCK) k_rg_propose(GmDev d) {
  * loaded together.  The parents retire here, beside the waiting for the claims.  The
  * partition into blocks (one region per block) is the commit pass's.  The launch's
  * first nrec blocks write the recycled slots. */
-__global__ void __launch_bounds__(64) k_rg_decide(GmDev d, uint32_t nrec, uint32_t nbp, uint32_t top_pos) {
+__global__ void __launch_bounds__(64) k_rg_decide(GmDev d, uint32_t nrec, uint32_t top_pos) {
     __shared__ uint4 sq2[64];
     __shared__ uint32_t sI[64], sB[64], sH[64], scnt[GM_RROWS];
     __shared__ uint16_t wl[26 * 64];
     if (d.st->halt) return;
     if (blockIdx.x < nrec) {
-        rg_recycle(d, blockIdx.x, nrec, nbp);
+        rg_recycle(d, blockIdx.x, nrec);
         return;
     }
     const uint32_t lane = threadIdx.x, blk = blockIdx.x - nrec;
@@ -680,71 +697,68 @@ __global__ void __launch_bounds__(64) k_rg_decide(GmDev d, uint32_t nrec, uint32
  * Border list (after its own winners, in its neighbour order: the infecting
  * region S = nbor[nb] parked them in its halo opp(nb)); the new records per
  * list, the lists' new lengths (recycled slots first, then appended) and their
- * prefixes for the next step. */
+ * prefixes for the next step.  A thread has a region: what it needs of the tables is
+ * loaded beside the scan, and the regions' counts go through LDS (at most
+ * 1025 x 11 of them). */
 __global__ void __launch_bounds__(1024) k_rg_decide_scan(GmDev d, uint32_t nb) {
-    __shared__ uint32_t acc[2];
+    __shared__ uint32_t acc[2], tot[GM_RROWS + 1], srs[(1024 + 1) * GM_RROWS];
     GmStats *st = d.st;
-    if (st->halt) return;
-    /* only the blocks in use hold counts */
-    const uint32_t nused = d.L.bstart[d.nreg];
-    __shared__ uint32_t tot[GM_RROWS + 1];
-    scan_rows(d.bcnt + RW_ROW0 * GM_MAX_BLOCKS, GM_RROWS + 1, nused < nb ? nused : nb, tot);
-    if (threadIdx.x < 2) acc[threadIdx.x] = 0;
-    if (threadIdx.x == 0) {
+    const uint32_t q = threadIdx.x, r = q < d.nreg ? q : 0u;
+    const uint32_t halt = st->halt, nused = d.L.bstart[d.nreg], b = d.L.bstart[r];
+    const uint32_t oI = d.L.n[2u * r], oB = d.L.n[2u * r + 1u], rlI = d.L.rlen[2u * r], rlB = d.L.rlen[2u * r + 1u];
+    const uint32_t left0 = d.win->left[0];
+    uint32_t S[GM_NHALO];
+#pragma unroll
+    for (uint32_t j = 0; j < GM_NHALO; j++) S[j] = d.reg[r].nbor[c_hdir[j]];
+    if (halt) return;
+    /* (blocks past the ones in use counted nothing) */
+    scan_rows(d.bcnt + RW_ROW0 * GM_MAX_BLOCKS, GM_RROWS + 1, nb, tot);
+    if (q < 2) acc[q] = 0;
+    if (q == 0) {
         st->nattempt = tot[GM_RW_A];
         if (tot[GM_RROWS]) { /* the cells left of the grain that sets rhomax */
-            const uint32_t left = d.win->left[0] - tot[GM_RROWS];
+            const uint32_t left = left0 - tot[GM_RROWS];
             d.win->left[0] = left;
             if (left == 0u) d.win->top_hit = 1u;
         }
     }
     /* each region's counts at its first parent: the offset of its first block
      * (the next region's, or the totals, for a region without parents) */
-    for (uint32_t r = threadIdx.x; r <= d.nreg; r += 1024) {
-        const uint32_t b = d.L.bstart[r];
+    if (q < d.nreg) {
+        uint32_t v[GM_RROWS];
 #pragma unroll
-        for (int c = 0; c < GM_RROWS; c++)
-            d.L.rs[r * GM_RROWS + c] = b < nused ? d.bcnt[(RW_ROW0 + c) * GM_MAX_BLOCKS + b] : tot[c];
+        for (int c = 0; c < GM_RROWS; c++) v[c] = b < nused ? d.bcnt[(RW_ROW0 + c) * GM_MAX_BLOCKS + b] : tot[c];
+#pragma unroll
+        for (int c = 0; c < GM_RROWS; c++) d.L.rs[q * GM_RROWS + c] = srs[q * GM_RROWS + c] = v[c];
     }
+    if (q < GM_RROWS) d.L.rs[d.nreg * GM_RROWS + q] = srs[d.nreg * GM_RROWS + q] = tot[q];
     __syncthreads();
-    for (uint32_t q = threadIdx.x; q < d.nreg; q += 1024) {
-        /* every load first (the stores below could alias them), then the prefix */
-        const uint32_t *a = d.L.rs + q * GM_RROWS, *b = a + GM_RROWS;
-        const uint32_t dI = b[GM_RW_I] - a[GM_RW_I], dB = b[GM_RW_B] - a[GM_RW_B];
-        uint32_t S[GM_NHALO], cnt[GM_NHALO];
-#pragma unroll
-        for (uint32_t j = 0; j < GM_NHALO; j++) S[j] = d.reg[q].nbor[c_hdir[j]];
+    uint32_t nI = 0, nB = 0, wI = 0, wB = 0;
+    if (q < d.nreg) {
+        const uint32_t *a = srs + q * GM_RROWS, *e = a + GM_RROWS;
+        wI = e[GM_RW_I] - a[GM_RW_I];
+        wB = e[GM_RW_B] - a[GM_RW_B];
 #pragma unroll
         for (uint32_t j = 0; j < GM_NHALO; j++) {
             const uint32_t hs = GM_RW_H0 + c_hidx[c_opp[c_hdir[j]]];
-            cnt[j] = S[j] != q ? d.L.rs[(S[j] + 1u) * GM_RROWS + hs] - d.L.rs[S[j] * GM_RROWS + hs] : 0u;
+            d.L.hoff[q * GM_NHALO + j] = wB;
+            if (S[j] != q) wB += srs[(S[j] + 1u) * GM_RROWS + hs] - srs[S[j] * GM_RROWS + hs];
         }
-        uint32_t run = dB;
-#pragma unroll
-        for (uint32_t j = 0; j < GM_NHALO; j++) {
-            d.L.hoff[q * GM_NHALO + j] = run;
-            run += cnt[j];
-        }
-        d.L.win[2u * q] = dI;
-        d.L.win[2u * q + 1u] = run;
-    }
-    __syncthreads();
-    uint32_t wI = 0, wB = 0;
-    for (uint32_t l = threadIdx.x; l < d.nlists; l += 1024) {
-        const uint32_t n = d.L.n[l], w = d.L.win[l], rl = d.L.rlen[l];
-        d.L.nold[l] = n;
-        d.L.n[l] = w > rl ? n + (w - rl) : n;
-        if (l & 1u) wB += w;
-        else wI += w;
+        nI = wI > rlI ? oI + (wI - rlI) : oI;
+        nB = wB > rlB ? oB + (wB - rlB) : oB;
+        d.L.nold[2u * q] = oI;
+        d.L.nold[2u * q + 1u] = oB;
+        d.L.n[2u * q] = nI;
+        d.L.n[2u * q + 1u] = nB;
     }
     if (wI) atomicAdd(&acc[0], wI);
     if (wB) atomicAdd(&acc[1], wB);
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (q == 0) {
         st->winI = acc[0];
         st->winB = acc[1];
     }
-    rg_prefix_block(d);
+    rg_prefix_block(d, nI, nB);
 }
 
 /* New records as the one-region commit pass writes them;
@@ -898,11 +912,9 @@ hipError_t gm_launch_rg_infect(const GmDev &d, const GmPParams &pp, const GmSwee
                                const GmWindow &w, GmStats *out, hipStream_t s, hipEvent_t *ev) {
     hipError_t e;
     if ((e = mark(ev, 4, s)) != hipSuccess) return e;
-    const uint32_t nbp = std::min(GM_PB, grid_for(parents_upper, 64u));
-    k_rg_propose<<<nbp, GM_BLOCK, 0, s>>>(d);
     const uint32_t nb = rg_infect_blocks(d, parents_upper), nrec = rg_sweep_blocks(d, a);
     if ((e = mark(ev, 5, s)) != hipSuccess) return e;
-    k_rg_decide<<<nrec + nb, 64, 0, s>>>(d, nrec, nbp, w.top_pos);
+    k_rg_decide<<<nrec + nb, 64, 0, s>>>(d, nrec, w.top_pos);
     if ((e = mark(ev, 6, s)) != hipSuccess) return e;
     k_rg_decide_scan<<<1, 1024, 0, s>>>(d, nb);
     if ((e = mark(ev, 7, s)) != hipSuccess || (e = mark(ev, 8, s)) != hipSuccess) return e;
