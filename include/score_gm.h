@@ -199,10 +199,10 @@ typedef struct score_gm_result {
     double loop_seconds;          /* host wall time spent inside step/run calls */
 } score_gm_result;
 
-/* Kernels of one growth step, in launch order (index into ms_kernel).  With one
- * region DECIDE includes the recycled slots and the ranking needs no scan of its
- * own, so DECIDE_SCAN and RECYCLE stay near 0, and so does SWEEP_SCAN on fronts of
- * up to 2^19 slots. */
+/* Kernels of one growth step, in launch order (index into ms_kernel).  DECIDE
+ * includes the recycled slots, so RECYCLE stays near 0.  With one region the ranking
+ * needs no scan of its own (DECIDE_SCAN) and short lists none after the sweep
+ * (SWEEP_SCAN); with several regions COMPACT includes the propose pass. */
 #define SCORE_GM_K_REANCHOR 0    /* steps whose scalars changed: every cell advanced and predicted again */
 #define SCORE_GM_K_SWEEP 1       /* calcGrowthStepInside/Border over the occupied slots */
 #define SCORE_GM_K_SWEEP_SCAN 2  /* list offsets of the sweep's blocks */

@@ -21,7 +21,8 @@
  *   k_compact      the completed slots of every step in FullRX order (Inside list,
  *                  then Border), and the INACTIVE slots as masks.  Short fronts: the
  *                  first step's propose pass too.
- *   k_window_end   closes the last step and hands the stats to the host.
+ *   (k_window_end  closes the last step and hands the stats to the host, where the last
+ *                  commit pass has not done it: a halted window)
  * per step
  *   k_propose      block 0 closes the step before (its row, list lengths, recycling
  *                  tables).  The others copy what the infection needs of each
@@ -32,21 +33,24 @@
  *                  attempts exactly as the serial loop issues them.
  *   k_decide       an attempt wins iff its key is the minimum; winners per parent
  *                  and destination list as bit masks, counted per 64 parents and per
- *                  block.  Further blocks write the recycled slots that may be handed
- *                  out, ascending.
+ *                  block; the parents retire.  Further blocks write the recycled
+ *                  slots that may be handed out, ascending.
  *   k_commit       the winners before a block rank its own: rank k into a list takes
  *                  the k-th recycled slot, else appends.  One thread per winner writes
  *                  the new record with its increment and completion step (certified
  *                  from the real sums, gm_radd_count_to_one), and clears the cell's
- *                  bitmap bit; the parents retire.
+ *                  bitmap bit.  The window's last one ends it (window_end).
  *
  * Three passes a step, where sweep, scan, compaction, ranking scan, recycling and
  * the step's row were seven more launches: on the 24x20x18 domain of ten nuclei a
- * step went from 48 to 24 us, at 100^3 from 62 to 33, at 320^3 from 90 to 62, at
- * 512^3 from 165 to 135.
+ * step went from 48 to 20 us, at 100^3 from 62 to 26, at 320^3 from 90 to 54, at
+ * 512^3 from 165 to 132.  A pass costs 2.4 us whatever it does and 0.7 us more for
+ * every load that waits for another, so on fronts of a few thousand parents the length
+ * of these chains and the number of passes are the time.
  *
  * No kernel waits on another block: every cross-block dependency is a kernel
- * boundary, so the passes use only relaxed device atomics.  FP64 throughout,
+ * boundary, but for the end of a window, which the last block to finish takes over,
+ * so the passes use only relaxed device atomics.  FP64 throughout,
  * compiled with -ffp-contract=off so every product and sum is rounded exactly as
  * in the reference's build without FMA.
  */

@@ -68,6 +68,10 @@ static __constant__ uint8_t c_hidx[27] = {0xFF, 0xFF, 0xFF, 0, 1, 2, 3, 0xFF, 0x
 #define RS_R 1
 #define RS_UN 2
 #define RW_ROW0 3
+/* sweep blocks (of 2048 slots) up to which compaction blocks do the propose pass; runs in
+ * eight regions, so and apart: 160^3 (0.8M slots at most) 29.9 and 31.2 ms, 200^3 (1.5M)
+ * 34.5 and 34.6, 256^3 (3.1M) 49.7 and 42.2, 320^3 80.3 and 53.5 */
+#define GM_RG_FUSE 1024u
 /* and, after its own, the row of its parents in the grain that sets rhomax */
 #define RW_TOP (RW_ROW0 + GM_RROWS)
 
@@ -394,7 +398,14 @@ __global__ void __launch_bounds__(1024) k_rg_sweep_scan(GmDev d, uint32_t nb, ui
             sR[l] = er;
         }
     }
-    scan_rows(d.bcnt, 3u, nb, tot);
+    if (nb <= GM_RG_FUSE) {
+        scan_rows(d.bcnt, 3u, nb, tot);
+    } else { /* sixteen rounds of a wave a row took 17 us, this 11 */
+        uint32_t v[3];
+        scan_block_counts<3>(d.bcnt, nb, v);
+        if (threadIdx.x < 3u) tot[threadIdx.x] = threadIdx.x == 0u ? v[0] : threadIdx.x == 1u ? v[1] : v[2];
+        __syncthreads();
+    }
     if (threadIdx.x == 0) {
         if (tot[RS_UN]) st->err |= GM_ERRF_MISSED;
         /* infection keys are (halo, neighbour, p, rank) in 32 bits, p < 2^23 */
@@ -514,51 +525,82 @@ static __device__ __forceinline__ uint32_t rg_propose(const GmDev &d, RgWave &W,
     return na;
 }
 
-/* The sweep's partition: a block's first wave, one lane per tile, lists its completed
- * slots in FullRX order (append_to_fullrx_*_list, SCORE_Kernel.cpp:3994-4042,
- * :4133-4180), the lists one after another; then all its waves take these parents
- * through the propose pass, which in a launch of its own read them back (5 us a step). */
-__global__ void __launch_bounds__(GM_BLOCK) k_rg_compact(GmDev d) {
-    __shared__ RgWave sw[GM_BLOCK / 64];
-    __shared__ uint32_t send, satt[GM_BLOCK / 64];
-    GmStats *st = d.st;
-    if (st->halt) return;
-    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-    const uint32_t T = d.L.tile[d.nlists], nfull = st->nfullI + st->nfullB, k = st->kcur;
-    const unsigned long long nret = st->nret;
-    uint32_t lo, hi;
-    part_of(T, GM_SW_TPC, lo, hi);
-    const uint32_t first = d.bcnt[RS_F * GM_MAX_BLOCKS + blockIdx.x];
-    const bool logged = nret + nfull <= d.rlogCap;
-    if (!logged && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&st->err, GM_ERRF_RLOG_FULL);
-    if (w == 0) {
-        uint32_t runF = first;
-        for (uint32_t batch = lo; batch < hi; batch += 64) {
-            const uint32_t t = batch + lane;
-            const uint64_t bf = t < hi ? d.mF[t] : 0ull;
-            const uint32_t cf = (uint32_t)__popcll(bf);
-            const uint32_t incf = wave_incl_scan(cf);
-            uint32_t of = runF + incf - cf;
-            runF += __shfl(incf, 63, 64);
-            if (bf) {
-                const uint32_t l = upper_index(d.L.tile, d.nlists, t);
-                const uint32_t s0 = d.L.base[l] + (t - d.L.tile[l]) * 64u;
-                for (uint64_t m = bf; m; m &= m - 1ull) {
-                    d.plist[of] = l;
-                    d.pslot[of++] = s0 + (uint32_t)__ffsll((long long)m) - 1u;
-                }
+/* The completed slots of tiles [lo, hi) in FullRX order (append_to_fullrx_*_list,
+ * SCORE_Kernel.cpp:3994-4042, :4133-4180) from position `first` on, the lists one after
+ * another, by one wave, a lane per tile; the position behind them. */
+static __device__ __forceinline__ uint32_t rg_list(const GmDev &d, uint32_t lo, uint32_t hi, uint32_t first) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t runF = first;
+    for (uint32_t batch = lo; batch < hi; batch += 64) {
+        const uint32_t t = batch + lane;
+        const uint64_t bf = t < hi ? d.mF[t] : 0ull;
+        const uint32_t cf = (uint32_t)__popcll(bf);
+        const uint32_t incf = wave_incl_scan(cf);
+        uint32_t of = runF + incf - cf;
+        runF += __shfl(incf, 63, 64);
+        if (bf) {
+            const uint32_t l = upper_index(d.L.tile, d.nlists, t);
+            const uint32_t s0 = d.L.base[l] + (t - d.L.tile[l]) * 64u;
+            for (uint64_t m = bf; m; m &= m - 1ull) {
+                d.plist[of] = l;
+                d.pslot[of++] = s0 + (uint32_t)__ffsll((long long)m) - 1u;
             }
         }
-        if (lane == 0) send = runF;
     }
-    __syncthreads();
+    return runF;
+}
+
+/* Long fronts (more than GM_RG_FUSE sweep blocks): the list alone, a wave per block,
+ * and the propose pass in a launch of its own, with full waves.  A sweep block has some
+ * 30 parents, half a wave: on 512^3 in eight regions the two passes take less than the
+ * fused one (81 us with four waves a block, 97 with one). */
+__global__ void __launch_bounds__(64) k_rg_list(GmDev d) {
+    if (d.st->halt) return;
+    uint32_t lo, hi;
+    part_of(d.L.tile[d.nlists], GM_SW_TPC, lo, hi);
+    rg_list(d, lo, hi, d.bcnt[RS_F * GM_MAX_BLOCKS + blockIdx.x]);
+}
+
+/* Parents [p0, p1) by the block, 64 a wave, `step` parents on for the next; their
+ * attempts are added to the step's. */
+static __device__ __forceinline__ void rg_propose_block(const GmDev &d, uint32_t p0, uint32_t p1, uint32_t step) {
+    __shared__ RgWave sw[GM_BLOCK / 64];
+    __shared__ uint32_t satt[GM_BLOCK / 64];
+    GmStats *st = d.st;
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    const uint32_t nfull = st->nfullI + st->nfullB, k = st->kcur;
+    const unsigned long long nret = st->nret;
+    const bool logged = nret + nfull <= d.rlogCap;
+    if (!logged && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&st->err, GM_ERRF_RLOG_FULL);
     uint32_t natt = 0;
-    for (uint32_t p = first + w * 64u; p < send; p += GM_BLOCK)
-        natt += rg_propose(d, sw[w], p, send - p < 64u ? send - p : 64u, k, logged ? d.rlog + nret : nullptr);
+    for (uint32_t p = p0 + w * 64u; p < p1; p += step)
+        natt += rg_propose(d, sw[w], p, p1 - p < 64u ? p1 - p : 64u, k, logged ? d.rlog + nret : nullptr);
     if (lane == 0) satt[w] = natt;
     __syncthreads();
     natt = satt[0] + satt[1] + satt[2] + satt[3];
     if (threadIdx.x == 0 && natt) atomicAdd(&st->ntried, natt);
+}
+
+__global__ void __launch_bounds__(GM_BLOCK) k_rg_propose(GmDev d) {
+    if (d.st->halt) return;
+    rg_propose_block(d, blockIdx.x * GM_BLOCK, d.st->nfullI + d.st->nfullB, gridDim.x * GM_BLOCK);
+}
+
+/* The sweep's partition: a block's first wave lists its completed slots, then all its
+ * waves take these parents through the propose pass, which in a launch of its own read
+ * them back (5 us a step). */
+__global__ void __launch_bounds__(GM_BLOCK) k_rg_compact(GmDev d) {
+    __shared__ uint32_t send;
+    if (d.st->halt) return;
+    uint32_t lo, hi;
+    part_of(d.L.tile[d.nlists], GM_SW_TPC, lo, hi);
+    const uint32_t first = d.bcnt[RS_F * GM_MAX_BLOCKS + blockIdx.x];
+    if (threadIdx.x < 64u) {
+        const uint32_t end = rg_list(d, lo, hi, first);
+        if (threadIdx.x == 0) send = end;
+    }
+    __syncthreads();
+    rg_propose_block(d, first, send, GM_BLOCK);
 }
 
 /* Each list's INACTIVE slots in ascending order (append_to_recycling_*_list,
@@ -612,7 +654,12 @@ hipError_t gm_launch_rg_sweep(const GmDev &d, const GmSweepArgs &a, uint32_t par
     if ((e = mark(ev, 2, s)) != hipSuccess) return e;
     k_rg_sweep_scan<<<1, 1024, 0, s>>>(d, nb, rg_infect_blocks(d, parents_upper));
     if ((e = mark(ev, 3, s)) != hipSuccess) return e;
-    k_rg_compact<<<nb, GM_BLOCK, 0, s>>>(d);
+    if (nb <= GM_RG_FUSE) {
+        k_rg_compact<<<nb, GM_BLOCK, 0, s>>>(d);
+    } else {
+        k_rg_list<<<nb, 64, 0, s>>>(d);
+        k_rg_propose<<<grid_for(parents_upper, GM_BLOCK), GM_BLOCK, 0, s>>>(d);
+    }
     return hipGetLastError();
 }
 
