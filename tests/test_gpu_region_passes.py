@@ -33,3 +33,17 @@ def test_parents_at_block_edges(require_gpu, T, nuclei):
     e = 24 if nuclei < 1000 else 72
     dom = synth.make_voronoi_domain(e, 2 * e, 2 * e - 1, n_grains=20, n_nuclei=nuclei, seed=T + nuclei)
     _same(dom, ParamsSpec(n_regions=T, xmax=0.5 if nuclei > 1000 else 0.99), T)
+
+
+def test_long_front(require_gpu):
+    """A front of more sweep blocks than compaction and propose pass share a launch for,
+    on either side of the line within one run."""
+    dom = synth.make_voronoi_domain(228, 216, 210, n_grains=600, n_nuclei=7700, seed=2)
+    prm = ParamsSpec(n_regions=4, xmax=0.8)
+    o, g = Oracle(dom, prm), _gm(dom, prm)
+    o.solve_rxgrowth()
+    g.solve_rxgrowth()
+    tr = g.trajectory()
+    slots = (tr["nslots_inside"] + tr["nslots_border"]).astype(np.int64)
+    assert slots.min() * 3 // 2 < 1024 * 2048 < slots.max() * 3 // 2
+    assert_final_equal_regions(o, g, 4)
