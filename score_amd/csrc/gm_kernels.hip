@@ -656,7 +656,8 @@ static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, 
  * sets rhomax, Xcells at a threshold, weights the window cannot wait for, a step
  * that found too few slots), or step j has more parents than the planes hold.  Every
  * input was written by an earlier kernel, so all blocks of the propose pass find
- * the same; it records the answer in st->halt for the step's other passes. */
+ * the same; it records the answer in st->halt for the step's other passes and for
+ * the steps queued behind it, which do nothing then. */
 static __device__ __forceinline__ bool must_halt_at(const GmDev &d, const GmWindow &w, uint32_t nfull) {
     const GmStats *st = d.st;
     /* every word loaded before the first test */
@@ -717,7 +718,10 @@ __global__ void __launch_bounds__(GM_BLOCK) k_propose(GmDev d, GmPart P, GmWindo
     GmStats *st = d.st;
     const GmWin *win = d.win;
     const uint32_t nfull = win->full[j], off = win->off[j];
-    const bool halt = must_halt(d, wd, j);
+    /* the window may have halted at an earlier step: the one before this did not run, and
+     * nothing is left to close.  (Block 0 sets the word only where every block halts.) */
+    const bool halted = agent_load(&st->halt) != 0u, halt = must_halt(d, wd, j);
+    if (halted) return;
     if (blockIdx.x == 0) {
         /* a step whose commit pass found too few slots is not done */
         const uint32_t undone = st->grow;
