@@ -70,6 +70,10 @@ static __device__ __forceinline__ uint64_t rdlane64(uint64_t v, uint32_t j) {
 static __device__ __forceinline__ uint32_t agent_load(const uint32_t *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+/* a word that another block may be changing, where the value before and the one after do equally well */
+static __device__ __forceinline__ uint32_t either_load(const uint32_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 static __device__ __forceinline__ void agent_store(uint32_t *p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

@@ -256,17 +256,14 @@ __global__ void __launch_bounds__(GM_BLOCK) k_sweep(GmDev d, GmPart P, uint32_t 
 static __device__ void window_totals(const GmDev &d, const GmPart &P, const uint32_t *tot, uint32_t recI, uint32_t recB,
                                      const uint32_t *totI) {
     GmWin *win = d.win;
-    uint32_t off = 0, err = 0;
+    uint32_t off = 0;
     for (uint32_t i = 0; i < P.W; i++) {
         win->full[i] = tot[i];
         win->fullI[i] = totI[i];
         win->off[i] = off;
         off += tot[i];
-        /* infection keys are p*32 + rank in 32 bits, p < full */
-        if (tot[i] > (1u << 27)) err = GM_ERRF_KEYS;
     }
     win->off[P.W] = off;
-    if (err) atomicOr(&d.st->err, err);
     GmWinStep &s = win->step[0];
     s.csz = P.csz0;
     s.nI = d.st->nI;
@@ -651,26 +648,38 @@ static __device__ void close_step(const GmDev &d, const GmPart &P, uint32_t js, 
     }
 }
 
-/* Whether step j of the window must not run: the host has to act on what step
- * j-1 left (an error, a count that wrapped, the exhaustion of the grain that
- * sets rhomax, Xcells at a threshold, weights the window cannot wait for, a step
- * that found too few slots), or step j has more parents than the planes hold.  Every
- * input was written by an earlier kernel, so all blocks of the propose pass find
- * the same; it records the answer in st->halt for the step's other passes and for
- * the steps queued behind it, which do nothing then. */
-static __device__ __forceinline__ bool must_halt_at(const GmDev &d, const GmWindow &w, uint32_t nfull) {
+/* Why step j of the window must not run.  HOST: the host has to act on what step j-1
+ * left (an error, a count that wrapped, the exhaustion of the grain that sets rhomax,
+ * Xcells at a threshold, weights the window cannot wait for, a step that found too few
+ * slots).  Else an error of the step's own: infection keys are p*32 + rank in 32 bits, p
+ * below its nfull parents, and the retirement log, of which it takes the entries from
+ * `ret` on, has an end.  Else PLANES: it has more parents than the planes hold.
+ * The inputs were written by earlier kernels, but for st->err, to which block 0 of the
+ * propose pass adds only where every block finds one of the step's own errors: all
+ * blocks halt, or none.  Block 0 records it in st->halt for the step's other passes and
+ * for the steps queued behind it, which do nothing then. */
+#define HALT_HOST 0x80000000u
+#define HALT_PLANES 0x40000000u
+#define HALT_ERRF (GM_ERRF_KEYS | GM_ERRF_RLOG_FULL)
+static __device__ __forceinline__ uint32_t halt_reason(const GmDev &d, const GmWindow &w, uint32_t nfull,
+                                                       unsigned long long ret, bool at_stop) {
     const GmStats *st = d.st;
     /* every word loaded before the first test */
-    const uint32_t flags = st->err | st->cwrap | st->novf | d.win->top_hit | st->grow, npend = st->npend;
-    return (flags != 0u) | ((npend != 0u) & !w.defer) | (npend > w.pend_limit) | (nfull > d.parentCap);
+    const uint32_t flags = either_load(&st->err) | st->cwrap | st->novf | d.win->top_hit | st->grow, npend = st->npend;
+    const bool host = (flags != 0u) | ((npend != 0u) & !w.defer) | (npend > w.pend_limit) | at_stop;
+    const uint32_t err = (nfull > (1u << 27) ? GM_ERRF_KEYS : 0u) | (ret + nfull > d.rlogCap ? GM_ERRF_RLOG_FULL : 0u);
+    return host ? HALT_HOST : err ? err : nfull > d.parentCap ? HALT_PLANES : 0u;
 }
-static __device__ __forceinline__ bool must_halt(const GmDev &d, const GmWindow &w, uint32_t j) {
-    const double xc = d.win->xcells0 + (double)d.win->off[j];
-    return must_halt_at(d, w, d.win->full[j]) | ((j != 0u) & (xc >= w.xstop));
+/* by one thread of block 0 */
+static __device__ __forceinline__ void record_halt(const GmDev &d, uint32_t why, uint32_t nfull, uint32_t j) {
+    d.st->halt = why ? 1u : 0u;
+    if (why & HALT_PLANES) d.st->need_par = nfull;
+    if (why & HALT_ERRF) atomicOr(&d.st->err, why);
+    if (d.prog) __hip_atomic_store(d.prog, (j << 1) | (why ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 /* Step k's parent p, in slot s: see k_propose; returns its attempts.  rlog: where the
- * step's retirements go in the log (null: they do not fit). */
+ * step's retirements go in the log. */
 static __device__ __forceinline__ uint32_t propose_parent(const GmDev &d, uint32_t s, uint32_t p, uint32_t k, uint2 *rlog) {
     const GmRec *r = d.rec + s;
     const RecC rc = rec_c(r);
@@ -699,7 +708,7 @@ static __device__ __forceinline__ uint32_t propose_parent(const GmDev &d, uint32
     d.pmA[p] = am;
     par_plane(d, GM_PAR1_CELL)[p] = make_uint4(x | y << 16, z | (fromB ? 1u << 16 : 0u), rc.defg, rxg);
     reinterpret_cast<double2 *>(par_plane(d, GM_PAR1_FP))[p] = make_double2(fin, rc.P);
-    if (rlog) rlog[p] = make_uint2(cell, d.ndefg + rxg);
+    rlog[p] = make_uint2(cell, d.ndefg + rxg);
     return (uint32_t)__popc(am);
 }
 
@@ -720,31 +729,26 @@ __global__ void __launch_bounds__(GM_BLOCK) k_propose(GmDev d, GmPart P, GmWindo
     const uint32_t nfull = win->full[j], off = win->off[j];
     /* the window may have halted at an earlier step: the one before this did not run, and
      * nothing is left to close.  (Block 0 sets the word only where every block halts.) */
-    const bool halted = agent_load(&st->halt) != 0u, halt = must_halt(d, wd, j);
+    const uint32_t halted = either_load(&st->halt);
+    const unsigned long long nret = win->nret0 + off;
+    const uint32_t halt = halt_reason(d, wd, nfull, nret, (j != 0u) & (win->xcells0 + (double)off >= wd.xstop));
     if (halted) return;
     if (blockIdx.x == 0) {
         /* a step whose commit pass found too few slots is not done */
         const uint32_t undone = st->grow;
         if (j && !undone) close_step(d, P, j - 1u, !halt);
-        if (threadIdx.x == 0) {
-            st->halt = halt ? 1u : 0u;
-            if (nfull > d.parentCap) st->need_par = nfull;
-            if (d.prog)
-                __hip_atomic_store(d.prog, (j << 1) | (halt ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
+        if (threadIdx.x == 0) record_halt(d, halt, nfull, j);
         return;
     }
     if (halt) return;
     /* the step's parents retire into the log at [nret, nret + nfull) */
-    const unsigned long long nret = win->nret0 + off;
-    const bool logged = nret + nfull <= d.rlogCap;
+    uint2 *rlog = d.rlog + nret;
     const uint32_t blk = blockIdx.x - 1u, lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-    if (!logged && blk == 0 && threadIdx.x == 0) atomicOr(&st->err, GM_ERRF_RLOG_FULL);
     uint32_t natt = 0;
     for (uint32_t c = w * P.nbp + blk; c * 64u < nfull; c += P.nbp * (GM_BLOCK / 64u)) {
         const uint32_t p = c * 64u + lane;
         if (p >= nfull) break;
-        natt += propose_parent(d, d.pslot[off + p], p, k, logged ? d.rlog + nret : nullptr);
+        natt += propose_parent(d, d.pslot[off + p], p, k, rlog);
     }
     for (int o = 32; o > 0; o >>= 1) natt += __shfl_xor(natt, o, 64);
     if (lane == 0) satt[w] = natt;
@@ -877,21 +881,14 @@ __global__ void __launch_bounds__(GM_BLOCK) k_compact(GmDev d, GmPart P, GmWindo
     if (!PROPOSE) return;
     /* the first step's attempts by the blocks that list its parents */
     const uint32_t nfull = stot[0], first = spre[0], cnt = d.wcnt[b];
-    GmStats *st = d.st;
-    const bool halt = must_halt_at(d, wd, nfull);
-    const unsigned long long nret = st->nret;
-    const bool logged = nret + nfull <= d.rlogCap;
-    if (b == 0 && t == 0) {
-        st->halt = halt ? 1u : 0u;
-        if (nfull > d.parentCap) st->need_par = nfull;
-        if (d.prog) __hip_atomic_store(d.prog, halt ? 1u : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        if (!halt && !logged) atomicOr(&st->err, GM_ERRF_RLOG_FULL);
-    }
+    const unsigned long long nret = d.st->nret;
+    const uint32_t halt = halt_reason(d, wd, nfull, nret, false);
+    if (b == 0 && t == 0) record_halt(d, halt, nfull, 0u);
     if (halt) return;
     __syncthreads();
     uint32_t natt = 0;
     for (uint32_t i = t; i < cnt; i += GM_BLOCK)
-        natt += propose_parent(d, d.pslot[first + i], first + i, k0, logged ? d.rlog + nret : nullptr);
+        natt += propose_parent(d, d.pslot[first + i], first + i, k0, d.rlog + nret);
     for (int o = 32; o > 0; o >>= 1) natt += __shfl_xor(natt, o, 64);
     if (lane == 0) run[w][0] = natt;
     __syncthreads();

@@ -1,0 +1,53 @@
+"""A step that the retirement log has no room for is refused before it runs, by every
+block of its propose pass alike: the error comes back and the state is the one before
+the step.  Cells retire twice where a defragmentation follows another with no
+completions between (the reference's search revives the records left behind); here
+12,000 records of slow cells are, and the last class of cells completes in one step."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from oracle.oracle import Oracle
+from score_amd import abi, synth
+from score_amd.growth import GrowthMachine
+from score_amd.synth import ParamsSpec
+
+pytestmark = pytest.mark.gpu
+
+LAST = 45
+
+
+def _case():
+    e = 38
+    a = np.arange(2, e - 2, 3)
+    dom = synth.make_voronoi_domain(e, e, e, n_grains=2, n_nuclei=len(a) ** 3, seed=3, rho_values=np.array([1e15, 1e14]))
+    z, y, x = np.meshgrid(a, a, a, indexing="ij")
+    dom.rxg_site[:] = (x + e * (y + e * z)).ravel()
+    dom.rxg_ori[:] = dom.rxg_ori[0]
+    dom.cellgrid = np.repeat(np.arange(e) >= 15, e * e).astype(np.uint32)
+    return dom, ParamsSpec(xmax=5.0, defrag_at=(0.36 * dom.N,) * 2)
+
+
+@pytest.mark.parametrize("first", [LAST, LAST - 1, LAST - 3])
+def test_step_beyond_the_log(require_gpu, first):
+    dom, prm = _case()
+    o = Oracle(dom, prm)
+    o.step(LAST)
+    defg, rxg = o.counts()
+    full = int(rxg.sum(dtype=np.int64))
+    cap = dom.N + 6 * 38 * 38 + 4096
+    with GrowthMachine(dom, prm) as g:
+        # the refused step is the first of its window, or a later one
+        g.step(first)
+        with pytest.raises(abi.ScoreGmError) as err:
+            g.step(1000)
+        assert err.value.code == abi.ERR_CAPACITY
+        assert np.array_equal(g.counts()[0], defg) and np.array_equal(g.counts()[1], rxg)
+        if first == LAST:
+            assert np.array_equal(g.grainmap(), o.grainmap())
+        with pytest.raises(abi.ScoreGmError):
+            g.step(1)
+    o.step(1)
+    t = o.trajectory()
+    assert full <= cap < full + int(t["nfull_inside"][LAST]) + int(t["nfull_border"][LAST])
