@@ -218,6 +218,7 @@ struct score_gm_handle {
     std::vector<GmRegion> reg;
     std::vector<uint32_t> lbase, lcap, lrcap, lrbase;
     char *stage = nullptr; /* pinned buffers of copy_staged; null: plain copies */
+    unsigned stage_workers = 0; /* how many workers they are for */
     /* arena of the arrays made at creation */
     struct Planned {
         void **p;
@@ -328,12 +329,16 @@ hipError_t copy_plain(void *dev, void *host, size_t bytes, bool to_host, hipStre
     return e != hipSuccess ? e : hipStreamSynchronize(s);
 }
 
-unsigned stage_workers() { return std::min(kStageWorkers, std::max(1u, std::thread::hardware_concurrency() / 2)); }
+/* (the count of processors may be another one later) */
+unsigned stage_workers_now() { return std::min(kStageWorkers, std::max(1u, std::thread::hardware_concurrency() / 2)); }
 
-/* `pin`: 2 chunks for each worker, or null (the plain copy) */
-hipError_t copy_staged(int device, char *pin, void *dev, void *host, size_t bytes, bool to_host, hipStream_t s) {
+/* through the handle's buffers, 2 chunks for each worker they were made for, or plainly */
+hipError_t copy_staged(const score_gm_handle *h, void *dev, void *host, size_t bytes, bool to_host) {
     const size_t chunks = (bytes + kStageChunk - 1) / kStageChunk;
-    const unsigned T = stage_workers();
+    const unsigned T = h->stage_workers;
+    const int device = h->device;
+    const hipStream_t s = h->stream;
+    char *const pin = h->stage;
     if (!pin || bytes < kStageMin) return copy_plain(dev, host, bytes, to_host, s);
     std::atomic<int> err{hipSuccess};
     auto work = [&](unsigned k) {
@@ -2038,14 +2043,15 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
     auto setup = [&]() -> int {
         hipStream_t s = h->stream;
         /* without them (no pinned memory left) the grid and the maps are copied plainly */
-        if (sizeof(uint32_t) * d.N >= kStageMin && stage_workers() > 1 &&
-            hipHostMalloc((void **)&h->stage, 2 * kStageChunk * stage_workers(), hipHostMallocDefault) != hipSuccess) {
+        h->stage_workers = stage_workers_now();
+        if (sizeof(uint32_t) * d.N >= kStageMin && h->stage_workers > 1 &&
+            hipHostMalloc((void **)&h->stage, 2 * kStageChunk * h->stage_workers, hipHostMallocDefault) != hipSuccess) {
             (void)hipGetLastError();
             h->stage = nullptr;
         }
         /* the grid arrives in the record array, which nothing uses yet */
         uint32_t *src = reinterpret_cast<uint32_t *>(d.rec);
-        HIPCHK(copy_staged(device, h->stage, src, const_cast<uint32_t *>(dom->cellgrid), sizeof(uint32_t) * d.N, false, s));
+        HIPCHK(copy_staged(h, src, const_cast<uint32_t *>(dom->cellgrid), sizeof(uint32_t) * d.N, false));
         HIPCHK(gm_launch_fill_u32(d.defcnt, 0u, d.ndefg, s));
         HIPCHK(gm_launch_fill_u32(d.defsub, 0u, (size_t)GM_SUBS * d.ndefg, s));
         HIPCHK(gm_launch_fill_u32((uint32_t *)d.st, 0u, sizeof(GmStats) / 4, s));
@@ -2198,7 +2204,7 @@ int score_gm_get_grainmap(score_gm_handle *h, uint32_t *out, int32_t encoding) {
     auto copy = [&]() -> int {
         HIPCHK(gm_launch_overlay_infected(h->d, h->nI, h->nB, h->step, tmp, h->stream));
         if (encoding == SCORE_GM_MAP_RAW2GID) HIPCHK(gm_launch_raw2gid(tmp, h->d.N, h->stream));
-        HIPCHK(copy_staged(h->device, h->stage, tmp, out, sizeof(uint32_t) * h->d.N, true, h->stream));
+        HIPCHK(copy_staged(h, tmp, out, sizeof(uint32_t) * h->d.N, true));
         return 0;
     };
     rc = copy();
