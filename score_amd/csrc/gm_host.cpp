@@ -226,6 +226,7 @@ struct score_gm_handle {
     };
     std::vector<Planned> plan;
     bool planning = false;
+    std::vector<std::pair<const void *, size_t>> held; /* what dalloc has given out */
     char *arena = nullptr;
     size_t arena_bytes = 0;
     uint32_t last_full = 0xFFFFFFFFu; /* most cells completed in one step of the last window */
@@ -399,6 +400,22 @@ hipError_t copy_staged(const score_gm_handle *h, void *dev, void *host, size_t b
     return e;
 }
 
+/* Device memory that the process's handles hold, and how much they may hold: all of the
+ * device's, or SCORE_GM_MEM_LIMIT bytes (for a device that is shared; checked when a
+ * handle is created). */
+std::atomic<uint64_t> g_held{0};
+
+uint64_t held_limit(bool *ok = nullptr) {
+    const char *ev = getenv("SCORE_GM_MEM_LIMIT");
+    if (ok) *ok = true;
+    if (!ev) return UINT64_MAX;
+    char *end = nullptr;
+    const long long v = strtoll(ev, &end, 10);
+    if (end != ev && *end == '\0' && v >= 1) return (uint64_t)v;
+    if (ok) *ok = false;
+    return UINT64_MAX;
+}
+
 /* Device memory comes from the device's stream-ordered pool on the handle's
  * stream: a free does not wait for the whole device (as hipFree does), so
  * handles created and destroyed next to running ones do not stall them, and
@@ -413,21 +430,38 @@ int dalloc(score_gm_handle *h, T **p, size_t n) {
         h->arena_bytes += (n * sizeof(T) + 255) / 256 * 256;
         return 0;
     }
-    hipError_t e = hipMallocFromPoolAsync((void **)p, n * sizeof(T), h->pool, h->stream);
+    const size_t bytes = n * sizeof(T);
+    try {
+        h->held.emplace_back(nullptr, bytes);
+    } catch (...) {
+        return fail(SCORE_GM_ERR_OOM, "host memory");
+    }
+    const bool fits = g_held.fetch_add(bytes) + bytes <= held_limit();
+    hipError_t e = fits ? hipMallocFromPoolAsync((void **)p, bytes, h->pool, h->stream) : hipErrorOutOfMemory;
     if (e != hipSuccess) {
+        g_held.fetch_sub(bytes);
+        h->held.pop_back();
         *p = nullptr;
         (void)hipGetLastError();
         g_last_error = std::string("hipMallocFromPoolAsync: ") + hipGetErrorString(e);
         return SCORE_GM_ERR_OOM;
     }
+    h->held.back().first = *p;
     return 0;
 }
 
 void dfree(score_gm_handle *h, void *p) {
     /* what lies in the arena goes with it */
     const char *c = static_cast<const char *>(p);
-    if (h->arena && c >= h->arena && c < h->arena + h->arena_bytes) return;
-    if (p) (void)hipFreeAsync(p, h->stream);
+    if (!p || (h->arena && c >= h->arena && c < h->arena + h->arena_bytes)) return;
+    for (auto &q : h->held)
+        if (q.first == p) {
+            g_held.fetch_sub(q.second);
+            q = h->held.back();
+            h->held.pop_back();
+            break;
+        }
+    (void)hipFreeAsync(p, h->stream);
 }
 
 /* The arrays a handle is created with, in one block: some 50 allocations and frees
@@ -457,9 +491,10 @@ void free_device(score_gm_handle *h) {
                     d.L.occ, d.L.tile, d.L.tile_s, d.L.par, d.L.rst, d.L.rbuf, d.L.rs, d.L.bstart, d.L.breg,
                     d.L.hoff, d.plist};
     for (void *q : ptrs) dfree(h, q);
-    if (h->arena) (void)hipFreeAsync(h->arena, h->stream);
+    char *const arena = h->arena;
     h->arena = nullptr;
     h->arena_bytes = 0;
+    dfree(h, arena);
     memset(&h->d, 0, sizeof(h->d));
     if (h->stage) (void)hipHostFree(h->stage);
     h->stage = nullptr;
@@ -986,56 +1021,69 @@ int grow_front(score_gm_handle *h, uint32_t need) {
     uint64_t nc = (std::max<uint64_t>(need, 2ull * d.capI) + 63) / 64 * 64;
     const bool staged = nc + d.capI > d.capImax;
     if (staged) nc = d.capImax;
-    const size_t used = (size_t)d.baseI + d.capI, tot = (size_t)d.baseI + nc + GM_SW_CHUNK;
-    GmRec *rec = d.rec;
-    gm_cs_t *cs = d.cstep;
-    char *keep = nullptr;
-    if (staged) {
-        keep = static_cast<char *>(malloc(used * (sizeof(GmRec) + sizeof(gm_cs_t))));
-        if (!keep) return fail(SCORE_GM_ERR_OOM, "host memory for the front list");
-        hipError_t e;
-        if ((e = hipMemcpyAsync(keep, rec, sizeof(GmRec) * used, hipMemcpyDeviceToHost, h->stream)) != hipSuccess ||
-            (e = hipMemcpyAsync(keep + sizeof(GmRec) * used, cs, sizeof(gm_cs_t) * used, hipMemcpyDeviceToHost,
-                                h->stream)) != hipSuccess ||
-            (e = hipStreamSynchronize(h->stream)) != hipSuccess) {
-            free(keep);
+    const size_t used = (size_t)d.baseI + d.capI;
+    /* the lists in new arrays of n Inside slots, copied from rec and cs */
+    auto place = [&](uint64_t n, const GmRec *rec, const gm_cs_t *cs) -> int {
+        const size_t tot = (size_t)d.baseI + n + GM_SW_CHUNK;
+        const hipMemcpyKind kind = staged ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
+        GmRec *nrec = nullptr;
+        gm_cs_t *ncs = nullptr;
+        int rc;
+        if ((rc = dalloc(h, &nrec, tot)) || (rc = dalloc(h, &ncs, tot))) {
+            dfree(h, nrec);
+            return rc;
+        }
+        hipError_t e = gm_launch_fill_u32((uint32_t *)ncs, 0xFFFFFFFFu, tot / 2, h->stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(nrec, rec, sizeof(GmRec) * used, kind, h->stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(ncs, cs, sizeof(gm_cs_t) * used, kind, h->stream);
+        if (e == hipSuccess && staged) e = hipStreamSynchronize(h->stream);
+        if (e != hipSuccess) {
+            dfree(h, nrec);
+            dfree(h, ncs);
             return hip_fail(e, "growing the Inside list");
         }
+        d.rec = nrec;
+        d.cstep = ncs;
+        d.capI = (uint32_t)n;
+        return 0;
+    };
+    GmRec *const rec = d.rec;
+    gm_cs_t *const cs = d.cstep;
+    int rc;
+    if (!staged) {
+        if ((rc = place(nc, rec, cs))) return rc;
         dfree(h, rec);
         dfree(h, cs);
-        d.rec = nullptr;
-        d.cstep = nullptr;
+        return 0;
     }
-    GmRec *nrec = nullptr;
-    gm_cs_t *ncs = nullptr;
-    int rc;
-    if ((rc = dalloc(h, &nrec, tot)) || (rc = dalloc(h, &ncs, tot))) {
-        dfree(h, nrec);
+    char *keep = static_cast<char *>(malloc(used * (sizeof(GmRec) + sizeof(gm_cs_t))));
+    if (!keep) return fail(SCORE_GM_ERR_OOM, "host memory for the front list");
+    GmRec *const krec = reinterpret_cast<GmRec *>(keep);
+    gm_cs_t *const kcs = reinterpret_cast<gm_cs_t *>(keep + sizeof(GmRec) * used);
+    hipError_t e;
+    if ((e = hipMemcpyAsync(krec, rec, sizeof(GmRec) * used, hipMemcpyDeviceToHost, h->stream)) != hipSuccess ||
+        (e = hipMemcpyAsync(kcs, cs, sizeof(gm_cs_t) * used, hipMemcpyDeviceToHost, h->stream)) != hipSuccess ||
+        (e = hipStreamSynchronize(h->stream)) != hipSuccess) {
         free(keep);
-        return rc;
-    }
-    const hipMemcpyKind kind = staged ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
-    const void *from = staged ? (const void *)keep : (const void *)rec;
-    const void *fromcs = staged ? (const void *)(keep + sizeof(GmRec) * used) : (const void *)cs;
-    hipError_t e = gm_launch_fill_u32((uint32_t *)ncs, 0xFFFFFFFFu, tot / 2, h->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(nrec, from, sizeof(GmRec) * used, kind, h->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(ncs, fromcs, sizeof(gm_cs_t) * used, kind, h->stream);
-    if (e == hipSuccess && staged) e = hipStreamSynchronize(h->stream);
-    free(keep);
-    if (e != hipSuccess) {
-        dfree(h, nrec);
-        dfree(h, ncs);
         return hip_fail(e, "growing the Inside list");
     }
-    if (!staged) {
-        dfree(h, rec);
-        dfree(h, cs);
+    dfree(h, rec);
+    dfree(h, cs);
+    d.rec = nullptr;
+    d.cstep = nullptr;
+    if ((rc = place(nc, krec, kcs))) {
+        /* as they were, if that still fits; else the handle has lost its front (front_lost) */
+        const std::string why = g_last_error;
+        (void)place(d.capI, krec, kcs);
+        g_last_error = why;
     }
-    d.rec = nrec;
-    d.cstep = ncs;
-    d.capI = (uint32_t)nc;
-    return 0;
+    free(keep);
+    return rc;
 }
+
+/* The front lists could not be brought back to the device after a growth that failed: the
+ * handle is in error and has nothing to show. */
+bool front_lost(const score_gm_handle *h) { return h->d.rec == nullptr; }
 
 /* per-step lists, tile masks and per-parent masks sized for the current
  * occupancy and the next step's arrivals (to either list) */
@@ -1791,6 +1839,9 @@ int score_gm_device_count(void) {
 
 static int create_handle(const score_gm_domain *dom, const score_gm_params *prm, int device, score_gm_handle **out) {
     int rc;
+    bool ok;
+    (void)held_limit(&ok);
+    if (!ok) return fail(SCORE_GM_ERR_ARG, "SCORE_GM_MEM_LIMIT must be a positive integer");
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || device < 0 || device >= ndev) {
         (void)hipGetLastError();
@@ -2196,6 +2247,7 @@ int score_gm_get_grainmap(score_gm_handle *h, uint32_t *out, int32_t encoding) {
     if (!h || !out) return fail(SCORE_GM_ERR_ARG, "null argument");
     if (encoding != SCORE_GM_MAP_CELLGRID && encoding != SCORE_GM_MAP_RAW2GID)
         return fail(SCORE_GM_ERR_ARG, "unknown encoding");
+    if (front_lost(h)) return h->err;
     HIPCHK(hipSetDevice(h->device));
     /* the grid with the front's cells marked infected, assembled in a device buffer */
     uint32_t *tmp = nullptr;
@@ -2247,6 +2299,7 @@ int score_gm_get_front(score_gm_handle *h, int32_t list, uint32_t cap, uint32_t 
                        uint8_t *infector, uint32_t *cell, double *rxfrac, double *P, uint32_t *defg, uint32_t *rxg) {
     if (!h || !n) return fail(SCORE_GM_ERR_ARG, "null argument");
     if (list < 0 || (uint32_t)list >= h->d.nlists) return fail(SCORE_GM_ERR_ARG, "unknown list");
+    if (front_lost(h)) return h->err;
     HIPCHK(hipSetDevice(h->device));
     uint32_t cnt = list == SCORE_GM_LIST_INSIDE ? h->nI : h->nB;
     uint32_t base = list == SCORE_GM_LIST_INSIDE ? h->d.baseI : 0u;
