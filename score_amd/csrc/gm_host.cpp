@@ -1612,11 +1612,27 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
                        : gm_launch_window_end(d, P, launched, w.top_pos, h->hst_dev, h->stream);
     if (e != hipSuccess || (e = prof ? hipStreamSynchronize(h->stream) : wait_window(h)) != hipSuccess)
         return h->err = hip_fail(e, "growth step");
+    /* an error that the steps before it are not part of: they count, and the handle is in
+     * error after the last of them */
+    int failed = 0;
+    std::string why;
+    auto stop = [&](int code) {
+        failed = code;
+        why = g_last_error;
+    };
     /* a step that found too few Inside slots or parents' entries waits for them:
      * step nexec runs on from its commit pass, or the first step from its start */
+    bool undone = false;
     while (d.nreg <= 1 && !h->hst->err && (h->hst->grow || (h->hst->need_par && h->hst->nexec == 0))) {
         const uint32_t j0 = h->hst->nexec, grow = h->hst->grow;
-        if ((rc = grow ? grow_front(h, grow) : grow_parents(h, h->hst->need_par))) return h->err = rc;
+        if ((rc = grow ? grow_front(h, grow) : grow_parents(h, h->hst->need_par))) {
+            if (front_lost(h)) return h->err = rc;
+            stop(rc);
+            /* the step's decide pass has retired its parents already */
+            undone = grow != 0;
+            if (grow && (e = gm_launch_unretire(d, j0, h->stream)) != hipSuccess) return h->err = hip_fail(e, "growth step");
+            break;
+        }
         if ((e = gm_launch_fill_u32(&d.st->grow, 0u, 2, h->stream)) != hipSuccess ||
             (e = gm_launch_fill_u32(&d.st->halt, 0u, 1, h->stream)) != hipSuccess ||
             (grow && (e = gm_launch_commit(d, h->pp, a, P, w, j0, nullptr, h->stream, ev)) != hipSuccess))
@@ -1631,7 +1647,7 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
             (e = hipStreamSynchronize(h->stream)) != hipSuccess)
             return h->err = hip_fail(e, "growth step");
     }
-    if (d.nreg <= 1 && !h->hst->err && h->hst->need_par && (rc = grow_parents(h, h->hst->need_par))) return h->err = rc;
+    if (d.nreg <= 1 && !failed && !h->hst->err && h->hst->need_par && (rc = grow_parents(h, h->hst->need_par))) stop(rc);
     h->last_sp = sp;
     h->have_last_sp = true;
     h->force_reanchor = false;
@@ -1639,7 +1655,10 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
      * and nothing rewrites the mirror before the next window's end */
     const GmStats &st = *h->hst;
     const uint32_t nexec = st.nexec;
-    if (st.err) return h->err = step_error(st.err);
+    if (st.err) stop(step_error(st.err));
+    /* (one region: a step that the log or the keys do not hold has not begun) */
+    if (st.err && (d.nreg > 1 || (st.err & ~(GM_ERRF_KEYS | GM_ERRF_RLOG_FULL)))) return h->err = failed;
+    if (failed && nexec == 0) return h->err = failed;
     if (nexec < 1 || nexec > W) return h->err = fail(SCORE_GM_ERR_STATE, "internal error: window step count");
     if (prof) {
         /* one step per window when profiling */
@@ -1741,11 +1760,12 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
         h->sum_sv += sv;
         if (j + 1 == nexec) {
             /* the grain that set rhomax and those after it that hold no cells leave the
-             * search; before the last step of a window it was not gone */
-            if (st.top_hit)
+             * search; before the last step of a window it was not gone (nor in it, where
+             * the step behind was undone: that one would have found it) */
+            if (st.top_hit && !undone)
                 for (uint32_t i = w.top_pos; i < std::min(st.top_next, d.ndefg); i++) h->alive[h->rho_order[i]] = 0;
             /* a count went below zero and wrapped: cellcount > 0 again, as in SCORE */
-            if (st.cwrap && (rc = refresh_alive(h))) return h->err = rc;
+            if (st.cwrap && !undone && (rc = refresh_alive(h))) return h->err = rc;
         }
         if (h->p.recovery_mode != 0) {
             /* update_mydgoptimize_rho (SCORE_RecoveryModels.cpp:128-135): re-sorted by the
@@ -1798,6 +1818,10 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
     *nsteps = nexec;
     h->windows++;
     if (prof) h->profc.ms_host += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - th0).count();
+    if (failed) {
+        g_last_error = why;
+        return h->err = failed;
+    }
     return 0;
 }
 
@@ -2266,6 +2290,7 @@ int score_gm_get_grainmap(score_gm_handle *h, uint32_t *out, int32_t encoding) {
 
 int score_gm_get_counts(score_gm_handle *h, uint32_t *defg_counts, uint32_t *rxg_counts) {
     if (!h) return fail(SCORE_GM_ERR_ARG, "null handle");
+    if (front_lost(h)) return h->err;
     HIPCHK(hipSetDevice(h->device));
     if (defg_counts) HIPCHK(gm_launch_fold_counts(h->d, h->stream));
     if (defg_counts)

@@ -461,6 +461,8 @@ hipError_t gm_launch_infect(const GmDev &d, const GmPParams &pp, const GmSweepAr
 /* its last pass alone, after the Inside list has grown for it */
 hipError_t gm_launch_commit(const GmDev &d, const GmPParams &pp, const GmSweepArgs &a, const GmPart &P,
                             const GmWindow &w, uint32_t j, GmStats *out, hipStream_t s, hipEvent_t *ev);
+/* step j's parents taken back into the grains' counts: its decide pass has run, its commit pass will not */
+hipError_t gm_launch_unretire(const GmDev &d, uint32_t j, hipStream_t s);
 /* the end of a window whose last step was launched without it, after `launched` steps: the last step's row, the stats into the host's mirror */
 hipError_t gm_launch_window_end(const GmDev &d, const GmPart &P, uint32_t launched, uint32_t top_pos, GmStats *out,
                                 hipStream_t s);

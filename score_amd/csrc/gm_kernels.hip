@@ -1337,6 +1337,21 @@ hipError_t gm_launch_commit(const GmDev &d, const GmPParams &pp, const GmSweepAr
     return hipGetLastError();
 }
 
+/* what the decide pass of step j retired, back (the parts of a count are only ever added up) */
+__global__ void k_unretire(GmDev d, uint32_t j) {
+    const uint32_t nfull = d.win->full[j];
+    for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < nfull; p += gridDim.x * blockDim.x) {
+        const uint4 q = par_plane(d, GM_PAR1_CELL)[p];
+        atomicSub(&d.defsub[q.z], 1u);
+        atomicSub(&d.rxcnt[q.w], 1u);
+    }
+}
+
+hipError_t gm_launch_unretire(const GmDev &d, uint32_t j, hipStream_t s) {
+    k_unretire<<<GM_DB, GM_BLOCK, 0, s>>>(d, j);
+    return hipGetLastError();
+}
+
 /* exported map, SCORE's raw file encoding: 1 for an infected cell, else 2 + id */
 __global__ void k_raw2gid(uint32_t *m, uint64_t n) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)

@@ -5,10 +5,12 @@ from __future__ import annotations
 
 import gc
 
+import numpy as np
 import pytest
 
+from oracle.oracle import Oracle
 from score_amd import abi, synth
-from score_amd.growth import GrowthMachine
+from score_amd.growth import GrowthMachine, same_trajectory
 from score_amd.synth import ParamsSpec
 
 pytestmark = pytest.mark.gpu
@@ -58,6 +60,95 @@ def test_no_memory_for_the_list(require_gpu, monkeypatch):
     assert answered and refused
 
 
+def _as_whole_steps(g, dom, prm):
+    """The state is the oracle's after the steps the trajectory has."""
+    o = Oracle(dom, prm)
+    tg = g.trajectory()
+    if len(tg):
+        o.step(len(tg))
+    assert same_trajectory(o.trajectory(), tg)
+    for a, b in zip(o.counts(), g.counts()):
+        assert np.array_equal(a, b)
+    assert np.array_equal(o.grainmap(), g.grainmap())
+    for lst in (abi.LIST_INSIDE, abi.LIST_BORDER):
+        fo, fg = o.front(lst), g.front(lst)
+        act = fo["activity"] != 0
+        assert np.array_equal(fo["activity"], fg["activity"])
+        for f in ("cell", "rxfrac", "rxg", "P"):
+            assert np.array_equal(fo[f][act], fg[f][act]), (lst, f)
+    return len(tg)
+
+
+@pytest.mark.parametrize("grains", [1, 12])
+def test_state_after_a_failed_list_growth(require_gpu, monkeypatch, grains):
+    """The step that needed the slots has not been, whether it is the first of its window
+    or a later one."""
+    monkeypatch.setenv("SCORE_GM_FRONT_SLOTS", "1")
+    dom = synth.make_voronoi_domain(34, 31, 29, n_grains=grains, n_nuclei=400, seed=3)
+    prm = ParamsSpec(grainlog_at=tuple(0.02 * i * dom.N for i in range(1, 40)))
+    ahead = set()
+    for s in range(0, 40):
+        with GrowthMachine(dom, prm) as g:
+            g.step(s)
+            monkeypatch.setenv("SCORE_GM_MEM_LIMIT", "1")
+            try:
+                g.step(1000)
+                failed = False
+            except abi.ScoreGmError:
+                failed = True
+            monkeypatch.delenv("SCORE_GM_MEM_LIMIT")
+            if not failed:
+                continue
+            try:
+                g.counts()
+            except abi.ScoreGmError as e:
+                # the list is lost: nothing is shown
+                assert e.code == abi.ERR_OOM
+                continue
+            ahead.add(_as_whole_steps(g, dom, prm) - s)
+    assert 0 in ahead and max(ahead) > 0
+
+
+def _least_limit(monkeypatch, run, hi=1 << 30):
+    """The least SCORE_GM_MEM_LIMIT, to 4 KiB, under which `run` ends."""
+    lo = 1
+    while hi - lo > 4096:
+        m = (lo + hi) // 2
+        monkeypatch.setenv("SCORE_GM_MEM_LIMIT", str(m))
+        try:
+            run()
+            hi = m
+        except abi.ScoreGmError as e:
+            assert e.code == abi.ERR_OOM
+            lo = m
+    monkeypatch.delenv("SCORE_GM_MEM_LIMIT")
+    return hi
+
+
+@pytest.mark.parametrize("start", [11, 12, 13])
+def test_state_after_failed_parents_planes(require_gpu, monkeypatch, start):
+    """Step 13 has more parents than the planes hold (4 MB more of them; the window's list of
+    completed cells, 1 MB, still fits)."""
+    e, n = 64, 30000
+    dom = synth.make_voronoi_domain(e, e, e, n_grains=1, n_nuclei=n, seed=3)
+    i = np.random.default_rng(1).choice((e - 4) ** 3, n, replace=False)
+    dom.rxg_site[:] = (i % 60 + 2) + e * (i // 60 % 60 + 2) + e * e * (i // 3600 + 2)
+
+    def steps(k):
+        with GrowthMachine(dom) as g:
+            g.step(k)
+
+    limit = _least_limit(monkeypatch, lambda: steps(13)) + (2 << 20)
+    with GrowthMachine(dom) as g:
+        g.step(start)
+        monkeypatch.setenv("SCORE_GM_MEM_LIMIT", str(limit))
+        with pytest.raises(abi.ScoreGmError) as err:
+            g.step(1000)
+        monkeypatch.delenv("SCORE_GM_MEM_LIMIT")
+        assert err.value.code == abi.ERR_OOM
+        assert _as_whole_steps(g, dom, ParamsSpec()) == 13
+
+
 def test_limit_must_be_a_number(require_gpu, monkeypatch):
     monkeypatch.setenv("SCORE_GM_MEM_LIMIT", "some")
     with pytest.raises(abi.ScoreGmError) as e:
@@ -73,20 +164,10 @@ def test_all_memory_is_given_back(require_gpu, monkeypatch):
     with GrowthMachine(dom) as g:
         g.solve_rxgrowth()
         g.grainmap(), g.counts(), g.front(abi.LIST_INSIDE)
-    lo, hi = 1 << 10, 1 << 30
-    # the least limit under which the run ends; it would creep up with bytes that stay counted
-    need = []
-    for _ in range(2):
-        a, b = lo, hi
-        while b - a > 4096:
-            m = (a + b) // 2
-            monkeypatch.setenv("SCORE_GM_MEM_LIMIT", str(m))
-            try:
-                with GrowthMachine(dom) as g:
-                    g.solve_rxgrowth()
-                b = m
-            except abi.ScoreGmError as e:
-                assert e.code == abi.ERR_OOM
-                a = m
-        need.append(b)
-    assert need[0] == need[1] < hi
+
+    def run():
+        with GrowthMachine(dom) as g:
+            g.solve_rxgrowth()
+
+    # it would creep up with bytes that stay counted
+    assert _least_limit(monkeypatch, run) == _least_limit(monkeypatch, run) < 1 << 30

@@ -10,7 +10,7 @@ import pytest
 
 from oracle.oracle import Oracle
 from score_amd import abi, synth
-from score_amd.growth import GrowthMachine
+from score_amd.growth import GrowthMachine, same_trajectory
 from score_amd.synth import ParamsSpec
 
 pytestmark = pytest.mark.gpu
@@ -44,8 +44,8 @@ def test_step_beyond_the_log(require_gpu, first):
             g.step(1000)
         assert err.value.code == abi.ERR_CAPACITY
         assert np.array_equal(g.counts()[0], defg) and np.array_equal(g.counts()[1], rxg)
-        if first == LAST:
-            assert np.array_equal(g.grainmap(), o.grainmap())
+        assert np.array_equal(g.grainmap(), o.grainmap())
+        assert same_trajectory(o.trajectory(), g.trajectory())
         with pytest.raises(abi.ScoreGmError):
             g.step(1)
     o.step(1)
