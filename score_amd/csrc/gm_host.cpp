@@ -2426,48 +2426,49 @@ int score_gm_get_status_noalloc(score_gm_handle *h, double rxthreshold, uint32_t
 
 namespace {
 
-/* one domain of a batch, create to destroy; a domain that does not fit into
- * device memory retries each time another one finishes */
+/* The domains of a batch or server that hold device memory.  One that meets the end of
+ * it (its lists grow while it runs) gives all of its own back and runs again: when
+ * another one is done, or when none holds memory any more.  Only a domain that had the
+ * memory to itself from its start to its end does not fit.  Several may fail at once,
+ * each for what the others held, so that none waits is no sign of that. */
 struct BatchGate {
     std::mutex m;
     std::condition_variable cv;
-    uint32_t inflight = 0; /* domains taken, including those waiting for memory */
-    uint32_t waiting = 0;
-    uint64_t finished = 0;
+    uint32_t holding = 0;  /* domains between their creation and their end */
+    uint64_t started = 0;
+    uint64_t finished = 0; /* of those, the ones that are done */
 };
 
-int batch_one(score_gm_batch_item &it, int32_t device, BatchGate &gate) {
+/* one domain, create to destroy */
+int batch_attempt(score_gm_batch_item &it, int32_t device) {
     score_gm_handle *h = nullptr;
-    int rc;
-    for (;;) {
-        uint64_t seen;
-        {
-            std::lock_guard<std::mutex> lk(gate.m);
-            seen = gate.finished;
-        }
-        rc = score_gm_create(it.domain, it.params, device, &h);
-        if (rc == SCORE_GM_OK) {
-            /* the front list may ask for more memory while the domain grows */
-            rc = score_gm_run(h, &it.result);
-            if (rc != SCORE_GM_ERR_OOM) break;
-            score_gm_destroy(h);
-            h = nullptr;
-            memset(&it.result, 0, sizeof(it.result));
-        }
-        if (rc != SCORE_GM_ERR_OOM) break;
-        /* wait for a running domain to give its memory back; with none running
-         * besides the waiting ones, it does not fit */
-        std::unique_lock<std::mutex> lk(gate.m);
-        if (gate.finished == seen && gate.inflight - gate.waiting <= 1) break;
-        gate.waiting++;
-        gate.cv.wait(lk, [&] { return gate.finished != seen; });
-        gate.waiting--;
-    }
-    if (!h) return rc;
+    memset(&it.result, 0, sizeof(it.result));
+    int rc = score_gm_create(it.domain, it.params, device, &h);
+    if (rc) return rc;
+    rc = score_gm_run(h, &it.result);
     if (!rc && (it.defg_counts || it.rxg_counts)) rc = score_gm_get_counts(h, it.defg_counts, it.rxg_counts);
     if (!rc && it.grainmap) rc = score_gm_get_grainmap(h, it.grainmap, it.map_encoding);
     score_gm_destroy(h);
     return rc;
+}
+
+int batch_one(score_gm_batch_item &it, int32_t device, BatchGate &gate) {
+    std::unique_lock<std::mutex> lk(gate.m);
+    for (;;) {
+        const bool first = ++gate.holding == 1;
+        const uint64_t mine = ++gate.started;
+        lk.unlock();
+        const int rc = batch_attempt(it, device);
+        lk.lock();
+        gate.holding--;
+        const bool alone = first && gate.started == mine;
+        const bool again = rc == SCORE_GM_ERR_OOM && !alone;
+        if (!again) gate.finished++;
+        gate.cv.notify_all();
+        if (!again) return rc;
+        const uint64_t seen = gate.finished;
+        gate.cv.wait(lk, [&] { return gate.finished != seen || gate.holding == 0; });
+    }
 }
 
 }  // namespace
@@ -2488,20 +2489,10 @@ int score_gm_batch_run(score_gm_batch_item *items, uint32_t n, int32_t device, u
         for (;;) {
             const uint32_t i = next.fetch_add(1);
             if (i >= n) return;
-            {
-                std::lock_guard<std::mutex> lk(gate.m);
-                gate.inflight++;
-            }
             const auto t0 = std::chrono::steady_clock::now();
             items[i].queued_seconds = std::chrono::duration<double>(t0 - tcall).count();
             items[i].status = batch_one(items[i], device, gate);
             items[i].seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-            {
-                std::lock_guard<std::mutex> lk(gate.m);
-                gate.inflight--;
-                gate.finished++;
-            }
-            gate.cv.notify_all();
         }
     };
     std::vector<std::thread> pool;
@@ -2610,18 +2601,8 @@ struct score_gm_server {
             }
             const auto t0 = std::chrono::steady_clock::now();
             r.item->queued_seconds = std::chrono::duration<double>(t0 - r.submitted).count();
-            {
-                std::lock_guard<std::mutex> lk(gate.m);
-                gate.inflight++;
-            }
             r.item->status = batch_one(*r.item, device, gate);
             r.item->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-            {
-                std::lock_guard<std::mutex> lk(gate.m);
-                gate.inflight--;
-                gate.finished++;
-            }
-            gate.cv.notify_all();
             {
                 std::lock_guard<std::mutex> lk(m);
                 running--;
