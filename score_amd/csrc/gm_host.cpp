@@ -1013,19 +1013,21 @@ int grow_parents(score_gm_handle *h, uint32_t need) {
 
 /* The Inside list grows by doubling, as SCORE's does, to at least `need` slots: it
  * lies behind the Border list, so no slot changes its number.  New slots are
- * INACTIVE.  Where both copies would hold more than a slot per cell the old one
- * waits in host memory, so that a domain never needs more device memory than lists
- * of full length (score_gm_footprint). */
+ * INACTIVE.  A domain never needs more device memory than lists of full length
+ * (score_gm_footprint): the longer list takes no more than the old one leaves of that,
+ * and where that is too little the old one waits in host memory. */
 int grow_front(score_gm_handle *h, uint32_t need) {
     GmDev &d = h->d;
     uint64_t nc = (std::max<uint64_t>(need, 2ull * d.capI) + 63) / 64 * 64;
-    const bool staged = nc + d.capI > d.capImax;
+    /* (both copies hold the Border list) */
+    const uint64_t beside = (uint64_t)d.capI + d.baseI + GM_SW_CHUNK, room = d.capImax > beside ? d.capImax - beside : 0u;
+    if (nc > room && room / 64 * 64 >= need) nc = room / 64 * 64;
+    const bool staged = nc > room;
     if (staged) nc = d.capImax;
     const size_t used = (size_t)d.baseI + d.capI;
     /* the lists in new arrays of n Inside slots, copied from rec and cs */
     auto place = [&](uint64_t n, const GmRec *rec, const gm_cs_t *cs) -> int {
         const size_t tot = (size_t)d.baseI + n + GM_SW_CHUNK;
-        const hipMemcpyKind kind = staged ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
         GmRec *nrec = nullptr;
         gm_cs_t *ncs = nullptr;
         int rc;
@@ -1034,9 +1036,13 @@ int grow_front(score_gm_handle *h, uint32_t need) {
             return rc;
         }
         hipError_t e = gm_launch_fill_u32((uint32_t *)ncs, 0xFFFFFFFFu, tot / 2, h->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(nrec, rec, sizeof(GmRec) * used, kind, h->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(ncs, cs, sizeof(gm_cs_t) * used, kind, h->stream);
-        if (e == hipSuccess && staged) e = hipStreamSynchronize(h->stream);
+        if (staged) {
+            if (e == hipSuccess) e = copy_staged(h, nrec, const_cast<GmRec *>(rec), sizeof(GmRec) * used, false);
+            if (e == hipSuccess) e = copy_staged(h, ncs, const_cast<gm_cs_t *>(cs), sizeof(gm_cs_t) * used, false);
+        } else {
+            if (e == hipSuccess) e = hipMemcpyAsync(nrec, rec, sizeof(GmRec) * used, hipMemcpyDeviceToDevice, h->stream);
+            if (e == hipSuccess) e = hipMemcpyAsync(ncs, cs, sizeof(gm_cs_t) * used, hipMemcpyDeviceToDevice, h->stream);
+        }
         if (e != hipSuccess) {
             dfree(h, nrec);
             dfree(h, ncs);
@@ -1061,9 +1067,8 @@ int grow_front(score_gm_handle *h, uint32_t need) {
     GmRec *const krec = reinterpret_cast<GmRec *>(keep);
     gm_cs_t *const kcs = reinterpret_cast<gm_cs_t *>(keep + sizeof(GmRec) * used);
     hipError_t e;
-    if ((e = hipMemcpyAsync(krec, rec, sizeof(GmRec) * used, hipMemcpyDeviceToHost, h->stream)) != hipSuccess ||
-        (e = hipMemcpyAsync(kcs, cs, sizeof(gm_cs_t) * used, hipMemcpyDeviceToHost, h->stream)) != hipSuccess ||
-        (e = hipStreamSynchronize(h->stream)) != hipSuccess) {
+    if ((e = copy_staged(h, rec, krec, sizeof(GmRec) * used, true)) != hipSuccess ||
+        (e = copy_staged(h, cs, kcs, sizeof(gm_cs_t) * used, true)) != hipSuccess) {
         free(keep);
         return hip_fail(e, "growing the Inside list");
     }
@@ -1914,10 +1919,16 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
         /* several regions: per-region lists (build_regions); the one-region sizes stay 0 */
         build_regions(h, (uint32_t)prm->n_regions);
     } else {
-        /* SCORE starts with a cache of rel_cell_caching*N cells and doubles it (0.2 in
-         * its decks; of the measured domains the front never took more than 0.4);
-         * small domains get every cell's slot */
-        const double frac = std::min(1.0, std::max(0.125, prm->rel_cell_caching));
+        /* SCORE starts with a cache of rel_cell_caching*N cells (0.2 in its decks) and
+         * doubles it.  The list grows here too, but a growth costs more than the slots: its
+         * longest over a run goes with the cube root of the nuclei per cell, d (nuclei at
+         * random, 100^3 and 200^3: 1.8 to 2.4 d^(1/3) of the cells with many deformed grains,
+         * d from 7.5e-4 on, 2.7 to 3.1 with one; below, at most 0.2), so that much is there
+         * from the start.  256^3 at d = 3e-2 took 203 ms in a list that started with 0.2 N
+         * and had to grow by way of host memory, 21 so (the
+         * whole call 230 and 50).  Small domains get every cell's slot. */
+        const double dense = 3.2 * cbrt((double)d.nrxg / (double)d.N);
+        const double frac = std::min(1.0, std::max({0.125, prm->rel_cell_caching, dense}));
         uint64_t slots = std::max<uint64_t>((uint64_t)(frac * (double)d.N) + 1, std::max<uint64_t>(kMinFrontSlots, d.nrxg));
         if (const char *ev = getenv("SCORE_GM_FRONT_SLOTS")) { /* tests make the list grow with it */
             char *end = nullptr;
@@ -2273,10 +2284,15 @@ int score_gm_get_grainmap(score_gm_handle *h, uint32_t *out, int32_t encoding) {
         return fail(SCORE_GM_ERR_ARG, "unknown encoding");
     if (front_lost(h)) return h->err;
     HIPCHK(hipSetDevice(h->device));
-    /* the grid with the front's cells marked infected, assembled in a device buffer */
-    uint32_t *tmp = nullptr;
-    int rc = dalloc(h, &tmp, h->d.N);
-    if (rc) return rc;
+    /* the grid with the front's cells marked infected, assembled where the Inside list's
+     * records end, which nothing reads before they are written, or in a buffer of its own
+     * (whose fresh memory takes 4 of 9 ms at 320^3) */
+    const GmDev &d = h->d;
+    uint32_t *own = nullptr, *tmp = reinterpret_cast<uint32_t *>(d.rec + d.baseI + h->nI);
+    int rc = 0;
+    if ((d.nreg > 1 || (uint64_t)(d.capI - h->nI) * sizeof(GmRec) < sizeof(uint32_t) * d.N) && (rc = dalloc(h, &own, d.N)))
+        return rc;
+    if (own) tmp = own;
     auto copy = [&]() -> int {
         HIPCHK(gm_launch_overlay_infected(h->d, h->nI, h->nB, h->step, tmp, h->stream));
         if (encoding == SCORE_GM_MAP_RAW2GID) HIPCHK(gm_launch_raw2gid(tmp, h->d.N, h->stream));
@@ -2284,7 +2300,7 @@ int score_gm_get_grainmap(score_gm_handle *h, uint32_t *out, int32_t encoding) {
         return 0;
     };
     rc = copy();
-    dfree(h, tmp);
+    dfree(h, own);
     return rc;
 }
 
