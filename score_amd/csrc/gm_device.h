@@ -11,6 +11,7 @@
 
 #include "gm_internal.h"
 #include "gm_radd.h"
+#include "gm_weight.h"
 
 #define GM_RH 2
 #define GM_RHO_RX (1.0e11)
@@ -93,30 +94,6 @@ static __device__ __forceinline__ uint32_t hash_slot(unsigned long long k, uint3
     k *= 0xc4ceb9fe1a85ec53ull;
     k ^= k >> 33;
     return (uint32_t)k & (cap - 1u);
-}
-
-/* largest |component| over the six Grimmer candidates of q_def^-1 * q_rx
- * (SCORE_Math.cpp:230-239, :558-608); only + - * fabs and compares, so the
- * value is bit-identical to the host's.  The 24 candidates are the sums and
- * differences of two components times 1/sqrt(2), of all four (left to right) times
- * 1/2, and the components.  Rounding is monotone and symmetric, so no sign pattern
- * exceeds the one that adds the magnitudes, and among the pairs the two largest
- * magnitudes win: three candidates remain (24 kept 48 registers alive, which held
- * the commit pass at 12 waves a CU). */
-static __device__ __forceinline__ double grimmer_omega(const double *p, const double *q, double fac) {
-    double m0 = q[0], m1 = -1.0 * q[1], m2 = -1.0 * q[2], m3 = -1.0 * q[3];
-    const double a = fabs(m0 * p[0] - m1 * p[1] - m2 * p[2] - m3 * p[3]);
-    const double b = fabs(p[0] * m1 + m0 * p[1] + (m2 * p[3] - m3 * p[2]));
-    const double c = fabs(p[0] * m2 + m0 * p[2] + (-(m1 * p[3]) + m3 * p[1]));
-    const double d = fabs(p[0] * m3 + m0 * p[3] + (m1 * p[2] - m2 * p[1]));
-    const double ab = a > b ? a : b, ba = a > b ? b : a, cd = c > d ? c : d, dc = c > d ? d : c;
-    const double l1 = ab > cd ? ab : cd;
-    const double lo = ab > cd ? cd : ab, in = ab > cd ? ba : dc;
-    const double l2 = lo > in ? lo : in;
-    const double two = (l1 + l2) * fac, four = (((a + b) + c) + d) * 0.5;
-    double omega = l1 > two ? l1 : two;
-    if (four > omega) omega = four;
-    return omega;
 }
 
 /* Mobility weight of (nucleus rxg, deformed grain g).  Rollett-Holm pairs whose

@@ -30,14 +30,13 @@
 
 #include "../../include/score_gm.h"
 #include "gm_internal.h"
+#include "gm_weight.h"
 #include "score_orient.h"
 
 namespace {
 
 /* constants (SCORE_Defs_Physics.h:51-160, SCORE_Math.h:61) */
 const double kBoltzmann = 1.3806488e-23;
-const double kPi = 3.1415926535897932384626433832795;
-const double kLagbHagb = ((15.0) / (180.0) * (kPi));
 const double kMaxDev40_111 = ((10.0) / (180.0) * (kPi));
 const double kInitialDeltaT = 1e-6;
 const double kInfinite = 1e36;
@@ -85,10 +84,6 @@ int hip_fail(hipError_t e, const char *where) {
 using score_orient::disori_angle;
 using score_orient::disori_quat;
 
-double rh_weight_of_theta(const score_gm_params &p, double theta) {
-    return 1.0 - (p.rh_cut * exp(-1.0 * p.rh_trans * pow((theta / kLagbHagb), p.rh_exponent)));
-}
-
 /* calc_mobilityweight_rollettholm / _sebaldgottstein (SCORE_GrainBoundaryPhysics.cpp:50-135),
  * identical arithmetic to reg_calc_mobilityweight (SCORE_Kernel.cpp:2460-2527) */
 double mobility_weight(const score_gm_params &p, const double *qrx, const double *qdef) {
@@ -108,42 +103,6 @@ double mobility_weight(const score_gm_params &p, const double *qrx, const double
         w = cc * cc;
     }
     return w;
-}
-
-/* Largest omega for which the Rollett-Holm weight is exactly 1.0 with margin:
- * the device returns P = 1.0 for omega <= this value and asks the host otherwise.
- * Returns -1 when no safe threshold exists (shortcut disabled). */
-double rh_omega_threshold(const score_gm_params &p) {
-    if (p.mobility_model != SCORE_GM_MOB_ROLLETTHOLM) return -1.0;
-    if (!(p.rh_cut > 0.0 && p.rh_trans > 0.0 && p.rh_exponent > 0.0)) return -1.0;
-    if (rh_weight_of_theta(p, kPi) != 1.0) return -1.0;
-    double lo = 0.0, hi = kPi; /* invariant: weight(hi) == 1.0 */
-    if (rh_weight_of_theta(p, lo) == 1.0) return 1.0; /* every pair has P == 1.0 */
-    for (int it = 0; it < 200; it++) {
-        double mid = 0.5 * (lo + hi);
-        if (rh_weight_of_theta(p, mid) == 1.0) hi = mid;
-        else lo = mid;
-    }
-    /* margin of 0.2 degree: the weight's deficit falls by a large factor over it */
-    const double theta_hi = hi + 0.2 / 180.0 * kPi;
-    if (theta_hi >= 2.0 * acos(0.85)) return -1.0; /* beyond the largest cubic disorientation */
-    /* The weight is 1.0 - x with x = cut * exp(-trans * (theta / 15 deg)^n), which falls
-     * with theta, and rounds to 1.0 once x <= 2^-54.  The computed x is off by at most
-     * a factor 1 + arg * (n + 4) * 2^-52 (arg = trans * (theta / 15 deg)^n), which the
-     * margin of 2 below covers at theta_hi and, since x falls faster than arg grows,
-     * at every larger angle, while n and arg are moderate.  Other settings are checked
-     * at 200,001 angles (7 of the 8 ms a handle took to create). */
-    const double arg = p.rh_trans * pow((theta_hi / kLagbHagb), p.rh_exponent);
-    const bool sure = p.rh_exponent <= 1000.0 && arg >= 2.0 && arg <= 700.0 && p.rh_cut * exp(-1.0 * arg) <= 0x1p-55;
-    for (int i = 0; !sure && i <= 200000; i++) {
-        double th = theta_hi + (kPi - theta_hi) * (double)i / 200000.0;
-        if (rh_weight_of_theta(p, th) != 1.0) return -1.0;
-    }
-    double om = cos(0.5 * theta_hi);
-    /* a few ulps below, so that 2*acos(om') >= theta_hi whatever the last-bit behaviour of acos */
-    for (int i = 0; i < 4; i++) om = nextafter(om, 0.0);
-    if (!(2.0 * acos(om) >= theta_hi)) return -1.0;
-    return om;
 }
 
 }  // namespace
