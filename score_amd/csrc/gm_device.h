@@ -58,13 +58,9 @@ static __device__ __forceinline__ uint32_t lanemask_lt_count(uint64_t m) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-/* lane j's value of v (j uniform); unsigned, so the 64-bit form does not
- * sign-extend the low word */
+/* lane j's value of v (j uniform) */
 static __device__ __forceinline__ uint32_t rdlane(uint32_t v, uint32_t j) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)j);
-}
-static __device__ __forceinline__ uint64_t rdlane64(uint64_t v, uint32_t j) {
-    return ((uint64_t)rdlane((uint32_t)(v >> 32), j) << 32) | (uint64_t)rdlane((uint32_t)v, j);
 }
 
 /* a word that other blocks of the same launch change, by atomics */
@@ -232,7 +228,7 @@ static __device__ __forceinline__ uint32_t predict_values(const GmSweepArgs &A, 
     if (cell_increment(A.sp, P, rho, inf, inc)) {
         if (k <= A.stepcap && A.next_only) {
             /* the step's one addition; a cell it leaves below 1.0 is re-anchored
-             * and predicted again before the next step (GM_STEP_FAR_NEXT) */
+             * and predicted again before the next step */
             cs = f + inc >= 1.0 ? k : GM_STEP_NEXT;
         } else if (k <= A.stepcap) {
             const uint64_t j = gm_radd_count_to_one(f, inc, (uint64_t)(A.stepcap - k) + 1u);

@@ -1421,7 +1421,8 @@ bool wait_steps(score_gm_handle *h, uint32_t need) {
 }
 
 /* Waits until the window's stats are in the host's mirror: the word the device sets
- * after them (copy_stats), or, after a second without it, whatever the stream says. */
+ * after them (copy_stats), or, after a second without it, whatever the stream says.  One
+ * core is busy meanwhile; the stream's own wait returns 8 us later. */
 hipError_t wait_window(score_gm_handle *h) {
     const auto t0 = std::chrono::steady_clock::now();
     for (uint32_t it = 1; !__atomic_load_n(h->hprog + 1, __ATOMIC_ACQUIRE); it++) {

@@ -356,7 +356,8 @@ hipError_t gm_launch_reanchor(const GmDev &d, const GmSweepArgs &a, hipStream_t 
  * the last grain's sum until another one follows, since atomics on one address are
  * served one after another: a grain met in a long run of words costs few of them
  * (one grain in all: one per block).  The host's two loops over the grid that this
- * replaces took 123 ms at 512^3, the bitmap alone 0.58; the pass takes 0.26 (2 TB/s). */
+ * replaces took 123 ms at 512^3; the pass takes 0.88, and moves 3.3 GB where the ids,
+ * the pairs and the bitmap are 1.6. */
 __global__ void __launch_bounds__(GM_BLOCK) k_grid_init(GmDev d, const uint32_t *src, uint32_t nwords) {
     __shared__ uint32_t sid[GM_BLOCK / 64], scnt[GM_BLOCK / 64];
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
@@ -1084,11 +1085,7 @@ __global__ void __launch_bounds__(GM_BLOCK) k_decide(GmDev d, GmPart P, uint32_t
         const uint32_t rp = valid ? d.rpos[q0.z] : 0xFFFFFFFFu;
         W.mI[lane] = 0;
         W.mB[lane] = 0;
-        const uint32_t na = (uint32_t)__popc(am), incl = wave_incl_scan(na);
-        const uint32_t n = __shfl(incl, 63, 64);
-        uint32_t pos = incl - na;
-        for (uint32_t m = am; m; m &= m - 1u) W.wl[pos++] = (uint16_t)(lane | ((uint32_t)__ffs(m) - 1u) << 8);
-        wave_sync();
+        const uint32_t n = list_attempts(am, W.wl);
         for (uint32_t i = lane; i < n; i += 64u) {
             const uint32_t e = W.wl[i], q = e & 0xFFu, rk = e >> 8;
             const uint2 v = W.xyz[q];
@@ -1965,9 +1962,10 @@ __global__ void __launch_bounds__(1024) k_arrivals(GmDev d, GmSweepArgs A) {
 }
 
 /* ----------------------------------------------------------- launch windows
- * Up to GM_WMAX steps are launched back to back.  Every kernel of a step reads
- * the step index and list lengths from the stats and returns at once once a
- * step has set `halt`, so that the host takes over at the step after it. */
+ * Up to GM_WMAX steps are launched back to back.  Every kernel of a step takes the
+ * lists' lengths before it from the device (GmWin; with several regions the step's
+ * index too, from the stats) and returns at once once a step has set `halt`, so that
+ * the host takes over at the step after it. */
 
 __global__ void __launch_bounds__(64) k_window_begin(GmDev d, uint32_t k, double xcells, uint32_t top_pos) {
     GmStats *st = d.st;

@@ -36,8 +36,8 @@
  * count is the offset of the region's first block.
  *
  * At 160^3 in eight regions (477 steps of 8500 parents) a step of these passes went
- * from 135 to 63 us: compaction and propose pass 30 to 11, decide with the retirement and the recycled
- * slots 28 to 9.5, commit with the step's end 29 to 17, the two scans 27 to 14.5.
+ * from 135 to 62 us: compaction and propose pass 30 to 13, decide with the retirement and the recycled
+ * slots 28 to 8.5, commit with the step's end 29 to 17, the two scans 27 to 13.4.
  *
  * Per step, in the profiling slots of the one-region kernels:
  *   k_reanchor (shared)   k_rg_sweep   k_rg_sweep_scan (+ per-list starts)
