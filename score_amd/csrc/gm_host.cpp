@@ -131,6 +131,7 @@ struct score_gm_handle {
     double Pmax = kDefaultPmax, regPmax = kDefaultPmax;
     uint32_t step = 0;
     uint32_t nI = 0, nB = 0;
+    uint32_t nI_most = 0; /* the most Inside slots in use after any step */
     uint32_t nuclei = 0;
     int completed = 0;
     int err = 0;
@@ -1663,6 +1664,7 @@ int step_window(score_gm_handle *h, uint32_t wmax, uint32_t *nsteps) {
         const GmStepRow &last = st.rows[nexec - 1];
         h->nI = last.nI;
         h->nB = last.nB;
+        h->nI_most = std::max(h->nI_most, h->nI);
         h->last_csz = gm_chunk_size(last.nfullI + last.nfullB, last.winI + last.winB);
         h->last_full = 0;
         for (uint32_t j = 0; j < nexec; j++) h->last_full = std::max(h->last_full, st.rows[j].nfullI + st.rows[j].nfullB);
@@ -2147,6 +2149,7 @@ static int create_handle(const score_gm_domain *dom, const score_gm_params *prm,
     }
     h->nI = h->hst->nI;
     h->nB = h->hst->nB;
+    h->nI_most = h->nI;
 
     /* solve_RXGROWTH prologue (SCORE_Kernel.cpp:6501-6530): scalars and the first dt */
     h->rho_host.assign(dom->defg_rho, dom->defg_rho + d.ndefg);
@@ -2244,13 +2247,15 @@ int score_gm_get_grainmap(score_gm_handle *h, uint32_t *out, int32_t encoding) {
         return fail(SCORE_GM_ERR_ARG, "unknown encoding");
     if (front_lost(h)) return h->err;
     HIPCHK(hipSetDevice(h->device));
-    /* the grid with the front's cells marked infected, assembled where the Inside list's
-     * records end, which nothing reads before they are written, or in a buffer of its own
-     * (whose fresh memory takes 4 of 9 ms at 320^3) */
+    /* the grid with the front's cells marked infected, assembled in the Inside list's records
+     * beyond any it ever held (a defragmentation leaves records behind the list's end that a
+     * later one may take back), which nothing reads before they are written, or in a buffer
+     * of its own (whose fresh memory takes 4 of 9 ms at 320^3) */
     const GmDev &d = h->d;
-    uint32_t *own = nullptr, *tmp = reinterpret_cast<uint32_t *>(d.rec + d.baseI + h->nI);
+    uint32_t *own = nullptr, *tmp = reinterpret_cast<uint32_t *>(d.rec + d.baseI + h->nI_most);
     int rc = 0;
-    if ((d.nreg > 1 || (uint64_t)(d.capI - h->nI) * sizeof(GmRec) < sizeof(uint32_t) * d.N) && (rc = dalloc(h, &own, d.N)))
+    if ((d.nreg > 1 || (uint64_t)(d.capI - h->nI_most) * sizeof(GmRec) < sizeof(uint32_t) * d.N) &&
+        (rc = dalloc(h, &own, d.N)))
         return rc;
     if (own) tmp = own;
     auto copy = [&]() -> int {

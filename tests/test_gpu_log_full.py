@@ -2,7 +2,7 @@
 block of its propose pass alike: the error comes back and the state is the one before
 the step.  Cells retire twice where a defragmentation follows another with no
 completions between (the reference's search revives the records left behind); here
-12,000 records of slow cells are, and the last class of cells completes in one step."""
+19,152 records of slow cells are, and the last class of cells completes in one step."""
 from __future__ import annotations
 
 import numpy as np
