@@ -11,13 +11,13 @@
  *                      to the retirement log
  *   rlog   (cell, ndefg+rxg) per retired cell in retirement order, written
  *                      coalesced with the step's parent data; the exported map
- *                      is the grid with the log applied and the front's cells
- *                      marked INFECTED
+ *                      is the grid with the front's cells marked INFECTED and then
+ *                      the log applied
  *   dmap   1 bit per cell, set while the cell is deformed (infectable), blocked so
  *          that one 128-byte line holds a 16x8x8 brick of cells: a 3x3x3
  *          neighbourhood usually lies in one or two lines
  *   front  Border list slots [0,capB), then from baseI on the Inside list's, which
- *          starts with SCORE's initial cache of cells and grows
+ *          starts with what the nuclei's density asks for and grows
  *          cstep uint16[slots]   completion step (mod GM_CS_MOD) or a GM_CS_*
  *                                sentinel; the only array every step reads in full
  *          rec   GmRec[slots]    64-byte record, read and written only when a cell
@@ -500,9 +500,8 @@ hipError_t gm_launch_defrag_move(const GmDev &d, uint32_t base, uint32_t first, 
  * ixyz and gid hold nI+nB entries. */
 hipError_t gm_launch_status(const GmDev &d, uint32_t nI, uint32_t nB, uint32_t k, double thr, uint32_t *ixyz,
                             uint32_t *gid, hipStream_t s);
-/* the cell grid as SCORE holds it into `out`: every retired
- * cell set to ndefg+rxg from the log, every cell held by an active front record
- * marked INFECTED */
+/* the cell grid as SCORE holds it into `out`: every cell held by an active front record
+ * marked INFECTED, but every retired cell set to ndefg+rxg from the log */
 hipError_t gm_launch_overlay_infected(const GmDev &d, uint32_t nI, uint32_t nB, uint32_t k, uint32_t *out,
                                       hipStream_t s);
 /* that map in SCORE's raw file encoding, in place */

@@ -1371,8 +1371,8 @@ __global__ void k_grid_out(GmDev d, uint32_t *out) {
     if ((d.N & 1u) && blockIdx.x == 0 && threadIdx.x == 0) out[d.N - 1u] = d.cell[d.N - 1u].y;
 }
 
-/* exported map: retired cells from the log, in retirement order (a cell retired
- * twice keeps the later entry, as SCORE's grid keeps its last write) */
+/* exported map: retired cells from the log (a cell retired twice is its nucleus' both
+ * times) */
 __global__ void k_apply_rlog(GmDev d, uint32_t *out) {
     const unsigned long long n = d.st->nret < d.rlogCap ? d.st->nret : d.rlogCap;
     for (unsigned long long i = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -1394,9 +1394,10 @@ __global__ void k_overlay_infected(GmDev d, uint32_t nI, uint32_t nB, uint32_t k
 hipError_t gm_launch_overlay_infected(const GmDev &d, uint32_t nI, uint32_t nB, uint32_t k, uint32_t *out,
                                       hipStream_t s) {
     k_grid_out<<<fill_blocks((d.N + 1u) / 2u), GM_BLOCK, 0, s>>>(d, out);
+    /* a cell is infected once, and retired after that: where another record still holds it
+     * (a defragmentation took it back) SCORE's grid has the retirement */
+    if (nI + nB) k_overlay_infected<<<fill_blocks(nI + nB), GM_BLOCK, 0, s>>>(d, nI, nB, k, out);
     k_apply_rlog<<<8192, GM_BLOCK, 0, s>>>(d, out);
-    if (nI + nB == 0) return hipGetLastError();
-    k_overlay_infected<<<fill_blocks(nI + nB), GM_BLOCK, 0, s>>>(d, nI, nB, k, out);
     return hipGetLastError();
 }
 

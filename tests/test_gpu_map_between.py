@@ -65,3 +65,19 @@ def test_maps_between_windows(require_gpu, monkeypatch, slots):
             g.step(4)
             assert np.array_equal(o.grainmap(), g.grainmap())
         assert same_trajectory(o.trajectory(), g.trajectory())
+
+
+def test_retired_cells_with_another_record(require_gpu):
+    """A cell that is held twice and has retired once is its grain's in the map."""
+    dom = synth.make_voronoi_domain(20, 28, 22, n_grains=1, n_nuclei=65, seed=38)
+    prm = ParamsSpec(maxfill=0.045, xmax=0.7, defrag_at=(900.0, 1650.0, 5350.0, 5900.0, 6050.0, 8150.0, 8950.0))
+    o = Oracle(dom, prm)
+    o.solve_rxgrowth()
+    fo = [o.front(lst) for lst in (abi.LIST_INSIDE, abi.LIST_BORDER)]
+    held = np.concatenate([f["cell"][f["activity"] != 0] for f in fo])
+    m = o.grainmap()
+    assert (m[held] != abi.CURRENTLY_INFECTED).sum() > 100
+    with GrowthMachine(dom, prm) as g:
+        g.solve_rxgrowth()
+        assert same_trajectory(o.trajectory(), g.trajectory())
+        assert np.array_equal(m, g.grainmap())
